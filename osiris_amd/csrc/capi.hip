@@ -180,7 +180,7 @@ struct osr_sim {
   DBuf E, B, J, ctrl, fe_part, hist;
   int64_t hist_cap = 0;
   std::vector<std::unique_ptr<Species>> sp;
-  DBuf d_spec, d_work, d_fd, d_ywork, d_ework, d_fwork;
+  DBuf d_spec, d_work, d_fd, d_ywork, d_ework, d_dwork, d_fwork;
   FieldDesc fd{};
   hipStream_t stream = nullptr;
   hipGraphExec_t gexec = nullptr;    // one step
@@ -972,6 +972,8 @@ int launch_yee(osr_sim* s) {
   const FieldDesc* fd = s->d_fd.as<FieldDesc>();
   const int2* w = s->d_ywork.as<int2>();
   const int2* we = s->d_ework.as<int2>();
+  const int2* wd = s->d_dwork.as<int2>();  // the history columns, then the cell blocks
+  const unsigned nd = (unsigned)(kRedCols + s->nblk);
   if (s->vp_n) {  // advance_yee with VPML x walls: update_boundary_bfld step 1 advances
                    // the wall E, update_boundary_efld the wall B (os-emf-boundary.f90:930-935,
                    // 1036-1041)
@@ -981,13 +983,13 @@ int launch_yee(osr_sim* s) {
       if (s->desc.vpml_diffuse[0] || s->desc.vpml_diffuse[1])
         hipLaunchKernelGGL(vpml_diffuse, dim3(nb), dim3(256), 0, s->stream, fd);
       hipLaunchKernelGGL((vpml_update<0, 2>), dim3(nb), dim3(256), 0, s->stream, fd);
-      hipLaunchKernelGGL((yee_dedt<2>), dim3(s->nblk), dim3(256), 0, s->stream, fd, w);
+      hipLaunchKernelGGL((yee_dedt<2>), dim3(nd), dim3(256), 0, s->stream, fd, wd);
       hipLaunchKernelGGL((vpml_update<1, 2>), dim3(nb), dim3(256), 0, s->stream, fd);
       hipLaunchKernelGGL((yee_dbdt<2, false>), dim3(s->nblk), dim3(256), 0, s->stream, fd, w);
     } else {
       hipLaunchKernelGGL((yee_dbdt<3, true>), dim3(s->nblk_e), dim3(256), 0, s->stream, fd, we);
       hipLaunchKernelGGL((vpml_update<0, 3>), dim3(nb), dim3(256), 0, s->stream, fd);
-      hipLaunchKernelGGL((yee_dedt<3>), dim3(s->nblk), dim3(256), 0, s->stream, fd, w);
+      hipLaunchKernelGGL((yee_dedt<3>), dim3(nd), dim3(256), 0, s->stream, fd, wd);
       hipLaunchKernelGGL((vpml_update<1, 3>), dim3(nb), dim3(256), 0, s->stream, fd);
       hipLaunchKernelGGL((yee_dbdt<3, false>), dim3(s->nblk), dim3(256), 0, s->stream, fd, w);
     }
@@ -996,20 +998,19 @@ int launch_yee(osr_sim* s) {
   }
   if (s->g.open_nx) {  // advance_yee with Lindman x walls (os-emf-solver-yee.f03:542-568)
     const unsigned nb = (unsigned)ceil_div(s->g.ny * s->g.nz, 256);
-    const unsigned nbf = (unsigned)ceil_div(s->g.ny * s->g.nz, kFinNT);
     // the work list of the first B half step carries the wall's first B update
     if (s->dims == 2) {
       hipLaunchKernelGGL((yee_dbdt<2, true>), dim3(s->nwork_e), dim3(256), 0, s->stream, fd, we);
-      hipLaunchKernelGGL((yee_dedt<2>), dim3(s->nblk), dim3(256), 0, s->stream, fd, w);
+      hipLaunchKernelGGL((yee_dedt<2>), dim3(nd), dim3(256), 0, s->stream, fd, wd);
       hipLaunchKernelGGL(wall_e, dim3(nb), dim3(256), 0, s->stream, fd);
       hipLaunchKernelGGL((yee_dbdt<2, false>), dim3(s->nblk), dim3(256), 0, s->stream, fd, w);
-      hipLaunchKernelGGL((wall_b2_end<2>), dim3(nbf), dim3(kFinNT), 0, s->stream, fd);
+      hipLaunchKernelGGL((wall_b2_end<2>), dim3(nb), dim3(256), 0, s->stream, fd);
     } else {
       hipLaunchKernelGGL((yee_dbdt<3, true>), dim3(s->nwork_e), dim3(256), 0, s->stream, fd, we);
-      hipLaunchKernelGGL((yee_dedt<3>), dim3(s->nblk), dim3(256), 0, s->stream, fd, w);
+      hipLaunchKernelGGL((yee_dedt<3>), dim3(nd), dim3(256), 0, s->stream, fd, wd);
       hipLaunchKernelGGL(wall_e, dim3(nb), dim3(256), 0, s->stream, fd);
       hipLaunchKernelGGL((yee_dbdt<3, false>), dim3(s->nblk), dim3(256), 0, s->stream, fd, w);
-      hipLaunchKernelGGL((wall_b2_end<3>), dim3(nbf), dim3(kFinNT), 0, s->stream, fd);
+      hipLaunchKernelGGL((wall_b2_end<3>), dim3(nb), dim3(256), 0, s->stream, fd);
     }
     // the last wall kernel also restored the wall values and ended the step
     HIPC(hipGetLastError());
@@ -1017,22 +1018,22 @@ int launch_yee(osr_sim* s) {
   }
   if (s->dims == 2) {
     hipLaunchKernelGGL((yee_dbdt<2, true>), dim3(s->nblk_e), dim3(256), 0, s->stream, fd, we);
-    hipLaunchKernelGGL((yee_dedt<2>), dim3(s->nblk), dim3(256), 0, s->stream, fd, w);
+    hipLaunchKernelGGL((yee_dedt<2>), dim3(nd), dim3(256), 0, s->stream, fd, wd);
     hipLaunchKernelGGL((yee_dbdt<2, false>), dim3(s->nblk), dim3(256), 0, s->stream, fd, w);
   } else {
     hipLaunchKernelGGL((yee_dbdt<3, true>), dim3(s->nblk_e), dim3(256), 0, s->stream, fd, we);
-    hipLaunchKernelGGL((yee_dedt<3>), dim3(s->nblk), dim3(256), 0, s->stream, fd, w);
+    hipLaunchKernelGGL((yee_dedt<3>), dim3(nd), dim3(256), 0, s->stream, fd, wd);
     hipLaunchKernelGGL((yee_dbdt<3, false>), dim3(s->nblk), dim3(256), 0, s->stream, fd, w);
   }
   HIPC(hipGetLastError());
   return OSR_OK;
 }
 
-// End of the step: history row, step counter, halt protocol.  With Lindman walls the last
+// End of the step: step counter, halt protocol (the E step's launch wrote the history row).  With Lindman walls the last
 // wall kernel of launch_yee has done it.
 int launch_finalize(osr_sim* s) {
   if (s->g.open_nx && !s->vp_n) return OSR_OK;
-  hipLaunchKernelGGL(finalize_step, dim3(1), dim3(kFinNT), 0, s->stream, s->d_fd.as<FieldDesc>(),
+  hipLaunchKernelGGL(finalize_step, dim3(1), dim3(64), 0, s->stream, s->d_fd.as<FieldDesc>(),
                      s->d_fwork.as<int>());
   HIPC(hipGetLastError());
   return OSR_OK;
@@ -1357,6 +1358,11 @@ int osr_sim_create(const osr_sim_desc* desc, osr_sim** out) {
     std::vector<int2> ew(yw.begin(), yw.begin() + s->nblk_e);
     for (int b = 0; b < nwall_e; b++) ew.push_back(make_int2(0, -1 - b));
     TRY(copy_on(s->stream, s->d_ework.p, ew.data(), sizeof(int2) * ew.size(), hipMemcpyHostToDevice));
+    std::vector<int2> dw;
+    for (int c = 0; c < kRedCols; c++) dw.push_back(make_int2(0, -1 - c));
+    dw.insert(dw.end(), yw.begin(), yw.end());
+    TRY(s->d_dwork.alloc(sizeof(int2) * dw.size()));
+    TRY(copy_on(s->stream, s->d_dwork.p, dw.data(), sizeof(int2) * dw.size(), hipMemcpyHostToDevice));
     int z = 0;
     TRY(copy_on(s->stream, s->d_fwork.p, &z, sizeof(int), hipMemcpyHostToDevice));
   }

@@ -18,7 +18,7 @@ namespace osr {
 
 struct FieldDesc {
   GridDesc g;
-  double* fe_part;   // [nblk][6] B1,B2,B3,E1,E2,E3 partial sums of squares
+  double* fe_part;   // [6][nblk] partial sums of squares of B1, B2, B3, E1, E2, E3
   int nblk;          // energy partials: one per kEneBlk blocks of 256 cells
   // finalisation
   int nspec;
@@ -101,6 +101,9 @@ constexpr int kEneBlk = 4;
 // one row of the Lindman wall B update (defined with the wall kernels below)
 template <int STEP, int DIMS, bool RESTORE = false>
 OSR_DEV void wall_b_row(const FieldDesc& fd, long long r);
+
+// the sum of one history column (defined with the step end below)
+OSR_DEV void reduce_column(const FieldDesc& fd, int col);
 
 template <int DIMS, bool ENERGY>
 __global__ __launch_bounds__(256) void yee_dbdt(const FieldDesc* __restrict__ fds,
@@ -206,7 +209,7 @@ __global__ __launch_bounds__(256) void yee_dbdt(const FieldDesc* __restrict__ fd
     __syncthreads();
     if (threadIdx.x < 6) {
       const int c = threadIdx.x;
-      fd.fe_part[(long long)wk.y * 6 + c] =
+      fd.fe_part[(long long)c * fd.nblk + wk.y] =
           ((s_red[0][c] + s_red[1][c]) + s_red[2][c]) + s_red[3][c];
     }
   }
@@ -218,6 +221,10 @@ __global__ __launch_bounds__(256) void yee_dedt(const FieldDesc* __restrict__ fd
   const int2 wk = work[blockIdx.x];
   const FieldDesc& fd = fds[wk.x];
   const GridDesc& g = fd.g;
+  if (wk.y < 0) {  // a history column: its partial sums are complete before this launch
+    reduce_column(fd, -1 - wk.y);
+    return;
+  }
   if (g.ctrl->halt >= 2) return;
   const long long nc = g.ncell;
   const long long idx = (long long)wk.y * 256 + threadIdx.x;
@@ -656,161 +663,82 @@ OSR_DEV void kmerge(double& s, double& c, double s2, double c2) {
   s = t;
 }
 
-// One block per simulation: compensated reduction of the step's partial sums into one
-// history row, then the step counter and the halt protocol.  The order of every addition
-// is fixed (strided per-thread sums, then a fixed shuffle tree per wave and the waves in
-// order), so the row is reproducible bit for bit.  All 6 + nspec columns go through the
-// reduction together: the six field columns in one pass over the blocks (each thread
-// reads the six contiguous partials of its blocks, several blocks' loads issued before
-// they are accumulated), the shuffle trees of all columns interleaved, and the final
-// merge of the 16 wave sums done by one thread per column, so the dependent FP64 chains
-// of the columns overlap instead of following one another.
-constexpr int kFinNT = 1024;
-constexpr int kFinCols = 6 + kMaxSpecies;
+// Sum of one history column (field component or species) by one workgroup of 256 threads:
+// compensated strided sums per thread, a fixed shuffle tree per wave, the waves in order,
+// so the row is reproducible bit for bit.  The columns are extra work items of the E step,
+// whose launch follows the kernels that write the partial sums (push, first B half step);
+// nothing reads the row on the device, so the sums run beside the field cells instead of
+// in a launch of their own: one workgroup for all columns at the end of the step took
+// 12 us on a 64 x 64 grid and 29 us on 192^3.  A 100-step 64 x 64 run went from 5.44 to
+// 4.42 ms, 40 steps of 52 x 44 x 36 from 4.81 to 4.40 ms.
+constexpr int kRedNT = 256;
+constexpr int kRedCols = 6 + kMaxSpecies;
 
-// the reduction and the step-end protocol, run by one workgroup of kFinNT threads
-OSR_DEV void finalize_body(const FieldDesc& fd) {
-  __shared__ double w_s[kFinNT / 64][kFinCols], w_c[kFinNT / 64][kFinCols];
-  const GridDesc& g = fd.g;
-  Ctrl* ctrl = g.ctrl;
-  // read with the partial sums; a halted simulation writes nothing (the reduction itself
-  // only reads, so it need not wait for the flag)
-  const int halt = ctrl->halt;
-  const long long step = ctrl->steps;
-  const int nspec = fd.nspec;
-  const int ncol = 6 + nspec;
-  constexpr int U = 2;  // items per column loaded ahead per thread (the order of the adds
-                       // is the same for any U)
-  double s[kFinCols], c[kFinCols];
+OSR_DEV void reduce_column(const FieldDesc& fd, int col) {
+  __shared__ double w_s[kRedNT / 64], w_c[kRedNT / 64];
+  constexpr int U = 8;  // loads in flight per thread (the order of the adds does not change)
+  if (col >= 6 + fd.nspec) return;
+  const int halt = fd.g.ctrl->halt;
+  const long long step = fd.g.ctrl->steps;
+  const double* __restrict__ p = col < 6 ? fd.fe_part + (long long)col * fd.nblk : fd.ep[col - 6];
+  const int n = col < 6 ? fd.nblk : fd.ep_n[col - 6];
+  double s = 0.0, c = 0.0;
+  for (int b0 = threadIdx.x; b0 < n; b0 += kRedNT * U) {
+    double v[U];
 #pragma unroll
-  for (int col = 0; col < kFinCols; col++) s[col] = c[col] = 0.0;
-  const int tid = threadIdx.x;
-  const int nblk = fd.nblk;
-  // first pass: a thread's first U items of the field columns and of the first kPre
-  // species, all loads issued before the first addition (one memory round trip instead
-  // of one per column group); kPre bounds the registers the loads ahead take
-  constexpr int kPre = 2;
-  {
-    double vf[U][6], vs[kPre][U];
-    int epn[kPre];
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-      const int b = tid + u * kFinNT;
-#pragma unroll
-      for (int col = 0; col < 6; col++)
-        vf[u][col] = b < nblk ? fd.fe_part[(long long)b * 6 + col] : 0.0;
-    }
-#pragma unroll
-    for (int sp = 0; sp < kPre; sp++) {
-      epn[sp] = sp < nspec ? fd.ep_n[sp] : 0;
-      const double* ep = fd.ep[sp];
-#pragma unroll
-      for (int u = 0; u < U; u++) {
-        const int t = tid + u * kFinNT;
-        vs[sp][u] = t < epn[sp] ? ep[t] : 0.0;
-      }
-    }
+    for (int u = 0; u < U; u++) v[u] = b0 + u * kRedNT < n ? p[b0 + u * kRedNT] : 0.0;
 #pragma unroll
     for (int u = 0; u < U; u++)
-      if (tid + u * kFinNT < nblk)
-#pragma unroll
-        for (int col = 0; col < 6; col++) kadd(s[col], c[col], vf[u][col]);
-#pragma unroll
-    for (int sp = 0; sp < kPre; sp++)
-#pragma unroll
-      for (int u = 0; u < U; u++)
-        if (tid + u * kFinNT < epn[sp]) kadd(s[6 + sp], c[6 + sp], vs[sp][u]);
+      if (b0 + u * kRedNT < n) kadd(s, c, v[u]);
   }
-  // the remaining items of every column (many cell blocks or tiles, more species), in
-  // order
-  for (int b0 = tid + U * kFinNT; b0 < nblk; b0 += kFinNT * U) {
-    double v[U][6];
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-      const int b = b0 + u * kFinNT;
-#pragma unroll
-      for (int col = 0; col < 6; col++)
-        v[u][col] = b < nblk ? fd.fe_part[(long long)b * 6 + col] : 0.0;
-    }
-#pragma unroll
-    for (int u = 0; u < U; u++)
-      if (b0 + u * kFinNT < nblk)
-#pragma unroll
-        for (int col = 0; col < 6; col++) kadd(s[col], c[col], v[u][col]);
-  }
-#pragma unroll
-  for (int sp = 0; sp < kMaxSpecies; sp++) {
-    if (sp >= nspec) break;
-    const double* ep = fd.ep[sp];
-    const int n = fd.ep_n[sp];
-    for (int t0 = tid + (sp < kPre ? U * kFinNT : 0); t0 < n; t0 += kFinNT * U) {
-      double v[U];
-#pragma unroll
-      for (int u = 0; u < U; u++) v[u] = t0 + u * kFinNT < n ? ep[t0 + u * kFinNT] : 0.0;
-#pragma unroll
-      for (int u = 0; u < U; u++)
-        if (t0 + u * kFinNT < n) kadd(s[6 + sp], c[6 + sp], v[u]);
-    }
-  }
-  // per wave: the fixed shuffle tree, all columns at each level
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  for (int off = 32; off > 0; off >>= 1) {
 #pragma unroll
-    for (int col = 0; col < kFinCols; col++) {
-      if (col >= ncol) break;
-      const double s2 = __shfl_down(s[col], off), c2 = __shfl_down(c[col], off);
-      kmerge(s[col], c[col], s2, c2);
-    }
+  for (int off = 32; off > 0; off >>= 1) {
+    const double s2 = __shfl_down(s, off), c2 = __shfl_down(c, off);
+    kmerge(s, c, s2, c2);
   }
   if (lane == 0) {
-#pragma unroll
-    for (int col = 0; col < kFinCols; col++) {
-      w_s[wave][col] = s[col];
-      w_c[wave][col] = c[col];
-    }
+    w_s[wave] = s;
+    w_c[wave] = c;
   }
   __syncthreads();
-  if (halt >= 2) return;  // uniform over the block, after its last barrier
-  // the waves in order, one thread per column
-  if (threadIdx.x < ncol) {
-    const int col = threadIdx.x;
-    double ss = w_s[0][col], cc = w_c[0][col];
-    for (int w = 1; w < kFinNT / 64; w++) kmerge(ss, cc, w_s[w][col], w_c[w][col]);
-    if (step < fd.hist_cap)
-      fd.hist[step * ncol + col] = (ss + cc) * (col < 6 ? fd.fe_scale : fd.ep_scale[col - 6]);
-  }
-  __syncthreads();  // every read of the control block above precedes its update
-  if (threadIdx.x == 0) {
-    ctrl->steps = step + 1;
-    if (halt == 1)
-      ctrl->halt = 2;
-    else if (ctrl->target > 0 && step + 1 >= ctrl->target)
-      ctrl->halt = 3;
-  }
+  if (threadIdx.x != 0 || halt >= 2 || step >= fd.hist_cap) return;
+  for (int w = 1; w < kRedNT / 64; w++) kmerge(s, c, w_s[w], w_c[w]);
+  fd.hist[step * (6 + fd.nspec) + col] = (s + c) * (col < 6 ? fd.fe_scale : fd.ep_scale[col - 6]);
 }
 
-__global__ __launch_bounds__(kFinNT) void finalize_step(const FieldDesc* __restrict__ fds,
-                                                        const int* __restrict__ work) {
-  finalize_body(fds[work[blockIdx.x]]);
+// End of the step (one thread, after every other kernel of the step): the step counter and
+// the halt protocol.
+OSR_DEV void end_step(const GridDesc& g) {
+  Ctrl* ctrl = g.ctrl;
+  const int halt = ctrl->halt;
+  const long long step = ctrl->steps, target = ctrl->target;
+  if (halt >= 2) return;
+  ctrl->steps = step + 1;
+  if (halt == 1)
+    ctrl->halt = 2;
+  else if (target > 0 && step + 1 >= target)
+    ctrl->halt = 3;
+}
+
+__global__ __launch_bounds__(64) void finalize_step(const FieldDesc* __restrict__ fds,
+                                                    const int* __restrict__ work) {
+  if (threadIdx.x == 0) end_step(fds[work[blockIdx.x]].g);
 }
 
 // Lindman walls: the lower wall's second B update with the restore of the wall values
-// (wall_b<2, DIMS, true>), kFinNT rows per workgroup, and the end of the step in the
-// workgroup that finishes last (a ticket on Ctrl::done), so no kernel launch follows.
-// Every workgroup has read the halt flag before it takes its ticket, so the flag changes
-// only once none of them looks at it any more; the reduction reads partial sums of
-// earlier kernels only.
+// (wall_b<2, DIMS, true>) and the end of the step in the workgroup that finishes last (a
+// ticket on Ctrl::done), so no kernel launch follows.  Every workgroup has read the halt
+// flag before it takes its ticket, so the flag changes only once none of them looks at it
+// any more.
 template <int DIMS>
-__global__ __launch_bounds__(kFinNT) void wall_b2_end(const FieldDesc* __restrict__ fds) {
-  __shared__ int s_last;
+__global__ __launch_bounds__(256) void wall_b2_end(const FieldDesc* __restrict__ fds) {
   const FieldDesc& fd = *fds;
-  wall_b_row<2, DIMS, true>(fd, (long long)blockIdx.x * kFinNT + threadIdx.x);
+  wall_b_row<2, DIMS, true>(fd, (long long)blockIdx.x * 256 + threadIdx.x);
   __syncthreads();
-  if (threadIdx.x == 0) s_last = atomicAdd(&fd.g.ctrl->done, 1u) == gridDim.x - 1;
-  __syncthreads();
-  if (!s_last) return;
-  if (threadIdx.x == 0) fd.g.ctrl->done = 0;
-  finalize_body(fd);
+  if (threadIdx.x != 0 || atomicAdd(&fd.g.ctrl->done, 1u) != gridDim.x - 1) return;
+  fd.g.ctrl->done = 0;
+  end_step(fd.g);
 }
 
 // ------------------------------------------------------------------------------------
