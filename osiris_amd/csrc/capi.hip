@@ -180,7 +180,7 @@ struct osr_sim {
   DBuf E, B, J, ctrl, fe_part, hist;
   int64_t hist_cap = 0;
   std::vector<std::unique_ptr<Species>> sp;
-  DBuf d_spec, d_work, d_fd, d_ywork, d_ework, d_dwork, d_fwork;
+  DBuf d_spec, d_work, d_pwork, d_fd, d_ywork, d_ework, d_dwork, d_fwork;
   FieldDesc fd{};
   hipStream_t stream = nullptr;
   hipGraphExec_t gexec = nullptr;    // one step
@@ -190,7 +190,9 @@ struct osr_sim {
   int64_t relayouts = 0;
   bool plain = false;
   size_t lds_push = 0;
-  int push_waves = 4;  // waves per push workgroup (SpecDesc::waves)
+  int push_waves = 4;  // waves per push workgroup
+  int split = 1;       // push workgroups per tile (SpecDesc::split)
+  int tile_waves() const { return push_waves * split; }
   int reorder = 0;     // tile_reorder period in steps (0: off)
   int sm_order[3] = {0, 0, 0};  // current smoothing per direction (0: none)
   float sm_coef[3][31] = {};
@@ -350,7 +352,8 @@ void make_spec_descs(const osr_sim* s, SpecDesc* v) {
     d.inc = p.inc.as<int>();
     d.epart = p.epart.as<double>();
     d.tem = (float)(0.5 * s->dt / (double)p.rqm);
-    d.waves = s->push_waves;
+    d.waves = s->tile_waves();
+    d.split = s->split;
   }
 }
 
@@ -436,6 +439,26 @@ inline void cell_coords(const osr_sim* s, uint32_t c, int* ic) {
     unpack3(c, ic[0], ic[1], ic[2]);
 }
 
+// Slots a tile keeps free for its mover regions: the waves' regions are rounded up to 64
+// slots each, and the fill leaves as many (at least those of the largest workgroup).
+int mover_slack(int tile_waves) { return 64 * std::max(kMaxPushWaves, tile_waves); }
+
+// Push workgroups per tile (2D compile-time kernels).  One wave takes about 1.2 us of VALU
+// issue per 64 particles, and about 2 us when it has a SIMD to itself, so a grid with
+// fewer waves than the chip's 1024 SIMDs hold is bound by the longest wave: its tiles are
+// shared by several workgroups.  Each of them stages the tile's fields and folds a current
+// tile of its own, which costs more than it gains once the tiles fill the chip.  us per
+// step, 1 / 2 / 4 workgroups per tile: 16x16 tiles with 4 waves, 64 tiles (128 x 128 x 16)
+// 53.6 / 45.4 / 41.9, 247 tiles (300 x 200 x 16) 94.2 / 87.1 / 90.8, 561 tiles (two species
+// of 9) 90.9 / 92.4 / 107.6, 1024 tiles 216.9 / 228.1 / 245.0; 32x16 tiles with 8 waves
+// (2 workgroups per CU), 102 tiles 84.6 / 76.8, 528 tiles push 69.4 / 57.7 (one workgroup
+// per tile leaves a second round of 16).  3D keeps one: LDS lets two workgroups into a CU,
+// and 378 tiles of 8x8x4 went from 95.8 to 106.8.
+int pick_split(int ntiles, int waves) {
+  if (waves >= 8) return ntiles <= 640 ? 2 : 1;
+  return ntiles <= 128 ? 4 : (ntiles <= 384 ? 2 : 1);
+}
+
 // Allocate a species' arrays for the given per-tile counts and capacities.
 int alloc_species(osr_sim* s, Species& p, const std::vector<int>& cnt) {
   const int nt = s->ntiles;
@@ -443,7 +466,7 @@ int alloc_species(osr_sim* s, Species& p, const std::vector<int>& cnt) {
   int64_t total = 0;
   for (int t = 0; t < nt; t++) {
     const int c = cnt[t];
-    int64_t cp = (int64_t)c + std::max(c / 4, 64) + 64 * kMaxPushWaves;
+    int64_t cp = (int64_t)c + std::max(c / 4, 64) + mover_slack(s->tile_waves());
     cp = (cp + 63) / 64 * 64;
     if (total + cp > INT32_MAX) return fail(OSR_ERR_ARG, "species too large for int32 slots");
     cap[t] = (int)cp;
@@ -474,11 +497,11 @@ int alloc_species(osr_sim* s, Species& p, const std::vector<int>& cnt) {
   TRY(p.off.alloc(4 * (size_t)nt));
   TRY(p.cnt.alloc(4 * (size_t)nt));
   TRY(p.cap.alloc(4 * (size_t)nt));
-  TRY(p.mv_cnt.alloc(4 * (size_t)nt * kMaxPushWaves));
+  TRY(p.mv_cnt.alloc(4 * (size_t)nt * kMaxTileWaves));
   TRY(p.mv_stride.alloc(4 * (size_t)nt));
   TRY(p.newcnt.alloc(4 * (size_t)nt));
   TRY(p.inc.alloc(4 * (size_t)nt));
-  p.epart_n = s->plain ? (int)((total + 255) / 256) : nt;
+  p.epart_n = s->plain ? (int)((total + 255) / 256) : nt * s->split;
   TRY(p.epart.alloc(8 * (size_t)p.epart_n));
   if (s->plain) {
     TRY(p.pl_ep.alloc(12 * n));
@@ -489,7 +512,7 @@ int alloc_species(osr_sim* s, Species& p, const std::vector<int>& cnt) {
   TRY(copy_on(s->stream, p.off.p, off.data(), 4 * nt, hipMemcpyHostToDevice));
   TRY(copy_on(s->stream, p.cnt.p, cnt.data(), 4 * nt, hipMemcpyHostToDevice));
   TRY(copy_on(s->stream, p.cap.p, cap.data(), 4 * nt, hipMemcpyHostToDevice));
-  HIPC(hipMemsetAsync(p.mv_cnt.p, 0, 4 * (size_t)nt * kMaxPushWaves, s->stream));
+  HIPC(hipMemsetAsync(p.mv_cnt.p, 0, 4 * (size_t)nt * kMaxTileWaves, s->stream));
   HIPC(hipMemsetAsync(p.mv_stride.p, 0, 4 * (size_t)nt, s->stream));
   HIPC(hipMemsetAsync(p.epart.p, 0, 8 * (size_t)p.epart_n, s->stream));
   HIPC(hipMemsetAsync(p.inc.p, 0, 4 * (size_t)nt, s->stream));
@@ -611,7 +634,7 @@ int download(hipStream_t st, std::vector<T>& v, const DBuf& b, size_t n) {
 // into the mover buffer but the fill did not run (halted step).
 int collect(osr_sim* s, Species& p, bool pending, HostParts& hp) {
   const int nt = s->ntiles;
-  const int W = s->push_waves;  // wave count of the push that filled the mover buffers
+  const int W = s->tile_waves();  // wave count of the push that filled the mover buffers
   const size_t C = (size_t)p.cap_total;
   std::vector<int> cnt, mvc, mvs, midx;
   TRY(download(s->stream, cnt, p.cnt, nt));
@@ -749,7 +772,7 @@ int regrow_species(osr_sim* s, int sid, bool* ok) {
     // every tile gets room for half its count again (a density front that overflows one
     // tile usually reaches its neighbours next); no tile shrinks
     const int64_t r = inc[t] < 0 ? need[t] : cnt[t];
-    int64_t c = std::max<int64_t>(p.h_cap[t], r + std::max<int64_t>(r / 2, 64) + 64 * kMaxPushWaves);
+    int64_t c = std::max<int64_t>(p.h_cap[t], r + std::max<int64_t>(r / 2, 64) + mover_slack(s->tile_waves()));
     c = (c + 63) / 64 * 64;
     if (total + c > INT32_MAX) return OSR_OK;
     cap[t] = (int)c;
@@ -920,8 +943,9 @@ int launch_push(osr_sim* s, int first, int count = 1) {
                                s->lds_push, &lds, &nt);
   if (!f) return fail(OSR_ERR_ARG, "no push kernel for dims=%d order=%d", s->dims, s->order);
   if (nt != 64 * s->push_waves) return fail(OSR_ERR_STATE, "push wave count mismatch");
-  hipLaunchKernelGGL(f, dim3((unsigned)(count * s->ntiles)), dim3(nt), lds, s->stream,
-                     s->d_spec.as<SpecDesc>(), s->d_work.as<int2>() + (size_t)first * s->ntiles);
+  hipLaunchKernelGGL(f, dim3((unsigned)(count * s->ntiles * s->split)), dim3(nt), lds, s->stream,
+                     s->d_spec.as<SpecDesc>(),
+                     s->d_pwork.as<int2>() + (size_t)first * s->ntiles * s->split);
   HIPC(hipGetLastError());
   return OSR_OK;
 }
@@ -1309,6 +1333,9 @@ int osr_sim_create(const osr_sim_desc* desc, osr_sim** out) {
   if (desc->push_waves > 0 && desc->push_waves != s->push_waves)
     return fail(OSR_ERR_ARG, "no push kernel with %d waves per workgroup for this tile and kernel",
                 desc->push_waves);
+  if (!s->plain && dims == 2 && desc->kernel != 1 &&
+      pick_push2d_t(s->order, 0, g.tx, g.ty, s->push_waves))
+    s->split = pick_split(g.ntiles, s->push_waves);
   HIPC(hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking));
   const size_t nc = (size_t)g.ncell;
   TRY(s->E.alloc(3 * nc * 4));
@@ -1403,6 +1430,11 @@ int osr_sim_add_species(osr_sim* s, float rqm, int pusher, int* sid) {
   for (int i = 0; i < ns; i++)
     for (int t = 0; t < s->ntiles; t++) w[(size_t)i * s->ntiles + t] = make_int2(i, xcd_tile(s->dims, t, s->ntiles));
   TRY(copy_on(s->stream, s->d_work.p, w.data(), sizeof(int2) * w.size(), hipMemcpyHostToDevice));
+  // the push's list names every item once per workgroup of the tile
+  std::vector<int2> pw;
+  for (const int2& it : w) pw.insert(pw.end(), s->split, it);
+  TRY(s->d_pwork.alloc(sizeof(int2) * pw.size()));
+  TRY(copy_on(s->stream, s->d_pwork.p, pw.data(), sizeof(int2) * pw.size(), hipMemcpyHostToDevice));
   // history rows gain a column: restart the history buffer
   s->hist.release();
   s->hist_cap = 0;

@@ -96,10 +96,10 @@ int64_t job_footprint(const osr_job_desc& j) {
       const int64_t wy = std::min(tl[1], d.nx[1] - ty * tl[1]);
       const int64_t wz = D == 3 ? std::min(tl[2], d.nx[2] - tz * tl[2]) : 1;
       const int64_t c = wx * wy * wz * ppc;
-      int64_t cp = c + std::max<int64_t>(c / 4, 64) + 64 * kMaxPushWaves;
+      int64_t cp = c + std::max<int64_t>(c / 4, 64) + 64 * kMaxTileWaves;
       slots += (cp + 63) / 64 * 64;
     }
-    b += slots * slot + ntiles * (48 + 8);
+    b += slots * slot + ntiles * (24 + 4 * kMaxTileWaves + 8 * kMaxSplit);
   }
   return b + (1 << 20);
 }
@@ -219,7 +219,7 @@ int ens_build(osr_ensemble* e, EnsBatch* b) {
   std::vector<SpecDesc> specs;
   std::vector<FieldDesc> fds(b->jobs.size());
   std::vector<int2> wp[2], wf, wy, we, wd;
-  std::vector<int> wn;
+  std::vector<int> wn, spec0;
   for (size_t k = 0; k < b->jobs.size(); k++) {
     osr_sim* s = b->jobs[k]->sim;
     const int base = (int)specs.size();
@@ -228,14 +228,25 @@ int ens_build(osr_ensemble* e, EnsBatch* b) {
     make_field_desc(s, fds[k]);
     for (size_t i = 0; i < s->sp.size(); i++)
       for (int t = 0; t < s->ntiles; t++) {
-        wp[s->sp[i]->pusher == OSR_VAY ? 1 : 0].push_back(make_int2(base + (int)i, t));
         wf.push_back(make_int2(base + (int)i, t));
       }
     for (int blk = 0; blk < s->nblk; blk++) wy.push_back(make_int2((int)k, blk));
     for (int blk = 0; blk < s->nblk_e; blk++) we.push_back(make_int2((int)k, blk));
     for (int c = 0; c < 6 + (int)s->sp.size(); c++) wd.push_back(make_int2((int)k, -1 - c));
     wn.push_back((int)k);
+    spec0.push_back(base);
   }
+  // the push lists, jobs with the most workgroups per tile first: a tile's workgroups then
+  // start at a multiple of their number, from which each finds its part
+  for (int sp = kMaxSplit; sp >= 1; sp /= 2)
+    for (size_t k = 0; k < b->jobs.size(); k++) {
+      const osr_sim* s = b->jobs[k]->sim;
+      if (s->split != sp) continue;
+      for (size_t i = 0; i < s->sp.size(); i++)
+        for (int t = 0; t < s->ntiles; t++)
+          wp[s->sp[i]->pusher == OSR_VAY ? 1 : 0].insert(
+              wp[s->sp[i]->pusher == OSR_VAY ? 1 : 0].end(), sp, make_int2(spec0[k] + (int)i, t));
+    }
   wd.insert(wd.end(), wy.begin(), wy.end());  // the E step: history columns, then cell blocks
   auto put = [&](DBuf& d, const void* src, size_t bytes) -> int {
     if (bytes == 0) return OSR_OK;

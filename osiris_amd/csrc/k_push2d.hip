@@ -100,8 +100,12 @@ __global__ __launch_bounds__(64 * NW, 4) void push_deposit_2d_t(const SpecDesc* 
   // uniform per workgroup: keep them (and the array bases below) in scalar registers
   const int base = __builtin_amdgcn_readfirstlane(d.off[tile]);
   const int n = __builtin_amdgcn_readfirstlane(d.cnt[tile]);
-  const int per_wave = ((n + NT - 1) / NT) * 64;
-  const int w0 = wave * per_wave;
+  // this workgroup's waves among the split * NW of the tile (the work list names a tile
+  // once per workgroup, back to back)
+  const int split = d.split, part = (int)(blockIdx.x % (unsigned)split);
+  const int tw = part * NW + wave;
+  const int per_wave = ((n + NT * split - 1) / (NT * split)) * 64;
+  const int w0 = tw * per_wave;
   const int w1 = min(w0 + per_wave, n);
   const float tem = d.tem;
   const float dtdx1 = g.dt_dx[0], dtdx2 = g.dt_dx[1];
@@ -302,8 +306,8 @@ __global__ __launch_bounds__(64 * NW, 4) void push_deposit_2d_t(const SpecDesc* 
   if (qlen > 0) deposit_queue(qhead, qlen);
 
   if (bad) atomicOr(&g.ctrl->error, 1);
-  if (lane == 0) d.mv_cnt[tile * NW + wave] = mcount;
-  if (threadIdx.x == 0) d.mv_stride[tile] = per_wave;
+  if (lane == 0) d.mv_cnt[tile * NW * split + tw] = mcount;
+  if (threadIdx.x == 0 && part == 0) d.mv_stride[tile] = per_wave;
   ene = wave_sum(ene);
   if (lane == 0) s_ene[wave] = ene;
   __syncthreads();
@@ -311,7 +315,7 @@ __global__ __launch_bounds__(64 * NW, 4) void push_deposit_2d_t(const SpecDesc* 
     double t = s_ene[0];
 #pragma unroll
     for (int w = 1; w < NW; w++) t += s_ene[w];
-    d.epart[tile] = t;
+    d.epart[tile * split + part] = t;
   }
   // ---- fold the LDS current tile into the global fixed-point J (periodic wrap)
   gu64* __restrict__ GJ = (gu64*)g.J;

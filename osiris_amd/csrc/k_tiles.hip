@@ -629,14 +629,14 @@ constexpr int kFillPF = 8;  // candidate movers per thread whose cells are loade
 template <int NT, int INC_MAX, int TAIL_BITS>
 __global__ __launch_bounds__(NT) void tile_fill(const SpecDesc* __restrict__ descs,
                                                 const int2* __restrict__ work) {
-  constexpr int MAXL = 26 * 4;  // candidate lists: neighbours x waves
+  constexpr int MAXL = 26 * kMaxTileWaves;  // candidate lists: neighbours x waves
   __shared__ int s_nb[26];
   __shared__ int s_nnb;
   __shared__ int s_lofs[MAXL + 1];
   __shared__ int s_lbase[MAXL];
   __shared__ int s_wtot[NT / 64];
   __shared__ int s_pcnt[kFillPF][NT / 64];
-  __shared__ int s_hpre[17];
+  __shared__ int s_hpre[kMaxTileWaves + 1];
   __shared__ int s_inc[INC_MAX];
   __shared__ unsigned int s_bits[TAIL_BITS / 32];
   const int2 wk = work[blockIdx.x];
@@ -656,7 +656,7 @@ __global__ __launch_bounds__(NT) void tile_fill(const SpecDesc* __restrict__ des
   }
   __syncthreads();
   const int L = s_nnb * NW;
-  if (L > MAXL) {  // more mover lists than the LDS tables hold: never with 26 x 4 or 8 x 8
+  if (L > MAXL) {  // more mover lists than the LDS tables hold: never with 26 x 16
     if (threadIdx.x == 0) atomicOr(&g.ctrl->error, 2);
     return;
   }

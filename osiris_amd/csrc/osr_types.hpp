@@ -28,6 +28,11 @@ constexpr int kMaxSpecies = 8;
 // tiles in LDS are then shared by twice as many waves, so two workgroups (16 waves) fit in
 // a CU's LDS where three 4-wave ones (12 waves) did.
 constexpr int kMaxPushWaves = 8;
+// Workgroups per tile in the 2D push (its split), and the waves of a tile over all of them:
+// a grid of few tiles would leave CUs idle with one workgroup per tile.  Each wave of a tile
+// owns a contiguous slice of its particles and a mover region, whichever workgroup it is in.
+constexpr int kMaxSplit = 4;
+constexpr int kMaxTileWaves = 16;
 // capacity of the per-wave virtual-particle queue of the 3D push (pending < 64 plus up to
 // 64 appended per VP level)
 constexpr int kVpQueue3 = 128;
@@ -125,13 +130,14 @@ struct SpecDesc {
   int* off;
   int* cnt;
   int* cap;
-  int* mv_cnt;     // [ntiles][waves]
+  int* mv_cnt;     // [ntiles][waves] (every wave of the tile, over its workgroups)
   int* mv_stride;  // [ntiles] per-wave region size used by the last push
   int* newcnt;     // [ntiles]
   int* inc;        // [ntiles] incoming count
-  double* epart;   // [ntiles] time-centred energy partial sums (un-normalised)
+  double* epart;   // [ntiles][split] time-centred energy partial sums (un-normalised)
   float tem;       // (float)(0.5*dt/rqm)
-  int waves;       // waves per workgroup in the push kernel
+  int split;       // workgroups per tile in the push (1 in 3D and with the generic kernel)
+  int waves;       // waves per tile in the push: those of its workgroups times split
 };
 
 // Cell packing.  2D: ix | iy<<16.  3D: ix | iy<<11 | iz<<22.

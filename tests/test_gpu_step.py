@@ -1,0 +1,43 @@
+"""The work split of the step's kernels at the edges of their rules: every choice gives the
+bits of the generic kernels (integer current, order-independent), so the comparisons are
+exact; the FP64 energy sums are grouped differently and agree to round-off (1e-12)."""
+import numpy as np
+import pytest
+
+import osiris_amd as oa
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(dims, nx, order, steps, **kw):
+    with oa.Simulation(dims, nx, (0.1,) * dims, 0.04, order, **kw) as sim:
+        rng = np.random.default_rng(5)
+        n = 3 * int(np.prod(nx))
+        for rqm, drift in ((-1.0, 0.3), (1.0, -0.2)):
+            sid = sim.add_species(rqm)
+            ix = np.stack([rng.integers(1, m + 1, n) for m in nx], 1).astype(np.int32)
+            x = (rng.random((n, dims), np.float32) - np.float32(0.5)).astype(np.float32)
+            u = (rng.standard_normal((n, 3)) * 0.2).astype(np.float32)
+            u[:, 0] += np.float32(drift)
+            sim.set_particles(sid, ix, x, u, np.full(n, 0.05 * rqm, np.float32))
+        sim.run(steps)
+        return sim.get_fields(), sim.get_particles(0), sim.get_particles(1), sim.history()
+
+
+def _same(a, b):
+    for x, y in zip(a[0] + a[1] + a[2], b[0] + b[1] + b[2]):
+        assert np.array_equal(x.view(np.uint32), y.view(np.uint32))
+    for x, y in zip(a[3], b[3]):
+        assert np.allclose(x, y, rtol=1e-12, atol=0)
+
+
+@pytest.mark.parametrize("nx,tile,waves", [
+    ((16, 16), (16, 16), 4), ((16, 40), (16, 16), 4), ((128, 256), (16, 16), 4),
+    ((129, 256), (16, 16), 4), ((384, 256), (16, 16), 4), ((385, 250), (16, 16), 4),
+    ((64, 33), (32, 16), 8), ((640, 512), (32, 16), 8), ((641, 512), (32, 16), 8),
+    ((48, 40), (16, 16), 8), ((70, 30), (8, 8), 4)])
+def test_push_workgroups_per_tile(nx, tile, waves):
+    """1, 2 and 4 push workgroups per tile, on both sides of each limit, tiles cut by the
+    grid's edge, 1 and 2 tiles per direction."""
+    print(f"case nx={nx} tile={tile} waves={waves}", flush=True)
+    _same(_run(2, nx, 2, 6, tile=tile, push_waves=waves), _run(2, nx, 2, 6, tile=tile, kernel=1))
