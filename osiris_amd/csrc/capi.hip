@@ -186,6 +186,10 @@ struct osr_sim {
   hipGraphExec_t gexec = nullptr;    // one step
   hipGraphExec_t gexec_k = nullptr;  // kGraphSteps steps
   bool graph_ok = false;
+  unsigned par = 0;       // Ctrl::par of the last completed batch (GridDesc::pp)
+  bool fe_stale = false;  // the host changed the fields: the energy partials of the next row
+                          // (GridDesc::pp) are computed before the next step
+  int yv = 0;             // yee2d_step variant (0: 32x8 cells per workgroup, 1: 64x16)
   int64_t steps = 0;
   int64_t relayouts = 0;
   bool plain = false;
@@ -221,6 +225,12 @@ struct osr_sim {
 namespace {
 
 int ceil_div(int a, int b) { return (a + b - 1) / b; }
+
+// yee2d_step variant of a grid of nc cells: 32x8 cells per workgroup (latency: one or two
+// staged cells per thread), or 64x16 (less halo) once the grid has several such tiles per
+// CU.  us, 32x8 / 64x16: 64x64 5.8 / 8.4, 128x128 6.1 / 8.6, 1024x1024 39.3 / 34.3; the
+// whole step on 512x512 219.4 / 217.1.
+int pick_yv(size_t nc) { return nc >= 500000; }
 
 constexpr int kZpRows = 256;  // steps of laser values per host evaluation (the longest batch)
 
@@ -428,6 +438,21 @@ int upload_descs(osr_sim* s) {
   TRY(copy_on(s->stream, s->d_fd.p, &s->fd, sizeof(FieldDesc), hipMemcpyHostToDevice));
   s->desc_version++;
   return OSR_OK;
+}
+
+// E, B of the copy the next step reads, and the grid descriptor that names them (for the
+// kernels that take it by value)
+float* cur_E(const osr_sim* s) {
+  return s->E.as<float>() + (s->g.pp ? (size_t)s->par * 3 * s->g.ncell : 0);
+}
+float* cur_B(const osr_sim* s) {
+  return s->B.as<float>() + (s->g.pp ? (size_t)s->par * 3 * s->g.ncell : 0);
+}
+GridDesc cur_grid(const osr_sim* s) {
+  GridDesc g = s->g;
+  g.E = cur_E(s);
+  g.B = cur_B(s);
+  return g;
 }
 
 // Cell coordinates (0-based) of a packed cell.
@@ -869,6 +894,16 @@ int xcd_tile(int dims, int p, int ntiles) {
 
 // ---- kernel dispatch -------------------------------------------------------------
 typedef void (*push_fn)(const SpecDesc*, const int2*);
+typedef void (*yee2d_fn)(const FieldDesc*, const int2*, int);
+
+yee2d_fn pick_yee2d(int yv) {
+  if (yv) return yee2d_step<64, 16>;
+  return yee2d_step<32, 8>;
+}
+yee2d_fn pick_yee2d_energy(int yv) {
+  if (yv) return yee2d_energy<64, 16>;
+  return yee2d_energy<32, 8>;
+}
 
 push_fn pick_push(int dims, int order, int pusher) {
 #define OSR_P(D, O, P) \
@@ -1040,7 +1075,10 @@ int launch_yee(osr_sim* s) {
     HIPC(hipGetLastError());
     return OSR_OK;
   }
-  if (s->dims == 2) {
+  if (s->g.pp) {
+    hipLaunchKernelGGL(pick_yee2d(s->yv),
+                       dim3((unsigned)(kRedCols + s->nblk_e)), dim3(256), 0, s->stream, fd, wd, 0);
+  } else if (s->dims == 2) {
     hipLaunchKernelGGL((yee_dbdt<2, true>), dim3(s->nblk_e), dim3(256), 0, s->stream, fd, we);
     hipLaunchKernelGGL((yee_dedt<2>), dim3(nd), dim3(256), 0, s->stream, fd, wd);
     hipLaunchKernelGGL((yee_dbdt<2, false>), dim3(s->nblk), dim3(256), 0, s->stream, fd, w);
@@ -1050,6 +1088,18 @@ int launch_yee(osr_sim* s) {
     hipLaunchKernelGGL((yee_dbdt<3, false>), dim3(s->nblk), dim3(256), 0, s->stream, fd, w);
   }
   HIPC(hipGetLastError());
+  return OSR_OK;
+}
+
+// The energy partials of fields the host changed, for the next history row (two-copy grids;
+// on the others the first B half step sums them)
+int refresh_energy(osr_sim* s) {
+  if (!s->g.pp || !s->fe_stale) return OSR_OK;
+  hipLaunchKernelGGL(pick_yee2d_energy(s->yv), dim3((unsigned)s->nblk_e),
+                     dim3(256), 0, s->stream, s->d_fd.as<FieldDesc>(),
+                     s->d_dwork.as<int2>() + kRedCols, 0);
+  HIPC(hipGetLastError());
+  s->fe_stale = false;
   return OSR_OK;
 }
 
@@ -1338,9 +1388,11 @@ int osr_sim_create(const osr_sim_desc* desc, osr_sim** out) {
     s->split = pick_split(g.ntiles, s->push_waves);
   HIPC(hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking));
   const size_t nc = (size_t)g.ncell;
-  TRY(s->E.alloc(3 * nc * 4));
-  TRY(s->B.alloc(3 * nc * 4));
-  TRY(s->J.alloc(3 * nc * 8));
+  g.pp = dims == 2 && !s->plain && !open_x;  // grids whose field step is yee2d_step
+  const size_t ncp = g.pp ? 2 * nc : nc;
+  TRY(s->E.alloc(3 * ncp * 4));
+  TRY(s->B.alloc(3 * ncp * 4));
+  TRY(s->J.alloc(3 * ncp * 8));
   TRY(s->ctrl.alloc(sizeof(Ctrl)));
   s->vp_n = vp_n;
   if (open_x && vp_n) {
@@ -1357,9 +1409,9 @@ int osr_sim_create(const osr_sim_desc* desc, osr_sim** out) {
     TRY(s->wall.alloc(wb));
     HIPC(hipMemsetAsync(s->wall.p, 0, wb, s->stream));
   }
-  HIPC(hipMemsetAsync(s->E.p, 0, 3 * nc * 4, s->stream));
-  HIPC(hipMemsetAsync(s->B.p, 0, 3 * nc * 4, s->stream));
-  HIPC(hipMemsetAsync(s->J.p, 0, 3 * nc * 8, s->stream));
+  HIPC(hipMemsetAsync(s->E.p, 0, 3 * ncp * 4, s->stream));
+  HIPC(hipMemsetAsync(s->B.p, 0, 3 * ncp * 4, s->stream));
+  HIPC(hipMemsetAsync(s->J.p, 0, 3 * ncp * 8, s->stream));
   HIPC(hipMemsetAsync(s->ctrl.p, 0, sizeof(Ctrl), s->stream));
   HIPC(hipStreamSynchronize(s->stream));
   g.E = s->E.as<float>();
@@ -1368,8 +1420,13 @@ int osr_sim_create(const osr_sim_desc* desc, osr_sim** out) {
   g.ctrl = s->ctrl.as<Ctrl>();
   s->nblk = (int)((nc + 255) / 256);
   s->nblk_e = (s->nblk + kEneBlk - 1) / kEneBlk;
-  TRY(s->fe_part.alloc(sizeof(double) * 6 * (size_t)s->nblk_e));
-  HIPC(hipMemsetAsync(s->fe_part.p, 0, sizeof(double) * 6 * (size_t)s->nblk_e, s->stream));
+  if (g.pp) {
+    s->yv = pick_yv(nc);
+    s->nblk_e = s->yv ? ceil_div(g.nx, 64) * ceil_div(g.ny, 16) : ceil_div(g.nx, 32) * ceil_div(g.ny, 8);
+  }
+  const size_t fe_bytes = sizeof(double) * 6 * (size_t)s->nblk_e * (g.pp ? 2 : 1);
+  TRY(s->fe_part.alloc(fe_bytes));
+  HIPC(hipMemsetAsync(s->fe_part.p, 0, fe_bytes, s->stream));
   HIPC(hipStreamSynchronize(s->stream));
   TRY(s->d_spec.alloc(sizeof(SpecDesc) * kMaxSpecies));
   TRY(s->d_fd.alloc(sizeof(FieldDesc)));
@@ -1382,12 +1439,14 @@ int osr_sim_create(const osr_sim_desc* desc, osr_sim** out) {
     std::vector<int2> yw((size_t)s->nblk);
     for (int b = 0; b < s->nblk; b++) yw[b] = make_int2(0, b);
     TRY(copy_on(s->stream, s->d_ywork.p, yw.data(), sizeof(int2) * yw.size(), hipMemcpyHostToDevice));
-    std::vector<int2> ew(yw.begin(), yw.begin() + s->nblk_e);
+    std::vector<int2> ew;
+    for (int b = 0; b < s->nblk_e; b++) ew.push_back(make_int2(0, b));
     for (int b = 0; b < nwall_e; b++) ew.push_back(make_int2(0, -1 - b));
     TRY(copy_on(s->stream, s->d_ework.p, ew.data(), sizeof(int2) * ew.size(), hipMemcpyHostToDevice));
     std::vector<int2> dw;
     for (int c = 0; c < kRedCols; c++) dw.push_back(make_int2(0, -1 - c));
-    dw.insert(dw.end(), yw.begin(), yw.end());
+    const std::vector<int2>& cells = g.pp ? ew : yw;  // tiles of yee2d_step, or blocks
+    dw.insert(dw.end(), cells.begin(), cells.end());
     TRY(s->d_dwork.alloc(sizeof(int2) * dw.size()));
     TRY(copy_on(s->stream, s->d_dwork.p, dw.data(), sizeof(int2) * dw.size(), hipMemcpyHostToDevice));
     int z = 0;
@@ -1565,9 +1624,10 @@ int osr_species_generate(osr_sim* s, int sid, const int* ppc, double density,
   return OSR_OK;
 }
 
-// open x walls: the wall values of the buffers, as the reference's boundary update puts
+// After the host changed the fields.  Open x walls: the wall values of the buffers, as the reference's boundary update puts
 // them before every push (also after the host changed the fields)
-static int restore_walls(osr_sim* s) {
+static int fields_changed(osr_sim* s) {
+  s->fe_stale = true;
   if (!s->g.open_nx) return OSR_OK;
   TRY(launch_wall_restore(s));
   HIPC(hipStreamSynchronize(s->stream));
@@ -1586,8 +1646,8 @@ static int fields_xfer(osr_sim* s, float* e, float* b, const int* ld, const int*
   std::vector<float> pe(3 * nc), pb(3 * nc);
   if (set && s->g.open_nx) {  // the guard band keeps its values
     HIPC(hipStreamSynchronize(s->stream));
-    TRY(copy_on(s->stream, pe.data(), s->E.p, 12 * nc, hipMemcpyDeviceToHost));
-    TRY(copy_on(s->stream, pb.data(), s->B.p, 12 * nc, hipMemcpyDeviceToHost));
+    TRY(copy_on(s->stream, pe.data(), cur_E(s), 12 * nc, hipMemcpyDeviceToHost));
+    TRY(copy_on(s->stream, pb.data(), cur_B(s), 12 * nc, hipMemcpyDeviceToHost));
   }
   const long ld0 = ld[0], ld1 = ld[1];
   auto ref = [&](int i, int j, int k) -> size_t {
@@ -1607,13 +1667,13 @@ static int fields_xfer(osr_sim* s, float* e, float* b, const int* ld, const int*
           }
         }
     HIPC(hipStreamSynchronize(s->stream));
-    if (e) TRY(copy_on(s->stream, s->E.p, pe.data(), 12 * nc, hipMemcpyHostToDevice));
-    if (b) TRY(copy_on(s->stream, s->B.p, pb.data(), 12 * nc, hipMemcpyHostToDevice));
-    return restore_walls(s);
+    if (e) TRY(copy_on(s->stream, cur_E(s), pe.data(), 12 * nc, hipMemcpyHostToDevice));
+    if (b) TRY(copy_on(s->stream, cur_B(s), pb.data(), 12 * nc, hipMemcpyHostToDevice));
+    return fields_changed(s);
   }
   HIPC(hipStreamSynchronize(s->stream));
-  TRY(copy_on(s->stream, pe.data(), s->E.p, 12 * nc, hipMemcpyDeviceToHost));
-  TRY(copy_on(s->stream, pb.data(), s->B.p, 12 * nc, hipMemcpyDeviceToHost));
+  TRY(copy_on(s->stream, pe.data(), cur_E(s), 12 * nc, hipMemcpyDeviceToHost));
+  TRY(copy_on(s->stream, pb.data(), cur_B(s), 12 * nc, hipMemcpyDeviceToHost));
   // every array cell (guards included) gets its periodic image; with open x walls the x
   // guard cells come from the guard band of the ring
   const int ldk = D == 3 ? ld[2] : 1;
@@ -1654,9 +1714,9 @@ int osr_fields_fill(osr_sim* s, const double* e0, const double* b0) {
     const double* f = w == 0 ? e0 : b0;
     if (!f) continue;
     for (int m = 0; m < 3; m++) std::fill(v.begin() + m * nc, v.begin() + (m + 1) * nc, (float)f[m]);
-    TRY(copy_on(s->stream, w == 0 ? s->E.p : s->B.p, v.data(), 12 * nc, hipMemcpyHostToDevice));
+    TRY(copy_on(s->stream, w == 0 ? cur_E(s) : cur_B(s), v.data(), 12 * nc, hipMemcpyHostToDevice));
   }
-  return restore_walls(s);
+  return fields_changed(s);
 }
 
 // particles left after absorbing walls removed some: the sum of the tile counts
@@ -1677,6 +1737,7 @@ int osr_sim_run(osr_sim* s, int nsteps) {
   if (nsteps == 0) return OSR_OK;
   TRY(ensure_hist(s, s->steps + nsteps));
   if (!s->graph_ok) TRY(build_graph(s));
+  TRY(refresh_energy(s));
   int64_t left = nsteps;
   int batch = 8;
   while (left > 0) {
@@ -1690,6 +1751,7 @@ int osr_sim_run(osr_sim* s, int nsteps) {
     for (; i < nb; i++) HIPC(hipGraphLaunch(s->gexec, s->stream));
     Ctrl c;
     TRY(read_ctrl(s, c));
+    s->par = c.par;
     if (c.error & 1) return fail(OSR_ERR_LAYOUT, "particle found outside its tile");
     if (c.error) return fail(OSR_ERR_STATE, "mover lists exceed the tile fill tables");
     const int64_t done = c.steps - s->steps;
@@ -1762,8 +1824,8 @@ int osr_sim_save_field(osr_sim* s, int quant, const char* ms_dir, const double* 
   const size_t nc = (size_t)s->g.ncell;
   std::vector<float> v(nc);
   HIPC(hipStreamSynchronize(s->stream));
-  const DBuf& src = quant < 3 ? s->E : s->B;
-  TRY(copy_on(s->stream, v.data(), src.as<float>() + (size_t)(quant % 3) * nc, 4 * nc,
+  const float* src = quant < 3 ? cur_E(s) : cur_B(s);
+  TRY(copy_on(s->stream, v.data(), src + (size_t)(quant % 3) * nc, 4 * nc,
                  hipMemcpyDeviceToHost));
   if (s->g.open_nx) {  // interior columns of the x ring only
     const int nxi = s->g.open_nx, nxr = s->g.nx;
@@ -1817,7 +1879,7 @@ int osr_sim_gauss(osr_sim* s, double* res, double* rho_out, double* maxabs) {
     HIPC(hipGetLastError());
   }
   hipLaunchKernelGGL(gauss_residual, dim3((unsigned)((nc + 255) / 256)), dim3(256), 0, s->stream,
-                     s->g, rho.as<unsigned long long>(), 1.0 / scale, 1.0 / s->dx[0],
+                     cur_grid(s), rho.as<unsigned long long>(), 1.0 / scale, 1.0 / s->dx[0],
                      1.0 / s->dx[1], s->dims == 3 ? 1.0 / s->dx[2] : 0.0, dres.as<double>());
   HIPC(hipGetLastError());
   std::vector<double> h(nc);
@@ -1858,10 +1920,10 @@ int osr_sim_init_fields(osr_sim* s, int sid, float ufl1) {
                      s->d_work.as<int2>() + (size_t)sid * s->ntiles, rho.as<unsigned long long>(),
                      scale);
   const unsigned nb = (unsigned)((nt + 255) / 256);
-  hipLaunchKernelGGL(es_charge, dim3(nb), dim3(256), 0, s->stream, s->g,
+  hipLaunchKernelGGL(es_charge, dim3(nb), dim3(256), 0, s->stream, cur_grid(s),
                      rho.as<unsigned long long>(), 1.0 / scale, charge.as<double>());
   if (ufl1 == 0.0f) {  // es_solver
-    hipLaunchKernelGGL(es_direct_2d, dim3(nb), dim3(256), 0, s->stream, s->g, charge.as<double>(),
+    hipLaunchKernelGGL(es_direct_2d, dim3(nb), dim3(256), 0, s->stream, cur_grid(s), charge.as<double>(),
                        s->dx[0], s->dx[1], s->dx[0] * s->dx[1]);
   } else if (s->dims == 3) {  // es_solver_3d_beam
     const float u1sq = ufl1 * ufl1;
@@ -1871,9 +1933,9 @@ int osr_sim_init_fields(osr_sim* s, int sid, float ufl1) {
     TRY(e23u.alloc(8 * (size_t)nt));
     const long long ns = (long long)s->g.ny * s->g.nz;
     hipLaunchKernelGGL(es_beam3d_e, dim3((unsigned)((ns + 255) / 256), (unsigned)interior_nx(s->g)),
-                       dim3(256), 0, s->stream, s->g, charge.as<double>(), cn, s->dx[1], s->dx[2],
+                       dim3(256), 0, s->stream, cur_grid(s), charge.as<double>(), cn, s->dx[1], s->dx[2],
                        e23u.as<float>());
-    hipLaunchKernelGGL(es_beam3d_apply, dim3(nb), dim3(256), 0, s->stream, s->g, e23u.as<float>(),
+    hipLaunchKernelGGL(es_beam3d_apply, dim3(nb), dim3(256), 0, s->stream, cur_grid(s), e23u.as<float>(),
                        ufl1, gamma);
     HIPC(hipGetLastError());
     HIPC(hipStreamSynchronize(s->stream));
@@ -1883,15 +1945,16 @@ int osr_sim_init_fields(osr_sim* s, int sid, float ufl1) {
     const double cn = s->dx[1] / gamma / 2;
     DBuf e2u;
     TRY(e2u.alloc(4 * (size_t)nt));
-    hipLaunchKernelGGL(es_beam_e2, dim3(nb), dim3(256), 0, s->stream, s->g, charge.as<double>(),
+    hipLaunchKernelGGL(es_beam_e2, dim3(nb), dim3(256), 0, s->stream, cur_grid(s), charge.as<double>(),
                        cn, e2u.as<float>());
-    hipLaunchKernelGGL(es_beam_apply, dim3(nb), dim3(256), 0, s->stream, s->g, e2u.as<float>(),
+    hipLaunchKernelGGL(es_beam_apply, dim3(nb), dim3(256), 0, s->stream, cur_grid(s), e2u.as<float>(),
                        ufl1, gamma);
     HIPC(hipGetLastError());
     HIPC(hipStreamSynchronize(s->stream));
   }
   HIPC(hipGetLastError());
   HIPC(hipStreamSynchronize(s->stream));
+  s->fe_stale = true;
   return OSR_OK;
 }
 
@@ -1940,6 +2003,7 @@ int osr_sim_time_kernels(osr_sim* s, int nsteps, double* ms) {
   for (int i = 0; i < nev; i++) HIPC(hipEventCreate(&ev[i]));
   double acc[6] = {0, 0, 0, 0, 0, 0};
   int done = 0;
+  TRY(refresh_energy(s));
   for (int k = 0; k < nsteps; k++) {
     if (!s->zp.empty()) {  // the laser walls of the step, not timed
       TRY(zp_fill(s, s->steps, 1));
@@ -1964,6 +2028,7 @@ int osr_sim_time_kernels(osr_sim* s, int nsteps, double* ms) {
     HIPC(hipEventSynchronize(ev[4]));
     Ctrl c;
     TRY(read_ctrl(s, c));
+    s->par = c.par;
     if (c.error & 1) return fail(OSR_ERR_LAYOUT, "particle found outside its tile");
     if (c.error) return fail(OSR_ERR_STATE, "mover lists exceed the tile fill tables");
     s->steps = c.steps;
@@ -2587,8 +2652,8 @@ int osr_sim_add_zpulse(osr_sim* s, const osr_zpulse* zp) {
   const size_t nc = (size_t)s->g.ncell, gn = g.cells();
   std::vector<float> pe(3 * nc), pb(3 * nc), eb(3 * gn), bb(3 * gn);
   HIPC(hipStreamSynchronize(s->stream));
-  TRY(copy_on(s->stream, pe.data(), s->E.p, 12 * nc, hipMemcpyDeviceToHost));
-  TRY(copy_on(s->stream, pb.data(), s->B.p, 12 * nc, hipMemcpyDeviceToHost));
+  TRY(copy_on(s->stream, pe.data(), cur_E(s), 12 * nc, hipMemcpyDeviceToHost));
+  TRY(copy_on(s->stream, pb.data(), cur_B(s), 12 * nc, hipMemcpyDeviceToHost));
   const int ring = s->g.nx;
   double phase0 = w.phase0, pol = w.pol;
   for (int k = 0; k < (w.pol_type != 0 ? 2 : 1); k++) {
@@ -2621,9 +2686,9 @@ int osr_sim_add_zpulse(osr_sim* s, const osr_zpulse* zp) {
           }
         }
   }
-  TRY(copy_on(s->stream, s->E.p, pe.data(), 12 * nc, hipMemcpyHostToDevice));
-  TRY(copy_on(s->stream, s->B.p, pb.data(), 12 * nc, hipMemcpyHostToDevice));
-  return restore_walls(s);
+  TRY(copy_on(s->stream, cur_E(s), pe.data(), 12 * nc, hipMemcpyHostToDevice));
+  TRY(copy_on(s->stream, cur_B(s), pb.data(), 12 * nc, hipMemcpyHostToDevice));
+  return fields_changed(s);
 }
 
 int osr_sim_zpulse_column(osr_sim* s, int k, int second, double t, float* b12, float* b3,

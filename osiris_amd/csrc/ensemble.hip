@@ -34,7 +34,7 @@ struct EnsJob {
 };
 
 struct EnsBatch {
-  int dims = 2, order = 2, tile[3] = {1, 1, 1}, kernel = 0, waves = 4;
+  int dims = 2, order = 2, tile[3] = {1, 1, 1}, kernel = 0, waves = 4, yv = 0;
   hipStream_t stream = nullptr;
   hipEvent_t ev = nullptr;
   std::vector<EnsJob*> jobs;     // jobs stepped by the graph
@@ -82,7 +82,7 @@ int64_t job_footprint(const osr_job_desc& j) {
   }
   const int64_t ntiles = (int64_t)nt[0] * nt[1] * nt[2];
   const int64_t nblk = (nc + 255) / 256;
-  int64_t b = nc * (12 + 12 + 24) + nblk * (48 + 8);
+  int64_t b = nc * (12 + 12 + 24) * (D == 2 ? 2 : 1) + nblk * (2 * 48 + 8);
   const int64_t rows = std::max<int64_t>(j.nsteps, 1024);
   b += rows * (6 + j.nspecies) * 8;
   const int64_t slot = D == 2 ? 68 : 76;
@@ -166,6 +166,8 @@ int ens_admit(osr_ensemble* e, EnsJob* j) {
       jd.b0[2] != 0)
     TRY(osr_fields_fill(s, jd.e0, jd.b0));
   TRY(ensure_hist(s, jd.nsteps));
+  TRY(refresh_energy(s));
+  HIPC(hipStreamSynchronize(s->stream));  // the batch runs on another stream
   Ctrl c{};
   c.target = jd.nsteps;
   TRY(copy_on(s->stream, s->ctrl.p, &c, sizeof(Ctrl), hipMemcpyHostToDevice));
@@ -186,7 +188,7 @@ int ens_admit(osr_ensemble* e, EnsJob* j) {
   for (auto& bb : e->batches)
     if (bb->dims == s->dims && bb->order == s->order && bb->tile[0] == s->g.tx &&
         bb->tile[1] == s->g.ty && bb->tile[2] == s->g.tz && bb->kernel == jd.sim.kernel &&
-        bb->waves == s->push_waves) {
+        bb->waves == s->push_waves && bb->yv == s->yv) {
       b = bb.get();
       break;
     }
@@ -199,6 +201,7 @@ int ens_admit(osr_ensemble* e, EnsJob* j) {
     nb->tile[2] = s->g.tz;
     nb->kernel = jd.sim.kernel;
     nb->waves = s->push_waves;
+    nb->yv = s->yv;
     nb->lds = s->lds_push;
     HIPC(hipStreamCreateWithFlags(&nb->stream, hipStreamNonBlocking));
     HIPC(hipEventCreateWithFlags(&nb->ev, hipEventDisableTiming));
@@ -247,7 +250,10 @@ int ens_build(osr_ensemble* e, EnsBatch* b) {
           wp[s->sp[i]->pusher == OSR_VAY ? 1 : 0].insert(
               wp[s->sp[i]->pusher == OSR_VAY ? 1 : 0].end(), sp, make_int2(spec0[k] + (int)i, t));
     }
-  wd.insert(wd.end(), wy.begin(), wy.end());  // the E step: history columns, then cell blocks
+  // the launch with the history columns: these, then yee2d_step's tiles (2D) or the E step's
+  // cell blocks
+  const std::vector<int2>& cells = b->dims == 2 ? we : wy;
+  wd.insert(wd.end(), cells.begin(), cells.end());
   auto put = [&](DBuf& d, const void* src, size_t bytes) -> int {
     if (bytes == 0) return OSR_OK;
     if (d.n < bytes) TRY(d.alloc(bytes + bytes / 2));
@@ -309,9 +315,8 @@ int ens_build(osr_ensemble* e, EnsBatch* b) {
     const int2* we = b->wene.as<int2>();
     const int2* wd = b->wded.as<int2>();
     if (b->dims == 2) {
-      hipLaunchKernelGGL((yee_dbdt<2, true>), dim3(b->nene), dim3(256), 0, b->stream, fd, we);
-      hipLaunchKernelGGL((yee_dedt<2>), dim3(b->nded), dim3(256), 0, b->stream, fd, wd);
-      hipLaunchKernelGGL((yee_dbdt<2, false>), dim3(b->nyee), dim3(256), 0, b->stream, fd, w);
+      hipLaunchKernelGGL(pick_yee2d(b->yv), dim3(b->nded), dim3(256),
+                         0, b->stream, fd, wd, 0);
     } else {
       hipLaunchKernelGGL((yee_dbdt<3, true>), dim3(b->nene), dim3(256), 0, b->stream, fd, we);
       hipLaunchKernelGGL((yee_dedt<3>), dim3(b->nded), dim3(256), 0, b->stream, fd, wd);
@@ -356,6 +361,7 @@ int ens_collect(osr_ensemble* e, EnsBatch* b) {
     osr_sim* s = j->sim;
     j->steps = c.steps;
     s->steps = c.steps;
+    s->par = c.par;
     if (c.error) {
       ens_fail_job(e, j);
       b->dirty = true;

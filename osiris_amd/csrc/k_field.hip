@@ -18,8 +18,10 @@ namespace osr {
 
 struct FieldDesc {
   GridDesc g;
-  double* fe_part;   // [6][nblk] partial sums of squares of B1, B2, B3, E1, E2, E3
-  int nblk;          // energy partials: one per kEneBlk blocks of 256 cells
+  double* fe_part;   // [6][nblk] partial sums of squares of B1, B2, B3, E1, E2, E3; two such
+                     // arrays when the grid holds two copies (GridDesc::pp), one per copy
+  int nblk;          // energy partials: one per kEneBlk blocks of 256 cells, or one per
+                     // tile of yee2d_step
   // finalisation
   int nspec;
   double* ep[kMaxSpecies];  // per-species tile energy partials
@@ -290,6 +292,220 @@ __global__ __launch_bounds__(256) void yee_dedt(const FieldDesc* __restrict__ fd
   E1[idx] = e1;
   E2[idx] = e2;
   E3[idx] = e3;
+}
+
+// ------------------------------------------------------------------------------------
+// The whole 2D periodic field step in one launch: B half step, E step, B half step, with
+// the arithmetic of yee_dbdt<2> and yee_dedt<2> operation for operation.  A workgroup owns a
+// tile of TX x TY cells, stages E on the tile plus (1, 2) cells and B plus (1, 1), and
+// recomputes the half-step B and the new E on the halo its own cells need.  Neighbouring
+// workgroups still read the old values, so the results go to the other copy of E and B
+// (GridDesc::pp), and the J it clears is the one the next step deposits into.
+// Bound: HBM on large grids, the launch and its chain of loads and barriers on small ones.
+// E, B, J are read once, E, B written, J cleared: 96 B per cell (the halo comes from L2)
+// against 180 B for the three launches, which read B three times and E twice: 1024x1024
+// 45 -> 34 us (2.9 TB/s), 128x128 14.7 -> 6.1 us, 64x64 13.6 -> 5.8 us.
+// It also leaves the energy of the new fields per tile for the next step's history row (the
+// row's fields are those its push starts from); the sums of this step's row are work items
+// of this launch (wk.y < 0).
+// ------------------------------------------------------------------------------------
+// block sums of the six field components into the energy partials `out` of one tile
+OSR_DEV void tile_energy(const double (&acc)[6], double* out, int nblk, int tile) {
+  __shared__ double s_red[4][6];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int c = 0; c < 6; c++) {
+    const double v = wave_sum(acc[c]);
+    if (lane == 0) s_red[wave][c] = v;
+  }
+  __syncthreads();
+  if (threadIdx.x < 6) {
+    const int c = threadIdx.x;
+    out[(long long)c * nblk + tile] = ((s_red[0][c] + s_red[1][c]) + s_red[2][c]) + s_red[3][c];
+  }
+}
+
+OSR_DEV int wrap_any(int i, int n) {
+  while (i < 0) i += n;
+  while (i >= n) i -= n;
+  return i;
+}
+
+// The staged cells of a yee2d tile: -1 .. T + 1 in each direction, item q of a thread is
+// cell threadIdx.x + 256 q of them in row order.
+template <int TX, int TY>
+struct YeeTile {
+  static constexpr int EX = TX + 3, EY = TY + 3, EN = EX * EY, Q = (EN + 255) / 256;
+  int x0, y0;
+  OSR_DEV YeeTile(int tile, int nx) {
+    const int ntx = (nx + TX - 1) / TX;
+    x0 = (tile % ntx) * TX;
+    y0 = (tile / ntx) * TY;
+  }
+  // global cell of staged cell i (the last one again beyond the end)
+  OSR_DEV long long cell(int i, int nx, int ny) const {
+    const int k = i < EN ? i : EN - 1;
+    return wrap_any(x0 - 1 + k % EX, nx) + (long long)nx * wrap_any(y0 - 1 + k / EX, ny);
+  }
+  // staged cell i lies in lo .. T - 1 + hi in both directions
+  OSR_DEV static bool in(int i, int lo, int hi) {
+    const int cx = i % EX, cy = i / EX;
+    return i < EN && cx >= 1 + lo && cx <= TX + hi && cy >= 1 + lo && cy <= TY + hi;
+  }
+  // and is a cell of the tile inside the grid
+  OSR_DEV bool own(int i, int nx, int ny) const {
+    return in(i, 0, 0) && x0 - 1 + i % EX < nx && y0 - 1 + i / EX < ny;
+  }
+};
+
+template <int TX, int TY>
+__global__ __launch_bounds__(256) void yee2d_step(const FieldDesc* __restrict__ fds,
+                                                  const int2* __restrict__ work, int) {
+  using T = YeeTile<TX, TY>;
+  constexpr int EX = T::EX, EN = T::EN, Q = T::Q;
+  __shared__ float sE[3][EN], sB[3][EN];
+  const int2 wk = work[blockIdx.x];
+  const FieldDesc& fd = fds[wk.x];
+  const GridDesc& g = fd.g;
+  if (wk.y < 0) {
+    reduce_column(fd, -1 - wk.y);
+    return;
+  }
+  const int halt = g.ctrl->halt;
+  const unsigned par = g.ctrl->par;
+  if (halt >= 2) return;
+  const int nx = g.nx, ny = g.ny, tid = threadIdx.x;
+  const long long nc = g.ncell;
+  const long long in = (long long)par * 3 * nc, out = (long long)(par ^ 1u) * 3 * nc;
+  const T tile(wk.y, nx);
+  const float* __restrict__ Ei = g.E + in;
+  const float* __restrict__ Bi = g.B + in;
+  // every load of the thread is issued before its first use (cells of the halo whose B or J
+  // is not needed included: no branches between the loads)
+  float e[Q][3], b[Q][3], jv[Q][3];
+  long long c[Q];
+#pragma unroll
+  for (int q = 0; q < Q; q++) c[q] = tile.cell(tid + 256 * q, nx, ny);
+#pragma unroll
+  for (int q = 0; q < Q; q++)
+#pragma unroll
+    for (int m = 0; m < 3; m++) e[q][m] = Ei[m * nc + c[q]];
+#pragma unroll
+  for (int q = 0; q < Q; q++)
+#pragma unroll
+    for (int m = 0; m < 3; m++) b[q][m] = Bi[m * nc + c[q]];
+  if (fd.Jf) {
+    const float* __restrict__ Jf = fd.Jf;
+#pragma unroll
+    for (int q = 0; q < Q; q++)
+#pragma unroll
+      for (int m = 0; m < 3; m++) jv[q][m] = Jf[m * nc + c[q]];
+  } else {
+    const unsigned long long* __restrict__ Ji = g.J + in;
+    const double jinv = g.jinv;
+    long long v[Q][3];
+#pragma unroll
+    for (int q = 0; q < Q; q++)
+#pragma unroll
+      for (int m = 0; m < 3; m++) v[q][m] = (long long)Ji[m * nc + c[q]];
+#pragma unroll
+    for (int q = 0; q < Q; q++)
+#pragma unroll
+      for (int m = 0; m < 3; m++) jv[q][m] = (float)((double)v[q][m] * jinv);
+  }
+#pragma unroll
+  for (int q = 0; q < Q; q++) {
+    const int i = tid + 256 * q;
+    if (i < EN)
+#pragma unroll
+      for (int m = 0; m < 3; m++) sE[m][i] = e[q][m];
+  }
+  __syncthreads();
+  const float h1 = fd.bdt[0], h2 = fd.bdt[1];
+  auto half_b = [&](int i, const float* ev, float* bv) {
+    const float n1 = bv[0] - h2 * (sE[2][i + EX] - ev[2]);
+    const float n2 = bv[1] + h1 * (sE[2][i + 1] - ev[2]);
+    const float n3 = bv[2] - h1 * (sE[1][i + 1] - ev[1]) + h2 * (sE[0][i + EX] - ev[0]);
+    bv[0] = n1;
+    bv[1] = n2;
+    bv[2] = n3;
+  };
+#pragma unroll
+  for (int q = 0; q < Q; q++) {
+    const int i = tid + 256 * q;
+    if (T::in(i, -1, 1)) {
+      half_b(i, e[q], b[q]);
+#pragma unroll
+      for (int m = 0; m < 3; m++) sB[m][i] = b[q][m];
+    }
+  }
+  __syncthreads();
+  const float d1 = fd.edt[0], d2 = fd.edt[1], dtif = fd.dtif;
+#pragma unroll
+  for (int q = 0; q < Q; q++) {
+    const int i = tid + 256 * q;
+    if (T::in(i, 0, 1)) {
+      const float b1 = b[q][0], b2 = b[q][1], b3 = b[q][2];
+      e[q][0] = e[q][0] - dtif * jv[q][0] + d2 * (b3 - sB[2][i - EX]);
+      e[q][1] = e[q][1] - dtif * jv[q][1] - d1 * (b3 - sB[2][i - 1]);
+      e[q][2] = e[q][2] - dtif * jv[q][2] + d1 * (b2 - sB[1][i - 1]) - d2 * (b1 - sB[0][i - EX]);
+      // the old E was last read before the barrier
+#pragma unroll
+      for (int m = 0; m < 3; m++) sE[m][i] = e[q][m];
+    }
+  }
+  __syncthreads();
+  double acc[6] = {0, 0, 0, 0, 0, 0};
+  float* __restrict__ Eo = g.E + out;
+  float* __restrict__ Bo = g.B + out;
+  unsigned long long* __restrict__ Jo = g.J + out;
+#pragma unroll
+  for (int q = 0; q < Q; q++) {
+    const int i = tid + 256 * q;
+    if (tile.own(i, nx, ny)) {
+      half_b(i, e[q], b[q]);
+#pragma unroll
+      for (int m = 0; m < 3; m++) {
+        Eo[m * nc + c[q]] = e[q][m];
+        Bo[m * nc + c[q]] = b[q][m];
+        Jo[m * nc + c[q]] = 0ull;
+        acc[m] += (double)b[q][m] * b[q][m];
+        acc[3 + m] += (double)e[q][m] * e[q][m];
+      }
+    }
+  }
+  tile_energy(acc, fd.fe_part + (long long)(par ^ 1u) * 6 * fd.nblk, fd.nblk, wk.y);
+}
+
+// The energy partials of the current copy, as yee2d_step leaves them (same cells per thread,
+// same sums): run when the host changed the fields, before the next step.
+template <int TX, int TY>
+__global__ __launch_bounds__(256) void yee2d_energy(const FieldDesc* __restrict__ fds,
+                                                    const int2* __restrict__ work, int) {
+  using T = YeeTile<TX, TY>;
+  const int2 wk = work[blockIdx.x];
+  const FieldDesc& fd = fds[wk.x];
+  const GridDesc& g = fd.g;
+  const int nx = g.nx, ny = g.ny;
+  const long long nc = g.ncell;
+  const T tile(wk.y, nx);
+  const float* __restrict__ E = g.E + cur_copy(g);
+  const float* __restrict__ B = g.B + cur_copy(g);
+  double acc[6] = {0, 0, 0, 0, 0, 0};
+#pragma unroll
+  for (int q = 0; q < T::Q; q++) {
+    const int i = threadIdx.x + 256 * q;
+    if (tile.own(i, nx, ny)) {
+      const long long c = tile.cell(i, nx, ny);
+#pragma unroll
+      for (int m = 0; m < 3; m++) {
+        const float vb = B[m * nc + c], ve = E[m * nc + c];
+        acc[m] += (double)vb * vb;
+        acc[3 + m] += (double)ve * ve;
+      }
+    }
+  }
+  tile_energy(acc, fd.fe_part + (long long)g.ctrl->par * 6 * fd.nblk, fd.nblk, wk.y);
 }
 
 // ------------------------------------------------------------------------------------
@@ -680,7 +896,9 @@ OSR_DEV void reduce_column(const FieldDesc& fd, int col) {
   if (col >= 6 + fd.nspec) return;
   const int halt = fd.g.ctrl->halt;
   const long long step = fd.g.ctrl->steps;
-  const double* __restrict__ p = col < 6 ? fd.fe_part + (long long)col * fd.nblk : fd.ep[col - 6];
+  const long long fe0 = fd.g.pp ? (long long)fd.g.ctrl->par * 6 * fd.nblk : 0;
+  const double* __restrict__ p =
+      col < 6 ? fd.fe_part + fe0 + (long long)col * fd.nblk : fd.ep[col - 6];
   const int n = col < 6 ? fd.nblk : fd.ep_n[col - 6];
   double s = 0.0, c = 0.0;
   for (int b0 = threadIdx.x; b0 < n; b0 += kRedNT * U) {
@@ -715,6 +933,7 @@ OSR_DEV void end_step(const GridDesc& g) {
   const long long step = ctrl->steps, target = ctrl->target;
   if (halt >= 2) return;
   ctrl->steps = step + 1;
+  if (g.pp) ctrl->par ^= 1u;
   if (halt == 1)
     ctrl->halt = 2;
   else if (target > 0 && step + 1 >= target)
@@ -1037,6 +1256,10 @@ template __global__ void yee_dbdt<2, false>(const FieldDesc*, const int2*);
 template __global__ void yee_dbdt<3, true>(const FieldDesc*, const int2*);
 template __global__ void yee_dbdt<3, false>(const FieldDesc*, const int2*);
 template __global__ void yee_dedt<2>(const FieldDesc*, const int2*);
+template __global__ void yee2d_step<32, 8>(const FieldDesc*, const int2*, int);
+template __global__ void yee2d_step<64, 16>(const FieldDesc*, const int2*, int);
+template __global__ void yee2d_energy<32, 8>(const FieldDesc*, const int2*, int);
+template __global__ void yee2d_energy<64, 16>(const FieldDesc*, const int2*, int);
 template __global__ void wall_b2_end<2>(const FieldDesc*);
 template __global__ void wall_b2_end<3>(const FieldDesc*);
 template __global__ void vpml_update<0, 2>(const FieldDesc*);

@@ -78,11 +78,11 @@ __global__ __launch_bounds__(64 * NW, 4) void push_deposit_2d_t(const SpecDesc* 
   const int tile = wk.y;
   const int cx0 = (tile % g.ntx) * TX, cy0 = (tile / g.ntx) * TY;
   const int nx = g.nx, ny = g.ny;
-  const long long nc = g.ncell;
+  const long long nc = g.ncell, co = cur_copy(g);
 
   {
-    const gf32* __restrict__ E = (const gf32*)g.E;
-    const gf32* __restrict__ B = (const gf32*)g.B;
+    const gf32* __restrict__ E = (const gf32*)g.E + co;
+    const gf32* __restrict__ B = (const gf32*)g.B + co;
     for (int i = threadIdx.x; i < GX * GY; i += NT) {
       const int col = i % GX, row = i / GX, li = row * GS + col;
       const int gx = wrapi(cx0 + col - O::GLO, nx), gy = wrapi(cy0 + row - O::GLO, ny);
@@ -318,7 +318,7 @@ __global__ __launch_bounds__(64 * NW, 4) void push_deposit_2d_t(const SpecDesc* 
     d.epart[tile * split + part] = t;
   }
   // ---- fold the LDS current tile into the global fixed-point J (periodic wrap)
-  gu64* __restrict__ GJ = (gu64*)g.J;
+  gu64* __restrict__ GJ = (gu64*)g.J + co;
   for (int i = threadIdx.x; i < JX * JY; i += NT) {
     const int col = i % JX, row = i / JX, li = row * JS + col;
     const int gx = wrapi(cx0 + col - O::JLO, nx), gy = wrapi(cy0 + row - O::JLO, ny);

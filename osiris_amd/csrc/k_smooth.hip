@@ -58,7 +58,7 @@ __global__ __launch_bounds__(256) void smooth_pass(const FieldDesc* __restrict__
   }
   const long long row = idx - (long long)c * st;  // the line's first cell
   const int src = pass == 0 ? fd.sm_src : 2;
-  const unsigned long long* Jq = g.J;
+  const unsigned long long* Jq = g.J + cur_copy(g);
   const float* Jp = (const float*)g.J;
   const float* P = fd.sm_buf[(pass + 1) & 1];  // previous pass's output
   float* dst = fd.sm_buf[pass & 1];

@@ -9,6 +9,7 @@
 //                   columns, reached by the same index wrap from column 0, the lower
 //                   guard cells x = 0, -1, ... (1-based cell indices of the reference);
 //   current  J    : int64 fixed point, planar [3][nz][ny][nx]; the value is J * 2^jshift;
+//                   periodic 2D grids hold two copies of E, B and J (GridDesc::pp);
 //   particles     : structure of arrays, grouped by tile.  Tile t owns the slots
 //                   [off[t], off[t]+cap[t]) of every array and its first cnt[t] slots hold
 //                   particles whose cell lies inside the tile.  A particle is
@@ -75,7 +76,7 @@ struct Ctrl {
   long long target;  // park (halt = 3) once steps reaches target; 0 = no target
   unsigned done;     // workgroups of a step-ending kernel that have finished (the last one
                      // ends the step and sets it back to 0)
-  unsigned pad;
+  unsigned par;      // current copy of the fields and the current (GridDesc::pp)
 };
 
 struct GridDesc {
@@ -89,6 +90,8 @@ struct GridDesc {
   float* E;
   float* B;
   unsigned long long* J;
+  int pp;            // E, B and J hold two copies, 3 ncell values apart: the step reads those
+                     // of Ctrl::par, writes E and B of the other and clears its J
   double jscale;     // 2^jshift
   double jinv;       // 2^-jshift
   float dt_dx[3];    // (float)(dt/dx)
@@ -96,6 +99,11 @@ struct GridDesc {
   Ctrl* ctrl;
   FastDiv div_nx, div_ny;  // cell index c -> x = c mod nx, row c / nx; row -> y, z
 };
+
+// values from the start of E, B or J to the copy the step reads
+__device__ inline long long cur_copy(const GridDesc& g) {
+  return g.pp ? (long long)g.ctrl->par * 3 * g.ncell : 0;
+}
 
 // the divisors of a grid whose extents are set (host)
 __host__ inline void set_grid_divisors(GridDesc& g) {
