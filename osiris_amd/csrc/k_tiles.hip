@@ -21,6 +21,8 @@
 // 2691-2905 (split + DEP_CURRENT), simd/os-spec-push-avx2.c:471-760 (fused SIMD kernel),
 // particles/os-particles.f03:1416-1443 (private J + reduce), spec/os-species.f03:269-441
 // (counting sort of particles by cell).
+#include <type_traits>
+
 #include "osr_device.hpp"
 #include "osr_types.hpp"
 
@@ -32,29 +34,9 @@ OSR_DEV int wrapi(int i, int n) {
   return i;
 }
 
-// Exclusive rank of `flag` among the threads of the block in thread order, and the total.
-// Uses wave ballots and one LDS exchange; all threads must call it.
-template <int NT>
-OSR_DEV int block_rank(bool flag, int* s_wtot, int& total) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  unsigned long long m = __ballot(flag);
-  int r = __popcll(m & ((1ull << lane) - 1ull));
-  if (lane == 0) s_wtot[wave] = __popcll(m);
-  __syncthreads();
-  int before = 0;
-  total = 0;
-  for (int w = 0; w < NT / 64; w++) {
-    int c = s_wtot[w];
-    if (w < wave) before += c;
-    total += c;
-  }
-  __syncthreads();
-  return before + r;
-}
-
-// block_rank for PF flags per thread at once, ranked in the order (p, thread): item p of
-// thread t comes after every item p' < p and after item p of the threads below t.  One
-// LDS exchange (two barriers) for all PF; all threads must call it.
+// Exclusive ranks of PF flags per thread in the order (p, thread), and their total: item p
+// of thread t comes after every item p' < p and after item p of the threads below t.  Wave
+// ballots and one LDS exchange (two barriers) for all PF; all threads must call it.
 template <int NT, int PF>
 OSR_DEV void block_rank_multi(const bool (&flag)[PF], int (*s_cnt)[NT / 64], int (&rank)[PF],
                               int& total) {
@@ -546,33 +528,20 @@ __global__ __launch_bounds__(NT) void push_deposit_3d(const SpecDesc* __restrict
 // ------------------------------------------------------------------------------------
 // Tile maintenance
 // ------------------------------------------------------------------------------------
-// Distinct neighbour tiles of `tile` (excluding itself) in a fixed order.
-OSR_DEV int neighbours(const GridDesc& g, int tile, int* nb) {
-  int tx, ty, tz;
+// k-th neighbour tile (dz, dy, dx order, dx fastest, the tile itself left out) of the tile at
+// (tx, ty, tz)
+OSR_DEV int neighbour(const GridDesc& g, int tx, int ty, int tz, int k) {
+  int dz = 0;
   if (g.dims == 2) {
-    tx = tile % g.ntx;
-    ty = tile / g.ntx;
-    tz = 0;
+    k += k >= 4;
   } else {
-    tx = tile % g.ntx;
-    ty = (tile / g.ntx) % g.nty;
-    tz = tile / (g.ntx * g.nty);
+    k += k >= 13;
+    dz = k / 9 - 1;
+    k = k % 9;
   }
-  const int zr = g.dims == 2 ? 0 : 1;
-  int k = 0;
-  for (int dz = -zr; dz <= zr; dz++)
-    for (int dy = -1; dy <= 1; dy++)
-      for (int dx = -1; dx <= 1; dx++) {
-        if (dx == 0 && dy == 0 && dz == 0) continue;
-        const int nxt = wrapi(tx + dx, g.ntx), nyt = wrapi(ty + dy, g.nty);
-        const int nzt = g.dims == 2 ? 0 : wrapi(tz + dz, g.ntz);
-        const int t = nxt + g.ntx * (nyt + g.nty * nzt);
-        if (t == tile) continue;
-        bool dup = false;
-        for (int j = 0; j < k; j++) dup |= nb[j] == t;
-        if (!dup) nb[k++] = t;
-      }
-  return k;
+  const int x = wrapi(tx + k % 3 - 1, g.ntx), y = wrapi(ty + k / 3 - 1, g.nty);
+  const int z = g.dims == 2 ? 0 : wrapi(tz + dz, g.ntz);
+  return x + g.ntx * (y + g.nty * z);
 }
 
 OSR_DEV void copy_from_mover(const SpecDesc& d, int src, int dst, int dims) {
@@ -608,167 +577,208 @@ OSR_DEV void copy_particle(const SpecDesc& d, int src, int dst, int dims) {
 // itself with inc = -1 and raises Ctrl::halt; the host then re-lays the species out from
 // the tiles that did fill plus the mover buffers.
 // NT threads per tile; INC_MAX incoming movers and TAIL_BITS holes left in the tail are the
-// most one fill can handle (LDS lists); beyond them the tile flags an overflow.
-// Segment of item i in a concatenation of n lists with start offsets ofs[0..n]
-// (ofs[0] = 0, non-decreasing, 0 <= i < ofs[n]): the last l with ofs[l] <= i, which skips
-// empty lists.  Binary search: the fill walks up to 8 x 8 (2D) or 26 x 4 (3D) lists.
-OSR_DEV int seg_find(const int* ofs, int n, int i) {
-  int lo = 0, hi = n;  // ofs[lo] <= i < ofs[hi]
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (ofs[mid] <= i)
-      lo = mid;
-    else
-      hi = mid;
-  }
-  return lo;
-}
+// most one fill handles; beyond them the tile flags an overflow.
+//
+// Bound: the chain of dependent loads and barriers of a tile (a tile moves few particles),
+// so the loads that depend on the same thing go out together: every list's length and base
+// by a thread of its own, then the own holes and the candidates' cells, then the movers.
+// The binary searches run on LDS tables, branch-free and in step for all items of a thread.
+// us per launch, lists walked by thread 0 and wave 0 / this: 64x64 14.1 / 9.2, 52x44x36
+// 26 / 12.8, 96^3 two beams 118 / 69, 192^3 533 / 385, 1024x1024 two beams 98 / 90 (there
+// and on 192^3 the scattered 4-byte copies of the movers take most of it).
+constexpr int kFillPF = 8;      // candidate movers per thread whose cells are loaded together
+constexpr int kFillHoles = 1024;  // own holes held in LDS (the rest are read from memory)
 
-constexpr int kFillPF = 8;  // candidate movers per thread whose cells are loaded together
+// Last l with ofs[l] <= v[p], for PF values at once: ofs is non-decreasing, ofs[0] <= v, and
+// padded above its last entry with INT_MAX up to N (a power of two) entries.
+template <int N, int PF>
+OSR_DEV void seg_find_multi(const int* ofs, const int (&v)[PF], int (&l)[PF]) {
+#pragma unroll
+  for (int p = 0; p < PF; p++) l[p] = 0;
+#pragma unroll
+  for (int h = N / 2; h > 0; h >>= 1)
+#pragma unroll
+    for (int p = 0; p < PF; p++)
+      if (ofs[l[p] + h] <= v[p]) l[p] += h;
+}
 
 template <int NT, int INC_MAX, int TAIL_BITS>
 __global__ __launch_bounds__(NT) void tile_fill(const SpecDesc* __restrict__ descs,
                                                 const int2* __restrict__ work) {
   constexpr int MAXL = 26 * kMaxTileWaves;  // candidate lists: neighbours x waves
-  __shared__ int s_nb[26];
-  __shared__ int s_nnb;
-  __shared__ int s_lofs[MAXL + 1];
-  __shared__ int s_lbase[MAXL];
-  __shared__ int s_wtot[NT / 64];
+  constexpr int PERL = (MAXL + NT - 1) / NT, NTAB = 512, NHT = 2 * kMaxTileWaves;
+  static_assert(MAXL < NTAB, "list table");
+  __shared__ int s_lofs[NTAB], s_lbase[MAXL], s_hofs[NHT];
+  __shared__ int s_lsum[PERL][NT / 64];
   __shared__ int s_pcnt[kFillPF][NT / 64];
-  __shared__ int s_hpre[kMaxTileWaves + 1];
+  __shared__ int s_hole[kFillHoles];
   __shared__ int s_inc[INC_MAX];
-  __shared__ unsigned int s_bits[TAIL_BITS / 32];
   const int2 wk = work[blockIdx.x];
   const SpecDesc& d = descs[wk.x];
   const GridDesc& g = d.g;
-  if (g.ctrl->halt >= 2) return;
-  const int tile = wk.y;
-  const int NW = d.waves;
+  const int tile = wk.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int NW = d.waves, wsh = 31 - __clz(NW);  // a power of two
   const int dims = g.dims;
-  const int base = d.off[tile];
-  const int n = d.cnt[tile];
-  const int stride = d.mv_stride[tile];
-  if (threadIdx.x == 0) {
-    s_nnb = neighbours(g, tile, s_nb);
-    s_hpre[0] = 0;
-    for (int w = 0; w < NW; w++) s_hpre[w + 1] = s_hpre[w] + d.mv_cnt[tile * NW + w];
-  }
-  __syncthreads();
-  const int L = s_nnb * NW;
-  if (L > MAXL) {  // more mover lists than the LDS tables hold: never with 26 x 16
-    if (threadIdx.x == 0) atomicOr(&g.ctrl->error, 2);
-    return;
-  }
-  if (threadIdx.x < 64) {  // wave 0: list bases and the prefix of the list lengths
-    const int lane = threadIdx.x;
-    int carry = 0;
-    for (int c0 = 0; c0 < L; c0 += 64) {
-      const int l = c0 + lane;
-      int v = 0;
-      if (l < L) {
-        const int nt = s_nb[l / NW], w = l % NW;
-        v = d.mv_cnt[nt * NW + w];
-        s_lbase[l] = d.off[nt] + w * d.mv_stride[nt];
+  const int L = (dims == 2 ? 8 : 26) << wsh;
+  const int base = d.off[tile], n = d.cnt[tile], cap = d.cap[tile], stride = d.mv_stride[tile];
+  const int tx = tile % g.ntx, ty = (tile / g.ntx) % g.nty, tz = tile / (g.ntx * g.nty);
+  // a direction of one or two tiles names some neighbours twice, or the tile itself
+  const bool small = g.ntx < 3 || g.nty < 3 || (dims == 3 && g.ntz < 3);
+  if (g.ctrl->halt >= 2) return;
+  // list lengths and bases, and the prefix of the lengths
+  int cnt[PERL], pre[PERL];
+#pragma unroll
+  for (int j = 0; j < PERL; j++) {
+    const int l = tid + j * NT;
+    cnt[j] = 0;
+    if (l < L) {
+      const int k = l >> wsh, w = l & (NW - 1), nt = neighbour(g, tx, ty, tz, k);
+      bool dup = false;
+      if (small) {
+        dup = nt == tile;
+        for (int i = 0; i < k; i++) dup |= neighbour(g, tx, ty, tz, i) == nt;
       }
-      for (int o = 1; o < 64; o <<= 1) {  // inclusive scan over the wave
-        const int t = __shfl_up(v, o, 64);
-        if (lane >= o) v += t;
-      }
-      if (l < L) s_lofs[l + 1] = carry + v;
-      carry += __shfl(v, 63, 64);
+      if (!dup) cnt[j] = d.mv_cnt[(nt << wsh) + w];
+      s_lbase[l] = d.off[nt] + w * d.mv_stride[nt];
     }
-    if (lane == 0) s_lofs[0] = 0;
+  }
+  const int own = tid < NW ? d.mv_cnt[(tile << wsh) + tid] : 0;  // wave 0: the tile's own lists
+  for (int i = tid; i < NTAB; i += NT)
+    if (i == 0 || i > L) s_lofs[i] = i == 0 ? 0 : 0x7FFFFFFF;
+  auto wave_scan = [&](int v) {  // inclusive, over the wave
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int t = __shfl_up(v, o, 64);
+      if (lane >= o) v += t;
+    }
+    return v;
+  };
+#pragma unroll
+  for (int j = 0; j < PERL; j++) {
+    pre[j] = wave_scan(cnt[j]);
+    if (lane == 63) s_lsum[j][wave] = pre[j];
+  }
+  if (wave == 0) {
+    const int h = wave_scan(own);
+    if (lane == 0) s_hofs[0] = 0;
+    if (lane < NHT - 1) s_hofs[lane + 1] = lane < NW ? h : 0x7FFFFFFF;
   }
   __syncthreads();
+  int T = 0;
+#pragma unroll
+  for (int j = 0; j < PERL; j++) {
+    int before = T;
+#pragma unroll
+    for (int w = 0; w < NT / 64; w++) {
+      const int v = s_lsum[j][w];
+      if (w < wave) before += v;
+      T += v;
+    }
+    const int l = tid + j * NT;
+    if (l < L) s_lofs[l + 1] = before + pre[j];
+  }
+  const int H = s_hofs[NW];
   // a tile of the guard band of open x walls takes no movers: the particles that left
   // through a wall (ix < 1 or ix > nx) are dropped (spec/os-spec-boundary.f03:476-513)
-  const bool absorb = (tile % g.ntx) * g.tx >= interior_nx(g);
-  const int T = absorb ? 0 : s_lofs[L];
-  const int H = s_hpre[NW];
+  if (tx * g.tx >= interior_nx(g)) T = 0;
+  __syncthreads();
+  auto hole_at = [&](int k) -> int {  // own hole k from memory
+    const int v[1] = {k};
+    int w[1];
+    seg_find_multi<NHT, 1>(s_hofs, v, w);
+    return d.midx[base + w[0] * stride + (k - s_hofs[w[0]])];
+  };
+  // holes are ascending in k: each wave's movers are in slot order, and so are the waves
+  for (int k = tid; k < min(H, kFillHoles); k += NT) s_hole[k] = hole_at(k);
   // pass 1: collect the incoming movers, in candidate order.  Candidates are taken PF NT
   // at a time, candidate c0 + p NT + thread as item p of the thread, and the cells of all
   // of them are loaded before any is ranked: one memory round trip per PF NT candidates
   // (a tile's neighbours hold some 8 x 200 movers on the 2D two-stream workload).
+  const int cx0 = tx * g.tx, cy0 = ty * g.ty, cz0 = tz * g.tz;
+  auto in_tile = [&](uint32_t c) {
+    int ix, iy, iz = 0;
+    if (dims == 2)
+      unpack2(c, ix, iy);
+    else
+      unpack3(c, ix, iy, iz);
+    return (unsigned)(ix - cx0) < (unsigned)g.tx && (unsigned)(iy - cy0) < (unsigned)g.ty &&
+           (dims == 2 || (unsigned)(iz - cz0) < (unsigned)g.tz);
+  };
   int I = 0;
-  for (int c0 = 0; c0 < T; c0 += NT * kFillPF) {
-    uint32_t cell[kFillPF];
-    int src[kFillPF];
+  auto collect = [&](auto pf, int c0) {
+    constexpr int PF = decltype(pf)::value;
+    int v[PF], l[PF], src[PF], r[PF], tot;
+    uint32_t cell[PF];
+    bool f[PF];
 #pragma unroll
-    for (int p = 0; p < kFillPF; p++) {
-      const int i = c0 + p * NT + threadIdx.x;
-      src[p] = -1;
-      cell[p] = 0u;
-      if (i < T) {
-        const int l = seg_find(s_lofs, L, i);
-        src[p] = s_lbase[l] + (i - s_lofs[l]);
-        cell[p] = d.mcell[src[p]];
-      }
+    for (int p = 0; p < PF; p++) v[p] = min(c0 + p * NT + tid, T - 1);
+    seg_find_multi<NTAB, PF>(s_lofs, v, l);
+#pragma unroll
+    for (int p = 0; p < PF; p++) {
+      src[p] = s_lbase[l[p]] + (v[p] - s_lofs[l[p]]);
+      cell[p] = d.mcell[src[p]];
     }
-    bool f[kFillPF];
 #pragma unroll
-    for (int p = 0; p < kFillPF; p++) f[p] = src[p] >= 0 && tile_of(g, cell[p]) == tile;
-    int r[kFillPF], tot;
-    block_rank_multi<NT, kFillPF>(f, s_pcnt, r, tot);
+    for (int p = 0; p < PF; p++) f[p] = c0 + p * NT + tid < T && in_tile(cell[p]);
+    block_rank_multi<NT, PF>(f, s_pcnt, r, tot);
 #pragma unroll
-    for (int p = 0; p < kFillPF; p++)
+    for (int p = 0; p < PF; p++)
       if (f[p] && I + r[p] < INC_MAX) s_inc[I + r[p]] = src[p];
     I += tot;
+  };
+  for (int c0 = 0; c0 < T;) {  // T is uniform
+    if (T - c0 <= 2 * NT) {
+      collect(std::integral_constant<int, 2>(), c0);
+      c0 += 2 * NT;
+    } else {
+      collect(std::integral_constant<int, kFillPF>(), c0);
+      c0 += kFillPF * NT;
+    }
   }
-  // every wave's entries of s_inc are in LDS before any wave reads them in pass 2 (the
-  // hole count below has barriers only when the tile loses more movers than it gains)
+  // every wave's entries of s_inc and s_hole are in LDS before any wave reads them below
   __syncthreads();
   const int nn = n - H + I;
-  if (I > INC_MAX || nn > d.cap[tile] - 64 * NW || H - I > TAIL_BITS) {
-    if (threadIdx.x == 0) {
+  if (I > INC_MAX || nn > cap - 64 * NW || H - I > TAIL_BITS) {
+    if (tid == 0) {
       d.inc[tile] = -1;
       // the count the tile needs after this step, or -1 if more capacity would not help
-      // (the incoming or tail lists exceed this kernel's LDS tables)
+      // (the incoming or tail lists exceed this kernel's limits)
       d.newcnt[tile] = (I > INC_MAX || H - I > TAIL_BITS) ? -1 : nn;
       atomicOr(&g.ctrl->halt, 1);
     }
     return;
   }
-  auto hole = [&](int k) -> int {
-    const int w = seg_find(s_hpre, NW, k);
-    return d.midx[base + w * stride + (k - s_hpre[w])];
-  };
-  // number of holes below nn (holes are ascending)
+  auto hole = [&](int k) -> int { return k < kFillHoles ? s_hole[k] : hole_at(k); };
+  // holes below nn: the whole list unless the tile shrinks
   int hlo = H;
   if (I < H) {
-    int c = 0;
-    for (int k = threadIdx.x; k < H; k += NT) c += hole(k) < nn;
-    for (int off = 32; off > 0; off >>= 1) c += __shfl_down(c, off, 64);
-    if ((threadIdx.x & 63) == 0) s_wtot[threadIdx.x >> 6] = c;
-    __syncthreads();
-    hlo = 0;
-    for (int w = 0; w < NT / 64; w++) hlo += s_wtot[w];
-    __syncthreads();
-  }
-  auto target = [&](int k) -> int { return k < hlo ? hole(k) : n + (k - H); };
-  // pass 2: incoming movers into the holes / appended slots
-  for (int r = threadIdx.x; r < I; r += NT) copy_from_mover(d, s_inc[r], base + target(r), dims);
-  // pass 3: tail particles into the remaining holes
-  if (I < H) {
-    const int tail = n - nn;  // = H - I
-    for (int i = threadIdx.x; i < (tail + 31) / 32; i += NT) s_bits[i] = 0u;
-    __syncthreads();
-    for (int k = hlo + threadIdx.x; k < H; k += NT) {
-      const int t = hole(k) - nn;
-      atomicOr(&s_bits[t >> 5], 1u << (t & 31));
-    }
-    __syncthreads();
-    int r1 = 0;
-    for (int i0 = 0; i0 < tail; i0 += NT) {
-      const int i = i0 + threadIdx.x;
-      const bool f = i < tail && !((s_bits[i >> 5] >> (i & 31)) & 1u);
-      int tot;
-      const int r = block_rank<NT>(f, s_wtot, tot);
-      if (f) copy_particle(d, base + nn + i, base + target(I + r1 + r), dims);
-      r1 += tot;
+    int lo = 0;
+    while (lo < hlo) {
+      const int mid = (lo + hlo) >> 1;
+      if (hole(mid) < nn)
+        lo = mid + 1;
+      else
+        hlo = mid;
     }
   }
-  if (threadIdx.x == 0) {
+  // pass 2: incoming movers into the holes below nn, then the appended slots
+  for (int r = tid; r < I; r += NT)
+    copy_from_mover(d, s_inc[r], base + (r < hlo ? hole(r) : n + (r - H)), dims);
+  // pass 3: the particles of the tail [nn, n) into the remaining holes: the r-th of them is
+  // slot nn + r + m, m the number of tail holes at or before it (hole hlo + j of the tail
+  // has hole - nn - j particles below it, non-decreasing in j)
+  for (int r = tid; r < hlo - I; r += NT) {
+    int lo = 0, hi = H - hlo;
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      if (hole(hlo + mid) - nn - mid <= r)
+        lo = mid + 1;
+      else
+        hi = mid;
+    }
+    copy_particle(d, base + nn + r + lo, base + hole(I + r), dims);
+  }
+  if (tid == 0) {
     d.cnt[tile] = nn;
     d.inc[tile] = I;
   }
