@@ -362,6 +362,12 @@ void make_spec_descs(const osr_sim* s, SpecDesc* v) {
     d.inc = p.inc.as<int>();
     d.epart = p.epart.as<double>();
     d.tem = (float)(0.5 * s->dt / (double)p.rqm);
+    // A particle adds at most |q| to a node and component, over all its virtual particles:
+    // |q|/2 (its path is shorter than dt) times a weight sum of at most 2 along and across
+    // the component, |q vz|/3 times at most 3 for the third; 1% and one unit per virtual
+    // particle cover the roundings.
+    const int maxcap = p.h_cap.empty() ? 0 : *std::max_element(p.h_cap.begin(), p.h_cap.end());
+    d.jraw = (double)maxcap * (1.01 * p.qmax * s->g.jscale + 4.0) < std::ldexp(1.0, 50);
     d.waves = s->tile_waves();
     d.split = s->split;
   }

@@ -7,16 +7,25 @@
 //  * particle, mover and field arrays are accessed through global-address-space
 //    pointers: uniform base + 32-bit offset, no per-array 64-bit address arithmetic, and
 //    the loads do not share the LDS wait counter as flat accesses would;
-//  * the first virtual particle (VP) of every particle is deposited straight from
-//    registers, with the start-point splines of the gather (VP 0 starts at the old
-//    position); a trajectory that crosses a cell face has 1 or 2 more VPs, which each
-//    wave appends to a private LDS queue and deposits 64 at a time, so the deposit runs
-//    on full waves instead of looping max(#VP) times over partly idle lanes;
+//  * a particle that stays in its cell is one virtual particle (VP) and is deposited
+//    straight from registers, with the start-point splines of the gather; one that crosses a
+//    cell face (an eighth of them on the two-stream workload) is appended to a private LDS
+//    queue of its wave, which splits and deposits 64 of them at a time, so that neither the
+//    split nor the further VPs run on partly idle waves;
 //  * the current of all waves is accumulated into one int64 fixed-point LDS tile; integer
 //    adds are exact and order independent, so the deposit is bit-reproducible run to run
 //    (FP32 LDS atomics were measured to be far slower here: a 40x longer LDS wait).
+// What bounds it: LDS (bank conflicts of the 64-bit adds, whose lanes point at random nodes
+// once the particles have moved: 12.7 cycles of a CU per add against 7.4 without conflicts)
+// and VALU issue, together.  Two-stream 1024x1024, 64 per cell, quadratic, per 64 particles:
+// 557 -> 460 VALU instructions (raw fixed-point bits, 21; split and further VPs on full waves
+// only, about 70), 36 -> 18 LDS reads; 1.270 -> 1.147 ms per step (3.1 TB/s of the 52 B a
+// particle moves), VALU 71% and LDS about 80% of the cycles.  512x512, 16 per cell, cubic, Vay
+// 170 -> 153 us, 515x267 quadratic 58 -> 54.5, 300x200 37 -> 31.6.
 // The arithmetic of gather, push, position advance and split is the one of the generic
 // kernel (the reference's AVX2 kernel, simd/os-spec-push-avx2.c:471-760).
+#include <type_traits>
+
 #include "osr_device.hpp"
 #include "osr_types.hpp"
 
@@ -36,39 +45,41 @@ OSR_DEV P el(P b, uint32_t i) {
   return (P)((gch*)b + i * (uint32_t)sizeof(*b));
 }
 
-// extra row pitch of the LDS field and current tiles (bank-conflict tuning)
-#ifndef OSR_FIELD_PAD
-#define OSR_FIELD_PAD 0
-#endif
-#ifndef OSR_CUR_PAD
-#define OSR_CUR_PAD 0
-#endif
-constexpr int kFieldPad = OSR_FIELD_PAD;
-constexpr int kCurPad = OSR_CUR_PAD;
-
 // periodic wrap of a cell index at most one period outside [0, n)
 OSR_DEV int wrap1(int i, int n) { return i < 0 ? i + n : (i >= n ? i - n : i); }
+
+// LDS layout of the staged fields.  A ds_read_b128 takes about 10 cycles of a CU for 64
+// lanes wherever they point (measured, also at random addresses), four 4-byte or two 8-byte
+// reads 38 and 25 at random addresses (5 per 8 bytes without bank conflicts, which particles
+// in the order a few steps leave them do not give).  So a 16-byte element per node holds what
+// the node's x line needs next: the two components that share a stencil at the node and its
+// right neighbour ((E1, B2) at half x, full y; (E2, B1) at full x, half y), and for E3 (full,
+// full) and B3 (half, half) the node and the next three, or, with linear and cubic splines,
+// the node and the next one (which keeps 4 workgroups in a CU).
+template <int ORDER>
+struct Line2 {
+  static constexpr int W = ORDER >= 2 ? 4 : 2;  // E3, B3 values per node
+  typedef float V __attribute__((ext_vector_type(W)));
+};
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 
 template <int ORDER, int PUSHER, int TX, int TY, int NW>
 __global__ __launch_bounds__(64 * NW, 4) void push_deposit_2d_t(const SpecDesc* __restrict__ descs,
                                                                 const int2* __restrict__ work) {
   using O = Ord<ORDER>;
-  constexpr int NP = O::NP;
+  using LV = typename Line2<ORDER>::V;
+  constexpr int NP = O::NP, LW = Line2<ORDER>::W;
   constexpr int NT = 64 * NW;
-  // staged field tile GX x GY and current tile JX x JY, stored with row pitches GS / JS
-  constexpr int GX = TX + O::GLO + O::GHI, GY = TY + O::GLO + O::GHI;
-  constexpr int JX = TX + O::JLO + O::JHI, JY = TY + O::JLO + O::JHI;
-  constexpr int GS = GX + kFieldPad, GN = GS * GY;
-  constexpr int JS = JX + kCurPad, JN = JS * JY;
-  constexpr int QC = 128;  // VP queue capacity per wave (< 64 pending + 64 appended)
-  // staged fields: components that share a stencil are paired so that one 64-bit LDS
-  // read serves both: (E1, B2) at (half x, full y), (E2, B1) at (full x, half y);
-  // E3 (full, full) and B3 (half, half) are single
-  __shared__ float2 sEB12[GN], sEB21[GN];
-  __shared__ float sE3[GN], sB3[GN];
+  // staged field tile GX x GY and current tile JX x JY
+  constexpr int GX = TX + O::GLO + O::GHI, GY = TY + O::GLO + O::GHI, GN = GX * GY;
+  constexpr int JX = TX + O::JLO + O::JHI, JY = TY + O::JLO + O::JHI, JN = JX * JY;
+  constexpr int QC = 64;  // crossing particles queued per wave
+  static_assert((TX & (TX - 1)) == 0 && (TY & (TY - 1)) == 0, "tile sides are powers of two");
+  __shared__ f32x4 s12[GN], s21[GN];
+  __shared__ LV s3[GN], s6[GN];
   __shared__ unsigned long long sJ[3 * JN];
-  __shared__ float sQ[NW][6][QC];  // x0, y0, x1, y1, q, vz
-  __shared__ int sQn[NW][QC];      // LDS node index of the VP's first stencil point
+  __shared__ f32x4 sQ[NW][2][QC];  // (x0, y0, x1, y1), (q, vz, node and cell shifts)
   __shared__ double s_ene[NW];
 
   const int2 wk = work[blockIdx.x];
@@ -83,14 +94,26 @@ __global__ __launch_bounds__(64 * NW, 4) void push_deposit_2d_t(const SpecDesc* 
   {
     const gf32* __restrict__ E = (const gf32*)g.E + co;
     const gf32* __restrict__ B = (const gf32*)g.B + co;
-    for (int i = threadIdx.x; i < GX * GY; i += NT) {
-      const int col = i % GX, row = i / GX, li = row * GS + col;
+    for (int i = threadIdx.x; i < GN; i += NT) {
+      const int col = i % GX, row = i / GX;
       const int gx = wrapi(cx0 + col - O::GLO, nx), gy = wrapi(cy0 + row - O::GLO, ny);
       const long long gi = gx + (long long)nx * gy;
-      sEB12[li] = make_float2(E[gi], B[nc + gi]);
-      sEB21[li] = make_float2(E[nc + gi], B[gi]);
-      sE3[li] = E[2 * nc + gi];
-      sB3[li] = B[2 * nc + gi];
+      const f32x2 p12 = {E[gi], B[nc + gi]}, p21 = {E[nc + gi], B[gi]};
+      const float e3 = E[2 * nc + gi], b3 = B[2 * nc + gi];
+      // this node's part of its own element and of those of the nodes on its left, as stores
+      // of that part alone: other threads write the rest of each element
+      ((f32x2*)s12)[2 * i] = p12;
+      ((f32x2*)s21)[2 * i] = p21;
+      if (col > 0) {
+        ((f32x2*)s12)[2 * i - 1] = p12;
+        ((f32x2*)s21)[2 * i - 1] = p21;
+      }
+#pragma unroll
+      for (int k = 0; k < LW; k++)
+        if (col >= k) {
+          ((float*)s3)[LW * (i - k) + k] = e3;
+          ((float*)s6)[LW * (i - k) + k] = b3;
+        }
     }
   }
   for (int i = threadIdx.x; i < 3 * JN; i += NT) sJ[i] = 0ull;
@@ -103,7 +126,7 @@ __global__ __launch_bounds__(64 * NW, 4) void push_deposit_2d_t(const SpecDesc* 
   // this workgroup's waves among the split * NW of the tile (the work list names a tile
   // once per workgroup, back to back)
   const int split = d.split, part = (int)(blockIdx.x % (unsigned)split);
-  const int tw = part * NW + wave;
+  const int tw = __builtin_amdgcn_readfirstlane(part * NW + wave);
   const int per_wave = ((n + NT * split - 1) / (NT * split)) * 64;
   const int w0 = tw * per_wave;
   const int w1 = min(w0 + per_wave, n);
@@ -114,8 +137,6 @@ __global__ __launch_bounds__(64 * NW, 4) void push_deposit_2d_t(const SpecDesc* 
   unsigned long long* const J1 = sJ;
   unsigned long long* const J2 = sJ + JN;
   unsigned long long* const J3 = sJ + 2 * JN;
-  float(*const Q)[QC] = sQ[wave];
-  int* const QN = sQn[wave];
   // particle and mover arrays of this tile, global address space
   const gu32* __restrict__ Pcell = (const gu32*)d.cell + base;
   const gf32* __restrict__ Px = (const gf32*)d.x + base;
@@ -141,31 +162,49 @@ __global__ __launch_bounds__(64 * NW, 4) void push_deposit_2d_t(const SpecDesc* 
   gu32* __restrict__ Mpid = (gu32*)d.mpid + base;
   gi32* __restrict__ Midx = (gi32*)d.midx + base;
 
-  // deposit of the queued VPs in slots [head, head + cnt) (cnt <= 64, one per lane)
-  auto deposit_queue = [&](int head, int cnt) {
-    if (lane < cnt) {
-      const int s = (head + lane) & (QC - 1);
-      const float x0 = Q[0][s], y0 = Q[1][s];
-      float S0x[NP], S0y[NP];
-      spline<ORDER>(x0, S0x);
-      spline<ORDER>(y0, S0y);
-      dep_vp<ORDER>(J1, J2, J3, S0x, S0y, x0, y0, Q[2][s], Q[3][s], Q[4][s], Q[5][s], QN[s], JS,
-                     jn1, jn2, jscale);
-    }
-  };
-
   double ene = 0.0;
   int mcount = 0;
-  int qhead = 0, qlen = 0;
   bool bad = false;
-  // The particle loads of the next iteration are issued before the current one is
-  // processed (software pipelining): a wave otherwise waits a full memory latency per
-  // iteration, and the bytes in flight per CU would cap the bandwidth well below peak.
-  uint32_t f_cell = 0, f_pid = 0;
-  float f_x = 0.f, f_y = 0.f, f_u1 = 0.f, f_u2 = 0.f, f_u3 = 0.f, f_q = 0.f;
-  auto prefetch = [&](int pf) {
-    if (pf < w1) {
-      const unsigned upf = (unsigned)pf;
+  // cells of the tile inside the grid; a particle that leaves them changes tile, unless the
+  // tile is the only one of a direction (it wraps into itself)
+  const int tcx = min(TX, nx - cx0), tcy = min(TY, ny - cy0);
+  const bool lone = g.ntx == 1 || g.nty == 1;
+  const uint32_t cell0 = pack2(cx0, cy0);
+
+  // the wave's particles; RAW: how the deposit adds (fix_bits)
+  auto push_all = [&](auto raw) {
+    constexpr bool RAW = decltype(raw)::value;
+    int qlen = 0;
+    f32x4* const Q0 = sQ[wave][0];
+    f32x4* const Q1 = sQ[wave][1];
+    // split and deposit of the queued particles, one per lane
+    auto deposit_queue = [&]() {
+      if (lane < qlen) {
+        const f32x4 a = Q0[lane], b = Q1[lane];
+        const int code = __float_as_int(b.z), nb0 = code >> 4;
+        VP2 vp[3];
+        const int nvp = split2d_fast(a.x, a.y, a.z, a.w, (code & 3) - 1, ((code >> 2) & 3) - 1, b.x,
+                                     b.y, vp);
+#pragma unroll
+        for (int v = 0; v < 3; v++) {
+          if (v == 2 && nvp < 3) break;  // a queued particle has crossed one face at least
+          float S0x[NP], S0y[NP];
+          spline<ORDER>(vp[v].x0, S0x);
+          spline<ORDER>(vp[v].y0, S0y);
+          dep_vp<ORDER, RAW>(J1, J2, J3, S0x, S0y, vp[v].x0, vp[v].y0, vp[v].x1, vp[v].y1, vp[v].q,
+                             vp[v].vz, nb0 + vp[v].dj * JX + vp[v].di, JX, jn1, jn2, jscale);
+        }
+      }
+      qlen = 0;
+    };
+    // The particle loads of the next iteration are issued before the current one is
+    // processed (software pipelining): a wave otherwise waits a full memory latency per
+    // iteration, and the bytes in flight per CU would cap the bandwidth well below peak.
+    // Lanes past the end load the last particle again and are masked below.
+    uint32_t f_cell = 0, f_pid = 0;
+    float f_x = 0.f, f_y = 0.f, f_u1 = 0.f, f_u2 = 0.f, f_u3 = 0.f, f_q = 0.f;
+    auto prefetch = [&](int pf) {
+      const unsigned upf = (unsigned)min(pf, w1 - 1);
       f_cell = *el(Pcell, upf);
       f_x = *el(Px, upf);
       f_y = *el(Py, upf);
@@ -174,136 +213,150 @@ __global__ __launch_bounds__(64 * NW, 4) void push_deposit_2d_t(const SpecDesc* 
       f_u3 = *el(Puz, upf);
       f_q = *el(Pq, upf);
       f_pid = *el(Ppid, upf);
+    };
+    if (w0 < w1) prefetch(w0 + lane);
+    for (int p0 = w0;; p0 += 64) {
+      const bool more = p0 < w1;  // the pass after the last particles empties the queue
+      bool cross = false;
+      f32x4 qa, qb;
+      if (more) {
+        const int p = p0 + lane;
+        const unsigned up = (unsigned)p;  // 32-bit unsigned offsets from the scalar bases
+        const uint32_t cell = f_cell, pid = f_pid;
+        const float x = f_x, y = f_y, q = f_q;
+        float u1 = f_u1, u2 = f_u2, u3 = f_u3;
+        if (p0 + 64 < w1) prefetch(p + 64);
+        // cell within the tile: both halves of the difference in range (a borrow shows too)
+        const uint32_t dl = cell - cell0;
+        const bool out = (dl & ~((TX - 1u) | ((TY - 1u) << 16))) != 0u;
+        const bool act = p < w1 && !out;
+        bad |= p < w1 && out;
+        const int lx = (int)(dl & (TX - 1u)), ly = (int)((dl >> 16) & (TY - 1u));
+        // ---- gather
+        float wx[NP], wy[NP], wxh[NP], wyh[NP];
+        spline<ORDER>(x, wx);
+        spline<ORDER>(y, wy);
+        splineh<ORDER>(x, x < 0.f ? 1.f : 0.f, wxh);
+        splineh<ORDER>(y, y < 0.f ? 1.f : 0.f, wyh);
+        const int gb = (ly + O::GLO + O::LP) * GX + lx + O::GLO + O::LP;
+        const int gbx = gb - (x < 0.f ? 1 : 0);
+        const int gby = gb - (y < 0.f ? GX : 0);
+        const int gbxy = gbx - (y < 0.f ? GX : 0);
+        float e1 = 0.f, e2 = 0.f, e3 = 0.f, b1 = 0.f, b2 = 0.f, b3 = 0.f;
+#pragma unroll
+        for (int k2 = 0; k2 < NP; k2++) {
+          // the row's line of each stencil
+          float r12[2 * NP + 2], r21[2 * NP + 2], r3[NP + 1], r6[NP + 1];
+          auto pairs = [&](const f32x4* L, float* r) {
+#pragma unroll
+            for (int k1 = 0; k1 < NP; k1 += 2) {
+              f32x4 v = L[k1];
+              if (k1 + 1 == NP) asm("" : "+v"(v));  // a full read: the low half alone is slower
+              r[2 * k1] = v.x;
+              r[2 * k1 + 1] = v.y;
+              r[2 * k1 + 2] = v.z;
+              r[2 * k1 + 3] = v.w;
+            }
+          };
+          auto line = [&](const LV* L, float* r) {
+#pragma unroll
+            for (int k1 = 0; k1 < NP; k1 += LW) {
+              const LV v = L[k1];
+#pragma unroll
+              for (int k = 0; k < LW; k++)
+                if (k1 + k < NP) r[k1 + k] = v[k];
+            }
+          };
+          pairs(s12 + gbx + k2 * GX, r12);
+          pairs(s21 + gby + k2 * GX, r21);
+          line(s3 + gb + k2 * GX, r3);
+          line(s6 + gbxy + k2 * GX, r6);
+          float le1 = 0.f, le2 = 0.f, le3 = 0.f, lb1 = 0.f, lb2 = 0.f, lb3 = 0.f;
+#pragma unroll
+          for (int k1 = 0; k1 < NP; k1++) {
+            le1 = fma_(r12[2 * k1], wxh[k1], le1);
+            le2 = fma_(r21[2 * k1], wx[k1], le2);
+            le3 = fma_(r3[k1], wx[k1], le3);
+            lb1 = fma_(r21[2 * k1 + 1], wx[k1], lb1);
+            lb2 = fma_(r12[2 * k1 + 1], wxh[k1], lb2);
+            lb3 = fma_(r6[k1], wxh[k1], lb3);
+          }
+          e1 = fma_(le1, wy[k2], e1);
+          e2 = fma_(le2, wyh[k2], e2);
+          e3 = fma_(le3, wy[k2], e3);
+          b1 = fma_(lb1, wyh[k2], b1);
+          b2 = fma_(lb2, wy[k2], b2);
+          b3 = fma_(lb3, wyh[k2], b3);
+        }
+        // ---- push
+        const float ke = push<PUSHER>(tem, e1, e2, e3, b1, b2, b3, u1, u2, u3);
+        ene = __builtin_fma((double)(act ? q : 0.f), (double)ke, ene);
+        // ---- position
+        const float rg = rgamma(u1, u2, u3);
+        const float v1 = u1 * rg, v2 = u2 * rg, v3 = u3 * rg;
+        const float x1 = fma_(v1, dtdx1, x), y1 = fma_(v2, dtdx2, y);
+        const float tx = trim(x1), ty = trim(y1);
+        const int dix = (int)tx, diy = (int)ty;
+        // ---- deposit of the particles that stay in their cell: one VP, with the gather's
+        // splines; the others are queued for the split
+        const int nb0 = (ly + O::LP + O::JLO) * JX + lx + O::LP + O::JLO;
+        cross = act && (dix | diy) != 0;
+        qa = f32x4{x, y, x1, y1};
+        qb = f32x4{q, v3, __int_as_float(nb0 * 16 + (dix + 1) + 4 * (diy + 1)), 0.f};
+        if (act && !cross)
+          dep_vp<ORDER, RAW>(J1, J2, J3, wx, wy, x, y, x1, y1, q, v3, nb0, JX, jn1, jn2, jscale);
+        const unsigned long long below = (1ull << lane) - 1ull;
+        // ---- store: stay in place, or leave through the mover buffer
+        const int nlx = lx + dix, nly = ly + diy;
+        bool stay = (unsigned)nlx < (unsigned)tcx && (unsigned)nly < (unsigned)tcy;
+        uint32_t ncell = cell0 + pack2(0, nly) + (uint32_t)nlx;
+        if (lone || !__all(stay || !act)) {
+          const int nix = wrap1(nlx + cx0, nx), niy = wrap1(nly + cy0, ny);
+          ncell = pack2(nix, niy);
+          stay = (nix / TX + g.ntx * (niy / TY)) == tile;
+        }
+        const float xs = x1 - tx, ys = y1 - ty;
+        if (act && stay) {
+          *el(Wcell, up) = ncell;
+          *el(Wx, up) = xs;
+          *el(Wy, up) = ys;
+          *el(Wux, up) = u1;
+          *el(Wuy, up) = u2;
+          *el(Wuz, up) = u3;
+        }
+        const bool mv = act && !stay;
+        const unsigned long long mm = __ballot(mv);
+        if (mv) {
+          const unsigned slot = (unsigned)(w0 + mcount + __popcll(mm & below));
+          *el(Mcell, slot) = ncell;
+          *el(Mx, slot) = xs;
+          *el(My, slot) = ys;
+          *el(Mux, slot) = u1;
+          *el(Muy, slot) = u2;
+          *el(Muz, slot) = u3;
+          *el(Mq, slot) = q;
+          *el(Mpid, slot) = pid;
+          *el(Midx, slot) = p;
+        }
+        mcount += __popcll(mm);
+      }
+      const unsigned long long mc = __ballot(cross);
+      const int add = __popcll(mc);
+      if (qlen + add > QC || (!more && qlen > 0)) deposit_queue();
+      if (!more) break;
+      if (cross) {
+        const int s = qlen + __popcll(mc & ((1ull << lane) - 1ull));
+        Q0[s] = qa;
+        Q1[s] = qb;
+      }
+      qlen += add;
     }
   };
-  prefetch(w0 + lane);
-  for (int p0 = w0; p0 < w1; p0 += 64) {
-    const int p = p0 + lane;
-    const unsigned up = (unsigned)p;  // 32-bit unsigned offsets from the scalar bases
-    bool act = p < w1;
-    float x = 0.f, y = 0.f, u1 = 0.f, u2 = 0.f, u3 = 0.f, q = 0.f;
-    int lx = 0, ly = 0;
-    const uint32_t cell = f_cell, pid = f_pid;
-    if (act) {
-      x = f_x;
-      y = f_y;
-      u1 = f_u1;
-      u2 = f_u2;
-      u3 = f_u3;
-      q = f_q;
-    }
-    prefetch(p + 64);
-    if (act) {
-      int ix, iy;
-      unpack2(cell, ix, iy);
-      lx = ix - cx0;
-      ly = iy - cy0;
-      if (lx < 0 || lx >= TX || ly < 0 || ly >= TY) {
-        bad = true;
-        act = false;
-        lx = ly = 0;
-      }
-    }
-    // ---- gather
-    float wx[NP], wy[NP], wxh[NP], wyh[NP];
-    spline<ORDER>(x, wx);
-    spline<ORDER>(y, wy);
-    splineh<ORDER>(x, x < 0.f ? 1.f : 0.f, wxh);
-    splineh<ORDER>(y, y < 0.f ? 1.f : 0.f, wyh);
-    const int gb = (ly + O::GLO + O::LP) * GS + lx + O::GLO + O::LP;
-    const int gbx = gb - (x < 0.f ? 1 : 0);
-    const int gby = gb - (y < 0.f ? GS : 0);
-    const int gbxy = gbx - (y < 0.f ? GS : 0);
-    float e1 = 0.f, e2 = 0.f, e3 = 0.f, b1 = 0.f, b2 = 0.f, b3 = 0.f;
-#pragma unroll
-    for (int k2 = 0; k2 < NP; k2++) {
-      float le1 = 0.f, le2 = 0.f, le3 = 0.f, lb1 = 0.f, lb2 = 0.f, lb3 = 0.f;
-#pragma unroll
-      for (int k1 = 0; k1 < NP; k1++) {
-        const float2 p12 = sEB12[gbx + k2 * GS + k1];
-        const float2 p21 = sEB21[gby + k2 * GS + k1];
-        le1 = fma_(p12.x, wxh[k1], le1);
-        le2 = fma_(p21.x, wx[k1], le2);
-        le3 = fma_(sE3[gb + k2 * GS + k1], wx[k1], le3);
-        lb1 = fma_(p21.y, wx[k1], lb1);
-        lb2 = fma_(p12.y, wxh[k1], lb2);
-        lb3 = fma_(sB3[gbxy + k2 * GS + k1], wxh[k1], lb3);
-      }
-      e1 = fma_(le1, wy[k2], e1);
-      e2 = fma_(le2, wyh[k2], e2);
-      e3 = fma_(le3, wy[k2], e3);
-      b1 = fma_(lb1, wyh[k2], b1);
-      b2 = fma_(lb2, wy[k2], b2);
-      b3 = fma_(lb3, wyh[k2], b3);
-    }
-    // ---- push
-    const float ke = push<PUSHER>(tem, e1, e2, e3, b1, b2, b3, u1, u2, u3);
-    if (act) ene += (double)q * (double)ke;
-    // ---- position
-    const float rg = rgamma(u1, u2, u3);
-    const float v1 = u1 * rg, v2 = u2 * rg, v3 = u3 * rg;
-    const float x1 = fma_(v1, dtdx1, x), y1 = fma_(v2, dtdx2, y);
-    const float tx = trim(x1), ty = trim(y1);
-    const int dix = (int)tx, diy = (int)ty;
-    // ---- split; VP 0 is deposited in place, VPs 1 and 2 go through the queue
-    VP2 vp[3];
-    const int nvp = act ? split2d_fast(x, y, x1, y1, dix, diy, q, v3, vp) : 0;
-    const int nb0 = (ly + O::LP + O::JLO) * JS + lx + O::LP + O::JLO;
-    if (act)
-      dep_vp<ORDER>(J1, J2, J3, wx, wy, vp[0].x0, vp[0].y0, vp[0].x1, vp[0].y1, vp[0].q,
-                    vp[0].vz, nb0, JS, jn1, jn2, jscale);
-    const unsigned long long below = (1ull << lane) - 1ull;
-#pragma unroll
-    for (int v = 1; v < 3; v++) {
-      const unsigned long long m = __ballot(v < nvp);
-      if (m == 0ull) break;
-      if (v < nvp) {
-        const int s = (qhead + qlen + __popcll(m & below)) & (QC - 1);
-        Q[0][s] = vp[v].x0;
-        Q[1][s] = vp[v].y0;
-        Q[2][s] = vp[v].x1;
-        Q[3][s] = vp[v].y1;
-        Q[4][s] = vp[v].q;
-        Q[5][s] = vp[v].vz;
-        QN[s] = nb0 + vp[v].dj * JS + vp[v].di;
-      }
-      qlen += __popcll(m);
-      if (qlen >= 64) {
-        deposit_queue(qhead, 64);
-        qhead = (qhead + 64) & (QC - 1);
-        qlen -= 64;
-      }
-    }
-    // ---- store: stay in place, or leave through the mover buffer
-    const int nix = wrap1(lx + cx0 + dix, nx), niy = wrap1(ly + cy0 + diy, ny);
-    const uint32_t ncell = pack2(nix, niy);
-    const bool stay = (nix / TX + g.ntx * (niy / TY)) == tile;
-    const float xs = x1 - tx, ys = y1 - ty;
-    if (act && stay) {
-      *el(Wcell, up) = ncell;
-      *el(Wx, up) = xs;
-      *el(Wy, up) = ys;
-      *el(Wux, up) = u1;
-      *el(Wuy, up) = u2;
-      *el(Wuz, up) = u3;
-    }
-    const bool mv = act && !stay;
-    const unsigned long long mm = __ballot(mv);
-    if (mv) {
-      const unsigned slot = (unsigned)(w0 + mcount + __popcll(mm & below));
-      *el(Mcell, slot) = ncell;
-      *el(Mx, slot) = xs;
-      *el(My, slot) = ys;
-      *el(Mux, slot) = u1;
-      *el(Muy, slot) = u2;
-      *el(Muz, slot) = u3;
-      *el(Mq, slot) = q;
-      *el(Mpid, slot) = pid;
-      *el(Midx, slot) = p;
-    }
-    mcount += __popcll(mm);
-  }
-  if (qlen > 0) deposit_queue(qhead, qlen);
+  const bool raw = d.jraw != 0;
+  if (raw)
+    push_all(std::true_type());
+  else
+    push_all(std::false_type());
 
   if (bad) atomicOr(&g.ctrl->error, 1);
   if (lane == 0) d.mv_cnt[tile * NW * split + tw] = mcount;
@@ -319,13 +372,12 @@ __global__ __launch_bounds__(64 * NW, 4) void push_deposit_2d_t(const SpecDesc* 
   }
   // ---- fold the LDS current tile into the global fixed-point J (periodic wrap)
   gu64* __restrict__ GJ = (gu64*)g.J + co;
-  for (int i = threadIdx.x; i < JX * JY; i += NT) {
-    const int col = i % JX, row = i / JX, li = row * JS + col;
-    const int gx = wrapi(cx0 + col - O::JLO, nx), gy = wrapi(cy0 + row - O::JLO, ny);
+  for (int i = threadIdx.x; i < JN; i += NT) {
+    const int gx = wrapi(cx0 + i % JX - O::JLO, nx), gy = wrapi(cy0 + i / JX - O::JLO, ny);
     const long long gi = gx + (long long)nx * gy;
 #pragma unroll
     for (int c = 0; c < 3; c++) {
-      const unsigned long long v = sJ[c * JN + li];
+      const unsigned long long t = sJ[c * JN + i], v = raw ? fix_sum<true>(t) : t;
       if (v) __hip_atomic_fetch_add(&GJ[c * nc + gi], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
   }

@@ -34,9 +34,9 @@ OSR_DEV float fma_(float a, float b, float c) { return __builtin_fmaf(a, b, c); 
 // |a| >= 2^-79 (the remainder then stays normal) whose quotient is normal, and for +0
 // numerators (a -0 numerator gives +0).  The push path
 // uses them only there: sqrt_rn on 1 + u^2, div_rn on numerators that are tem, 1, 2 or
-// +-1/2 - x0 (at least 2^-25 in magnitude, or exactly +0).  The kinetic energy
-// u^2 / (gamma + 1), whose numerator can be denormal, and Vay's inner roots keep the
-// IEEE operations.  The compiler's IEEE sequences (-fhip-fp32-correctly-rounded-divide-
+// +-1/2 - x0 (at least 2^-25 in magnitude, or exactly +0), and on u^2 of Boris' kinetic
+// energy u^2 / (gamma + 1), where a numerator below 2^-24 meets the divisor 2.  Vay's
+// energy and inner roots keep the IEEE operations.  The compiler's IEEE sequences (-fhip-fp32-correctly-rounded-divide-
 // sqrt) also scale operands for the denormal and overflow ranges; the shorter forms
 // leave that out.
 // ------------------------------------------------------------------------------------
@@ -158,7 +158,9 @@ OSR_DEV float boris(float tem, float e1, float e2, float e3, float b1, float b2,
   float ut1 = u1 + e1, ut2 = u2 + e2, ut3 = u3 + e3;
   float utsq = fma_(ut3, ut3, fma_(ut2, ut2, ut1 * ut1));
   float gamma = sqrt_rn(utsq + 1.0f);
-  float ene = utsq / (gamma + 1.0f);  // IEEE: utsq can be denormal
+  // div_rn is exact here for every utsq: gamma + 1 differs from 2 only for utsq > 2^-24, and
+  // a / 2 is the correctly rounded half also when a or the half is denormal
+  float ene = div_rn(utsq, gamma + 1.0f);
   float tg = div_rn(tem, gamma);
   b1 = b1 * tg;
   b2 = b2 * tg;
@@ -244,9 +246,18 @@ OSR_DEV long long to_fix(float v, double scale) {
   double t = __builtin_fma((double)v, scale, 6755399441055744.0);
   return __double_as_longlong(t) - 0x4338000000000000LL;
 }
-// the integer held by t = fma(a, b, 1.5*2^52), as the 64-bit pattern of the sum
+// the integer held by t = fma(a, b, 1.5*2^52), as the 64-bit pattern of the sum.  RAW: the
+// bits of t as they are, the integer plus 0x4338 << 48, a multiple of 2^51: a sum of any
+// number of them holds the sum of the integers in its low 51 bits, and when that is known to
+// lie within +-2^50 fix_sum recovers it, which saves the subtraction of each term.
+template <bool RAW = false>
 OSR_DEV unsigned long long fix_bits(double t) {
+  if (RAW) return (unsigned long long)__double_as_longlong(t);
   return (unsigned long long)(__double_as_longlong(t) - 0x4338000000000000LL);
+}
+template <bool RAW>
+OSR_DEV unsigned long long fix_sum(unsigned long long v) {
+  return RAW ? (unsigned long long)((long long)(v << 13) >> 13) : v;
 }
 
 // Charge-conserving deposit of one VP into the LDS current tile (DEP_CURRENT_2D,
@@ -261,7 +272,7 @@ OSR_DEV unsigned long long fix_bits(double t) {
 // grid by fma(a, b, 1.5*2^52): one FMA and one integer add per contribution.  The j3 bracket
 // is evaluated as A S0y + B S1y with A = S0x + S1x/2, B = S1x + S0x/2 (two FP32 operations
 // per node).  |a b 2^s| < 2^51 for every contribution (bound of the scale choice).
-template <int ORDER>
+template <int ORDER, bool RAW = false>
 OSR_DEV void dep_vp(unsigned long long* __restrict__ J1, unsigned long long* __restrict__ J2,
                     unsigned long long* __restrict__ J3, const float* S0x, const float* S0y,
                     float x0, float y0, float x1, float y1, float q, float vz, int nb, int js,
@@ -294,9 +305,9 @@ OSR_DEV void dep_vp(unsigned long long* __restrict__ J1, unsigned long long* __r
     for (int k1 = 0; k1 < NP; k1++) {
       const int idx = nb + k2 * js + k1;
       const float t1 = fma_(B[k1], S1y[k2], A[k1] * S0y[k2]);
-      if (k1 < NP - 1) atomicAdd(&J1[idx], fix_bits(__builtin_fma(a1[k1], b1[k2], M)));
-      if (k2 < NP - 1) atomicAdd(&J2[idx], fix_bits(__builtin_fma(a2[k2], b2[k1], M)));
-      atomicAdd(&J3[idx], fix_bits(__builtin_fma(c3, (double)t1, M)));
+      if (k1 < NP - 1) atomicAdd(&J1[idx], fix_bits<RAW>(__builtin_fma(a1[k1], b1[k2], M)));
+      if (k2 < NP - 1) atomicAdd(&J2[idx], fix_bits<RAW>(__builtin_fma(a2[k2], b2[k1], M)));
+      atomicAdd(&J3[idx], fix_bits<RAW>(__builtin_fma(c3, (double)t1, M)));
     }
   }
 }

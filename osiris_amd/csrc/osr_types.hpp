@@ -144,6 +144,7 @@ struct SpecDesc {
   int* inc;        // [ntiles] incoming count
   double* epart;   // [ntiles][split] time-centred energy partial sums (un-normalised)
   float tem;       // (float)(0.5*dt/rqm)
+  int jraw;        // no node sum of a tile's current can leave +-2^50 (fix_bits, RAW)
   int split;       // workgroups per tile in the push (1 in 3D and with the generic kernel)
   int waves;       // waves per tile in the push: those of its workgroups times split
 };

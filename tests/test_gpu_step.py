@@ -43,6 +43,35 @@ def test_push_workgroups_per_tile(nx, tile, waves):
     _same(_run(2, nx, 2, 6, tile=tile, push_waves=waves), _run(2, nx, 2, 6, tile=tile, kernel=1))
 
 
+@pytest.mark.parametrize("dims,order,pusher", [(2, 1, 0), (2, 2, 1), (2, 3, 0), (3, 1, 1), (3, 2, 0), (3, 3, 1)])
+@pytest.mark.parametrize("case", ["all_cross", "none_cross", "one_cell"])
+def test_push_crossing_queue(dims, order, pusher, case):
+    """The queue of face-crossing particles: every particle of a wave crosses (up to all
+    faces at once), none does, and thousands pile up in one cell; grids large enough for the
+    raw fixed-point sums, against the generic kernel (bit for bit)."""
+    print(f"case dims={dims} order={order} pusher={pusher} {case}", flush=True)
+    nx = (256, 192) if dims == 2 else (48, 40, 24)
+    out = []
+    for kernel in (0, 1):
+        with oa.Simulation(dims, nx, (0.1,) * dims, 0.055, order, kernel=kernel) as sim:
+            rng = np.random.default_rng(3)
+            n = 150_001
+            ix = np.stack([rng.integers(1, m + 1, n) for m in nx], 1).astype(np.int32)
+            if case == "one_cell":
+                ix[:5000] = 17
+            x = (rng.random((n, dims), np.float32) - np.float32(0.5)).astype(np.float32)
+            u = (rng.standard_normal((n, 3)) * (1e-23 if case == "none_cross" else 0.1)).astype(np.float32)
+            if case == "all_cross":
+                u[:, :dims] = np.where(rng.random((n, dims)) < 0.5, -5.0, 5.0)
+                x[:, :dims] = np.sign(u[:, :dims]) * np.float32(0.49)
+            sid = sim.add_species(-1.0, pusher)
+            sim.set_particles(sid, ix, x, u, np.full(n, -0.01, np.float32))
+            sim.fill_fields(b0=(0.0, 0.0, 0.2) if case != "none_cross" else (0.0, 0.0, 0.0))
+            sim.run(3)
+            out.append((sim.get_fields(), sim.get_particles(0), (), sim.history()))
+    _same(*out)
+
+
 @pytest.mark.parametrize("nx,order", [((1, 1), 1), ((2, 3), 2), ((31, 7), 1), ((33, 9), 2), ((65, 17), 3),
                                       ((32, 8), 1), ((700, 600), 2), ((1024, 512), 1)])
 def test_fused_field_step(nx, order):
