@@ -34,9 +34,9 @@ OSR_DEV float fma_(float a, float b, float c) { return __builtin_fmaf(a, b, c); 
 // |a| >= 2^-79 (the remainder then stays normal) whose quotient is normal, and for +0
 // numerators (a -0 numerator gives +0).  The push path
 // uses them only there: sqrt_rn on 1 + u^2, div_rn on numerators that are tem, 1, 2 or
-// +-1/2 - x0 (at least 2^-25 in magnitude, or exactly +0), and on u^2 of Boris' kinetic
-// energy u^2 / (gamma + 1), where a numerator below 2^-24 meets the divisor 2.  Vay's
-// energy and inner roots keep the IEEE operations.  The compiler's IEEE sequences (-fhip-fp32-correctly-rounded-divide-
+// +-1/2 - x0 (at least 2^-25 in magnitude, or exactly +0), and on u^2 of the kinetic
+// energies u^2 / (gamma + 1), where a numerator below 2^-24 meets the divisor 2.  Vay's
+// inner roots take the IEEE operations outside that range.  The compiler's IEEE sequences (-fhip-fp32-correctly-rounded-divide-
 // sqrt) also scale operands for the denormal and overflow ranges; the shorter forms
 // leave that out.
 // ------------------------------------------------------------------------------------
@@ -207,8 +207,13 @@ OSR_DEV float vay(float tem, float e1, float e2, float e3, float b1, float b2, f
   float w1 = ut1 + e1, w2 = ut2 + e2, w3 = ut3 + e3;
   float ustar = w1 * b1 + w2 * b2 + w3 * b3;
   float sigma = 1.0f + w1 * w1 + w2 * w2 + w3 * w3 - bpsq;
-  rgam = 1.0f / __builtin_sqrtf(0.5f * (sigma + __builtin_sqrtf(sigma * sigma +
-                                                                 4.0f * (bpsq + ustar * ustar))));
+  // Both arguments are at least 1 up to rounding, except where sigma < 0 cancels (|tau|^2 far
+  // above 1 + u^2) or sigma^2 overflows: those waves take the IEEE operations.
+  const float in = sigma * sigma + 4.0f * (bpsq + ustar * ustar);
+  const bool in_ok = in >= 1.0e-29f && in <= 3.0e38f;
+  const float so = 0.5f * (sigma + (__all(in_ok) ? sqrt_rn(in) : __builtin_sqrtf(in)));
+  const bool so_ok = so >= 1.0e-29f && so <= 3.0e38f;
+  rgam = __all(so_ok) ? rcp_rn(sqrt_rn(so)) : 1.0f / __builtin_sqrtf(so);
   b1 *= rgam; b2 *= rgam; b3 *= rgam;
   float spar = rcp_rn(1.0f + b1 * b1 + b2 * b2 + b3 * b3);
   float uptp = w1 * b1 + w2 * b2 + w3 * b3;
@@ -219,7 +224,7 @@ OSR_DEV float vay(float tem, float e1, float e2, float e3, float b1, float b2, f
   float uc1 = 0.5f * (o1 + u1), uc2 = 0.5f * (o2 + u2), uc3 = 0.5f * (o3 + u3);
   float uc2s = uc1 * uc1 + uc2 * uc2 + uc3 * uc3;
   float gc = sqrt_rn(uc2s + 1.0f);
-  return uc2s / (gc + 1.0f);  // IEEE: uc2s can be denormal
+  return div_rn(uc2s, gc + 1.0f);  // as in boris
 }
 
 template <int PUSHER>
@@ -467,7 +472,7 @@ OSR_DEV VP3 pick(const VP3* vp, int v) {
 // int64 grid: one FMA and one integer add per node.  S0x/S0y/S0z are the splines of the
 // VP's start point, nb its first stencil node, jy/jz the row and plane pitches of the
 // tile, JN the size of one component plane.
-template <int ORDER>
+template <int ORDER, bool RAW = false>
 OSR_DEV void dep_vp3(unsigned long long* __restrict__ J, int JN, const float* S0x,
                      const float* S0y, const float* S0z, float x0, float y0, float z0, float x1,
                      float y1, float z1, float q, int nb, int jy, int jz, float jn1, float jn2,
@@ -500,14 +505,14 @@ OSR_DEV void dep_vp3(unsigned long long* __restrict__ J, int JN, const float* S0
 #pragma unroll
       for (int k1 = 0; k1 < NP; k1++) {
         const int idx = nb + k3 * jz + k2 * jy + k1;
-        if (k1 < NP - 1) atomicAdd(&J[idx], fix_bits(__builtin_fma(a1[k1], b1, M)));
+        if (k1 < NP - 1) atomicAdd(&J[idx], fix_bits<RAW>(__builtin_fma(a1[k1], b1, M)));
         if (k2 < NP - 1) {
           const double b2 = (double)wp(S0x[k1], S1x[k1], S0z[k3], S1z[k3]);
-          atomicAdd(&J[JN + idx], fix_bits(__builtin_fma(a2[k2], b2, M)));
+          atomicAdd(&J[JN + idx], fix_bits<RAW>(__builtin_fma(a2[k2], b2, M)));
         }
         if (k3 < NP - 1) {
           const double b3 = (double)wp(S0x[k1], S1x[k1], S0y[k2], S1y[k2]);
-          atomicAdd(&J[2 * JN + idx], fix_bits(__builtin_fma(a3[k3], b3, M)));
+          atomicAdd(&J[2 * JN + idx], fix_bits<RAW>(__builtin_fma(a3[k3], b3, M)));
         }
       }
     }

@@ -34,7 +34,9 @@ constexpr int kMaxPushWaves = 8;
 // owns a contiguous slice of its particles and a mover region, whichever workgroup it is in.
 constexpr int kMaxSplit = 4;
 constexpr int kMaxTileWaves = 16;
-// capacity of the per-wave virtual-particle queue of the 3D push (pending < 64 plus up to
+// waves per workgroup of the compile-time 3D push
+__host__ __device__ constexpr int push3d_waves(int order) { return order == 3 ? 4 : 8; }
+// capacity of the per-wave virtual-particle queue of the generic 3D push (pending < 64 plus up to
 // 64 appended per VP level)
 constexpr int kVpQueue3 = 128;
 // default waves per workgroup of the 2D compile-time tile kernels
@@ -153,7 +155,7 @@ struct SpecDesc {
 __host__ __device__ inline uint32_t pack2(int ix, int iy) {
   return (uint32_t)ix | ((uint32_t)iy << 16);
 }
-__host__ __device__ inline uint32_t pack3(int ix, int iy, int iz) {
+__host__ __device__ constexpr uint32_t pack3(int ix, int iy, int iz) {
   return (uint32_t)ix | ((uint32_t)iy << 11) | ((uint32_t)iz << 22);
 }
 __host__ __device__ inline void unpack2(uint32_t c, int& ix, int& iy) {
