@@ -80,6 +80,7 @@ __global__ __launch_bounds__(64 * NW, 4) void push_deposit_2d_t(const SpecDesc* 
   __shared__ LV s3[GN], s6[GN];
   __shared__ unsigned long long sJ[3 * JN];
   __shared__ f32x4 sQ[NW][2][QC];  // (x0, y0, x1, y1), (q, vz, node and cell shifts)
+  __shared__ int sQn[NW];
   __shared__ double s_ene[NW];
 
   const int2 wk = work[blockIdx.x];
@@ -177,17 +178,29 @@ __global__ __launch_bounds__(64 * NW, 4) void push_deposit_2d_t(const SpecDesc* 
     int qlen = 0;
     f32x4* const Q0 = sQ[wave][0];
     f32x4* const Q1 = sQ[wave][1];
-    // split and deposit of the queued particles, one per lane
-    auto deposit_queue = [&]() {
-      if (lane < qlen) {
-        const f32x4 a = Q0[lane], b = Q1[lane];
-        const int code = __float_as_int(b.z), nb0 = code >> 4;
-        VP2 vp[3];
-        const int nvp = split2d_fast(a.x, a.y, a.z, a.w, (code & 3) - 1, ((code >> 2) & 3) - 1, b.x,
-                                     b.y, vp);
+    const unsigned long long below = (1ull << lane) - 1ull;
+    // split and deposit of queued particles, one per lane (on: the lane holds one, (a, b));
+    // the third virtual particles of double crossings are queued again, as particles that
+    // cross nothing
+    auto deposit_queue = [&](bool on, const f32x4& a, const f32x4& b) {
+      VP2 vp[3];
+      int nvp = 0, nb0 = 0;
+      if (on) {
+        const int code = __float_as_int(b.z);
+        nb0 = code >> 4;
+        nvp = split2d_fast(a.x, a.y, a.z, a.w, (code & 3) - 1, ((code >> 2) & 3) - 1, b.x, b.y, vp);
+      }
+      const unsigned long long m2 = __ballot(nvp > 2);
+      qlen = __popcll(m2);
+      if (nvp > 2) {
+        const int s = __popcll(m2 & below);
+        Q0[s] = f32x4{vp[2].x0, vp[2].y0, vp[2].x1, vp[2].y1};
+        Q1[s] = f32x4{vp[2].q, vp[2].vz,
+                      __int_as_float((nb0 + vp[2].dj * JX + vp[2].di) * 16 + 1 + 4), 0.f};
+      }
 #pragma unroll
-        for (int v = 0; v < 3; v++) {
-          if (v == 2 && nvp < 3) break;  // a queued particle has crossed one face at least
+      for (int v = 0; v < 2; v++) {
+        if (v < nvp) {
           float S0x[NP], S0y[NP];
           spline<ORDER>(vp[v].x0, S0x);
           spline<ORDER>(vp[v].y0, S0y);
@@ -195,7 +208,6 @@ __global__ __launch_bounds__(64 * NW, 4) void push_deposit_2d_t(const SpecDesc* 
                              vp[v].vz, nb0 + vp[v].dj * JX + vp[v].di, JX, jn1, jn2, jscale);
         }
       }
-      qlen = 0;
     };
     // The particle loads of the next iteration are issued before the current one is
     // processed (software pipelining): a wave otherwise waits a full memory latency per
@@ -215,141 +227,156 @@ __global__ __launch_bounds__(64 * NW, 4) void push_deposit_2d_t(const SpecDesc* 
       f_pid = *el(Ppid, upf);
     };
     if (w0 < w1) prefetch(w0 + lane);
-    for (int p0 = w0;; p0 += 64) {
-      const bool more = p0 < w1;  // the pass after the last particles empties the queue
-      bool cross = false;
-      f32x4 qa, qb;
-      if (more) {
-        const int p = p0 + lane;
-        const unsigned up = (unsigned)p;  // 32-bit unsigned offsets from the scalar bases
-        const uint32_t cell = f_cell, pid = f_pid;
-        const float x = f_x, y = f_y, q = f_q;
-        float u1 = f_u1, u2 = f_u2, u3 = f_u3;
-        if (p0 + 64 < w1) prefetch(p + 64);
-        // cell within the tile: both halves of the difference in range (a borrow shows too)
-        const uint32_t dl = cell - cell0;
-        const bool out = (dl & ~((TX - 1u) | ((TY - 1u) << 16))) != 0u;
-        const bool act = p < w1 && !out;
-        bad |= p < w1 && out;
-        const int lx = (int)(dl & (TX - 1u)), ly = (int)((dl >> 16) & (TY - 1u));
-        // ---- gather
-        float wx[NP], wy[NP], wxh[NP], wyh[NP];
-        spline<ORDER>(x, wx);
-        spline<ORDER>(y, wy);
-        splineh<ORDER>(x, x < 0.f ? 1.f : 0.f, wxh);
-        splineh<ORDER>(y, y < 0.f ? 1.f : 0.f, wyh);
-        const int gb = (ly + O::GLO + O::LP) * GX + lx + O::GLO + O::LP;
-        const int gbx = gb - (x < 0.f ? 1 : 0);
-        const int gby = gb - (y < 0.f ? GX : 0);
-        const int gbxy = gbx - (y < 0.f ? GX : 0);
-        float e1 = 0.f, e2 = 0.f, e3 = 0.f, b1 = 0.f, b2 = 0.f, b3 = 0.f;
+    for (int p0 = w0; p0 < w1; p0 += 64) {
+      const int p = p0 + lane;
+      const unsigned up = (unsigned)p;  // 32-bit unsigned offsets from the scalar bases
+      const uint32_t cell = f_cell, pid = f_pid;
+      const float x = f_x, y = f_y, q = f_q;
+      float u1 = f_u1, u2 = f_u2, u3 = f_u3;
+      if (p0 + 64 < w1) prefetch(p + 64);
+      // cell within the tile: both halves of the difference in range (a borrow shows too)
+      const uint32_t dl = cell - cell0;
+      const bool out = (dl & ~((TX - 1u) | ((TY - 1u) << 16))) != 0u;
+      const bool act = p < w1 && !out;
+      bad |= p < w1 && out;
+      const int lx = (int)(dl & (TX - 1u)), ly = (int)((dl >> 16) & (TY - 1u));
+      // ---- gather
+      float wx[NP], wy[NP], wxh[NP], wyh[NP];
+      spline<ORDER>(x, wx);
+      spline<ORDER>(y, wy);
+      splineh<ORDER>(x, x < 0.f ? 1.f : 0.f, wxh);
+      splineh<ORDER>(y, y < 0.f ? 1.f : 0.f, wyh);
+      const int gb = (ly + O::GLO + O::LP) * GX + lx + O::GLO + O::LP;
+      const int gbx = gb - (x < 0.f ? 1 : 0);
+      const int gby = gb - (y < 0.f ? GX : 0);
+      const int gbxy = gbx - (y < 0.f ? GX : 0);
+      float e1 = 0.f, e2 = 0.f, e3 = 0.f, b1 = 0.f, b2 = 0.f, b3 = 0.f;
 #pragma unroll
-        for (int k2 = 0; k2 < NP; k2++) {
-          // the row's line of each stencil
-          float r12[2 * NP + 2], r21[2 * NP + 2], r3[NP + 1], r6[NP + 1];
-          auto pairs = [&](const f32x4* L, float* r) {
+      for (int k2 = 0; k2 < NP; k2++) {
+        // the row's line of each stencil
+        float r12[2 * NP + 2], r21[2 * NP + 2], r3[NP + 1], r6[NP + 1];
+        auto pairs = [&](const f32x4* L, float* r) {
 #pragma unroll
-            for (int k1 = 0; k1 < NP; k1 += 2) {
-              f32x4 v = L[k1];
-              if (k1 + 1 == NP) asm("" : "+v"(v));  // a full read: the low half alone is slower
-              r[2 * k1] = v.x;
-              r[2 * k1 + 1] = v.y;
-              r[2 * k1 + 2] = v.z;
-              r[2 * k1 + 3] = v.w;
-            }
-          };
-          auto line = [&](const LV* L, float* r) {
-#pragma unroll
-            for (int k1 = 0; k1 < NP; k1 += LW) {
-              const LV v = L[k1];
-#pragma unroll
-              for (int k = 0; k < LW; k++)
-                if (k1 + k < NP) r[k1 + k] = v[k];
-            }
-          };
-          pairs(s12 + gbx + k2 * GX, r12);
-          pairs(s21 + gby + k2 * GX, r21);
-          line(s3 + gb + k2 * GX, r3);
-          line(s6 + gbxy + k2 * GX, r6);
-          float le1 = 0.f, le2 = 0.f, le3 = 0.f, lb1 = 0.f, lb2 = 0.f, lb3 = 0.f;
-#pragma unroll
-          for (int k1 = 0; k1 < NP; k1++) {
-            le1 = fma_(r12[2 * k1], wxh[k1], le1);
-            le2 = fma_(r21[2 * k1], wx[k1], le2);
-            le3 = fma_(r3[k1], wx[k1], le3);
-            lb1 = fma_(r21[2 * k1 + 1], wx[k1], lb1);
-            lb2 = fma_(r12[2 * k1 + 1], wxh[k1], lb2);
-            lb3 = fma_(r6[k1], wxh[k1], lb3);
+          for (int k1 = 0; k1 < NP; k1 += 2) {
+            f32x4 v = L[k1];
+            if (k1 + 1 == NP) asm("" : "+v"(v));  // a full read: the low half alone is slower
+            r[2 * k1] = v.x;
+            r[2 * k1 + 1] = v.y;
+            r[2 * k1 + 2] = v.z;
+            r[2 * k1 + 3] = v.w;
           }
-          e1 = fma_(le1, wy[k2], e1);
-          e2 = fma_(le2, wyh[k2], e2);
-          e3 = fma_(le3, wy[k2], e3);
-          b1 = fma_(lb1, wyh[k2], b1);
-          b2 = fma_(lb2, wy[k2], b2);
-          b3 = fma_(lb3, wyh[k2], b3);
+        };
+        auto line = [&](const LV* L, float* r) {
+#pragma unroll
+          for (int k1 = 0; k1 < NP; k1 += LW) {
+            const LV v = L[k1];
+#pragma unroll
+            for (int k = 0; k < LW; k++)
+              if (k1 + k < NP) r[k1 + k] = v[k];
+          }
+        };
+        pairs(s12 + gbx + k2 * GX, r12);
+        pairs(s21 + gby + k2 * GX, r21);
+        line(s3 + gb + k2 * GX, r3);
+        line(s6 + gbxy + k2 * GX, r6);
+        float le1 = 0.f, le2 = 0.f, le3 = 0.f, lb1 = 0.f, lb2 = 0.f, lb3 = 0.f;
+#pragma unroll
+        for (int k1 = 0; k1 < NP; k1++) {
+          le1 = fma_(r12[2 * k1], wxh[k1], le1);
+          le2 = fma_(r21[2 * k1], wx[k1], le2);
+          le3 = fma_(r3[k1], wx[k1], le3);
+          lb1 = fma_(r21[2 * k1 + 1], wx[k1], lb1);
+          lb2 = fma_(r12[2 * k1 + 1], wxh[k1], lb2);
+          lb3 = fma_(r6[k1], wxh[k1], lb3);
         }
-        // ---- push
-        const float ke = push<PUSHER>(tem, e1, e2, e3, b1, b2, b3, u1, u2, u3);
-        ene = __builtin_fma((double)(act ? q : 0.f), (double)ke, ene);
-        // ---- position
-        const float rg = rgamma(u1, u2, u3);
-        const float v1 = u1 * rg, v2 = u2 * rg, v3 = u3 * rg;
-        const float x1 = fma_(v1, dtdx1, x), y1 = fma_(v2, dtdx2, y);
-        const float tx = trim(x1), ty = trim(y1);
-        const int dix = (int)tx, diy = (int)ty;
-        // ---- deposit of the particles that stay in their cell: one VP, with the gather's
-        // splines; the others are queued for the split
-        const int nb0 = (ly + O::LP + O::JLO) * JX + lx + O::LP + O::JLO;
-        cross = act && (dix | diy) != 0;
-        qa = f32x4{x, y, x1, y1};
-        qb = f32x4{q, v3, __int_as_float(nb0 * 16 + (dix + 1) + 4 * (diy + 1)), 0.f};
-        if (act && !cross)
-          dep_vp<ORDER, RAW>(J1, J2, J3, wx, wy, x, y, x1, y1, q, v3, nb0, JX, jn1, jn2, jscale);
-        const unsigned long long below = (1ull << lane) - 1ull;
-        // ---- store: stay in place, or leave through the mover buffer
-        const int nlx = lx + dix, nly = ly + diy;
-        bool stay = (unsigned)nlx < (unsigned)tcx && (unsigned)nly < (unsigned)tcy;
-        uint32_t ncell = cell0 + pack2(0, nly) + (uint32_t)nlx;
-        if (lone || !__all(stay || !act)) {
-          const int nix = wrap1(nlx + cx0, nx), niy = wrap1(nly + cy0, ny);
-          ncell = pack2(nix, niy);
-          stay = (nix / TX + g.ntx * (niy / TY)) == tile;
-        }
-        const float xs = x1 - tx, ys = y1 - ty;
-        if (act && stay) {
-          *el(Wcell, up) = ncell;
-          *el(Wx, up) = xs;
-          *el(Wy, up) = ys;
-          *el(Wux, up) = u1;
-          *el(Wuy, up) = u2;
-          *el(Wuz, up) = u3;
-        }
-        const bool mv = act && !stay;
-        const unsigned long long mm = __ballot(mv);
-        if (mv) {
-          const unsigned slot = (unsigned)(w0 + mcount + __popcll(mm & below));
-          *el(Mcell, slot) = ncell;
-          *el(Mx, slot) = xs;
-          *el(My, slot) = ys;
-          *el(Mux, slot) = u1;
-          *el(Muy, slot) = u2;
-          *el(Muz, slot) = u3;
-          *el(Mq, slot) = q;
-          *el(Mpid, slot) = pid;
-          *el(Midx, slot) = p;
-        }
-        mcount += __popcll(mm);
+        e1 = fma_(le1, wy[k2], e1);
+        e2 = fma_(le2, wyh[k2], e2);
+        e3 = fma_(le3, wy[k2], e3);
+        b1 = fma_(lb1, wyh[k2], b1);
+        b2 = fma_(lb2, wy[k2], b2);
+        b3 = fma_(lb3, wyh[k2], b3);
       }
+      // ---- push
+      const float ke = push<PUSHER>(tem, e1, e2, e3, b1, b2, b3, u1, u2, u3);
+      ene = __builtin_fma((double)(act ? q : 0.f), (double)ke, ene);
+      // ---- position
+      const float rg = rgamma(u1, u2, u3);
+      const float v1 = u1 * rg, v2 = u2 * rg, v3 = u3 * rg;
+      const float x1 = fma_(v1, dtdx1, x), y1 = fma_(v2, dtdx2, y);
+      const float tx = trim(x1), ty = trim(y1);
+      const int dix = (int)tx, diy = (int)ty;
+      // ---- deposit of the particles that stay in their cell: one VP, with the gather's
+      // splines; the others are queued for the split
+      const int nb0 = (ly + O::LP + O::JLO) * JX + lx + O::LP + O::JLO;
+      const bool cross = act && (dix | diy) != 0;
+      const f32x4 qa = {x, y, x1, y1};
+      const f32x4 qb = {q, v3, __int_as_float(nb0 * 16 + (dix + 1) + 4 * (diy + 1)), 0.f};
+      if (act && !cross)
+        dep_vp<ORDER, RAW>(J1, J2, J3, wx, wy, x, y, x1, y1, q, v3, nb0, JX, jn1, jn2, jscale);
+      // ---- store: stay in place, or leave through the mover buffer
+      const int nlx = lx + dix, nly = ly + diy;
+      bool stay = (unsigned)nlx < (unsigned)tcx && (unsigned)nly < (unsigned)tcy;
+      uint32_t ncell = cell0 + pack2(0, nly) + (uint32_t)nlx;
+      if (lone || !__all(stay || !act)) {
+        const int nix = wrap1(nlx + cx0, nx), niy = wrap1(nly + cy0, ny);
+        ncell = pack2(nix, niy);
+        stay = (nix / TX + g.ntx * (niy / TY)) == tile;
+      }
+      const float xs = x1 - tx, ys = y1 - ty;
+      if (act && stay) {
+        *el(Wcell, up) = ncell;
+        *el(Wx, up) = xs;
+        *el(Wy, up) = ys;
+        *el(Wux, up) = u1;
+        *el(Wuy, up) = u2;
+        *el(Wuz, up) = u3;
+      }
+      const bool mv = act && !stay;
+      const unsigned long long mm = __ballot(mv);
+      if (mv) {
+        const unsigned slot = (unsigned)(w0 + mcount + __popcll(mm & below));
+        *el(Mcell, slot) = ncell;
+        *el(Mx, slot) = xs;
+        *el(My, slot) = ys;
+        *el(Mux, slot) = u1;
+        *el(Muy, slot) = u2;
+        *el(Muz, slot) = u3;
+        *el(Mq, slot) = q;
+        *el(Mpid, slot) = pid;
+        *el(Midx, slot) = p;
+      }
+      mcount += __popcll(mm);
       const unsigned long long mc = __ballot(cross);
       const int add = __popcll(mc);
-      if (qlen + add > QC || (!more && qlen > 0)) deposit_queue();
-      if (!more) break;
+      // twice at most: what a first call queues again crosses nothing
+      while (qlen + add > QC) deposit_queue(lane < qlen, Q0[lane], Q1[lane]);
       if (cross) {
-        const int s = qlen + __popcll(mc & ((1ull << lane) - 1ull));
+        const int s = qlen + __popcll(mc & below);
         Q0[s] = qa;
         Q1[s] = qb;
       }
       qlen += add;
+    }
+    // What is left in the queues, shared over the waves so that it runs on full ones: at most
+    // NW QC entries, one batch per wave.  The second round takes what the first queued again.
+    for (;;) {
+      if (lane == 0) sQn[wave] = qlen;
+      __syncthreads();
+      int left = 64 * wave + lane, total = 0, w = 0;  // this lane's entry: `left` of queue w
+#pragma unroll
+      for (int k = 0; k < NW; k++) {
+        const int c = sQn[k];
+        total += c;
+        if (w == k && left >= c) {
+          left -= c;
+          w = k + 1;
+        }
+      }
+      const bool on = w < NW;
+      const f32x4 a = sQ[on ? w : 0][0][on ? left : 0], b = sQ[on ? w : 0][1][on ? left : 0];
+      __syncthreads();  // every wave has its entries before the queues are written again
+      if (total == 0) break;
+      deposit_queue(on, a, b);
     }
   };
   const bool raw = d.jraw != 0;
