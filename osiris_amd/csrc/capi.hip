@@ -19,6 +19,7 @@
 #include "k_field.hip"
 #include "k_smooth.hip"
 #include "k_loader.hip"
+#include "k_readback.hip"
 #include "k_tiles.hip"
 #include "k_push2d.hip"
 #include "k_push3d.hip"
@@ -142,6 +143,7 @@ struct Species {
   float rqm = -1.f;
   int pusher = OSR_BORIS;
   int64_t np = 0;
+  int64_t npid = 0;  // particles given at first: their pids are 0 .. npid - 1
   int64_t cap_total = 0;
   double qabs = 0.0, qmax = 0.0;
   DBuf cell, x, y, z, ux, uy, uz, q, pid;
@@ -739,28 +741,6 @@ int collect(osr_sim* s, Species& p, bool pending, HostParts& hp) {
             push(mcell, mpid, mx, my, mz, mux, muy, muz, mq, m);
         }
   return OSR_OK;
-}
-
-// Stable order by pid, used to return particles in the order they were given.
-void sort_by_pid(HostParts& hp) {
-  const size_t n = hp.size();
-  std::vector<size_t> idx(n);
-  for (size_t i = 0; i < n; i++) idx[i] = i;
-  std::stable_sort(idx.begin(), idx.end(), [&](size_t a, size_t b) { return hp.pid[a] < hp.pid[b]; });
-  HostParts o;
-  o.reserve(n);
-  for (size_t i : idx) {
-    o.cell.push_back(hp.cell[i]);
-    o.pid.push_back(hp.pid[i]);
-    o.x.push_back(hp.x[i]);
-    o.y.push_back(hp.y[i]);
-    o.z.push_back(hp.z[i]);
-    o.ux.push_back(hp.ux[i]);
-    o.uy.push_back(hp.uy[i]);
-    o.uz.push_back(hp.uz[i]);
-    o.q.push_back(hp.q[i]);
-  }
-  hp = std::move(o);
 }
 
 // Fill kernel and its launch shape (4 waves per tile; LDS lists for up to 4096 incoming
@@ -1545,6 +1525,7 @@ int osr_species_set(osr_sim* s, int sid, int64_t np, const int* ix, const float*
   }
   HIPC(hipStreamSynchronize(s->stream));
   TRY(layout_upload(s, *s->sp[sid], hp));
+  s->sp[sid]->npid = np;
   update_jscale(s);
   TRY(upload_descs(s));
   s->graph_ok = false;
@@ -1561,28 +1542,51 @@ int osr_species_count(osr_sim* s, int sid, int64_t* np) {
 int osr_species_get(osr_sim* s, int sid, int* ix, float* x, float* u, float* q) {
   TRY(check_sim(s));
   if (sid < 0 || sid >= (int)s->sp.size()) return fail(OSR_ERR_ARG, "bad species id");
-  HIPC(hipStreamSynchronize(s->stream));
-  HostParts hp;
-  TRY(collect(s, *s->sp[sid], false, hp));
-  sort_by_pid(hp);
-  const int D = s->dims;
-  for (size_t i = 0; i < hp.size(); i++) {
-    int c[3];
-    cell_coords(s, hp.cell[i], c);
-    if (ix)
-      for (int d = 0; d < D; d++) ix[D * i + d] = c[d] + 1;
-    if (x) {
-      x[D * i] = hp.x[i];
-      x[D * i + 1] = hp.y[i];
-      if (D == 3) x[D * i + 2] = hp.z[i];
-    }
-    if (u) {
-      u[3 * i] = hp.ux[i];
-      u[3 * i + 1] = hp.uy[i];
-      u[3 * i + 2] = hp.uz[i];
-    }
-    if (q) q[i] = hp.q[i];
+  Species& p = *s->sp[sid];
+  const int nt = s->ntiles, D = s->dims;
+  const SpecDesc* spec = s->d_spec.as<SpecDesc>();
+  std::vector<int> cnt;
+  TRY(download(s->stream, cnt, p.cnt, nt));
+  int64_t n = 0;
+  for (int c : cnt) n += c;
+  if (n == 0) return OSR_OK;
+  // ranks in upload order: the pids themselves, or with gaps their prefix in a bitmap
+  DBuf map;
+  ParticlesOut a{};
+  if (n != p.npid) {
+    const long long nw = (p.npid + 31) / 32;
+    const unsigned ng = (unsigned)((nw + kPidWords - 1) / kPidWords);
+    TRY(map.alloc(sizeof(unsigned) * (2 * (size_t)nw + ng)));
+    unsigned* bits = map.as<unsigned>();
+    HIPC(hipMemsetAsync(bits, 0, sizeof(unsigned) * (size_t)nw, s->stream));
+    hipLaunchKernelGGL(pids_mark, dim3(nt), dim3(256), 0, s->stream, spec, sid, bits);
+    hipLaunchKernelGGL(pids_count, dim3(ng), dim3(256), 0, s->stream, bits, nw, bits + 2 * nw);
+    hipLaunchKernelGGL(pids_prefix, dim3(ng), dim3(256), 0, s->stream, bits, nw, bits + 2 * nw,
+                       bits + nw);
+    HIPC(hipGetLastError());
+    a.bits = bits;
+    a.pre = bits + nw;
   }
+  // in pieces of at most 2^22 particles (the device buffer stays below 170 MB)
+  const int64_t piece = std::min<int64_t>(n, 1 << 22);
+  DBuf out;
+  TRY(out.alloc(4 * (size_t)piece * (2 * D + 4)));
+  a.ix = out.as<int>();
+  a.x = (float*)(a.ix + D * piece);
+  a.u = a.x + D * piece;
+  a.q = a.u + 3 * piece;
+  for (int64_t r0 = 0; r0 < n; r0 += piece) {
+    const size_t m = (size_t)std::min(piece, n - r0);
+    a.r0 = (uint32_t)r0;
+    a.n = (uint32_t)m;
+    hipLaunchKernelGGL(particles_out, dim3(nt), dim3(256), 0, s->stream, spec, sid, a);
+    HIPC(hipGetLastError());
+    if (ix) TRY(copy_on(s->stream, ix + D * r0, a.ix, 4 * D * m, hipMemcpyDeviceToHost));
+    if (x) TRY(copy_on(s->stream, x + D * r0, a.x, 4 * D * m, hipMemcpyDeviceToHost));
+    if (u) TRY(copy_on(s->stream, u + 3 * r0, a.u, 12 * m, hipMemcpyDeviceToHost));
+    if (q) TRY(copy_on(s->stream, q + r0, a.q, 4 * m, hipMemcpyDeviceToHost));
+  }
+  HIPC(hipStreamSynchronize(s->stream));
   return OSR_OK;
 }
 
@@ -1609,6 +1613,7 @@ int osr_species_generate(osr_sim* s, int sid, const int* ppc, double density,
   }
   HIPC(hipStreamSynchronize(s->stream));
   TRY(alloc_species(s, p, cnt));
+  p.npid = p.np;
   const float q = (float)((p.rqm < 0 ? -1.0 : 1.0) * density / tot);
   p.qabs = std::fabs((double)q) * (double)p.np;
   p.qmax = std::fabs((double)q);
@@ -1654,8 +1659,32 @@ static int fields_xfer(osr_sim* s, float* e, float* b, const int* ld, const int*
   for (int d = 0; d < D; d++)
     if (ld[d] < nin[d] + gcl[d] || gcl[d] < 0) return fail(OSR_ERR_ARG, "bad field extents");
   const size_t nc = (size_t)s->g.ncell;
+  if (!set) {
+    // every array cell (guards included) gets its periodic image; with open x walls the x
+    // guard cells come from the guard band of the ring.  In pieces of whole rows, at most
+    // about 64 MB each.
+    FieldsOut a{s->g.nx, s->g.ny, s->g.nz, s->g.ncell, ld[0], ld[1],
+                {gcl[0], gcl[1], D == 3 ? gcl[2] : 0}, 0, 0};
+    const long long rows = (long long)ld[1] * (D == 3 ? ld[2] : 1);
+    const long long piece = std::min(rows, std::max(1ll, (64ll << 20) / (12ll * ld[0])));
+    DBuf out;
+    TRY(out.alloc(12 * (size_t)piece * ld[0]));
+    for (int w = 0; w < 2; w++) {
+      float* h = w == 0 ? e : b;
+      if (!h) continue;
+      for (a.row0 = 0; a.row0 < rows; a.row0 += piece) {
+        a.rows = std::min(piece, rows - a.row0);
+        hipLaunchKernelGGL(fields_out, dim3((unsigned)((a.rows * ld[0] + 255) / 256)), dim3(256), 0,
+                           s->stream, w == 0 ? cur_E(s) : cur_B(s), out.as<float>(), a);
+        HIPC(hipGetLastError());
+        TRY(copy_on(s->stream, h + 3 * (size_t)a.row0 * ld[0], out.p, 12 * (size_t)a.rows * ld[0],
+                    hipMemcpyDeviceToHost));
+      }
+    }
+    return OSR_OK;
+  }
   std::vector<float> pe(3 * nc), pb(3 * nc);
-  if (set && s->g.open_nx) {  // the guard band keeps its values
+  if (s->g.open_nx) {  // the guard band keeps its values
     HIPC(hipStreamSynchronize(s->stream));
     TRY(copy_on(s->stream, pe.data(), cur_E(s), 12 * nc, hipMemcpyDeviceToHost));
     TRY(copy_on(s->stream, pb.data(), cur_B(s), 12 * nc, hipMemcpyDeviceToHost));
@@ -1666,42 +1695,20 @@ static int fields_xfer(osr_sim* s, float* e, float* b, const int* ld, const int*
     if (D == 3) o += (size_t)ld0 * ld1 * (size_t)(k + gcl[2]);
     return 3 * o;
   };
-  if (set) {
-    for (int k = 0; k < nin[2]; k++)
-      for (int j = 0; j < nin[1]; j++)
-        for (int i = 0; i < nin[0]; i++) {
-          const size_t c = (size_t)i + (size_t)nxs[0] * (j + (size_t)nxs[1] * k);
-          const size_t r = ref(i, j, k);
-          for (int m = 0; m < 3; m++) {
-            pe[m * nc + c] = e ? e[r + m] : 0.f;
-            pb[m * nc + c] = b ? b[r + m] : 0.f;
-          }
-        }
-    HIPC(hipStreamSynchronize(s->stream));
-    if (e) TRY(copy_on(s->stream, cur_E(s), pe.data(), 12 * nc, hipMemcpyHostToDevice));
-    if (b) TRY(copy_on(s->stream, cur_B(s), pb.data(), 12 * nc, hipMemcpyHostToDevice));
-    return fields_changed(s);
-  }
-  HIPC(hipStreamSynchronize(s->stream));
-  TRY(copy_on(s->stream, pe.data(), cur_E(s), 12 * nc, hipMemcpyDeviceToHost));
-  TRY(copy_on(s->stream, pb.data(), cur_B(s), 12 * nc, hipMemcpyDeviceToHost));
-  // every array cell (guards included) gets its periodic image; with open x walls the x
-  // guard cells come from the guard band of the ring
-  const int ldk = D == 3 ? ld[2] : 1;
-  for (int k = 0; k < ldk; k++)
-    for (int j = 0; j < ld[1]; j++)
-      for (int i = 0; i < ld[0]; i++) {
-        const int ii = ((i - gcl[0]) % nxs[0] + nxs[0]) % nxs[0];
-        const int jj = ((j - gcl[1]) % nxs[1] + nxs[1]) % nxs[1];
-        const int kk = D == 3 ? ((k - gcl[2]) % nxs[2] + nxs[2]) % nxs[2] : 0;
-        const size_t c = (size_t)ii + (size_t)nxs[0] * (jj + (size_t)nxs[1] * kk);
-        const size_t r = 3 * ((size_t)i + (size_t)ld0 * (j + (size_t)ld1 * k));
+  for (int k = 0; k < nin[2]; k++)
+    for (int j = 0; j < nin[1]; j++)
+      for (int i = 0; i < nin[0]; i++) {
+        const size_t c = (size_t)i + (size_t)nxs[0] * (j + (size_t)nxs[1] * k);
+        const size_t r = ref(i, j, k);
         for (int m = 0; m < 3; m++) {
-          if (e) e[r + m] = pe[m * nc + c];
-          if (b) b[r + m] = pb[m * nc + c];
+          pe[m * nc + c] = e ? e[r + m] : 0.f;
+          pb[m * nc + c] = b ? b[r + m] : 0.f;
         }
       }
-  return OSR_OK;
+  HIPC(hipStreamSynchronize(s->stream));
+  if (e) TRY(copy_on(s->stream, cur_E(s), pe.data(), 12 * nc, hipMemcpyHostToDevice));
+  if (b) TRY(copy_on(s->stream, cur_B(s), pb.data(), 12 * nc, hipMemcpyHostToDevice));
+  return fields_changed(s);
 }
 
 int osr_fields_set(osr_sim* s, const float* e, const float* b, const int* ld, const int* gcl) {

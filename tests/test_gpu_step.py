@@ -108,3 +108,36 @@ def test_fused_field_step(nx, order):
         fld, _ = sim.history()
     want = 0.5 * dx[0] * dx[1] * np.array(rows)
     assert np.allclose(fld, want, rtol=1e-12, atol=0)
+
+
+@pytest.mark.parametrize("dims,n", [(2, 1), (2, 2047), (2, 200_000), (3, 70_000)])
+def test_particles_come_back_in_upload_order(dims, n):
+    """get_particles after absorbing walls removed some: the survivors in upload order (the
+    charges number the particles), each with its own cell, position and momentum (free
+    motion without charge-weighted forces is checked through u, which stays as given up to
+    the tiny fields of 1e-12 charges)."""
+    print(f"case dims={dims} n={n}", flush=True)
+    rng = np.random.default_rng(9)
+    nx = (64, 40, 24)[:dims]
+    ix = np.stack([rng.integers(1, m + 1, n) for m in nx], 1).astype(np.int32)
+    x = (rng.random((n, dims), np.float32) - np.float32(0.5)).astype(np.float32)
+    u = (rng.standard_normal((n, 3)) * 3.0).astype(np.float32)
+    q = (-(np.arange(n) + 1) * 1e-14).astype(np.float32)
+    with oa.Simulation(dims, nx, (0.1,) * dims, 0.05, 2, xbnd="lindman") as sim:
+        sid = sim.add_species(-1.0)
+        sim.set_particles(sid, ix, x, u, q)
+        got0 = sim.get_particles(sid)
+        for a, b in zip(got0, (ix, x, u, q)):
+            assert np.array_equal(a, b)
+        sim.run(25)
+        jx, jp, ju, jq = sim.get_particles(sid)
+        assert len(jq) == sim.count(sid) and (n < 100 or len(jq) < n)
+    k = np.searchsorted(-q, -jq)  # ascending and unique
+    assert np.array_equal(q[k], jq) and np.all(np.diff(k) > 0)
+    assert np.allclose(ju, u[k], rtol=0, atol=1e-5)
+    v = u[k].astype(np.float64) / np.sqrt(1 + (u[k].astype(np.float64) ** 2).sum(1, keepdims=True))
+    end = (ix[k] + x[k] + 25 * 0.5 * v[:, :dims])
+    d = jx + jp - end
+    for m in range(1, dims):
+        d[:, m] -= nx[m] * np.round(d[:, m] / nx[m])
+    assert np.abs(d).max() < 1e-3
