@@ -75,13 +75,14 @@ struct DBuf {
   void* p = nullptr;
   size_t n = 0;
   bool async = false;
+  bool own = true;  // false: a part of another buffer
   hipStream_t st = nullptr;
   DBuf() = default;
   DBuf(const DBuf&) = delete;
   DBuf& operator=(const DBuf&) = delete;
   ~DBuf() { release(); }
   void release() {
-    if (p) {
+    if (p && own) {
       if (async)
         (void)hipFreeAsync(p, st);
       else
@@ -90,6 +91,14 @@ struct DBuf {
     p = nullptr;
     n = 0;
     async = false;
+    own = true;
+  }
+  // name a part of another buffer, which keeps it
+  void view(void* part, size_t bytes) {
+    release();
+    p = part;
+    n = bytes;
+    own = false;
   }
   int alloc(size_t bytes) {
     release();
@@ -118,6 +127,7 @@ struct DBuf {
     std::swap(p, o.p);
     std::swap(n, o.n);
     std::swap(async, o.async);
+    std::swap(own, o.own);
     std::swap(st, o.st);
   }
   template <class T>
@@ -146,6 +156,9 @@ struct Species {
   int64_t npid = 0;  // particles given at first: their pids are 0 .. npid - 1
   int64_t cap_total = 0;
   double qabs = 0.0, qmax = 0.0;
+  // the particle and mover arrays and the tile tables are parts of one allocation each: an
+  // allocation or release costs 100 to 200 us whatever its size, and a re-layout makes both
+  DBuf slots, tables;
   DBuf cell, x, y, z, ux, uy, uz, q, pid;
   DBuf mcell, mx, my, mz, mux, muy, muz, mq, mpid, midx;
   DBuf off, cnt, cap, mv_cnt, mv_stride, newcnt, inc, epart;
@@ -492,6 +505,27 @@ int pick_split(int ntiles, int waves) {
   return ntiles <= 128 ? 4 : (ntiles <= 384 ? 2 : 1);
 }
 
+// The 19 particle and mover arrays of a species in the order of RegrowArrays
+void particle_arrays(Species& p, DBuf* (&arr)[19]) {
+  DBuf* const v[19] = {&p.cell, &p.x, &p.y, &p.z, &p.ux, &p.uy, &p.uz, &p.q, &p.pid,
+                       &p.mcell, &p.mx, &p.my, &p.mz, &p.mux, &p.muy, &p.muz, &p.mq, &p.mpid,
+                       &p.midx};
+  std::copy(v, v + 19, arr);
+}
+
+// Their places in one allocation of n slots each (z and mz of a 2D species: none)
+int alloc_slots(int dims, DBuf& slots, size_t n, uint32_t* (&at)[19]) {
+  const size_t bytes = (4 * n + 255) / 256 * 256;
+  TRY(slots.alloc(bytes * (dims == 3 ? 19 : 17)));
+  char* b = (char*)slots.p;
+  for (int a = 0; a < 19; a++) {
+    const bool none = dims != 3 && (a == 3 || a == 12);
+    at[a] = (uint32_t*)b;
+    if (!none) b += bytes;
+  }
+  return OSR_OK;
+}
+
 // Allocate a species' arrays for the given per-tile counts and capacities.
 int alloc_species(osr_sim* s, Species& p, const std::vector<int>& cnt) {
   const int nt = s->ntiles;
@@ -508,48 +542,34 @@ int alloc_species(osr_sim* s, Species& p, const std::vector<int>& cnt) {
   }
   p.cap_total = total;
   const size_t n = (size_t)total;
-  TRY(p.cell.alloc(4 * n));
-  TRY(p.x.alloc(4 * n));
-  TRY(p.y.alloc(4 * n));
-  TRY(p.z.alloc(s->dims == 3 ? 4 * n : 4));
-  TRY(p.ux.alloc(4 * n));
-  TRY(p.uy.alloc(4 * n));
-  TRY(p.uz.alloc(4 * n));
-  TRY(p.q.alloc(4 * n));
-  TRY(p.pid.alloc(4 * n));
-  TRY(p.mcell.alloc(4 * n));
-  TRY(p.mx.alloc(4 * n));
-  TRY(p.my.alloc(4 * n));
-  TRY(p.mz.alloc(s->dims == 3 ? 4 * n : 4));
-  TRY(p.mux.alloc(4 * n));
-  TRY(p.muy.alloc(4 * n));
-  TRY(p.muz.alloc(4 * n));
-  TRY(p.mq.alloc(4 * n));
-  TRY(p.mpid.alloc(4 * n));
-  TRY(p.midx.alloc(4 * n));
-  TRY(p.off.alloc(4 * (size_t)nt));
-  TRY(p.cnt.alloc(4 * (size_t)nt));
-  TRY(p.cap.alloc(4 * (size_t)nt));
-  TRY(p.mv_cnt.alloc(4 * (size_t)nt * kMaxTileWaves));
-  TRY(p.mv_stride.alloc(4 * (size_t)nt));
-  TRY(p.newcnt.alloc(4 * (size_t)nt));
-  TRY(p.inc.alloc(4 * (size_t)nt));
+  uint32_t* at[19];
+  DBuf* arr[19];
+  particle_arrays(p, arr);
+  for (int a = 0; a < 19; a++) arr[a]->release();
+  TRY(alloc_slots(s->dims, p.slots, n, at));
+  for (int a = 0; a < 19; a++) arr[a]->view(at[a], 4 * n);
   p.epart_n = s->plain ? (int)((total + 255) / 256) : nt * s->split;
-  TRY(p.epart.alloc(8 * (size_t)p.epart_n));
+  // the tile tables: off, cnt, cap (uploaded together), then those that start at zero
+  const size_t tb = (4 * (size_t)nt + 255) / 256 * 256, mb = tb * kMaxTileWaves;
+  const size_t eb = 8 * (size_t)p.epart_n;
+  TRY(p.tables.alloc(6 * tb + mb + eb));
+  char* t0 = (char*)p.tables.p;
+  DBuf* const tab[6] = {&p.off, &p.cnt, &p.cap, &p.mv_stride, &p.newcnt, &p.inc};
+  for (int k = 0; k < 6; k++) tab[k]->view(t0 + k * tb, 4 * (size_t)nt);
+  p.mv_cnt.view(t0 + 6 * tb, 4 * (size_t)nt * kMaxTileWaves);
+  p.epart.view(t0 + 6 * tb + mb, eb);
   if (s->plain) {
     TRY(p.pl_ep.alloc(12 * n));
     TRY(p.pl_bp.alloc(12 * n));
     TRY(p.pl_vp.alloc(7 * 3 * 4 * n));
     TRY(p.pl_nvp.alloc(4 * n));
   }
-  TRY(copy_on(s->stream, p.off.p, off.data(), 4 * nt, hipMemcpyHostToDevice));
-  TRY(copy_on(s->stream, p.cnt.p, cnt.data(), 4 * nt, hipMemcpyHostToDevice));
-  TRY(copy_on(s->stream, p.cap.p, cap.data(), 4 * nt, hipMemcpyHostToDevice));
-  HIPC(hipMemsetAsync(p.mv_cnt.p, 0, 4 * (size_t)nt * kMaxTileWaves, s->stream));
-  HIPC(hipMemsetAsync(p.mv_stride.p, 0, 4 * (size_t)nt, s->stream));
-  HIPC(hipMemsetAsync(p.epart.p, 0, 8 * (size_t)p.epart_n, s->stream));
-  HIPC(hipMemsetAsync(p.inc.p, 0, 4 * (size_t)nt, s->stream));
-  HIPC(hipStreamSynchronize(s->stream));
+  std::vector<char> h(3 * tb, 0);
+  std::memcpy(h.data(), off.data(), 4 * (size_t)nt);
+  std::memcpy(h.data() + tb, cnt.data(), 4 * (size_t)nt);
+  std::memcpy(h.data() + 2 * tb, cap.data(), 4 * (size_t)nt);
+  HIPC(hipMemsetAsync(t0 + 3 * tb, 0, 3 * tb + mb + eb, s->stream));
+  TRY(copy_on(s->stream, t0, h.data(), h.size(), hipMemcpyHostToDevice));
   p.h_off = off;
   p.h_cap = cap;
   int64_t np = 0;
@@ -791,18 +811,12 @@ int regrow_species(osr_sim* s, int sid, bool* ok) {
     total += c;
   }
   const size_t n = (size_t)total;
-  const bool three = s->dims == 3;
-  DBuf* arr[19] = {&p.cell, &p.x, &p.y, &p.z, &p.ux, &p.uy, &p.uz, &p.q, &p.pid,
-                   &p.mcell, &p.mx, &p.my, &p.mz, &p.mux, &p.muy, &p.muz, &p.mq, &p.mpid,
-                   &p.midx};
-  DBuf nb[19];
+  DBuf* arr[19];
+  particle_arrays(p, arr);
+  DBuf slots;
   RegrowArrays src{}, dst{};
-  for (int a = 0; a < 19; a++) {
-    const bool dummy = !three && (a == 3 || a == 12);  // z and mz of a 2D species
-    TRY(nb[a].alloc(dummy ? 4 : 4 * n));
-    src.a[a] = arr[a]->as<uint32_t>();
-    dst.a[a] = nb[a].as<uint32_t>();
-  }
+  TRY(alloc_slots(s->dims, slots, n, dst.a));
+  for (int a = 0; a < 19; a++) src.a[a] = arr[a]->as<uint32_t>();
   DBuf d_off, d_work;
   TRY(d_off.alloc(4 * (size_t)nt));
   TRY(d_work.alloc(sizeof(int2) * over.size()));
@@ -812,7 +826,8 @@ int regrow_species(osr_sim* s, int sid, bool* ok) {
                      s->d_spec.as<SpecDesc>(), sid, src, dst, d_off.as<int>());
   HIPC(hipGetLastError());
   HIPC(hipStreamSynchronize(s->stream));
-  for (int a = 0; a < 19; a++) arr[a]->swap(nb[a]);  // the old arrays go with nb
+  p.slots.swap(slots);  // the old arrays go with the local
+  for (int a = 0; a < 19; a++) arr[a]->view(dst.a[a], 4 * n);
   TRY(copy_on(s->stream, p.off.p, off.data(), 4 * (size_t)nt, hipMemcpyHostToDevice));
   TRY(copy_on(s->stream, p.cap.p, cap.data(), 4 * (size_t)nt, hipMemcpyHostToDevice));
   p.h_off = off;
@@ -1780,7 +1795,7 @@ int osr_sim_run(osr_sim* s, int nsteps) {
       Ctrl z = c;
       z.halt = 0;
       TRY(copy_on(s->stream, s->ctrl.p, &z, sizeof(Ctrl), hipMemcpyHostToDevice));
-      TRY(build_graph(s));
+      // the captured steps name the descriptors and work lists, which keep their places
       batch = 8;
     } else if (done != nb) {
       return fail(OSR_ERR_STATE, "step counter advanced by %lld instead of %d",
@@ -1988,11 +2003,7 @@ int osr_sim_footprint(osr_sim* s, int64_t* bytes) {
   if (!bytes) return fail(OSR_ERR_ARG, "null argument");
   size_t b = s->E.n + s->B.n + s->J.n + s->fe_part.n + s->hist.n;
   for (auto& p : s->sp) {
-    const DBuf* all[] = {&p->cell, &p->x, &p->y, &p->z, &p->ux, &p->uy, &p->uz, &p->q, &p->pid,
-                         &p->mcell, &p->mx, &p->my, &p->mz, &p->mux, &p->muy, &p->muz, &p->mq,
-                         &p->mpid, &p->midx, &p->off, &p->cnt, &p->cap, &p->mv_cnt,
-                         &p->mv_stride, &p->newcnt, &p->inc, &p->epart};
-    for (const DBuf* d : all) b += d->n;
+    b += p->slots.n + p->tables.n;
   }
   *bytes = (int64_t)b;
   return OSR_OK;
