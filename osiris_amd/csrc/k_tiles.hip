@@ -833,17 +833,26 @@ __global__ __launch_bounds__(256) void regrow_move(const SpecDesc* __restrict__ 
 // fill overflowed is skipped (the host re-lays those particles out), as are tiles with
 // more than MAXN particles or RMAX particles in one cell.
 // ------------------------------------------------------------------------------------
+//
+// Bound: latency, then HBM (each array is read and written once, 72 B per particle).  Every
+// wave ranks a quarter of the slots, with counts of its own that the next waves start from,
+// and each array's loads are issued before the previous one is stored.  us per launch, one
+// launch in four active, one ranking wave / this: 52x44x36 18 / 12, 96^3 two beams 107 / 78,
+// 192^3 8 per cell 629 / 450 (an active one moves 4.1 GB in 1.8 ms).
 template <int NT, int RMAX, int MAXC, int MAXN>
 __global__ __launch_bounds__(NT) void tile_reorder(const SpecDesc* __restrict__ descs,
                                                    const int2* __restrict__ work, int period) {
-  constexpr int MAXW = RMAX * MAXC / 32;
-  __shared__ int s_cnt[MAXC];
+  constexpr int MAXW = RMAX * MAXC / 32, NW = NT / 64;
+  constexpr int CB = 10;  // bits of a cell key in s_key
+  static_assert(MAXC <= 1 << CB, "cell keys");
+  __shared__ int s_cnt[NW][MAXC];  // particles of the cell in the wave's slots, then before them
+  __shared__ int s_tot[MAXC];      // particles of the cell
   __shared__ unsigned int s_bits[MAXW];
   __shared__ int s_wpre[MAXW];
   __shared__ int s_key[MAXN];
-  __shared__ uint32_t s_tmp[MAXN];
-  __shared__ int s_tot[NT / 64];
-  __shared__ int s_abort;
+  __shared__ __align__(16) uint32_t s_tmp[MAXN];
+  __shared__ int s_sum[NW];
+  __shared__ int s_abort, s_rows;
   const int2 wk = work[blockIdx.x];
   const SpecDesc& d = descs[wk.x];
   const GridDesc& g = d.g;
@@ -855,25 +864,29 @@ __global__ __launch_bounds__(NT) void tile_reorder(const SpecDesc* __restrict__ 
   if (n < 2 || n > MAXN || C > MAXC) return;
   const int cx0 = (tile % g.ntx) * g.tx, cy0 = ((tile / g.ntx) % g.nty) * g.ty;
   const int cz0 = dims == 3 ? (tile / (g.ntx * g.nty)) * g.tz : 0;
-  for (int c = threadIdx.x; c < C; c += NT) s_cnt[c] = 0;
-  if (threadIdx.x == 0) s_abort = 0;
-  // the tile's packed cells, coalesced, into s_key (each entry is replaced by its key)
-  for (int p = threadIdx.x; p < n; p += NT) s_key[p] = (int)d.cell[base + p];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  for (int c = tid; c < NW * MAXC; c += NT) (&s_cnt[0][0])[c] = 0;
+  if (tid == 0) s_abort = s_rows = 0;
   __syncthreads();
   int nbits = 0;  // bits of a local cell index
   while ((1 << nbits) < C) nbits++;
-  if (threadIdx.x < 64) {  // one wave: ranks within the cell in slot order
-    const int lane = threadIdx.x;
+  // ranks within the cell in slot order, each wave over its own slots
+  const int per = ((n + 64 * NW - 1) / (64 * NW)) * 64;
+  {
+    const int p0 = wave * per, p1 = min(p0 + per, n);
     const unsigned long long below = (1ull << lane) - 1ull;
-    for (int c0 = 0; c0 < n; c0 += 64) {
+    uint32_t next = p0 + lane < p1 ? d.cell[base + p0 + lane] : 0u;
+    for (int c0 = p0; c0 < p1; c0 += 64) {
       const int p = c0 + lane;
+      const uint32_t cell = next;
+      next = p + 64 < p1 ? d.cell[base + p + 64] : 0u;
       int lc = -1 - lane;  // distinct for the lanes past the end
-      if (p < n) {
+      if (p < p1) {
         int ix, iy, iz = 0;
         if (dims == 2)
-          unpack2((uint32_t)s_key[p], ix, iy);
+          unpack2(cell, ix, iy);
         else
-          unpack3((uint32_t)s_key[p], ix, iy, iz);
+          unpack3(cell, ix, iy, iz);
         const int lx = ix - cx0, ly = iy - cy0, lz = iz - cz0;
         if (lx < 0 || lx >= g.tx || ly < 0 || ly >= g.ty || lz < 0 ||
             lz >= (dims == 3 ? g.tz : 1))
@@ -889,25 +902,37 @@ __global__ __launch_bounds__(NT) void tile_reorder(const SpecDesc* __restrict__ 
       }
       const int before = __popcll(same & below);
       const int after = __popcll(same & ~below) - 1;
-      if (lc >= 0) {
-        const int r = s_cnt[lc] + before;
-        if (r >= RMAX) s_abort = 1;
-        s_key[p] = r * C + lc;
-      }
+      if (lc >= 0) s_key[p] = ((s_cnt[wave][lc] + before) << CB) | lc;
       __builtin_amdgcn_wave_barrier();
-      if (lc >= 0 && after == 0) s_cnt[lc] += before + 1;
+      if (lc >= 0 && after == 0) s_cnt[wave][lc] += before + 1;
       __builtin_amdgcn_wave_barrier();
     }
   }
   __syncthreads();
-  if (s_abort) return;
+  // per cell: what the waves before hold, and the total
+  int rows = 0;
+  for (int c = tid; c < C; c += NT) {
+    int run = 0;
+#pragma unroll
+    for (int w = 0; w < NW; w++) {
+      const int v = s_cnt[w][c];
+      s_cnt[w][c] = run;
+      run += v;
+    }
+    s_tot[c] = run;
+    rows = max(rows, run);
+  }
+  if (rows > 0) atomicMax(&s_rows, rows);
+  __syncthreads();
+  rows = s_rows;
+  if (s_abort || rows > RMAX) return;
   // occupancy of the keys (rank, cell): occupied iff the cell holds more than rank
-  const int nw = (RMAX * C + 31) / 32;
-  for (int w = threadIdx.x; w < nw; w += NT) {
+  const int nw = (rows * C + 31) / 32;
+  for (int w = tid; w < nw; w += NT) {
     unsigned int m = 0u;
     int r = (32 * w) / C, c = (32 * w) % C;  // key 32 w = r C + c, walked bit by bit
     for (int b = 0; b < 32; b++) {
-      if (r < RMAX && s_cnt[c] > r) m |= 1u << b;
+      if (s_tot[c] > r) m |= 1u << b;
       if (++c == C) {
         c = 0;
         r++;
@@ -917,74 +942,83 @@ __global__ __launch_bounds__(NT) void tile_reorder(const SpecDesc* __restrict__ 
   }
   __syncthreads();
   // exclusive prefix of the word populations: each thread owns consecutive words
-  constexpr int PER = (MAXW + NT - 1) / NT;
-  const int w0 = threadIdx.x * PER;
+  const int own_w = (nw + NT - 1) / NT;
+  const int w0 = tid * own_w;
   int own = 0;
-  for (int k = 0; k < PER; k++)
+  for (int k = 0; k < own_w; k++)
     if (w0 + k < nw) own += __popc(s_bits[w0 + k]);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   int inc = own;
   for (int o = 1; o < 64; o <<= 1) {
     const int t = __shfl_up(inc, o, 64);
     if (lane >= o) inc += t;
   }
-  if (lane == 63) s_tot[wave] = inc;
+  if (lane == 63) s_sum[wave] = inc;
   __syncthreads();
   int run = inc - own;
-  for (int w = 0; w < wave; w++) run += s_tot[w];
-  for (int k = 0; k < PER; k++)
+  for (int w = 0; w < wave; w++) run += s_sum[w];
+  for (int k = 0; k < own_w; k++)
     if (w0 + k < nw) {
       s_wpre[w0 + k] = run;
       run += __popc(s_bits[w0 + k]);
     }
   __syncthreads();
-  // new slot of every particle, in place of its key
-  for (int p = threadIdx.x; p < n; p += NT) {
-    const int k = s_key[p];
-    s_key[p] = s_wpre[k >> 5] + __popc(s_bits[k >> 5] & ((1u << (k & 31)) - 1u));
-  }
-  __syncthreads();
-  // permute each array through LDS: coalesced 16-byte reads of 4 consecutive slots per
-  // thread (tile bases are multiples of 64 slots), LDS scatter, coalesced writes back
+  // new slot of every particle, in groups of 4 consecutive slots per thread (tile bases are
+  // multiples of 64 slots)
   constexpr int PT = MAXN / (4 * NT);  // 4-slot groups per thread
   int dst[PT][4];
 #pragma unroll
   for (int j = 0; j < PT; j++)
 #pragma unroll
     for (int e = 0; e < 4; e++) {
-      const int p = 4 * (threadIdx.x + NT * j) + e;
-      dst[j][e] = p < n ? s_key[p] : -1;
+      const int p = 4 * (tid + NT * j) + e;
+      dst[j][e] = -1;
+      if (p < n) {
+        const int v = s_key[p], lc = v & ((1 << CB) - 1);
+        const int k = ((v >> CB) + s_cnt[p / per][lc]) * C + lc;
+        dst[j][e] = s_wpre[k >> 5] + __popc(s_bits[k >> 5] & ((1u << (k & 31)) - 1u));
+      }
     }
+  // permute each array through LDS: coalesced 16-byte reads, LDS scatter, coalesced writes
   uint32_t* arr[9] = {d.cell, (uint32_t*)d.x, (uint32_t*)d.y, (uint32_t*)d.z, (uint32_t*)d.ux,
                       (uint32_t*)d.uy, (uint32_t*)d.uz, (uint32_t*)d.q, d.pid};
+  uint4 v[PT];
+  auto load = [&](int a) {
+    const uint32_t* A = arr[a] + base;
+#pragma unroll
+    for (int j = 0; j < PT; j++) {
+      const int q = 4 * (tid + NT * j);
+      v[j] = make_uint4(0u, 0u, 0u, 0u);
+      if (q + 3 < n) {
+        v[j] = *(const uint4*)(A + q);
+      } else if (q < n) {
+        v[j].x = A[q];
+        if (q + 1 < n) v[j].y = A[q + 1];
+        if (q + 2 < n) v[j].z = A[q + 2];
+      }
+    }
+  };
+  load(0);
 #pragma unroll
   for (int a = 0; a < 9; a++) {
     if (a == 3 && dims != 3) continue;
     uint32_t* A = arr[a] + base;
 #pragma unroll
     for (int j = 0; j < PT; j++) {
-      const int q = 4 * (threadIdx.x + NT * j);
-      if (q + 3 < n) {
-        const uint4 v = *(const uint4*)(A + q);
-        s_tmp[dst[j][0]] = v.x;
-        s_tmp[dst[j][1]] = v.y;
-        s_tmp[dst[j][2]] = v.z;
-        s_tmp[dst[j][3]] = v.w;
-      } else {
+      const uint32_t w[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
 #pragma unroll
-        for (int e = 0; e < 4; e++)
-          if (q + e < n) s_tmp[dst[j][e]] = A[q + e];
-      }
+      for (int e = 0; e < 4; e++)
+        if (dst[j][e] >= 0) s_tmp[dst[j][e]] = w[e];
     }
+    if (a < 8) load(a == 2 && dims != 3 ? 4 : a + 1);
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < PT; j++) {
-      const int q = 4 * (threadIdx.x + NT * j);
+      const int q = 4 * (tid + NT * j);
       if (q + 3 < n) {
-        *(uint4*)(A + q) = make_uint4(s_tmp[q], s_tmp[q + 1], s_tmp[q + 2], s_tmp[q + 3]);
+        *(uint4*)(A + q) = *(const uint4*)(s_tmp + q);
       } else {
 #pragma unroll
-        for (int e = 0; e < 4; e++)
+        for (int e = 0; e < 3; e++)
           if (q + e < n) A[q + e] = s_tmp[q + e];
       }
     }
