@@ -1143,6 +1143,11 @@ int launch_plain(osr_sim* s, int sid) {
 int launch_smooth(osr_sim* s) {
   int np = 0;
   for (int d = 0; d < s->dims; d++) np += s->sm_order[d] > 0;
+  if (np > 0 && s->dims == 2) {
+    const int nt = ceil_div(s->g.nx, kSmX) * ceil_div(s->g.ny, kSmY);
+    hipLaunchKernelGGL(smooth2d, dim3(3 * nt), dim3(256), 0, s->stream, s->d_fd.as<FieldDesc>());
+    np = 0;
+  }
   for (int p = 0; p < np; p++)
     hipLaunchKernelGGL(smooth_pass, dim3(s->nblk), dim3(256), 0, s->stream,
                        s->d_fd.as<FieldDesc>(), s->d_ywork.as<int2>(), p);

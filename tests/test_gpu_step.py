@@ -110,6 +110,41 @@ def test_fused_field_step(nx, order):
     assert np.allclose(fld, want, rtol=1e-12, atol=0)
 
 
+@pytest.mark.parametrize("nx,order", [((6, 5), (15, 15)), ((32, 16), (1, 2)), ((33, 17), (3, 3)), ((31, 70), (15, 0)),
+                                      ((90, 15), (0, 15)), ((300, 200), (3, 3))])
+def test_smoothed_current_2d(nx, order):
+    """After one step from zero fields E = -dt J; with dt a power of two the product is
+    exact, so the smoothed run's E is the filter (x before y, taps summed left to right with
+    each product rounded) of the unsmoothed run's E bit for bit."""
+    print(f"case nx={nx} order={order}", flush=True)
+    rng = np.random.default_rng(3)
+    n = 5 * nx[0] * nx[1]
+    ix = np.stack([rng.integers(1, m + 1, n) for m in nx], 1).astype(np.int32)
+    x = (rng.random((n, 2), np.float32) - np.float32(0.5)).astype(np.float32)
+    u = (rng.standard_normal((n, 3)) * 0.5).astype(np.float32)
+    q = (-rng.random(n)).astype(np.float32)
+    coef = np.zeros((3, 31), np.float32)
+    for d in range(2):
+        coef[d, 15 - order[d]:16 + order[d]] = rng.standard_normal(2 * order[d] + 1)
+    e = []
+    for smooth in (False, True):
+        with oa.Simulation(2, nx, (0.1, 0.1), 0.0625, 2) as sim:
+            sim.set_particles(sim.add_species(-1.0), ix, x, u, q)
+            if smooth:
+                sim.set_smooth(order + (0,), coef)
+            sim.run(1)
+            e.append(sim.get_fields()[0])
+    want = e[0]
+    for d in range(2):
+        if order[d]:
+            k = order[d]
+            taps = [np.roll(want, -m, 1 - d) * coef[d, 15 + m] for m in range(-k, k + 1)]
+            want = taps[0]
+            for t in taps[1:]:
+                want = want + t
+    assert np.array_equal(e[1], want)  # the sign of a zero sum is not the product's
+
+
 @pytest.mark.parametrize("dims,n", [(2, 1), (2, 2047), (2, 200_000), (3, 70_000)])
 def test_particles_come_back_in_upload_order(dims, n):
     """get_particles after absorbing walls removed some: the survivors in upload order (the
