@@ -188,8 +188,10 @@ struct osr_sim {
   int ntiles = 0;
   int nblk = 0;  // Yee blocks of 256 cells
   int nblk_e = 0;  // energy workgroups of the first B half step (kEneBlk blocks each)
-  int nwork_e = 0;  // its work items: the nblk_e blocks, then (Lindman walls) the blocks of
-                    // 256 rows of the lower wall's first B update, as (0, -1 - block)
+  int nwork_e = 0;  // its work items: the nblk_e blocks, then (x walls) as (0, -1 - block) the
+                    // blocks of 256 rows of the lower Lindman wall's first B update or of 256
+                    // cells of the VPML walls
+  int nwall_v = 0;  // blocks of 256 cells of the VPML walls
   double dx[3] = {1, 1, 1};
   double dt = 0;
   DBuf E, B, J, ctrl, fe_part, hist;
@@ -1029,51 +1031,43 @@ int launch_wall_restore(osr_sim* s) {
   return OSR_OK;
 }
 
-int launch_yee(osr_sim* s) {
+// next_laser: the next step's laser values join the last half step (its own launch_laser is
+// left out; only where that step's kernels follow in the stream).
+int launch_yee(osr_sim* s, bool next_laser = false) {
   const FieldDesc* fd = s->d_fd.as<FieldDesc>();
   const int2* w = s->d_ywork.as<int2>();
   const int2* we = s->d_ework.as<int2>();
   const int2* wd = s->d_dwork.as<int2>();  // the history columns, then the cell blocks
   const unsigned nd = (unsigned)(kRedCols + s->nblk);
-  if (s->vp_n) {  // advance_yee with VPML x walls: update_boundary_bfld step 1 advances
-                   // the wall E, update_boundary_efld the wall B (os-emf-boundary.f90:930-935,
-                   // 1036-1041)
-    const unsigned nb = (unsigned)((2ll * s->vp_n * s->g.ny * s->g.nz + 255) / 256);
-    if (s->dims == 2) {
-      hipLaunchKernelGGL((yee_dbdt<2, true>), dim3(s->nblk_e), dim3(256), 0, s->stream, fd, we);
-      if (s->desc.vpml_diffuse[0] || s->desc.vpml_diffuse[1])
-        hipLaunchKernelGGL(vpml_diffuse, dim3(nb), dim3(256), 0, s->stream, fd);
-      hipLaunchKernelGGL((vpml_update<0, 2>), dim3(nb), dim3(256), 0, s->stream, fd);
-      hipLaunchKernelGGL((yee_dedt<2>), dim3(nd), dim3(256), 0, s->stream, fd, wd);
-      hipLaunchKernelGGL((vpml_update<1, 2>), dim3(nb), dim3(256), 0, s->stream, fd);
-      hipLaunchKernelGGL((yee_dbdt<2, false>), dim3(s->nblk), dim3(256), 0, s->stream, fd, w);
-    } else {
-      hipLaunchKernelGGL((yee_dbdt<3, true>), dim3(s->nblk_e), dim3(256), 0, s->stream, fd, we);
-      hipLaunchKernelGGL((vpml_update<0, 3>), dim3(nb), dim3(256), 0, s->stream, fd);
-      hipLaunchKernelGGL((yee_dedt<3>), dim3(nd), dim3(256), 0, s->stream, fd, wd);
-      hipLaunchKernelGGL((vpml_update<1, 3>), dim3(nb), dim3(256), 0, s->stream, fd);
-      hipLaunchKernelGGL((yee_dbdt<3, false>), dim3(s->nblk), dim3(256), 0, s->stream, fd, w);
+  if (s->g.open_nx) {
+    // VPML x walls: update_boundary_bfld step 1 advances the wall E, update_boundary_efld the
+    // wall B (os-emf-boundary.f90:930-935, 1036-1041).  Lindman x walls
+    // (os-emf-solver-yee.f03:542-568): the work list of the first B half step carries the
+    // wall's first B update.
+    typedef void (*fk)(const FieldDesc*, const int2*);
+    const bool vp = s->vp_n > 0, d3 = s->dims == 3;
+    const unsigned nwv = (unsigned)s->nwall_v;
+    const bool diffuse = vp && (s->desc.vpml_diffuse[0] || s->desc.vpml_diffuse[1]);
+    const fk b1 = d3 ? (vp ? (fk)yee_dbdt<3, true, true> : (fk)yee_dbdt<3, true>)
+                     : (vp && !diffuse ? (fk)yee_dbdt<2, true, true> : (fk)yee_dbdt<2, true>);
+    const fk e = d3 ? (vp ? (fk)yee_dedt<3, 2> : (fk)yee_dedt<3, 1>)
+                    : (vp ? (fk)yee_dedt<2, 2> : (fk)yee_dedt<2, 1>);
+    const fk b2 = d3 ? (next_laser ? (fk)yee_dbdt<3, false, false, true> : (fk)yee_dbdt<3, false>)
+                     : (next_laser ? (fk)yee_dbdt<2, false, false, true> : (fk)yee_dbdt<2, false>);
+    hipLaunchKernelGGL(b1, dim3(diffuse ? s->nblk_e : s->nwork_e), dim3(256), 0, s->stream, fd, we);
+    if (diffuse) {
+      hipLaunchKernelGGL(vpml_diffuse, dim3(nwv), dim3(256), 0, s->stream, fd);
+      hipLaunchKernelGGL(vpml_update_e, dim3(nwv), dim3(256), 0, s->stream, fd);
     }
-    HIPC(hipGetLastError());
-    return OSR_OK;
-  }
-  if (s->g.open_nx) {  // advance_yee with Lindman x walls (os-emf-solver-yee.f03:542-568)
-    const unsigned nb = (unsigned)ceil_div(s->g.ny * s->g.nz, 256);
-    // the work list of the first B half step carries the wall's first B update
-    if (s->dims == 2) {
-      hipLaunchKernelGGL((yee_dbdt<2, true>), dim3(s->nwork_e), dim3(256), 0, s->stream, fd, we);
-      hipLaunchKernelGGL((yee_dedt<2>), dim3(nd), dim3(256), 0, s->stream, fd, wd);
-      hipLaunchKernelGGL(wall_e, dim3(nb), dim3(256), 0, s->stream, fd);
-      hipLaunchKernelGGL((yee_dbdt<2, false>), dim3(s->nblk), dim3(256), 0, s->stream, fd, w);
-      hipLaunchKernelGGL((wall_b2_end<2>), dim3(nb), dim3(256), 0, s->stream, fd);
-    } else {
-      hipLaunchKernelGGL((yee_dbdt<3, true>), dim3(s->nwork_e), dim3(256), 0, s->stream, fd, we);
-      hipLaunchKernelGGL((yee_dedt<3>), dim3(nd), dim3(256), 0, s->stream, fd, wd);
-      hipLaunchKernelGGL(wall_e, dim3(nb), dim3(256), 0, s->stream, fd);
-      hipLaunchKernelGGL((yee_dbdt<3, false>), dim3(s->nblk), dim3(256), 0, s->stream, fd, w);
-      hipLaunchKernelGGL((wall_b2_end<3>), dim3(nb), dim3(256), 0, s->stream, fd);
+    hipLaunchKernelGGL(e, dim3(nd + nwv), dim3(256), 0, s->stream, fd, wd);
+    hipLaunchKernelGGL(b2, dim3(s->nblk), dim3(256), 0, s->stream, fd, w);
+    if (!vp) {  // also restores the wall values and ends the step
+      const unsigned nb = (unsigned)ceil_div(s->g.ny * s->g.nz, 256);
+      if (d3)
+        hipLaunchKernelGGL((wall_b2_end<3>), dim3(nb), dim3(256), 0, s->stream, fd);
+      else
+        hipLaunchKernelGGL((wall_b2_end<2>), dim3(nb), dim3(256), 0, s->stream, fd);
     }
-    // the last wall kernel also restored the wall values and ended the step
     HIPC(hipGetLastError());
     return OSR_OK;
   }
@@ -1192,12 +1186,15 @@ int zp_fill(osr_sim* s, int64_t first, int n) {
   return OSR_OK;
 }
 
-int enqueue_step(osr_sim* s) {
-  TRY(launch_laser(s));
+// One of several steps put into the stream without a stop between them: `laser`, the step's
+// laser launch is its own (the step before did not take it along), `next`, another follows.
+int enqueue_step(osr_sim* s, bool laser = true, bool next = false) {
+  if (laser) TRY(launch_laser(s));
+  const bool next_laser = next && !s->zp.empty();
   if (s->plain) {
     for (size_t i = 0; i < s->sp.size(); i++) TRY(launch_plain(s, (int)i));
     TRY(launch_smooth(s));
-    TRY(launch_yee(s));
+    TRY(launch_yee(s, next_laser));
     TRY(launch_finalize(s));
     return OSR_OK;
   }
@@ -1205,7 +1202,7 @@ int enqueue_step(osr_sim* s) {
   if (!s->sp.empty()) TRY(launch_fill(s));
   if (!s->sp.empty()) TRY(launch_reorder(s));
   TRY(launch_smooth(s));
-  TRY(launch_yee(s));
+  TRY(launch_yee(s, next_laser));
   TRY(launch_finalize(s));
   return OSR_OK;
 }
@@ -1219,7 +1216,7 @@ int capture_steps(osr_sim* s, int nsteps, hipGraphExec_t* out) {
   hipGraph_t graph = nullptr;
   HIPC(hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
   int r = OSR_OK;
-  for (int k = 0; k < nsteps && r == OSR_OK; k++) r = enqueue_step(s);
+  for (int k = 0; k < nsteps && r == OSR_OK; k++) r = enqueue_step(s, k == 0, k + 1 < nsteps);
   hipError_t e = hipStreamEndCapture(s->stream, &graph);
   if (r != OSR_OK) {
     if (graph) (void)hipGraphDestroy(graph);
@@ -1450,7 +1447,8 @@ int osr_sim_create(const osr_sim_desc* desc, osr_sim** out) {
   TRY(s->d_spec.alloc(sizeof(SpecDesc) * kMaxSpecies));
   TRY(s->d_fd.alloc(sizeof(FieldDesc)));
   TRY(s->d_ywork.alloc(sizeof(int2) * (size_t)s->nblk));
-  const int nwall_e = (g.open_nx && !vp_n) ? ceil_div(g.ny * g.nz, 256) : 0;
+  s->nwall_v = vp_n ? (int)((2ll * vp_n * g.ny * g.nz + 255) / 256) : 0;
+  const int nwall_e = g.open_nx ? (vp_n ? s->nwall_v : ceil_div(g.ny * g.nz, 256)) : 0;
   s->nwork_e = s->nblk_e + nwall_e;
   TRY(s->d_ework.alloc(sizeof(int2) * (size_t)s->nwork_e));
   TRY(s->d_fwork.alloc(sizeof(int)));
@@ -1466,6 +1464,7 @@ int osr_sim_create(const osr_sim_desc* desc, osr_sim** out) {
     for (int c = 0; c < kRedCols; c++) dw.push_back(make_int2(0, -1 - c));
     const std::vector<int2>& cells = g.pp ? ew : yw;  // tiles of yee2d_step, or blocks
     dw.insert(dw.end(), cells.begin(), cells.end());
+    for (int b = 0; b < s->nwall_v; b++) dw.push_back(make_int2(0, -1 - kRedCols - b));
     TRY(s->d_dwork.alloc(sizeof(int2) * dw.size()));
     TRY(copy_on(s->stream, s->d_dwork.p, dw.data(), sizeof(int2) * dw.size(), hipMemcpyHostToDevice));
     int z = 0;

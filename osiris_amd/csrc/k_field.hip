@@ -104,10 +104,41 @@ constexpr int kEneBlk = 4;
 template <int STEP, int DIMS, bool RESTORE = false>
 OSR_DEV void wall_b_row(const FieldDesc& fd, long long r);
 
-// the sum of one history column (defined with the step end below)
+// one row of a Lindman wall's E update (UPPER: the wall at nx+2), from the row's new E2, E3
+// next to it (defined with the wall kernels below)
+template <bool UPPER>
+OSR_DEV void wall_e_row(const FieldDesc& fd, long long r, int j, int k, float e2, float e3);
+
+// the VPML walls (defined with their update below): a workgroup's share of the wall cells, a
+// row's interface cell inside the box, a row's interface cell inside the wall
+template <int EB, int DIMS>
+OSR_DEV void vpml_cells(const FieldDesc& fd, long long t);
+template <int EB, int DIMS>
+OSR_DEV void vpml_from_box(const FieldDesc& fd, int wl, long long r, int j, int k, float v1,
+                           float v2, float v3);
+template <int EB, int DIMS>
+OSR_DEV void vpml_to_box(const FieldDesc& fd, int wl, long long r, float (&v)[3]);
+
+// the laser launches of table row `row` into B2, B3 of column i, row r
+OSR_DEV void laser_add(const FieldDesc& fd, long long row, int i, long long r, float& b2,
+                       float& b3);
+
+// history columns; the sum of one (defined with the step end below)
+constexpr int kRedCols = 6 + kMaxSpecies;
 OSR_DEV void reduce_column(const FieldDesc& fd, int col);
 
-template <int DIMS, bool ENERGY>
+// The walls' and lasers' work that needs only a cell's own new values and its wall row's
+// buffers rides on the launches of the field cells; as launches of their own they take 4 to
+// 5 us each per step with hardly a wave in flight, and the gap to the next: 60 steps of 512x96
+// with VPML walls and a laser went from 4.01 to 3.57 ms with six launches per step for nine,
+// of 1024x256 with Lindman walls from 10.3 to 9.7 ms with seven (counting a laser launch every
+// fourth step) for eight.
+//  * VPML (first half step): the walls' E cells are work items (wk.y < 0); the threads of
+//    the box cells x = 1, nx+1 hand their new B to the wall, those of x = 0, nx+2 take theirs
+//    from it.
+//  * LASER (last half step): adds the next step's laser values, if that step will run; the
+//    launch that follows it in the stream must be that step's.
+template <int DIMS, bool ENERGY, bool VPML = false, bool LASER = false>
 __global__ __launch_bounds__(256) void yee_dbdt(const FieldDesc* __restrict__ fds,
                                                 const int2* __restrict__ work) {
   __shared__ double s_red[4][6];
@@ -117,11 +148,20 @@ __global__ __launch_bounds__(256) void yee_dbdt(const FieldDesc* __restrict__ fd
   const GridDesc& g = fd.g;
   if (ENERGY && wk.y < 0) {
     // a block of rows of the lower Lindman wall: its B update after the first half step
-    // (wall_b<1>) reads E and its own buffer only, neither of which this kernel writes
-    wall_b_row<1, DIMS>(fd, (long long)(-1 - wk.y) * 256 + threadIdx.x);
+    // (wall_b_row<1>) reads E and its own buffer only, neither of which this kernel writes
+    const long long t = (long long)(-1 - wk.y) * 256 + threadIdx.x;
+    if (VPML)
+      vpml_cells<0, DIMS>(fd, t);
+    else
+      wall_b_row<1, DIMS>(fd, t);
     return;
   }
-  if (g.ctrl->halt >= 2) return;
+  const int halt = g.ctrl->halt;
+  // the step ends after this launch: it halts where end_step will
+  const long long step = LASER ? g.ctrl->steps : 0, target = LASER ? g.ctrl->target : 0;
+  const long long las_row = LASER ? step + 1 - *fd.las_first : 0;
+  const bool las = LASER && halt == 0 && !(target > 0 && step + 1 >= target);
+  if (halt >= 2) return;
   const long long nc = g.ncell;
   const float d1 = fd.bdt[0], d2 = fd.bdt[1], d3 = fd.bdt[2];
   const int nx = g.nx, ny = g.ny;
@@ -137,13 +177,13 @@ __global__ __launch_bounds__(256) void yee_dbdt(const FieldDesc* __restrict__ fd
   // every load of the workgroup's NB cells per thread is issued before the first store
   // (E and B are distinct arrays)
   long long idx[NB];
-  int ii[NB];
+  int ii[NB], jj[NB], kk[NB];
   float e1[NB], e2[NB], e3[NB], b1[NB], b2[NB], b3[NB];
   float e3j[NB], e3i[NB], e2i[NB], e1j[NB], e2k[NB], e1k[NB];
 #pragma unroll
   for (int qb = 0; qb < NB; qb++) {
     idx[qb] = ((long long)wk.y * NB + qb) * 256 + threadIdx.x;
-    ii[qb] = 0;
+    ii[qb] = jj[qb] = kk[qb] = 0;
     e1[qb] = e2[qb] = e3[qb] = b1[qb] = b2[qb] = b3[qb] = 0.f;
     e3j[qb] = e3i[qb] = e2i[qb] = e1j[qb] = e2k[qb] = e1k[qb] = 0.f;
     if (idx[qb] >= nc) continue;
@@ -153,6 +193,8 @@ __global__ __launch_bounds__(256) void yee_dbdt(const FieldDesc* __restrict__ fd
     const long long ip = id - i + wrp(i + 1, nx);
     const long long jp = id + (long long)(wrp(j + 1, ny) - j) * nx;
     ii[qb] = i;
+    jj[qb] = j;
+    kk[qb] = k;
     e1[qb] = E1[id];
     e2[qb] = E2[id];
     e3[qb] = E3[id];
@@ -194,12 +236,24 @@ __global__ __launch_bounds__(256) void yee_dbdt(const FieldDesc* __restrict__ fd
       n2 = b2[qb] + d1 * (e3i[qb] - e3[qb]) - d3 * (e1k[qb] - e1[qb]);
       n3 = b3[qb] - d1 * (e2i[qb] - e2[qb]) + d2 * (e1j[qb] - e1[qb]);
     }
-    if (live) {
+    const long long row = jj[qb] + (long long)ny * kk[qb];
+    if (LASER && las) laser_add(fd, las_row, i, row, n2, n3);
+    const bool wall = VPML && (i == nx - 1 || i == nxi + 1);  // x = 0, nx+2
+    if (wall) {
+      float v[3];
+      vpml_to_box<0, DIMS>(fd, i == nxi + 1, row, v);
+      n1 = v[0];
+      n2 = v[1];
+      n3 = v[2];
+    }
+    if (live || wall) {
       const long long id = idx[qb];
       B1[id] = n1;
       B2[id] = n2;
       B3[id] = n3;
     }
+    if (VPML && (i == 0 || i == nxi))
+      vpml_from_box<0, DIMS>(fd, i == nxi, row, jj[qb], kk[qb], n1, n2, n3);
   }
   if (ENERGY) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -217,14 +271,20 @@ __global__ __launch_bounds__(256) void yee_dbdt(const FieldDesc* __restrict__ fd
   }
 }
 
-template <int DIMS>
+// WALL: 1 Lindman, the walls' E update by the threads of x = 1 and nx+1 (it writes x = 0,
+// nx+2, which no thread advances or reads); 2 VPML, as in yee_dbdt with the walls' B cells as
+// work items.
+template <int DIMS, int WALL = 0>
 __global__ __launch_bounds__(256) void yee_dedt(const FieldDesc* __restrict__ fds,
                                                 const int2* __restrict__ work) {
   const int2 wk = work[blockIdx.x];
   const FieldDesc& fd = fds[wk.x];
   const GridDesc& g = fd.g;
   if (wk.y < 0) {  // a history column: its partial sums are complete before this launch
-    reduce_column(fd, -1 - wk.y);
+    if (WALL == 2 && wk.y < -kRedCols)
+      vpml_cells<1, DIMS>(fd, (long long)(-1 - kRedCols - wk.y) * 256 + threadIdx.x);
+    else
+      reduce_column(fd, -1 - wk.y);
     return;
   }
   if (g.ctrl->halt >= 2) return;
@@ -288,10 +348,24 @@ __global__ __launch_bounds__(256) void yee_dedt(const FieldDesc* __restrict__ fd
   }
   // open x walls: E is advanced on x = 1 .. nx+1 only (dedt_2d loops); the current of
   // every column is still converted and cleared above
-  if (i > interior_nx(g)) return;
+  const int nxi = interior_nx(g);
+  const long long row = j + (long long)ny * k;
+  if (WALL == 2 && (i == nx - 1 || i == nxi + 1)) {
+    float v[3];
+    vpml_to_box<1, DIMS>(fd, i == nxi + 1, row, v);
+    e1 = v[0];
+    e2 = v[1];
+    e3 = v[2];
+  } else if (i > nxi) {
+    return;
+  }
   E1[idx] = e1;
   E2[idx] = e2;
   E3[idx] = e3;
+  if (WALL == 1 && i == 0) wall_e_row<false>(fd, row, j, k, e2, e3);
+  if (WALL == 1 && i == nxi) wall_e_row<true>(fd, row, j, k, e2, e3);
+  if (WALL == 2 && (i == 0 || i == nxi))
+    vpml_from_box<1, DIMS>(fd, i == nxi, row, j, k, e1, e2, e3);
 }
 
 // ------------------------------------------------------------------------------------
@@ -521,12 +595,12 @@ OSR_DEV float* wall_at(const FieldDesc& fd, int k, long long R) { return fd.wall
 // B buffer of the lower wall.  STEP 2: the reference reads E3(0, ny+1, z) and E2(0, y,
 // nz+1), guard cells that nothing refreshes between the start of the step and the second
 // B half step, so they still hold E3(0, 1, z) and E2(0, y, 1) of the start of the step
-// (saved by wall_e).  E1 on the wall is always zero.
+// (saved by wall_e_row).  E1 on the wall is always zero.
 // RESTORE (after the second B half step): the same thread then puts its row's wall values
 // back into the box, as wall_restore does.  The B update reads E only at x = 0 and x = 1;
-// there the restore rewrites the values the box already holds (wall_e left E2, E3 at x = 0
-// equal to their buffers, E1 there is never advanced and stays zero, and no kernel since
-// wall_e writes E).  The writes that change the box (B at x = 0, E1 at x = nx+1) touch
+// there the restore rewrites the values the box already holds (wall_e_row left E2, E3 at
+// x = 0 equal to their buffers, E1 there is never advanced and stays zero, and no kernel
+// since writes E).  The writes that change the box (B at x = 0, E1 at x = nx+1) touch
 // cells no B update reads, so the rows need no ordering and one launch does both.
 template <int STEP, int DIMS, bool RESTORE>
 OSR_DEV void wall_b_row(const FieldDesc& fd, long long r) {
@@ -589,55 +663,42 @@ OSR_DEV void wall_b_row(const FieldDesc& fd, long long r) {
   }
 }
 
-template <int STEP, int DIMS, bool RESTORE = false>
-__global__ __launch_bounds__(256) void wall_b(const FieldDesc* __restrict__ fds) {
-  wall_b_row<STEP, DIMS, RESTORE>(*fds, (long long)blockIdx.x * 256 + threadIdx.x);
-}
-
-__global__ __launch_bounds__(256) void wall_e(const FieldDesc* __restrict__ fds) {
-  const FieldDesc& fd = *fds;
+template <bool UPPER>
+OSR_DEV void wall_e_row(const FieldDesc& fd, long long r, int j, int k, float e2, float e3) {
   const GridDesc& g = fd.g;
-  const int halt = g.ctrl->halt;  // checked before the first store, the loads in flight
-  const int ny = g.ny, nz = g.nz, nx = g.nx, nxi = g.open_nx;
-  const long long R = (long long)ny * nz;
-  const long long r = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (r >= R) return;
-  int j, k;
-  row_yz(g, r, j, k);
-  const long long nc = g.ncell;
+  const int nx = g.nx, nxi = g.open_nx;
+  const long long R = (long long)g.ny * g.nz, nc = g.ncell, row = r * nx;
   const float dc = fd.wall_dc;
-  float* ebl = wall_at(fd, 0, R);
-  float* ebu = wall_at(fd, 9, R);
-  float* stale3 = wall_at(fd, 15, R);
-  float* stale2 = stale3 + nz;
-  const long long row = r * nx;
   // lower wall: E(0) = buf(1) + dc (buf(0) - E(1)); buffers <- E(0), E(1)
   // upper wall: E(nx+2) = buf(nx+1) + dc (buf(nx+2) - E(nx+1)); buffers <- E(nx+1), E(nx+2)
-  float lb0[3], lb1[3], e1v[3], ub1[3], ub2[3], env[3];
+  float* eb = wall_at(fd, UPPER ? 9 : 0, R);
+  const float ev[3] = {0.f, e2, e3};
+  float b0[3], b1[3];
 #pragma unroll
   for (int p = 1; p <= 2; p++) {
-    const float* E = g.E + p * nc + row;
-    lb0[p] = ebl[(2 * p + 0) * R + r];
-    lb1[p] = ebl[(2 * p + 1) * R + r];
-    e1v[p] = E[0];
-    ub1[p] = ebu[(2 * p + 0) * R + r];
-    ub2[p] = ebu[(2 * p + 1) * R + r];
-    env[p] = E[nxi];
+    b0[p] = eb[(2 * p + 0) * R + r];
+    b1[p] = eb[(2 * p + 1) * R + r];
   }
-  if (halt >= 2) return;
-  if (j == 0) stale3[k] = lb0[2];  // E3(0, 1, z) before this update
-  if (k == 0) stale2[j] = lb0[1];  // E2(0, y, 1)
+  if (!UPPER) {
+    float* stale3 = wall_at(fd, 15, R);
+    float* stale2 = stale3 + g.nz;
+    if (j == 0) stale3[k] = b0[2];  // E3(0, 1, z) before this update
+    if (k == 0) stale2[j] = b0[1];  // E2(0, y, 1)
+  }
 #pragma unroll
   for (int p = 1; p <= 2; p++) {
     float* E = g.E + p * nc + row;
-    const float v = lb1[p] + dc * (lb0[p] - e1v[p]);
-    E[nx - 1] = v;
-    ebl[(2 * p + 0) * R + r] = v;
-    ebl[(2 * p + 1) * R + r] = e1v[p];
-    const float w = ub1[p] + dc * (ub2[p] - env[p]);
-    E[nxi + 1] = w;
-    ebu[(2 * p + 0) * R + r] = env[p];
-    ebu[(2 * p + 1) * R + r] = w;
+    if (UPPER) {
+      const float w = b0[p] + dc * (b1[p] - ev[p]);
+      E[nxi + 1] = w;
+      eb[(2 * p + 0) * R + r] = ev[p];
+      eb[(2 * p + 1) * R + r] = w;
+    } else {
+      const float v = b1[p] + dc * (b0[p] - ev[p]);
+      E[nx - 1] = v;
+      eb[(2 * p + 0) * R + r] = v;
+      eb[(2 * p + 1) * R + r] = ev[p];
+    }
   }
 }
 
@@ -720,57 +781,27 @@ __global__ __launch_bounds__(256) void vpml_diffuse(const FieldDesc* __restrict_
   zy[o] = keep * b + rate * a;
 }
 
+// the wall cell next to the box (box_to_vpml) and the one after it (vpml_to_box)
+OSR_DEV int vp_btv(int wl, int n) { return wl == 0 ? n - 1 : 0; }
+OSR_DEV int vp_vtb(int wl, int n) { return wl == 0 ? n - 2 : 1; }
+
+// Update of wall cell (wl, l, row r).  bY, bZ: the box's second and third component at the
+// interface, which stand for the neighbouring wall cell where that one is box_to_vpml.
 template <int EB, int DIMS>
-__global__ __launch_bounds__(256) void vpml_update(const FieldDesc* __restrict__ fds) {
+OSR_DEV void vpml_cell(const FieldDesc& fd, int wl, int l, long long r, int j, int k, float bY,
+                       float bZ) {
   constexpr int NC = DIMS == 3 ? 6 : 4;
-  const FieldDesc& fd = *fds;
   const GridDesc& g = fd.g;
-  if (g.ctrl->halt >= 2) return;
-  const int n = fd.vp_n, ny = g.ny, nz = g.nz, nx = g.nx;
+  const int n = fd.vp_n, ny = g.ny, nz = g.nz;
   const long long R = (long long)ny * nz;
-  const long long t = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (t >= 2 * n * R) return;
-  const long long r = t % R;
-  const int l = (int)((t / R) % n);
-  const int wl = (int)(t / (R * n));
-  int j, k;
-  row_yz(g, r, j, k);
-  const long long nc = g.ncell;
-  // ring columns of the wall's interface cells: x = 1 and 0 (lower), nx+1 and nx+2 (upper)
-  const int btv = wl == 0 ? n - 1 : 0, vtb = wl == 0 ? n - 2 : 1;
-  const long long cb = r * nx + (wl == 0 ? 0 : g.open_nx);
-  const long long cv = r * nx + (wl == 0 ? nx - 1 : g.open_nx + 1);
   const long long o = (long long)l * R + r;
-  float* const F = EB == 0 ? g.B : g.E;  // the box field of the interface
-  float* W[NC];                          // its wall counterpart
-  float* U[NC];                          // the wall field updated
+  const int btv = vp_btv(wl, n);
+  const float* W[NC];  // the wall counterpart of the field the interface exchanges
+  float* U[NC];        // the wall field updated
 #pragma unroll
   for (int c = 0; c < NC; c++) {
     W[c] = vp_arr<DIMS>(fd, wl, EB == 0 ? 1 : 0, c);
     U[c] = vp_arr<DIMS>(fd, wl, EB == 0 ? 0 : 1, c);
-  }
-  if (l == btv) {
-    if (DIMS == 2) {
-      W[0][o] = F[cb];
-      W[1][o] = F[nc + cb];
-      W[2][o] = F[2 * nc + cb];
-      W[3][o] = 0.0f;
-    } else {
-#pragma unroll
-      for (int c = 0; c < 3; c++) {
-        W[2 * c][o] = F[c * nc + cb];
-        W[2 * c + 1][o] = 0.0f;
-      }
-    }
-  } else if (l == vtb && !(DIMS == 2 && EB == 0 && fd.vp_diff[wl])) {  // else vpml_diffuse
-    if (DIMS == 2) {
-      F[cv] = W[0][o];
-      F[nc + cv] = W[1][o];
-      F[2 * nc + cv] = W[2][o] + W[3][o];
-    } else {
-#pragma unroll
-      for (int c = 0; c < 3; c++) F[c * nc + cv] = W[2 * c][o] + W[2 * c + 1][o];
-    }
   }
   const float d2 = fd.vp_dt2, d3 = fd.vp_dt3;
   const float* cf = fd.wall + (size_t)4 * NC * n * R + (size_t)(wl * 2 + EB) * 3 * n;
@@ -784,24 +815,24 @@ __global__ __launch_bounds__(256) void vpml_update(const FieldDesc* __restrict__
     const float c1 = cf[ci], c2 = cf[n + ci], c3 = cf[2 * n + ci];
     const long long ol = o - R;  // cell x-1
     const bool from_box = l - 1 == btv;  // upper wall, first updated cell: x-1 = nx+1
-    if (DIMS == 2) {
-      const float bl1 = from_box ? F[nc + cb] : W[1][ol];
-      const float bl23 = from_box ? F[2 * nc + cb] + 0.0f : W[2][ol] + W[3][ol];
+    if constexpr (DIMS == 2) {
+      const float bl1 = from_box ? bY : W[1][ol];
+      const float bl23 = from_box ? bZ + 0.0f : W[2][ol] + W[3][ol];
       const float b0 = W[0][o], b1 = W[1][o], b2 = W[2][o], b3 = W[3][o];
       U[0][o] = U[0][o] + d2 * (b2 + b3 - W[2][ojm] - W[3][ojm]);
       U[3][o] = U[3][o] - d2 * (b0 - W[0][ojm]);
       U[1][o] = c1 * U[1][o] - c2 * (b2 + b3) + c3 * bl23;
       U[2][o] = c1 * U[2][o] + c2 * b1 - c3 * bl1;
     } else {
-      const float blY = from_box ? F[nc + cb] + 0.0f : W[2][ol] + W[3][ol];
-      const float blZ = from_box ? F[2 * nc + cb] + 0.0f : W[4][ol] + W[5][ol];
-      const float bX = W[0][o] + W[1][o], bY = W[2][o] + W[3][o], bZ = W[4][o] + W[5][o];
-      U[0][o] = U[0][o] + d2 * (bZ - W[4][ojm] - W[5][ojm]);
-      U[5][o] = U[5][o] - d2 * (bX - W[0][ojm] - W[1][ojm]);
-      U[1][o] = U[1][o] - d3 * (bY - W[2][okm] - W[3][okm]);
-      U[3][o] = U[3][o] + d3 * (bX - W[0][okm] - W[1][okm]);
-      U[2][o] = c1 * U[2][o] - c2 * bZ + c3 * blZ;
-      U[4][o] = c1 * U[4][o] + c2 * bY - c3 * blY;
+      const float blY = from_box ? bY + 0.0f : W[2][ol] + W[3][ol];
+      const float blZ = from_box ? bZ + 0.0f : W[4][ol] + W[5][ol];
+      const float wX = W[0][o] + W[1][o], wY = W[2][o] + W[3][o], wZ = W[4][o] + W[5][o];
+      U[0][o] = U[0][o] + d2 * (wZ - W[4][ojm] - W[5][ojm]);
+      U[5][o] = U[5][o] - d2 * (wX - W[0][ojm] - W[1][ojm]);
+      U[1][o] = U[1][o] - d3 * (wY - W[2][okm] - W[3][okm]);
+      U[3][o] = U[3][o] + d3 * (wX - W[0][okm] - W[1][okm]);
+      U[2][o] = c1 * U[2][o] - c2 * wZ + c3 * blZ;
+      U[4][o] = c1 * U[4][o] + c2 * wY - c3 * blY;
     }
   } else {
     if (l < (wl == 0 ? 0 : 1) || l > n - 2) return;
@@ -809,17 +840,17 @@ __global__ __launch_bounds__(256) void vpml_update(const FieldDesc* __restrict__
     const float c1 = cf[ci], c2 = cf[n + ci], c3 = cf[2 * n + ci];
     const long long or1 = o + R;  // cell x+1
     const bool from_box = l + 1 == btv;  // lower wall, last updated cell: x+1 = 1
-    if (DIMS == 2) {
-      const float el1 = from_box ? F[nc + cb] : W[1][or1];
-      const float el23 = from_box ? F[2 * nc + cb] + 0.0f : W[2][or1] + W[3][or1];
+    if constexpr (DIMS == 2) {
+      const float el1 = from_box ? bY : W[1][or1];
+      const float el23 = from_box ? bZ + 0.0f : W[2][or1] + W[3][or1];
       const float e0 = W[0][o], e1 = W[1][o], e2 = W[2][o], e3 = W[3][o];
       U[0][o] = U[0][o] - d2 * (W[2][ojp] + W[3][ojp] - e2 - e3);
       U[3][o] = U[3][o] + d2 * (W[0][ojp] - e0);
       U[1][o] = c1 * U[1][o] + c2 * el23 - c3 * (e2 + e3);
       U[2][o] = c1 * U[2][o] - c2 * el1 + c3 * e1;
     } else {
-      const float elY = from_box ? F[nc + cb] + 0.0f : W[2][or1] + W[3][or1];
-      const float elZ = from_box ? F[2 * nc + cb] + 0.0f : W[4][or1] + W[5][or1];
+      const float elY = from_box ? bY + 0.0f : W[2][or1] + W[3][or1];
+      const float elZ = from_box ? bZ + 0.0f : W[4][or1] + W[5][or1];
       const float e0 = W[0][o], e1 = W[1][o], e2 = W[2][o], e3 = W[3][o];
       const float e4 = W[4][o], e5 = W[5][o];
       U[0][o] = U[0][o] - d2 * (W[4][ojp] + W[5][ojp] - e4 - e5);
@@ -830,6 +861,102 @@ __global__ __launch_bounds__(256) void vpml_update(const FieldDesc* __restrict__
       U[4][o] = c1 * U[4][o] - c2 * elY + c3 * (e2 + e3);
     }
   }
+}
+
+// wall, cell and row of wall item t
+OSR_DEV bool vp_item(const FieldDesc& fd, long long t, int& wl, int& l, long long& r, int& j,
+                     int& k) {
+  const GridDesc& g = fd.g;
+  const long long R = (long long)g.ny * g.nz;
+  if (t >= 2 * fd.vp_n * R) return false;
+  r = t % R;
+  l = (int)((t / R) % fd.vp_n);
+  wl = (int)(t / (R * fd.vp_n));
+  row_yz(g, r, j, k);
+  return true;
+}
+
+// the one cell of a wall whose neighbour is box_to_vpml: updated by the box cell's thread
+template <int EB>
+OSR_DEV bool vp_by_box(int wl, int l, int n) {
+  return EB == 0 ? wl == 1 && l == 1 : wl == 0 && l == n - 2;
+}
+
+template <int EB, int DIMS>
+OSR_DEV void vpml_cells(const FieldDesc& fd, long long t) {
+  if (fd.g.ctrl->halt >= 2) return;
+  int wl, l, j, k;
+  long long r;
+  if (!vp_item(fd, t, wl, l, r, j, k) || vp_by_box<EB>(wl, l, fd.vp_n)) return;
+  vpml_cell<EB, DIMS>(fd, wl, l, r, j, k, 0.0f, 0.0f);
+}
+
+// box_to_vpml: the box cell's new values into the wall, and the wall cell that needs them.
+// No other thread of the launch reads the wall cell written.
+template <int EB, int DIMS>
+OSR_DEV void vpml_from_box(const FieldDesc& fd, int wl, long long r, int j, int k, float v1,
+                           float v2, float v3) {
+  const int n = fd.vp_n, l = EB == 0 ? 1 : n - 2;
+  const long long o = (long long)vp_btv(wl, n) * fd.g.ny * fd.g.nz + r;
+  constexpr int eb = EB == 0 ? 1 : 0;
+  if (vp_by_box<EB>(wl, l, n)) vpml_cell<EB, DIMS>(fd, wl, l, r, j, k, v2, v3);
+  if (DIMS == 2) {
+    vp_arr<DIMS>(fd, wl, eb, 0)[o] = v1;
+    vp_arr<DIMS>(fd, wl, eb, 1)[o] = v2;
+    vp_arr<DIMS>(fd, wl, eb, 2)[o] = v3;
+    vp_arr<DIMS>(fd, wl, eb, 3)[o] = 0.0f;
+  } else {
+    const float v[3] = {v1, v2, v3};
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      vp_arr<DIMS>(fd, wl, eb, 2 * c)[o] = v[c];
+      vp_arr<DIMS>(fd, wl, eb, 2 * c + 1)[o] = 0.0f;
+    }
+  }
+}
+
+// vpml_to_box: the sums of a wall cell's split pairs, which no thread of the launch writes
+template <int EB, int DIMS>
+OSR_DEV void vpml_to_box(const FieldDesc& fd, int wl, long long r, float (&v)[3]) {
+  const long long o = (long long)vp_vtb(wl, fd.vp_n) * fd.g.ny * fd.g.nz + r;
+  constexpr int eb = EB == 0 ? 1 : 0;
+  if (DIMS == 2) {
+    v[0] = vp_arr<DIMS>(fd, wl, eb, 0)[o];
+    v[1] = vp_arr<DIMS>(fd, wl, eb, 1)[o];
+    v[2] = vp_arr<DIMS>(fd, wl, eb, 2)[o] + vp_arr<DIMS>(fd, wl, eb, 3)[o];
+  } else {
+#pragma unroll
+    for (int c = 0; c < 3; c++)
+      v[c] = vp_arr<DIMS>(fd, wl, eb, 2 * c)[o] + vp_arr<DIMS>(fd, wl, eb, 2 * c + 1)[o];
+  }
+}
+
+// The B interface and the E update after vpml_diffuse, whose mixing comes between the first B
+// half step and the wall cells, as a launch of its own (2D).
+__global__ __launch_bounds__(256) void vpml_update_e(const FieldDesc* __restrict__ fds) {
+  const FieldDesc& fd = *fds;
+  const GridDesc& g = fd.g;
+  if (g.ctrl->halt >= 2) return;
+  int wl, l, j, k;
+  long long r;
+  if (!vp_item(fd, (long long)blockIdx.x * 256 + threadIdx.x, wl, l, r, j, k)) return;
+  const int n = fd.vp_n;
+  const long long nc = g.ncell;
+  const long long cb = r * g.nx + (wl == 0 ? 0 : g.open_nx);
+  if (l == vp_btv(wl, n)) {
+    const long long o = (long long)l * g.ny + r;
+    vp_arr<2>(fd, wl, 1, 0)[o] = g.B[cb];
+    vp_arr<2>(fd, wl, 1, 1)[o] = g.B[nc + cb];
+    vp_arr<2>(fd, wl, 1, 2)[o] = g.B[2 * nc + cb];
+    vp_arr<2>(fd, wl, 1, 3)[o] = 0.0f;
+  } else if (l == vp_vtb(wl, n) && !fd.vp_diff[wl]) {  // else vpml_diffuse
+    const long long cv = r * g.nx + (wl == 0 ? g.nx - 1 : g.open_nx + 1);
+    float v[3];
+    vpml_to_box<0, 2>(fd, wl, r, v);
+#pragma unroll
+    for (int c = 0; c < 3; c++) g.B[c * nc + cv] = v[c];
+  }
+  vpml_cell<0, 2>(fd, wl, l, r, j, k, g.B[nc + cb], g.B[2 * nc + cb]);
 }
 
 // zpulse_wall launches (launch_em_wall_2d, zpulse/os-zpulse-wall.f03:865-960): B2, B3 of
@@ -858,6 +985,19 @@ __global__ __launch_bounds__(256) void laser_wall(const FieldDesc* __restrict__ 
   }
 }
 
+OSR_DEV void laser_add(const FieldDesc& fd, long long row, int i, long long r, float& b2,
+                       float& b3) {
+  if (row < 0 || row >= fd.las_rows) return;
+  const long long R = (long long)fd.g.ny * fd.g.nz;
+  for (int k = 0; k < fd.las_k; k++) {
+    if (i != fd.las_col[k]) continue;
+    const long long e = row * fd.las_k + k;
+    if (!fd.las_mask[e]) continue;
+    const float* v = fd.las_tab + e * 2 * R;
+    b2 = b2 + v[r];
+    b3 = b3 + v[R + r];
+  }
+}
 
 // Neumaier compensated accumulation
 OSR_DEV void kadd(double& s, double& c, double v) {
@@ -888,7 +1028,6 @@ OSR_DEV void kmerge(double& s, double& c, double s2, double c2) {
 // 12 us on a 64 x 64 grid and 29 us on 192^3.  A 100-step 64 x 64 run went from 5.44 to
 // 4.42 ms, 40 steps of 52 x 44 x 36 from 4.81 to 4.40 ms.
 constexpr int kRedNT = 256;
-constexpr int kRedCols = 6 + kMaxSpecies;
 
 OSR_DEV void reduce_column(const FieldDesc& fd, int col) {
   __shared__ double w_s[kRedNT / 64], w_c[kRedNT / 64];
@@ -946,7 +1085,7 @@ __global__ __launch_bounds__(64) void finalize_step(const FieldDesc* __restrict_
 }
 
 // Lindman walls: the lower wall's second B update with the restore of the wall values
-// (wall_b<2, DIMS, true>) and the end of the step in the workgroup that finishes last (a
+// (wall_b_row<2, DIMS, true>) and the end of the step in the workgroup that finishes last (a
 // ticket on Ctrl::done), so no kernel launch follows.  Every workgroup has read the halt
 // flag before it takes its ticket, so the flag changes only once none of them looks at it
 // any more.
@@ -1255,18 +1394,22 @@ template __global__ void yee_dbdt<2, true>(const FieldDesc*, const int2*);
 template __global__ void yee_dbdt<2, false>(const FieldDesc*, const int2*);
 template __global__ void yee_dbdt<3, true>(const FieldDesc*, const int2*);
 template __global__ void yee_dbdt<3, false>(const FieldDesc*, const int2*);
+template __global__ void yee_dbdt<2, true, true>(const FieldDesc*, const int2*);
+template __global__ void yee_dbdt<3, true, true>(const FieldDesc*, const int2*);
+template __global__ void yee_dbdt<2, false, false, true>(const FieldDesc*, const int2*);
+template __global__ void yee_dbdt<3, false, false, true>(const FieldDesc*, const int2*);
 template __global__ void yee_dedt<2>(const FieldDesc*, const int2*);
+template __global__ void yee_dedt<2, 1>(const FieldDesc*, const int2*);
+template __global__ void yee_dedt<2, 2>(const FieldDesc*, const int2*);
+template __global__ void yee_dedt<3>(const FieldDesc*, const int2*);
+template __global__ void yee_dedt<3, 1>(const FieldDesc*, const int2*);
+template __global__ void yee_dedt<3, 2>(const FieldDesc*, const int2*);
 template __global__ void yee2d_step<32, 8>(const FieldDesc*, const int2*, int);
 template __global__ void yee2d_step<64, 16>(const FieldDesc*, const int2*, int);
 template __global__ void yee2d_energy<32, 8>(const FieldDesc*, const int2*, int);
 template __global__ void yee2d_energy<64, 16>(const FieldDesc*, const int2*, int);
 template __global__ void wall_b2_end<2>(const FieldDesc*);
 template __global__ void wall_b2_end<3>(const FieldDesc*);
-template __global__ void vpml_update<0, 2>(const FieldDesc*);
-template __global__ void vpml_update<1, 2>(const FieldDesc*);
-template __global__ void vpml_update<0, 3>(const FieldDesc*);
-template __global__ void vpml_update<1, 3>(const FieldDesc*);
-template __global__ void yee_dedt<3>(const FieldDesc*, const int2*);
 template __global__ void rho_deposit<1>(const SpecDesc*, const int2*, unsigned long long*, double);
 template __global__ void rho_deposit<2>(const SpecDesc*, const int2*, unsigned long long*, double);
 template __global__ void rho_deposit<3>(const SpecDesc*, const int2*, unsigned long long*, double);

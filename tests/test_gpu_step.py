@@ -176,3 +176,31 @@ def test_particles_come_back_in_upload_order(dims, n):
     for m in range(1, dims):
         d[:, m] -= nx[m] * np.round(d[:, m] / nx[m])
     assert np.abs(d).max() < 1e-3
+
+
+@pytest.mark.parametrize("dims,xbnd", [(2, "lindman"), (2, "vpml"), (3, "lindman"), (3, "vpml")])
+def test_laser_steps_in_one_call(dims, xbnd):
+    """Steps of one call against calls of one step: inside a call the last field launch of a
+    step adds the next step's laser values, the first step of a call has a launch of its
+    own.  The drifting block overflows tiles, so steps also stop between the two."""
+    print(f"case dims={dims} xbnd={xbnd}", flush=True)
+    nx = (32, 30, 10)[:dims]
+    rng = np.random.default_rng(21)
+    n = 6000
+    ix = np.stack([rng.integers(lo, hi, n) for lo, hi in ((17, 25), (1, 9), (1, 5))[:dims]], 1).astype(np.int32)
+    x = (rng.random((n, dims), np.float32) - np.float32(0.5)).astype(np.float32)
+    u = (rng.standard_normal((n, 3)) * 0.05 + (2.0, 1.5, 0.0)).astype(np.float32)
+    out = []
+    for calls in ((1,) * 23, (23,), (9, 2, 12)):
+        with oa.Simulation(dims, nx, (0.1,) * dims, 0.05, 2, xbnd=xbnd, tile=(8, 8, 4)[:dims]) as sim:
+            sim.set_particles(sim.add_species(-1.0), ix, x, u, np.full(n, -0.02, np.float32))
+            for prop in ("forward", "backward"):
+                sim.add_zpulse_wall(a0=0.7, omega0=5.0, pol=30.0, pol_type=1, propagation=prop,
+                                    tenv_type="sin2", tenv_rise=0.4, tenv_flat=0.5, tenv_fall=0.3)
+            for k in calls:
+                sim.run(k)
+            out.append((sim.get_fields(), sim.get_particles(0), (), sim.history()))
+            rel = sim.relayouts
+    assert rel >= 1
+    for o in out[1:]:
+        _same(out[0], o)
