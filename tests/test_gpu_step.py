@@ -204,3 +204,32 @@ def test_laser_steps_in_one_call(dims, xbnd):
     assert rel >= 1
     for o in out[1:]:
         _same(out[0], o)
+
+
+@pytest.mark.parametrize("dims,order", [(2, 1), (2, 2), (2, 3), (3, 1), (3, 2), (3, 3)])
+@pytest.mark.parametrize("n", [1, 256, 257, 9000])
+def test_dropin_current_in_any_particle_order(dims, order, n):
+    """Particles in cell order, whose workgroups sum their current in LDS, and the same ones
+    shuffled over the whole grid, whose workgroups add to memory: the integer sums agree, so
+    the currents have the same bits; so have the particles."""
+    print(f"case dims={dims} order={order} n={n}", flush=True)
+    rng = np.random.default_rng(17)
+    nx, lo, hi = (90, 70, 40)[:dims], 3, 4
+    ix = np.stack([rng.integers(1, m + 1, n) for m in nx], 1).astype(np.int32)
+    if dims == 3:  # dense enough for the sorted case to fit: 9000 in a 24 x 20 x 10 corner
+        ix = np.stack([rng.integers(1, m + 1, n) for m in (24, 20, 10)], 1).astype(np.int32)
+    ix = ix[np.lexsort(ix.T)]
+    x = (rng.random((n, dims), np.float32) - np.float32(0.5)).astype(np.float32)
+    u = (rng.standard_normal((n, 3)) * 2.0).astype(np.float32)
+    q = np.full(n, -0.0173, np.float32)
+    shape = tuple(m + lo + hi for m in reversed(nx)) + (3,)
+    e, b = (rng.standard_normal(shape).astype(np.float32) for _ in range(2))
+    out = []
+    for p in (np.arange(n), rng.permutation(n)):
+        j = np.zeros(shape, np.float32)
+        r = oa.advance_deposit(dims, order, ix[p], x[p], u[p], q, -1.0, e, b, lo, j, lo,
+                               (0.1,) * dims, 0.05)
+        back = np.argsort(p)
+        out.append([j] + [a[back] for a in r[:3]])
+    for a, c in zip(*out):
+        assert np.array_equal(a.view(np.uint32), c.view(np.uint32))
