@@ -1377,8 +1377,8 @@ int osr_sim_create(const osr_sim_desc* desc, osr_sim** out) {
   s->lds_push = s->plain ? 0 : push_lds_bytes(dims, s->order, tile);
   if (s->lds_push > 160 * 1024) return fail(OSR_ERR_ARG, "tile too large for LDS");
   // Default re-order period.  The cubic 3D push waits for its LDS passes, which the order of a
-  // tile's particles decides: a 192^3 step takes 7.43 ms with a period of 3 or 4, 7.50 with 2,
-  // 7.53 with 6 and 7.61 with 8.  Linear and quadratic lines are shorter and their push is not
+  // tile's particles decides: a 192^3 step takes 7.15 ms with a period of 3, 7.07 to 7.09 with
+  // 4 to 8, 7.19 with 16 and 7.58 without.  Linear and quadratic lines are shorter and their push is not
   // bound by them: a 96^3 quadratic step of drifting beams takes 703 us with a period of 4, 682
   // with 8 and 673 with 16, 32 and none, a 52x44x36 linear one 70.6, 66.7, 64.8, 64.1 and 61.6
   // without (a launch that finds nothing to do costs 2.5 us).

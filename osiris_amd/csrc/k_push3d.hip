@@ -1,7 +1,7 @@
 // k_push3d.hip -- fused 3D push + deposit with compile-time tile shape.
 //
-// One workgroup of 4 waves (cubic splines) or 8 per (species, tile).  Compared with the generic 3D kernel in
-// k_tiles.hip:
+// One workgroup of 4 waves (cubic splines) or 8 per (species, tile).  Compared with the
+// generic 3D kernel in k_tiles.hip:
 //  * TX/TY/TZ are template parameters, so the LDS pitches of the staged field and current
 //    tiles are constants and every stencil offset is an immediate (the generic kernel
 //    adds runtime row and plane pitches for each of the 4 x 4 lines of a cubic stencil,
@@ -13,11 +13,15 @@
 //  * a particle that stays in its cell is deposited from registers; one that crosses a face
 //    is queued in LDS, and the waves split and deposit 64 of them at a time (their third and
 //    fourth virtual particles go back into the queue, so they run on full waves too).
+//  * with cubic splines the lanes of a deposit are permuted first, so that the 64-bit adds of a
+//    16-lane group mostly fall into different banks (spread_lanes).
 // What bounds it: LDS.  Per 64 particles the cubic gather makes 192 paired 4-byte reads, whose
 // lanes conflict through their half-cell shifts (9 cycles of a CU each, 5 without conflicts),
-// and the deposit 161 64-bit adds (11 cycles each, 7.4 without): about 90% of the cycles on
-// 192^3, 8 per cell (6.4 ms), with the VALU 42% busy (55% with the split in the main path and
-// subtracted fixed-point bits, in the same time).  Linear and quadratic splines have room for
+// and the deposit 161 64-bit adds (11 cycles each as the particles come, some 9 on permuted
+// lanes, 7.4 without conflicts): about 90% of the cycles on 192^3, 8 per cell.  The permutation
+// takes 11 crossbar operations and the splines once more, and 6.4 ms became 6.0; quadratic
+// splines gain nothing from it (96^3, two beams of 4: 27.9 ms per 40 steps either way), linear
+// ones lose (52x44x36: 2.70 -> 2.80 ms).  Linear and quadratic splines have room for
 // 8 waves in 128 registers, 4 per SIMD instead of 2: 52x44x36 linear 34 -> 29.6 us, 96^3
 // quadratic, two beams of 4, 464 -> 428 us; cubic spills there and gains nothing.
 // The arithmetic (gather line/plane order, pusher, position advance, split, deposit) is
@@ -43,6 +47,39 @@ OSR_DEV lcf32* lds_line(const float* base, int elem) {
   return (lcf32*)(size_t)a;
 }
 
+// A permutation of the lanes (the lane whose values each lane takes) that spreads the lanes
+// with `on` over the 16-lane groups in which LDS makes 64-bit adds: lane 16 k + r takes the
+// k-th one whose `res` (its base node mod 16, the pair of banks its adds fall into) is r, and
+// what is over four of a kind fills the lanes left free.  Every lane is some lane's source.
+OSR_DEV int spread_lanes(bool on, int res, int lane) {
+  const unsigned long long m = __ballot(on);
+  const unsigned long long b0 = __ballot(res & 1), b1 = __ballot(res & 2), b2 = __ballot(res & 4),
+                           b3 = __ballot(res & 8);
+  auto kind = [&](int v) {  // the lanes with `on` and residue v
+    return m & (v & 1 ? b0 : ~b0) & (v & 2 ? b1 : ~b1) & (v & 4 ? b2 : ~b2) & (v & 8 ? b3 : ~b3);
+  };
+  const unsigned long long below = (1ull << lane) - 1ull;
+  const int rank = __popcll(kind(res) & below);
+  const bool placed = on && rank < 4;
+  const bool taken = __popcll(kind(lane & 15)) > (lane >> 4);
+  const unsigned long long mp = __ballot(placed), fr = ~__ballot(taken);
+  // the lanes not placed, in order, those with `on` first
+  const unsigned long long ov = m & ~mp, id = ~m;
+  const int nov = __popcll(ov), rest = nov + __popcll(id);
+  const int idx = on ? (placed ? rest + __popcll(mp & below) : __popcll(ov & below))
+                     : nov + __popcll(id & below);
+  const int order = __builtin_amdgcn_ds_permute(idx << 2, lane);
+  // every lane not placed sends to a free lane, whose value is not used
+  const int spare = fr ? __ffsll((long long)fr) - 1 : 0;
+  const int from = __builtin_amdgcn_ds_permute((placed ? 16 * rank + res : spare) << 2, lane);
+  const int fill = __builtin_amdgcn_ds_bpermute(__popcll(fr & below) << 2, order);
+  return taken ? from : fill;
+}
+
+OSR_DEV float lane_from(float v, int src) {
+  return __int_as_float(__builtin_amdgcn_ds_bpermute(src << 2, __float_as_int(v)));
+}
+
 template <int ORDER, int TX, int TY, int TZ>
 struct Tile3 {
   using O = Ord<ORDER>;
@@ -59,6 +96,7 @@ struct Tile3 {
   // planes of the current padded where LDS has room (13 x 13 nodes for cubic splines): 8%
   // fewer bank conflicts of the 64-bit adds in a model of the particle order
   static constexpr int JXY = JX * JY + (JX == 13 ? 5 : 0), JN = JXY * JZ;
+  static constexpr bool SPREAD = ORDER == 3;
   static constexpr int NW = push3d_waves(ORDER), NT = 64 * NW, QC = 64;
 };
 
@@ -347,9 +385,25 @@ __global__ __launch_bounds__(64 * push3d_waves(ORDER), push3d_waves(ORDER) / 2) 
       }
       mcount += __popcll(mm);
       // ---- deposit of the particles that stay in their cell, with the gather's splines
-      if (act && !cross)
+      const bool in = act && !cross;
+      if constexpr (T::SPREAD) {
+        const int src = spread_lanes(in, nb0 & 15, lane);
+        const float X = lane_from(x, src), Y = lane_from(y, src), Z = lane_from(z, src);
+        const float X1 = lane_from(x1, src), Y1 = lane_from(y1, src), Z1 = lane_from(z1, src);
+        const float Q = lane_from(q, src);
+        const int nb = __builtin_amdgcn_ds_bpermute(src << 2, in ? nb0 : -1);
+        if (nb >= 0) {
+          float S0x[NP], S0y[NP], S0z[NP];
+          spline<ORDER>(X, S0x);
+          spline<ORDER>(Y, S0y);
+          spline<ORDER>(Z, S0z);
+          dep_vp3<ORDER, RAW>(sJ, JN, S0x, S0y, S0z, X, Y, Z, X1, Y1, Z1, Q, nb, JX, JXY, jn1,
+                              jn2, jn3, jscale);
+        }
+      } else if (in) {
         dep_vp3<ORDER, RAW>(sJ, JN, wx, wy, wz, x, y, z, x1, y1, z1, q, nb0, JX, JXY, jn1, jn2,
                             jn3, jscale);
+      }
       const unsigned long long mc = __ballot(cross);
       const int add = __popcll(mc);
       // twice at most: what a first call queues again crosses nothing

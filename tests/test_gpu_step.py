@@ -233,3 +233,25 @@ def test_dropin_current_in_any_particle_order(dims, order, n):
         out.append([j] + [a[back] for a in r[:3]])
     for a, c in zip(*out):
         assert np.array_equal(a.view(np.uint32), c.view(np.uint32))
+
+
+@pytest.mark.parametrize("n", [1, 4, 5, 64, 65, 700])
+@pytest.mark.parametrize("cells", [1, 3, 40])
+def test_cubic_deposit_lanes(n, cells):
+    """The cubic 3D deposit permutes its lanes by their base node: few particles, full waves
+    and remainders, all of a kind or of many kinds, against the generic kernel (bit for
+    bit)."""
+    print(f"case n={n} cells={cells}", flush=True)
+    rng = np.random.default_rng(n + cells)
+    nx = (24, 16, 12)
+    at = np.stack([rng.integers(1, m + 1, cells) for m in nx], 1).astype(np.int32)
+    ix = at[rng.integers(0, cells, n)]
+    x = (rng.random((n, 3), np.float32) - np.float32(0.5)).astype(np.float32)
+    u = (rng.standard_normal((n, 3)) * 0.3).astype(np.float32)
+    out = []
+    for kernel in (0, 1):
+        with oa.Simulation(3, nx, (0.1,) * 3, 0.055, 3, kernel=kernel) as sim:
+            sim.set_particles(sim.add_species(-1.0), ix, x, u, np.full(n, -0.01, np.float32))
+            sim.run(5)
+            out.append((sim.get_fields(), sim.get_particles(0), (), sim.history()))
+    _same(*out)
