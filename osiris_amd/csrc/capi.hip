@@ -453,9 +453,37 @@ void make_field_desc(const osr_sim* s, FieldDesc& f) {
   }
 }
 
+// The field work on the tile fill's launch and its workgroups (field_beside_fill): what comes
+// first in the field advance and needs only the fields and the current, while the fill moves
+// particles.  On small grids both are chains of latencies that leave most of the chip idle, so
+// the shorter one and the gap between two launches are saved.  ms per pass, launches of their
+// own / beside the fill: 64x64 job of 100 steps 3.37 / 2.77, 128x128 4.91 / 4.30, 515x267 3.57
+// / 3.30, 512x512 11.46 / 11.08, 52x44x36 2.71 / 2.50, 1024x256 with Lindman walls 9.88 / 9.35,
+// 512x96 with VPML walls 3.57 / 3.22, 96^3 29.3 / 28.9; 192^3 the same (302).  Left out:
+// yee2d_step<64, 16>, whose 108 registers would leave the fill too few waves (with the 32x8
+// variant in its place 1024x1024 takes the same 128 ms), 3D VPML walls for the same reason,
+// and vpml_diffuse, which comes between the half step and the walls.
+int ride_kind(const osr_sim* s) {
+  if (s->plain || s->sp.empty()) return kRideNone;
+  if (s->g.pp) return s->yv == 0 ? kRideStep2d : kRideNone;
+  if (s->desc.vpml_diffuse[0] || s->desc.vpml_diffuse[1]) return kRideNone;
+  if (s->vp_n) return s->dims == 2 ? kRideVpml2d : kRideNone;
+  return kRideHalfB;
+}
+int ride_items(const osr_sim* s) {
+  const int k = ride_kind(s);
+  return k == kRideStep2d ? kRedCols + s->nblk_e : (k != kRideNone ? s->nwork_e : 0);
+}
+
 int upload_descs(osr_sim* s) {
   std::vector<SpecDesc> v(kMaxSpecies);
   make_spec_descs(s, v.data());
+  if (ride_kind(s) != kRideNone)
+    for (SpecDesc& d : v) {
+      d.fd = s->d_fd.p;
+      d.fd_first = (int)s->sp.size() * s->ntiles;
+      d.fd_kind = ride_kind(s);
+    }
   TRY(copy_on(s->stream, s->d_spec.p, v.data(), sizeof(SpecDesc) * kMaxSpecies, hipMemcpyHostToDevice));
   make_field_desc(s, s->fd);
   TRY(copy_on(s->stream, s->d_fd.p, &s->fd, sizeof(FieldDesc), hipMemcpyHostToDevice));
@@ -1013,8 +1041,9 @@ int launch_reorder(osr_sim* s) {
   return OSR_OK;
 }
 
-int launch_fill(osr_sim* s) {
-  const int nw = (int)s->sp.size() * s->ntiles;
+// ride: with the field work that runs beside it, which launch_yee then leaves out
+int launch_fill(osr_sim* s, bool ride = false) {
+  const int nw = (int)s->sp.size() * s->ntiles + (ride ? ride_items(s) : 0);
   const FillKernel k = pick_fill();
   hipLaunchKernelGGL(k.f, dim3(nw), dim3(k.nt), 0, s->stream, s->d_spec.as<SpecDesc>(),
                      s->d_work.as<int2>());
@@ -1033,7 +1062,8 @@ int launch_wall_restore(osr_sim* s) {
 
 // next_laser: the next step's laser values join the last half step (its own launch_laser is
 // left out; only where that step's kernels follow in the stream).
-int launch_yee(osr_sim* s, bool next_laser = false) {
+int launch_yee(osr_sim* s, bool next_laser = false, bool rode = false) {
+  rode = rode && ride_kind(s) != kRideNone;
   const FieldDesc* fd = s->d_fd.as<FieldDesc>();
   const int2* w = s->d_ywork.as<int2>();
   const int2* we = s->d_ework.as<int2>();
@@ -1054,7 +1084,9 @@ int launch_yee(osr_sim* s, bool next_laser = false) {
                     : (vp ? (fk)yee_dedt<2, 2> : (fk)yee_dedt<2, 1>);
     const fk b2 = d3 ? (next_laser ? (fk)yee_dbdt<3, false, false, true> : (fk)yee_dbdt<3, false>)
                      : (next_laser ? (fk)yee_dbdt<2, false, false, true> : (fk)yee_dbdt<2, false>);
-    hipLaunchKernelGGL(b1, dim3(diffuse ? s->nblk_e : s->nwork_e), dim3(256), 0, s->stream, fd, we);
+    if (!rode)
+      hipLaunchKernelGGL(b1, dim3(diffuse ? s->nblk_e : s->nwork_e), dim3(256), 0, s->stream, fd,
+                         we);
     if (diffuse) {
       hipLaunchKernelGGL(vpml_diffuse, dim3(nwv), dim3(256), 0, s->stream, fd);
       hipLaunchKernelGGL(vpml_update_e, dim3(nwv), dim3(256), 0, s->stream, fd);
@@ -1072,14 +1104,17 @@ int launch_yee(osr_sim* s, bool next_laser = false) {
     return OSR_OK;
   }
   if (s->g.pp) {
-    hipLaunchKernelGGL(pick_yee2d(s->yv),
-                       dim3((unsigned)(kRedCols + s->nblk_e)), dim3(256), 0, s->stream, fd, wd, 0);
+    if (!rode)
+      hipLaunchKernelGGL(pick_yee2d(s->yv), dim3((unsigned)(kRedCols + s->nblk_e)), dim3(256), 0,
+                         s->stream, fd, wd, 0);
   } else if (s->dims == 2) {
-    hipLaunchKernelGGL((yee_dbdt<2, true>), dim3(s->nblk_e), dim3(256), 0, s->stream, fd, we);
+    if (!rode)
+      hipLaunchKernelGGL((yee_dbdt<2, true>), dim3(s->nblk_e), dim3(256), 0, s->stream, fd, we);
     hipLaunchKernelGGL((yee_dedt<2>), dim3(nd), dim3(256), 0, s->stream, fd, wd);
     hipLaunchKernelGGL((yee_dbdt<2, false>), dim3(s->nblk), dim3(256), 0, s->stream, fd, w);
   } else {
-    hipLaunchKernelGGL((yee_dbdt<3, true>), dim3(s->nblk_e), dim3(256), 0, s->stream, fd, we);
+    if (!rode)
+      hipLaunchKernelGGL((yee_dbdt<3, true>), dim3(s->nblk_e), dim3(256), 0, s->stream, fd, we);
     hipLaunchKernelGGL((yee_dedt<3>), dim3(nd), dim3(256), 0, s->stream, fd, wd);
     hipLaunchKernelGGL((yee_dbdt<3, false>), dim3(s->nblk), dim3(256), 0, s->stream, fd, w);
   }
@@ -1199,10 +1234,10 @@ int enqueue_step(osr_sim* s, bool laser = true, bool next = false) {
     return OSR_OK;
   }
   TRY(launch_pushes(s));
-  if (!s->sp.empty()) TRY(launch_fill(s));
-  if (!s->sp.empty()) TRY(launch_reorder(s));
   TRY(launch_smooth(s));
-  TRY(launch_yee(s, next_laser));
+  if (!s->sp.empty()) TRY(launch_fill(s, true));
+  if (!s->sp.empty()) TRY(launch_reorder(s));
+  TRY(launch_yee(s, next_laser, true));
   TRY(launch_finalize(s));
   return OSR_OK;
 }
@@ -1500,16 +1535,18 @@ int osr_sim_add_species(osr_sim* s, float rqm, int pusher, int* sid) {
   std::vector<int> cnt(s->ntiles, 0);
   TRY(alloc_species(s, *p, cnt));
   s->sp.push_back(std::move(p));
-  // the work list covers (species, tile) pairs, each species' tiles in XCD order
+  // the work list covers (species, tile) pairs, each species' tiles in XCD order, then an entry
+  // (of the first pair; only the place in the list counts) for each workgroup of field work
   const int ns = (int)s->sp.size();
-  TRY(s->d_work.alloc(sizeof(int2) * (size_t)ns * s->ntiles));
-  std::vector<int2> w((size_t)ns * s->ntiles);
+  const size_t nw = (size_t)ns * s->ntiles, nall = nw + ride_items(s);
+  TRY(s->d_work.alloc(sizeof(int2) * nall));
+  std::vector<int2> w(nall, make_int2(0, 0));
   for (int i = 0; i < ns; i++)
     for (int t = 0; t < s->ntiles; t++) w[(size_t)i * s->ntiles + t] = make_int2(i, xcd_tile(s->dims, t, s->ntiles));
   TRY(copy_on(s->stream, s->d_work.p, w.data(), sizeof(int2) * w.size(), hipMemcpyHostToDevice));
   // the push's list names every item once per workgroup of the tile
   std::vector<int2> pw;
-  for (const int2& it : w) pw.insert(pw.end(), s->split, it);
+  for (size_t i = 0; i < nw; i++) pw.insert(pw.end(), s->split, w[i]);
   TRY(s->d_pwork.alloc(sizeof(int2) * pw.size()));
   TRY(copy_on(s->stream, s->d_pwork.p, pw.data(), sizeof(int2) * pw.size(), hipMemcpyHostToDevice));
   // history rows gain a column: restart the history buffer

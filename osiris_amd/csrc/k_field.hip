@@ -139,17 +139,14 @@ OSR_DEV void reduce_column(const FieldDesc& fd, int col);
 //  * LASER (last half step): adds the next step's laser values, if that step will run; the
 //    launch that follows it in the stream must be that step's.
 template <int DIMS, bool ENERGY, bool VPML = false, bool LASER = false>
-__global__ __launch_bounds__(256) void yee_dbdt(const FieldDesc* __restrict__ fds,
-                                                const int2* __restrict__ work) {
+OSR_DEV void yee_dbdt_item(const FieldDesc& fd, int item) {
   __shared__ double s_red[4][6];
   constexpr int NB = ENERGY ? kEneBlk : 1;
-  const int2 wk = work[blockIdx.x];
-  const FieldDesc& fd = fds[wk.x];
   const GridDesc& g = fd.g;
-  if (ENERGY && wk.y < 0) {
+  if (ENERGY && item < 0) {
     // a block of rows of the lower Lindman wall: its B update after the first half step
     // (wall_b_row<1>) reads E and its own buffer only, neither of which this kernel writes
-    const long long t = (long long)(-1 - wk.y) * 256 + threadIdx.x;
+    const long long t = (long long)(-1 - item) * 256 + threadIdx.x;
     if (VPML)
       vpml_cells<0, DIMS>(fd, t);
     else
@@ -182,7 +179,7 @@ __global__ __launch_bounds__(256) void yee_dbdt(const FieldDesc* __restrict__ fd
   float e3j[NB], e3i[NB], e2i[NB], e1j[NB], e2k[NB], e1k[NB];
 #pragma unroll
   for (int qb = 0; qb < NB; qb++) {
-    idx[qb] = ((long long)wk.y * NB + qb) * 256 + threadIdx.x;
+    idx[qb] = ((long long)item * NB + qb) * 256 + threadIdx.x;
     ii[qb] = jj[qb] = kk[qb] = 0;
     e1[qb] = e2[qb] = e3[qb] = b1[qb] = b2[qb] = b3[qb] = 0.f;
     e3j[qb] = e3i[qb] = e2i[qb] = e1j[qb] = e2k[qb] = e1k[qb] = 0.f;
@@ -238,22 +235,32 @@ __global__ __launch_bounds__(256) void yee_dbdt(const FieldDesc* __restrict__ fd
     }
     const long long row = jj[qb] + (long long)ny * kk[qb];
     if (LASER && las) laser_add(fd, las_row, i, row, n2, n3);
-    const bool wall = VPML && (i == nx - 1 || i == nxi + 1);  // x = 0, nx+2
-    if (wall) {
-      float v[3];
-      vpml_to_box<0, DIMS>(fd, i == nxi + 1, row, v);
-      n1 = v[0];
-      n2 = v[1];
-      n3 = v[2];
-    }
-    if (live || wall) {
+    if (live) {
       const long long id = idx[qb];
       B1[id] = n1;
       B2[id] = n2;
       B3[id] = n3;
     }
-    if (VPML && (i == 0 || i == nxi))
-      vpml_from_box<0, DIMS>(fd, i == nxi, row, jj[qb], kk[qb], n1, n2, n3);
+  }
+  // the cells at the walls, one copy of the code for the NB cells of a thread (registers)
+  if (VPML) {
+#pragma unroll 1
+    for (int qb = 0; qb < NB; qb++) {
+      const long long id = ((long long)item * NB + qb) * 256 + threadIdx.x;
+      if (id >= nc) break;
+      int i, j, k;
+      cell_xyz(g, id, i, j, k);
+      const long long row = j + (long long)ny * k;
+      if (i == 0 || i == nxi) {  // x = 1, nx+1
+        vpml_from_box<0, DIMS>(fd, i == nxi, row, j, k, B1[id], B2[id], B3[id]);
+      } else if (i == nx - 1 || i == nxi + 1) {  // x = 0, nx+2
+        float v[3];
+        vpml_to_box<0, DIMS>(fd, i == nxi + 1, row, v);
+        B1[id] = v[0];
+        B2[id] = v[1];
+        B3[id] = v[2];
+      }
+    }
   }
   if (ENERGY) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -265,10 +272,17 @@ __global__ __launch_bounds__(256) void yee_dbdt(const FieldDesc* __restrict__ fd
     __syncthreads();
     if (threadIdx.x < 6) {
       const int c = threadIdx.x;
-      fd.fe_part[(long long)c * fd.nblk + wk.y] =
+      fd.fe_part[(long long)c * fd.nblk + item] =
           ((s_red[0][c] + s_red[1][c]) + s_red[2][c]) + s_red[3][c];
     }
   }
+}
+
+template <int DIMS, bool ENERGY, bool VPML = false, bool LASER = false>
+__global__ __launch_bounds__(256) void yee_dbdt(const FieldDesc* __restrict__ fds,
+                                                const int2* __restrict__ work) {
+  const int2 wk = work[blockIdx.x];
+  yee_dbdt_item<DIMS, ENERGY, VPML, LASER>(fds[wk.x], wk.y);
 }
 
 // WALL: 1 Lindman, the walls' E update by the threads of x = 1 and nx+1 (it writes x = 0,
@@ -432,26 +446,24 @@ struct YeeTile {
   }
 };
 
+// LDS floats of the staged E and half-step B
 template <int TX, int TY>
-__global__ __launch_bounds__(256) void yee2d_step(const FieldDesc* __restrict__ fds,
-                                                  const int2* __restrict__ work, int) {
+constexpr int kYeeLds = 6 * YeeTile<TX, TY>::EN;
+
+template <int TX, int TY>
+OSR_DEV void yee2d_tile(const FieldDesc& fd, int item, float* lds) {
   using T = YeeTile<TX, TY>;
   constexpr int EX = T::EX, EN = T::EN, Q = T::Q;
-  __shared__ float sE[3][EN], sB[3][EN];
-  const int2 wk = work[blockIdx.x];
-  const FieldDesc& fd = fds[wk.x];
+  float(*const sE)[EN] = (float(*)[EN])lds;
+  float(*const sB)[EN] = (float(*)[EN])(lds + 3 * EN);
   const GridDesc& g = fd.g;
-  if (wk.y < 0) {
-    reduce_column(fd, -1 - wk.y);
-    return;
-  }
   const int halt = g.ctrl->halt;
   const unsigned par = g.ctrl->par;
   if (halt >= 2) return;
   const int nx = g.nx, ny = g.ny, tid = threadIdx.x;
   const long long nc = g.ncell;
   const long long in = (long long)par * 3 * nc, out = (long long)(par ^ 1u) * 3 * nc;
-  const T tile(wk.y, nx);
+  const T tile(item, nx);
   const float* __restrict__ Ei = g.E + in;
   const float* __restrict__ Bi = g.B + in;
   // every load of the thread is issued before its first use (cells of the halo whose B or J
@@ -548,7 +560,39 @@ __global__ __launch_bounds__(256) void yee2d_step(const FieldDesc* __restrict__ 
       }
     }
   }
-  tile_energy(acc, fd.fe_part + (long long)(par ^ 1u) * 6 * fd.nblk, fd.nblk, wk.y);
+  tile_energy(acc, fd.fe_part + (long long)(par ^ 1u) * 6 * fd.nblk, fd.nblk, item);
+}
+
+// work items (simulation, tile) or (simulation, -1 - history column)
+template <int TX, int TY>
+__global__ __launch_bounds__(256) void yee2d_step(const FieldDesc* __restrict__ fds,
+                                                  const int2* __restrict__ work, int) {
+  __shared__ float lds[kYeeLds<TX, TY>];
+  const int2 wk = work[blockIdx.x];
+  if (wk.y < 0)
+    reduce_column(fds[wk.x], -1 - wk.y);
+  else
+    yee2d_tile<TX, TY>(fds[wk.x], wk.y, lds);
+}
+
+// A workgroup's share of the field work that needs nothing from the tile fill and rides on its
+// launch (SpecDesc::fd): the 2D periodic step with the history columns, or the first B half
+// step with the field energy and the walls.  item counts from 0.
+OSR_DEV void field_beside_fill(const FieldDesc& fd, int kind, int item, float* lds) {
+  if (kind == kRideStep2d) {
+    if (item < kRedCols)
+      reduce_column(fd, item);
+    else
+      yee2d_tile<32, 8>(fd, item - kRedCols, lds);
+  } else {
+    const int it = item < fd.nblk ? item : fd.nblk - 1 - item;
+    if (kind == kRideVpml2d)
+      yee_dbdt_item<2, true, true>(fd, it);
+    else if (fd.g.dims == 2)
+      yee_dbdt_item<2, true>(fd, it);
+    else
+      yee_dbdt_item<3, true>(fd, it);
+  }
 }
 
 // The energy partials of the current copy, as yee2d_step leaves them (same cells per thread,

@@ -616,6 +616,12 @@ __global__ __launch_bounds__(NT) void tile_fill(const SpecDesc* __restrict__ des
   const int2 wk = work[blockIdx.x];
   const SpecDesc& d = descs[wk.x];
   const GridDesc& g = d.g;
+  if (d.fd && (int)blockIdx.x >= d.fd_first) {  // a block of field work, in the list's arrays
+    static_assert(sizeof(s_inc) >= sizeof(float) * kYeeLds<32, 8>, "staged fields");
+    field_beside_fill(*(const FieldDesc*)d.fd, d.fd_kind, (int)blockIdx.x - d.fd_first,
+                      (float*)s_inc);
+    return;
+  }
   const int tile = wk.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int NW = d.waves, wsh = 31 - __clz(NW);  // a power of two
   const int dims = g.dims;

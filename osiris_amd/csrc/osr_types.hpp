@@ -149,7 +149,16 @@ struct SpecDesc {
   int jraw;        // no node sum of a tile's current can leave +-2^50 (fix_bits, RAW)
   int split;       // workgroups per tile in the push (1 in 3D and with the generic kernel)
   int waves;       // waves per tile in the push: those of its workgroups times split
+  // field work on the fill's launch (single simulations): its blocks from fd_first on belong to
+  // the field descriptor fd (field_beside_fill); null: none
+  const void* fd;
+  int fd_first;
+  int fd_kind;     // kRide...
 };
+
+// field work beside the tile fill: none; the whole 2D periodic step; the first B half step;
+// that with 2D VPML walls
+enum { kRideNone = 0, kRideStep2d = 1, kRideHalfB = 2, kRideVpml2d = 3 };
 
 // Cell packing.  2D: ix | iy<<16.  3D: ix | iy<<11 | iz<<22.
 __host__ __device__ inline uint32_t pack2(int ix, int iy) {

@@ -255,3 +255,31 @@ def test_cubic_deposit_lanes(n, cells):
             sim.run(5)
             out.append((sim.get_fields(), sim.get_particles(0), (), sim.history()))
     _same(*out)
+
+
+@pytest.mark.parametrize("dims,nx,kw,smooth", [
+    (2, (64, 48), {}, 0), (2, (64, 48), {}, 3), (2, (150, 90), dict(reorder=2), 0), (2, (1024, 512), {}, 0),
+    (3, (24, 20, 12), {}, 0), (3, (24, 20, 12), dict(reorder=3), 1), (2, (64, 48), dict(xbnd="lindman"), 0),
+    (3, (24, 20, 12), dict(xbnd="lindman"), 0), (2, (64, 48), dict(xbnd="vpml"), 0),
+    (2, (64, 48), dict(xbnd="vpml", vpml_diffuse=(True, False)), 0), (3, (24, 20, 12), dict(xbnd="vpml"), 0)])
+def test_field_work_beside_the_fill(dims, nx, kw, smooth):
+    """A run, whose tile fill carries the first part of the field advance, against steps with
+    every kernel in a launch of its own (the timed ones), bit for bit."""
+    print(f"case nx={nx} {kw} smooth={smooth}", flush=True)
+    rng = np.random.default_rng(29)
+    n = 4 * int(np.prod(nx))
+    out = []
+    ix = np.stack([rng.integers(1, m + 1, n) for m in nx], 1).astype(np.int32)
+    x = (rng.random((n, dims), np.float32) - np.float32(0.5)).astype(np.float32)
+    u = (rng.standard_normal((n, 3)) * 0.2).astype(np.float32)
+    e, b = (rng.standard_normal(tuple(reversed(nx)) + (3,)).astype(np.float32) * np.float32(0.1) for _ in range(2))
+    for timed in (False, True):
+        with oa.Simulation(dims, nx, (0.1,) * dims, 0.05, 2, **kw) as sim:
+            for rqm in (-1.0, 100.0):
+                sim.set_particles(sim.add_species(rqm), ix, x, u, np.full(n, 0.02 * np.sign(rqm), np.float32))
+            sim.set_fields(e, b)
+            if smooth:
+                sim.set_smooth(*oa.smooth_setup(dims, ["compensated"] * dims, (smooth,) * dims, (0.1,) * dims))
+            sim.time_kernels(9) if timed else sim.run(9)
+            out.append((sim.get_fields(), sim.get_particles(0), sim.get_particles(1), sim.history()))
+    _same(*out)
