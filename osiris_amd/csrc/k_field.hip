@@ -6,8 +6,8 @@
 // refresh (update_periodic_vdf, vdf/os-vdf-comm.f90:142-330) on every interior cell.
 // The arithmetic keeps the reference's operation order in FP32 (no contraction).
 //
-// The three sub-steps are memory-bound stencils over planar component arrays: one thread
-// per cell, consecutive threads on consecutive x (coalesced).  The E step also converts
+// Periodic 2D grids take the whole step in one launch (yee2d_step).  Otherwise the three
+// sub-steps are memory-bound stencils over planar component arrays: one thread per cell, consecutive threads on consecutive x (coalesced).  The E step also converts
 // the fixed-point current to float and clears it for the next deposit, and the first B
 // step accumulates the field energy of E^n, B^n (the fields the particles were pushed
 // with) into per-block FP64 partial sums.
