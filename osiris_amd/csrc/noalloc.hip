@@ -86,11 +86,26 @@ __global__ __launch_bounds__(256) void na_check(NoallocHdr* h, NaCheckArgs a) {
 }
 
 // sum and maximum of |q| in one workgroup: 256 strided partial sums, then the partials in
-// thread order (deterministic)
+// thread order (deterministic).  Bound by the latency of its loads, so each thread has 16 in
+// flight; the order of the additions is that of one at a time.  393216 charges: 619 us with one
+// load at a time, 100 us so.
 __global__ __launch_bounds__(256) void na_charge(NoallocHdr* h, const float* q, int np) {
   __shared__ double s_sum[256], s_max[256];
   double s = 0.0, m = 0.0;
-  for (int i = threadIdx.x; i < np; i += 256) {
+  constexpr int U = 16;
+  int i = threadIdx.x;
+  for (; i + (U - 1) * 256 < np; i += U * 256) {
+    float f[U];
+#pragma unroll
+    for (int k = 0; k < U; k++) f[k] = q[i + k * 256];
+#pragma unroll
+    for (int k = 0; k < U; k++) {
+      const double v = fabs((double)f[k]);
+      s += v;
+      m = fmax(m, v);
+    }
+  }
+  for (; i < np; i += 256) {
     const double v = fabs((double)q[i]);
     s += v;
     m = fmax(m, v);
@@ -109,12 +124,30 @@ __global__ __launch_bounds__(256) void na_charge(NoallocHdr* h, const float* q, 
   }
 }
 
-// energy partials summed in block order, as the host entry point sums them
-__global__ void na_energy(NoallocHdr* h, const double* ep, int nblk) {
-  if (blockIdx.x != 0 || threadIdx.x != 0) return;
-  double e = 0.0;
-  for (int b = 0; b < nblk; b++) e += ep[b];
-  h->ene = e;
+// energy partials summed in block order, as the host entry point sums them: a wave loads 64 at
+// a time, the next ones ahead, and adds them one after the other (1536 partials: 82 us by one
+// thread, 16 us so)
+__global__ __launch_bounds__(64) void na_energy(NoallocHdr* h, const double* ep, int nblk) {
+  const int lane = threadIdx.x;
+  double e = 0.0, next = lane < nblk ? ep[lane] : 0.0;
+  for (int b = 0; b < nblk; b += 64) {
+    const double v = next;
+    if (b + 64 + lane < nblk) next = ep[b + 64 + lane];
+    const int n = nblk - b < 64 ? nblk - b : 64;
+    const long long w = __double_as_longlong(v);
+    const int lo = (int)w, hi = (int)(w >> 32);
+    auto part = [&](int k) {
+      const unsigned l = (unsigned)__builtin_amdgcn_readlane(lo, k);
+      return __longlong_as_double((long long)__builtin_amdgcn_readlane(hi, k) << 32 | l);
+    };
+    if (n == 64) {
+#pragma unroll
+      for (int k = 0; k < 64; k++) e += part(k);
+    } else {
+      for (int k = 0; k < n; k++) e += part(k);
+    }
+  }
+  if (lane == 0) h->ene = e;
 }
 
 }  // namespace
@@ -222,7 +255,7 @@ int osr_advance_deposit_noalloc(int dims, int order, int pusher, int* ix, float*
 #undef OSR_D
     hipLaunchKernelGGL(f, dim3(nblk), dim3(256), 0, 0, a);
     HIPC(hipGetLastError());
-    hipLaunchKernelGGL(na_energy, dim3(1), dim3(1), 0, 0, hdr, (const double*)epart, nblk);
+    hipLaunchKernelGGL(na_energy, dim3(1), dim3(64), 0, 0, hdr, (const double*)epart, nblk);
     HIPC(hipGetLastError());
   }
   hipLaunchKernelGGL(dropin_jadd, dim3((unsigned)((nj + 255) / 256)), dim3(256), 0, 0, j,

@@ -283,3 +283,28 @@ def test_field_work_beside_the_fill(dims, nx, kw, smooth):
             sim.time_kernels(9) if timed else sim.run(9)
             out.append((sim.get_fields(), sim.get_particles(0), sim.get_particles(1), sim.history()))
     _same(*out)
+
+
+@pytest.mark.parametrize("n", [1, 4095, 4096, 4097, 16384, 16385, 33000])
+def test_noalloc_sums(n):
+    """The allocation-free drop-in sums |q| (which sets the current's scale) and the energy
+    partials in the order of the host entry point; sizes at the remainders of its 16 x 256
+    loads and 64 partials at a time.  Equal charges, so the scales agree and J too."""
+    from test_zz_no_alloc import _noalloc
+
+    print(f"case n={n}", flush=True)
+    rng = np.random.default_rng(n)
+    nx, lo, hi = (40, 30), 3, 4
+    ix = np.stack([rng.integers(1, m + 1, n) for m in nx], 1).astype(np.int32)
+    x = (rng.random((n, 2), np.float32) - np.float32(0.5)).astype(np.float32)
+    u = rng.standard_normal((n, 3)).astype(np.float32)
+    q = np.full(n, -0.25, np.float32)
+    shape = tuple(m + lo + hi for m in reversed(nx)) + (3,)
+    e, b = (rng.standard_normal(shape).astype(np.float32) for _ in range(2))
+    j0 = np.zeros(shape, np.float32)
+    jr = j0.copy()
+    want = oa.advance_deposit(2, 2, ix.copy(), x.copy(), u.copy(), q, -1.0, e, b, lo, jr, lo, (0.1, 0.1), 0.05)
+    got = _noalloc(2, 2, oa.OSR_BORIS, ix, x, u, q, e, b, lo, j0, (0.1, 0.1), 0.05)
+    for a, c in zip(want[:3], got[:3]):
+        assert np.array_equal(a.view(np.uint32), c.view(np.uint32))
+    assert np.array_equal(jr.view(np.uint32), got[3].view(np.uint32)) and want[3] == got[4]
