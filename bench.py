@@ -473,7 +473,7 @@ def main():
                     help="c4: field walls of the open x boundaries")
     ap.add_argument("--reorder", type=int, default=0,
                     help="in-tile particle order restored every N steps (0 = library default: "
-                         "4 for cubic splines in 3D, else off; negative = off)")
+                         "in 3D 4 for cubic and 16 for quadratic splines, else off; negative = off)")
     ap.add_argument("--push-waves", type=int, default=0,
                     help="waves per push workgroup without autotuning (0 = the tile's default)")
     ap.add_argument("--autotune", action="store_true", default=True)

@@ -153,8 +153,8 @@ typedef struct {
   int xbnd;       /* x walls: OSR_BND_PERIODIC (0), OSR_BND_LINDMAN (1, also named
                      OSR_BND_OPEN) or OSR_BND_VPML (2) */
   int reorder;    /* fused path: restore the (rank in cell, cell) particle order inside the
-                     tiles every this many steps; 0 = default (4 for cubic splines in
-                     3D, else off), negative = off.  Changes no result beyond FP64 round-off of the
+                     tiles every this many steps; 0 = default (in 3D 4 for cubic
+                     and 16 for quadratic splines, else off), negative = off.  Changes no result beyond FP64 round-off of the
                      energy sums (the counterpart of the reference's periodic sort,
                      sort_species, spec/os-species.f03:269-332) */
   int vpml_size;  /* OSR_BND_VPML: wall thickness in cells, 4..64; 0 = 8 (vpml_bnd_size,

@@ -1413,13 +1413,15 @@ int osr_sim_create(const osr_sim_desc* desc, osr_sim** out) {
   if (s->lds_push > 160 * 1024) return fail(OSR_ERR_ARG, "tile too large for LDS");
   // Default re-order period.  The cubic 3D push waits for its LDS passes, which the order of a
   // tile's particles decides: a 192^3 step takes 7.15 ms with a period of 3, 7.07 to 7.09 with
-  // 4 to 8, 7.19 with 16 and 7.58 without.  Linear and quadratic lines are shorter and their push is not
-  // bound by them: a 96^3 quadratic step of drifting beams takes 703 us with a period of 4, 682
-  // with 8 and 673 with 16, 32 and none, a 52x44x36 linear one 70.6, 66.7, 64.8, 64.1 and 61.6
-  // without (a launch that finds nothing to do costs 2.5 us).
-  s->reorder = desc->reorder > 0
-                   ? desc->reorder
-                   : (desc->reorder == 0 && dims == 3 && s->order == 3 ? 4 : 0);
+  // 4 to 8, 7.19 with 16 and 7.58 without.  Quadratic lines are shorter, and a longer period
+  // serves cold plasmas, which keep their order, as well as hot ones, which lose it at once: us
+  // per step with 4 / 8 / 16 / 32 / none, 96^3 of 8 per cell, u_th 0.005 399 / 374 / 366 / 369
+  // / 418, 0.02 434 / 416 / 413 / 424 / 457, 0.1 501 / 492 / 492 / 496 / 496; 160^3, 0.3 2681 /
+  // 2621 / 2597 / 2585 / 2565.  The linear push is not bound by the order: 160^3, 0.01 1195 /
+  // 1074 / 1005 / 976 / 946, 52x44x36 70.6 / 66.7 / 64.8 / 64.1 / 61.6 (a launch that finds
+  // nothing to do costs 2.5 us).
+  const int period = dims == 3 ? (s->order == 3 ? 4 : (s->order == 2 ? 16 : 0)) : 0;
+  s->reorder = desc->reorder > 0 ? desc->reorder : (desc->reorder == 0 ? period : 0);
   s->push_waves = kWaves;
   if (desc->push_waves != 0 && desc->push_waves != 4 && desc->push_waves != 8)
     return fail(OSR_ERR_ARG, "push_waves must be 0, 4 or 8");
