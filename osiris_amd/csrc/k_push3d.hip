@@ -407,7 +407,12 @@ __global__ __launch_bounds__(64 * push3d_waves(ORDER), push3d_waves(ORDER) / 2) 
       const unsigned long long mc = __ballot(cross);
       const int add = __popcll(mc);
       // twice at most: what a first call queues again crosses nothing
-      while (qlen + add > QC) deposit_queue(lane < qlen, Q0[lane], Q1[lane]);
+      while (qlen + add > QC) {
+        wave_lds_sync();  // the entries of the other lanes
+        const f32x4 a = Q0[lane], b = Q1[lane];
+        wave_lds_sync();  // read before any is written again
+        deposit_queue(lane < qlen, a, b);
+      }
       if (cross) {
         const int s = qlen + __popcll(mc & below);
         Q0[s] = qa;

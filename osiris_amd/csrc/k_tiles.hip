@@ -327,6 +327,7 @@ __global__ __launch_bounds__(NT) void push_deposit_3d(const SpecDesc* __restrict
   int qhead = 0, qlen = 0;
   // deposit of the queued VPs in slots [head, head + cnt) (cnt <= 64, one per lane)
   auto deposit_queue = [&](int head, int cnt) {
+    wave_lds_sync();  // the entries of the other lanes
     if (lane < cnt) {
       const int sl = (head + lane) & (QC - 1);
       const float x0 = Q[sl], y0 = Q[QC + sl], z0 = Q[2 * QC + sl];
@@ -337,6 +338,7 @@ __global__ __launch_bounds__(NT) void push_deposit_3d(const SpecDesc* __restrict
       dep_vp3<ORDER>(sJ, JN, S0x, S0y, S0z, x0, y0, z0, Q[3 * QC + sl], Q[4 * QC + sl],
                      Q[5 * QC + sl], Q[6 * QC + sl], QN[sl], JX, JXY, jn1, jn2, jn3, jscale);
     }
+    wave_lds_sync();  // read before any is written again
   };
 
   double ene = 0.0;
@@ -909,9 +911,9 @@ __global__ __launch_bounds__(NT) void tile_reorder(const SpecDesc* __restrict__ 
       const int before = __popcll(same & below);
       const int after = __popcll(same & ~below) - 1;
       if (lc >= 0) s_key[p] = ((s_cnt[wave][lc] + before) << CB) | lc;
-      __builtin_amdgcn_wave_barrier();
+      wave_lds_sync();
       if (lc >= 0 && after == 0) s_cnt[wave][lc] += before + 1;
-      __builtin_amdgcn_wave_barrier();
+      wave_lds_sync();
     }
   }
   __syncthreads();

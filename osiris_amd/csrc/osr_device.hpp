@@ -13,6 +13,18 @@
 
 namespace osr {
 
+// What the lanes of a wave stored to LDS before it is what they all read after it, and what
+// they read before it was read before any of them stores after it.  The hardware keeps a
+// wave's LDS accesses in order by itself; without the fences the compiler may not: each lane
+// is a thread of its own to it, so that a value one lane read may stand for a second read of
+// the same place after another lane's store.  No instruction results (wavefront scope, LDS
+// only).  Every lane of the wave must call it.
+OSR_DEV void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 OSR_DEV float fma_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 
 // ------------------------------------------------------------------------------------
