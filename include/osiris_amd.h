@@ -251,6 +251,11 @@ int osr_sim_footprint(osr_sim *sim, int64_t *bytes);
  * tile[3] in cells, waves per workgroup, and *compiled_tile = 1 when the compile-time
  * tile variant runs, 0 for the generic kernel (or the plain path). */
 int osr_sim_launch_config(osr_sim *sim, int *tile, int *waves, int *compiled_tile);
+/* *raw = 1 when the push of species sid adds the current's fixed-point terms as the raw bits
+ * of their FP64 form, which its present charges and layout allow if no sum of a tile can leave
+ * +-2^50; 0 when it converts each term (and with the generic kernel).  The bits of every
+ * result are the same. */
+int osr_species_raw_sums(osr_sim *sim, int sid, int *raw);
 
 /* ---------------------------------------------------------------------------------
  * 4. Ensemble serving (no counterpart in the reference, which runs one simulation per

@@ -59,6 +59,7 @@ SIGNATURES = {
     "osr_sim_time_kernels": (I, [P, I, P]),
     "osr_sim_footprint": (I, [P, P]),
     "osr_sim_launch_config": (I, [P, P, P, P]),
+    "osr_species_raw_sums": (I, [P, I, P]),
     "osr_ens_create": (I, [P, P]),
     "osr_ens_destroy": (I, [P]),
     "osr_ens_submit": (I, [P, P, P]),

@@ -344,6 +344,15 @@ void update_jscale(osr_sim* s) {
   s->g.jinv = std::ldexp(1.0, -sh);
 }
 
+// A particle adds at most |q| to a node and component, over all its virtual particles: |q|/2
+// (its path is shorter than dt) times a weight sum of at most 2 along and across the component,
+// |q vz|/3 times at most 3 for the third; 1% and one unit per virtual particle cover the
+// roundings.  Whether the sums of a tile's particles then stay within +-2^50 (fix_bits, RAW).
+bool raw_sums(const osr_sim* s, const Species& p) {
+  const int maxcap = p.h_cap.empty() ? 0 : *std::max_element(p.h_cap.begin(), p.h_cap.end());
+  return (double)maxcap * (1.01 * p.qmax * s->g.jscale + 4.0) < std::ldexp(1.0, 50);
+}
+
 // device descriptors of the species of s (v[0 .. nspecies)) and of its fields
 void make_spec_descs(const osr_sim* s, SpecDesc* v) {
   for (size_t i = 0; i < s->sp.size(); i++) {
@@ -379,12 +388,7 @@ void make_spec_descs(const osr_sim* s, SpecDesc* v) {
     d.inc = p.inc.as<int>();
     d.epart = p.epart.as<double>();
     d.tem = (float)(0.5 * s->dt / (double)p.rqm);
-    // A particle adds at most |q| to a node and component, over all its virtual particles:
-    // |q|/2 (its path is shorter than dt) times a weight sum of at most 2 along and across
-    // the component, |q vz|/3 times at most 3 for the third; 1% and one unit per virtual
-    // particle cover the roundings.
-    const int maxcap = p.h_cap.empty() ? 0 : *std::max_element(p.h_cap.begin(), p.h_cap.end());
-    d.jraw = (double)maxcap * (1.01 * p.qmax * s->g.jscale + 4.0) < std::ldexp(1.0, 50);
+    d.jraw = raw_sums(s, p);
     d.waves = s->tile_waves();
     d.split = s->split;
   }
@@ -2071,6 +2075,15 @@ int osr_sim_launch_config(osr_sim* s, int* tile, int* waves, int* compiled_tile)
   if (!s->plain && s->desc.kernel != 1)
     *compiled_tile = (s->dims == 2 ? pick_push2d_t(s->order, 0, s->g.tx, s->g.ty, s->push_waves)
                                    : pick_push3d_t(s->order, 0, s->g.tx, s->g.ty, s->g.tz)) != nullptr;
+  return OSR_OK;
+}
+
+int osr_species_raw_sums(osr_sim* s, int sid, int* raw) {
+  TRY(check_sim(s));
+  if (sid < 0 || sid >= (int)s->sp.size() || !raw) return fail(OSR_ERR_ARG, "bad argument");
+  int tile[3], waves, compiled = 0;
+  TRY(osr_sim_launch_config(s, tile, &waves, &compiled));
+  *raw = compiled && raw_sums(s, *s->sp[sid]);
   return OSR_OK;
 }
 

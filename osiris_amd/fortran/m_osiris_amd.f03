@@ -118,7 +118,7 @@ module m_osiris_amd
             osr_species_count, osr_species_get, osr_species_generate, osr_fields_set, &
             osr_fields_get, osr_fields_fill, osr_sim_run, osr_sim_steps, osr_sim_history, &
             osr_sim_gauss, osr_sim_relayouts, osr_sim_time_kernels, osr_sim_footprint, &
-            osr_sim_launch_config
+            osr_sim_launch_config, osr_species_raw_sums
   public :: osr_smooth_setup, osr_smooth_vdf, osr_sim_set_smooth
   public :: osr_sim_write_hist, osr_sim_save_field
   public :: osr_sim_add_zpulse_wall, osr_sim_zpulse_column, osr_sim_init_fields, &
@@ -344,6 +344,13 @@ module m_osiris_amd
       type(c_ptr), value :: sim
       integer(c_int), intent(out) :: tile(3), waves, compiled_tile
       integer(c_int) :: osr_sim_launch_config
+    end function
+    function osr_species_raw_sums(sim, sid, raw) bind(c, name="osr_species_raw_sums")
+      import :: c_int, c_ptr
+      type(c_ptr), value :: sim
+      integer(c_int), value :: sid
+      integer(c_int), intent(out) :: raw
+      integer(c_int) :: osr_species_raw_sums
     end function
 
     ! ---- 5. current smoothing

@@ -359,6 +359,12 @@ class Simulation:
     def push_waves(self):
         return self.launch_config["push_waves"]
 
+    def raw_sums(self, sid):
+        """Whether the push of species sid adds the current's fixed-point terms as raw bits."""
+        raw = C.c_int()
+        check(lib().osr_species_raw_sums(self._h, int(sid), C.byref(raw)))
+        return bool(raw.value)
+
     @property
     def footprint(self):
         n = C.c_int64()
