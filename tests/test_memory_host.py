@@ -1,0 +1,86 @@
+"""The library's use of device memory on the CPU, over the mock runtime of tests/hostcheck with
+a device memory that fills up (capi_mock_mem.hip)."""
+import json
+import os
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+HC = os.path.join(ROOT, "tests", "hostcheck")
+HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+
+
+@pytest.fixture(scope="module")
+def mem_lib():
+    if not os.path.exists(HIPCC):
+        pytest.skip("hipcc not available")
+    out = os.path.join(HC, "_build", "libosiris_hostcheck_mem.so")
+    os.makedirs(os.path.dirname(out), exist_ok=True)
+    csrc = os.path.join(ROOT, "osiris_amd", "csrc")
+    srcs = [os.path.join(HC, f) for f in os.listdir(HC) if f.endswith((".h", ".hip"))] + [
+        os.path.join(csrc, f) for f in os.listdir(csrc)]
+    if not os.path.exists(out) or os.path.getmtime(out) < max(os.path.getmtime(s) for s in srcs):
+        # host code only: the device code, which the mock never runs, is named but not there
+        tmp = f"{out}.{os.getpid()}.tmp"
+        subprocess.run([HIPCC, "--offload-arch=gfx950", "--offload-host-only", "-O1", "-w", "-std=c++17",
+                        "-fPIC", "-I", os.path.join(ROOT, "include"), "-c", "-o", tmp + ".o",
+                        os.path.join(HC, "capi_mock_mem.hip")], check=True)
+        syms = subprocess.run(["nm", "-u", tmp + ".o"], check=True, capture_output=True, text=True).stdout
+        subprocess.run([HIPCC, "-shared", "-rdynamic", "-o", tmp, tmp + ".o"] + [
+            f"-Wl,--defsym={s}=0" for s in syms.split() if s.startswith("__hip_fatbin")], check=True)
+        os.remove(tmp + ".o")
+        os.replace(tmp, out)
+    return out
+
+
+PRELUDE = """
+import ctypes as C, json, sys
+sys.path.insert(0, {root!r})
+import numpy as np
+import osiris_amd._lib as L
+L.LIB_PATH = {lib!r}
+L.lib()
+raw = C.CDLL({lib!r})
+for f in ("mock_errors", "mock_order_errors", "mock_live", "mock_large_allocs"):
+    getattr(raw, f).restype = C.c_longlong
+raw.mock_leave_free.argtypes = [C.c_longlong]
+from osiris_amd.sim import Simulation
+out = {{}}
+"""
+
+
+def _run(lib, body):
+    """Result of `body` (which fills the dict `out`) in a process of its own."""
+    code = PRELUDE.format(root=ROOT, lib=lib) + body + """
+out["errors"] = raw.mock_errors() + raw.mock_order_errors()
+out["live"] = raw.mock_live()
+print(json.dumps(out))
+"""
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stderr[-3000:]
+    res = json.loads(r.stdout.strip().splitlines()[-1])
+    assert res.pop("errors") == 0 and res.pop("live") == 0, r.stderr[-3000:]
+    return res
+
+
+@pytest.mark.parametrize("dims,nx,ppc,species", [(2, (300, 200), (2, 2), 0), (2, (64, 64), (2, 2), 0),
+                                                 (3, (48, 48, 48), (2, 1, 1), 0), (2, (512, 512), (4, 4), 2)])
+def test_no_large_allocation_for_small_arrays(mem_lib, dims, nx, ppc, species):
+    """An allocation of 2 MiB or more takes some 290 us and a smaller one 5 us: arrays below
+    that size (the copies of the fields and the current, the particle arrays) are not put
+    together into larger allocations, and larger ones are one allocation each, or, the particle
+    arrays, one in all (512x512: once for the empty species, once for the particles)."""
+    res = _run(mem_lib, f"""
+with Simulation({dims}, {nx}, (0.1,) * {dims}, 0.05, 2) as s:
+    out["grid"] = raw.mock_large_allocs()
+    sid = s.add_species(-1.0)
+    s.generate(sid, {ppc})
+    out["species"] = raw.mock_large_allocs() - out["grid"]
+    s.run(3)
+""")
+    cells = 1
+    for m in nx:
+        cells *= m
+    assert res == {"grid": 2 * (12 * cells >= 2 << 20) + (24 * cells >= 2 << 20), "species": species}
