@@ -1634,6 +1634,29 @@ int osr_species_count(osr_sim* s, int sid, int64_t* np) {
   return OSR_OK;
 }
 
+// osr_species_get without device memory of its own: the arrays as they are, ordered by the host
+static int species_get_host(osr_sim* s, Species& p, int* ix, float* x, float* u, float* q) {
+  HostParts hp;
+  TRY(collect(s, p, false, hp));
+  std::vector<uint32_t> by_pid(hp.size());
+  for (size_t i = 0; i < by_pid.size(); i++) by_pid[i] = (uint32_t)i;
+  std::sort(by_pid.begin(), by_pid.end(), [&](uint32_t a, uint32_t b) { return hp.pid[a] < hp.pid[b]; });
+  const int D = s->dims;
+  for (size_t o = 0; o < by_pid.size(); o++) {
+    const size_t i = by_pid[o];
+    int c[3];
+    cell_coords(s, hp.cell[i], c);
+    const float xi[3] = {hp.x[i], hp.y[i], hp.z[i]}, ui[3] = {hp.ux[i], hp.uy[i], hp.uz[i]};
+    for (int d = 0; d < D; d++) {
+      if (ix) ix[D * o + d] = c[d] + 1;
+      if (x) x[D * o + d] = xi[d];
+    }
+    if (u) std::copy(ui, ui + 3, u + 3 * o);
+    if (q) q[o] = hp.q[i];
+  }
+  return OSR_OK;
+}
+
 int osr_species_get(osr_sim* s, int sid, int* ix, float* x, float* u, float* q) {
   TRY(check_sim(s));
   if (sid < 0 || sid >= (int)s->sp.size()) return fail(OSR_ERR_ARG, "bad species id");
@@ -1651,7 +1674,8 @@ int osr_species_get(osr_sim* s, int sid, int* ix, float* x, float* u, float* q) 
   if (n != p.npid) {
     const long long nw = (p.npid + 31) / 32;
     const unsigned ng = (unsigned)((nw + kPidWords - 1) / kPidWords);
-    TRY(map.alloc(sizeof(unsigned) * (2 * (size_t)nw + ng)));
+    if (map.alloc(sizeof(unsigned) * (2 * (size_t)nw + ng)) != OSR_OK)
+      return species_get_host(s, p, ix, x, u, q);
     unsigned* bits = map.as<unsigned>();
     HIPC(hipMemsetAsync(bits, 0, sizeof(unsigned) * (size_t)nw, s->stream));
     hipLaunchKernelGGL(pids_mark, dim3(nt), dim3(256), 0, s->stream, spec, sid, bits);
@@ -1665,7 +1689,10 @@ int osr_species_get(osr_sim* s, int sid, int* ix, float* x, float* u, float* q) 
   // in pieces of at most 2^22 particles (the device buffer stays below 170 MB)
   const int64_t piece = std::min<int64_t>(n, 1 << 22);
   DBuf out;
-  TRY(out.alloc(4 * (size_t)piece * (2 * D + 4)));
+  if (out.alloc(4 * (size_t)piece * (2 * D + 4)) != OSR_OK) {
+    HIPC(hipStreamSynchronize(s->stream));  // the kernels on the bitmap, which goes
+    return species_get_host(s, p, ix, x, u, q);
+  }
   a.ix = out.as<int>();
   a.x = (float*)(a.ix + D * piece);
   a.u = a.x + D * piece;
@@ -1745,6 +1772,29 @@ static int fields_changed(osr_sim* s) {
   return OSR_OK;
 }
 
+// osr_fields_get without device memory of its own: the planar arrays, rearranged by the host
+static int fields_get_host(osr_sim* s, float* e, float* b, const int* ld, const int* gcl) {
+  const int D = s->dims, ldk = D == 3 ? ld[2] : 1, gk = D == 3 ? gcl[2] : 0;
+  const size_t nc = (size_t)s->g.ncell, nx = s->g.nx, ny = s->g.ny;
+  auto wrap = [](int i, int n) { return (i % n + n) % n; };
+  std::vector<float> v(3 * nc);
+  for (int w = 0; w < 2; w++) {
+    float* f = w == 0 ? e : b;
+    if (!f) continue;
+    TRY(copy_on(s->stream, v.data(), w == 0 ? cur_E(s) : cur_B(s), 12 * nc, hipMemcpyDeviceToHost));
+    for (int k = 0; k < ldk; k++)
+      for (int j = 0; j < ld[1]; j++) {
+        const size_t row = nx * (wrap(j - gcl[1], s->g.ny) + ny * wrap(k - gk, s->g.nz));
+        int ii = wrap(-gcl[0], s->g.nx);
+        for (int i = 0; i < ld[0]; i++, f += 3) {
+          for (int m = 0; m < 3; m++) f[m] = v[m * nc + row + ii];
+          if (++ii == s->g.nx) ii = 0;
+        }
+      }
+  }
+  return OSR_OK;
+}
+
 static int fields_xfer(osr_sim* s, float* e, float* b, const int* ld, const int* gcl, bool set) {
   const int D = s->dims;
   // nxs: device extents (with open x walls the x ring includes the guard band);
@@ -1757,13 +1807,16 @@ static int fields_xfer(osr_sim* s, float* e, float* b, const int* ld, const int*
   if (!set) {
     // every array cell (guards included) gets its periodic image; with open x walls the x
     // guard cells come from the guard band of the ring.  In pieces of whole rows, at most
-    // about 64 MB each.
+    // about 64 MB each.  Small arrays are rearranged by the host, in less time than the device
+    // memory for it takes (us for E and B, host / device: 69x69 cells 75 / 100, 17^3 66 / 101,
+    // 305x205 289 / 130), and so are all when there is no device memory left.
     FieldsOut a{s->g.nx, s->g.ny, s->g.nz, s->g.ncell, ld[0], ld[1],
                 {gcl[0], gcl[1], D == 3 ? gcl[2] : 0}, 0, 0};
     const long long rows = (long long)ld[1] * (D == 3 ? ld[2] : 1);
     const long long piece = std::min(rows, std::max(1ll, (64ll << 20) / (12ll * ld[0])));
     DBuf out;
-    TRY(out.alloc(12 * (size_t)piece * ld[0]));
+    if (rows * ld[0] <= 12000 || out.alloc(12 * (size_t)piece * ld[0]) != OSR_OK)
+      return fields_get_host(s, e, b, ld, gcl);
     for (int w = 0; w < 2; w++) {
       float* h = w == 0 ? e : b;
       if (!h) continue;

@@ -84,3 +84,29 @@ with Simulation({dims}, {nx}, (0.1,) * {dims}, 0.05, 2) as s:
     for m in nx:
         cells *= m
     assert res == {"grid": 2 * (12 * cells >= 2 << 20) + (24 * cells >= 2 << 20), "species": species}
+
+
+@pytest.mark.parametrize("dims,nx", [(2, (150, 110)), (3, (40, 30, 20))])
+def test_read_back_without_device_memory(mem_lib, dims, nx):
+    """Fields and particles come back when the device has no memory left for laying them out."""
+    res = _run(mem_lib, f"""
+dims, nx = {dims}, {nx}
+rng = np.random.default_rng(4)
+n = 20000
+ix = np.stack([rng.integers(1, m + 1, n) for m in nx], 1).astype(np.int32)
+x = (rng.random((n, dims), np.float32) - np.float32(0.5)).astype(np.float32)
+u = rng.standard_normal((n, 3)).astype(np.float32)
+q = (-rng.random(n)).astype(np.float32)
+e, b = (rng.standard_normal(tuple(reversed(nx)) + (3,)).astype(np.float32) for _ in range(2))
+with Simulation(dims, nx, (0.1,) * dims, 0.05, 2) as s:
+    sid = s.add_species(-1.0)
+    s.set_particles(sid, ix, x, u, q)
+    s.set_fields(e, b)
+    raw.mock_leave_free(0)
+    out["particles"] = all(np.array_equal(a, c) for a, c in zip(s.get_particles(sid), (ix, x, u, q)))
+    lo, up = [3, 1, 2][:dims], [2, 4, 1][:dims]
+    pad = [(l, h) for l, h in zip(reversed(lo), reversed(up))] + [(0, 0)]
+    out["fields"] = all(np.array_equal(a, np.pad(c, pad, "wrap")) for a, c in zip(s.get_fields(lo, up), (e, b)))
+    raw.mock_leave_free(-1)
+""")
+    assert res == {"particles": True, "fields": True}
