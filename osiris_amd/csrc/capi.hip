@@ -136,23 +136,6 @@ struct DBuf {
   }
 };
 
-// An allocation below this size comes out of a pool of the runtime's (about 5 us with its
-// release), a larger one is mapped by itself (290 us; 12 to 24 when it takes the place of one
-// released just before): measured at 4 KB to 1 GB, 17 at a time.
-constexpr size_t kLargeAlloc = size_t(2) << 20;
-
-// An array and, if wanted, a second copy of it, in one allocation unless that alone makes it
-// a large one
-int alloc_copies(DBuf& a, DBuf& b, size_t bytes, bool two) {
-  if (two && bytes < kLargeAlloc && 2 * bytes >= kLargeAlloc) {
-    TRY(a.alloc(bytes));
-    return b.alloc(bytes);
-  }
-  TRY(a.alloc(two ? 2 * bytes : bytes));
-  if (two) b.view((char*)a.p + bytes, bytes);
-  return OSR_OK;
-}
-
 // Copy between host and device ordered on stream `st`: it runs after the work already
 // queued there (a download sees the kernels launched on `st` before it) and is complete
 // when the call returns, so kernels launched afterwards on any stream see an upload and
@@ -173,9 +156,12 @@ struct Species {
   int64_t npid = 0;  // particles given at first: their pids are 0 .. npid - 1
   int64_t cap_total = 0;
   double qabs = 0.0, qmax = 0.0;
-  // the allocations that hold the particle and mover arrays (alloc_slots), and the one that
-  // holds the tile tables
-  DBuf slots[19], tables;
+  // The particle and mover arrays and the tile tables are parts of one allocation each: from 2 MiB
+  // on an allocation takes some 290 us whatever its size, and smaller ones, cheap where earlier
+  // releases left room for them, as much in a young process.  us to create and load a simulation
+  // in one, an allocation per array / this: 64x64 of 16 per cell 571 / 412, 128x128 2135 / 1015,
+  // 512x512 9607 / 1295, 48^3 of 8 per cell 5650 / 838.
+  DBuf slots, tables;
   DBuf cell, x, y, z, ux, uy, uz, q, pid;
   DBuf mcell, mx, my, mz, mux, muy, muz, mq, mpid, midx;
   DBuf off, cnt, cap, mv_cnt, mv_stride, newcnt, inc, epart;
@@ -211,7 +197,7 @@ struct osr_sim {
   int nwall_v = 0;  // blocks of 256 cells of the VPML walls
   double dx[3] = {1, 1, 1};
   double dt = 0;
-  DBuf E, B, J, E2, B2, J2, ctrl, fe_part, hist;
+  DBuf E, B, J, ctrl, fe_part, hist;
   int64_t hist_cap = 0;
   std::vector<std::unique_ptr<Species>> sp;
   DBuf d_spec, d_work, d_pwork, d_fd, d_ywork, d_ework, d_dwork, d_fwork;
@@ -515,10 +501,10 @@ int upload_descs(osr_sim* s) {
 // E, B of the copy the next step reads, and the grid descriptor that names them (for the
 // kernels that take it by value)
 float* cur_E(const osr_sim* s) {
-  return s->g.pp && s->par ? s->g.E2 : s->g.E;
+  return s->E.as<float>() + (s->g.pp ? (size_t)s->par * 3 * s->g.ncell : 0);
 }
 float* cur_B(const osr_sim* s) {
-  return s->g.pp && s->par ? s->g.B2 : s->g.B;
+  return s->B.as<float>() + (s->g.pp ? (size_t)s->par * 3 * s->g.ncell : 0);
 }
 GridDesc cur_grid(const osr_sim* s) {
   GridDesc g = s->g;
@@ -564,22 +550,15 @@ void particle_arrays(Species& p, DBuf* (&arr)[19]) {
   std::copy(v, v + 19, arr);
 }
 
-// Places for them, n slots each (z and mz of a 2D species: none), in as few allocations as the
-// price of a large one allows: all in one when an array is large by itself (17 arrays of 3 MB
-// 4985 us, 51 MB at once 290), else as many together as stay below.
-int alloc_slots(int dims, DBuf (&slots)[19], size_t n, uint32_t* (&at)[19]) {
-  const size_t bytes = std::max<size_t>(256, (4 * n + 255) / 256 * 256);
-  const size_t per = bytes >= kLargeAlloc ? 19 : (kLargeAlloc - 1) / bytes;
-  int real[19], nr = 0;
+// Their places in one allocation of n slots each (z and mz of a 2D species: none)
+int alloc_slots(int dims, DBuf& slots, size_t n, uint32_t* (&at)[19]) {
+  const size_t bytes = (4 * n + 255) / 256 * 256;
+  TRY(slots.alloc(bytes * (dims == 3 ? 19 : 17)));
+  char* b = (char*)slots.p;
   for (int a = 0; a < 19; a++) {
-    slots[a].release();
-    at[a] = nullptr;
-    if (dims == 3 || (a != 3 && a != 12)) real[nr++] = a;
-  }
-  for (int i = 0, k = 0; i < nr; k++) {
-    const int m = (int)std::min<size_t>(per, nr - i);
-    TRY(slots[k].alloc(bytes * m));
-    for (int j = 0; j < m; j++, i++) at[real[i]] = (uint32_t*)((char*)slots[k].p + j * bytes);
+    const bool none = dims != 3 && (a == 3 || a == 12);
+    at[a] = (uint32_t*)b;
+    if (!none) b += bytes;
   }
   return OSR_OK;
 }
@@ -605,7 +584,7 @@ int alloc_species(osr_sim* s, Species& p, const std::vector<int>& cnt) {
   particle_arrays(p, arr);
   for (int a = 0; a < 19; a++) arr[a]->release();
   TRY(alloc_slots(s->dims, p.slots, n, at));
-  for (int a = 0; a < 19; a++) arr[a]->view(at[a], at[a] ? 4 * n : 0);
+  for (int a = 0; a < 19; a++) arr[a]->view(at[a], 4 * n);
   p.epart_n = s->plain ? (int)((total + 255) / 256) : nt * s->split;
   // the tile tables: off, cnt, cap (uploaded together), then those that start at zero
   const size_t tb = (4 * (size_t)nt + 255) / 256 * 256, mb = tb * kMaxTileWaves;
@@ -871,7 +850,7 @@ int regrow_species(osr_sim* s, int sid, bool* ok) {
   const size_t n = (size_t)total;
   DBuf* arr[19];
   particle_arrays(p, arr);
-  DBuf slots[19];
+  DBuf slots;
   RegrowArrays src{}, dst{};
   TRY(alloc_slots(s->dims, slots, n, dst.a));
   for (int a = 0; a < 19; a++) src.a[a] = arr[a]->as<uint32_t>();
@@ -884,8 +863,8 @@ int regrow_species(osr_sim* s, int sid, bool* ok) {
                      s->d_spec.as<SpecDesc>(), sid, src, dst, d_off.as<int>());
   HIPC(hipGetLastError());
   HIPC(hipStreamSynchronize(s->stream));
-  for (int a = 0; a < 19; a++) p.slots[a].swap(slots[a]);  // the old arrays go with the local
-  for (int a = 0; a < 19; a++) arr[a]->view(dst.a[a], dst.a[a] ? 4 * n : 0);
+  p.slots.swap(slots);  // the old arrays go with the local
+  for (int a = 0; a < 19; a++) arr[a]->view(dst.a[a], 4 * n);
   TRY(copy_on(s->stream, p.off.p, off.data(), 4 * (size_t)nt, hipMemcpyHostToDevice));
   TRY(copy_on(s->stream, p.cap.p, cap.data(), 4 * (size_t)nt, hipMemcpyHostToDevice));
   p.h_off = off;
@@ -1470,9 +1449,10 @@ int osr_sim_create(const osr_sim_desc* desc, osr_sim** out) {
   HIPC(hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking));
   const size_t nc = (size_t)g.ncell;
   g.pp = dims == 2 && !s->plain && !open_x;  // grids whose field step is yee2d_step
-  TRY(alloc_copies(s->E, s->E2, 12 * nc, g.pp));
-  TRY(alloc_copies(s->B, s->B2, 12 * nc, g.pp));
-  TRY(alloc_copies(s->J, s->J2, 24 * nc, g.pp));
+  const size_t ncp = g.pp ? 2 * nc : nc;
+  TRY(s->E.alloc(3 * ncp * 4));
+  TRY(s->B.alloc(3 * ncp * 4));
+  TRY(s->J.alloc(3 * ncp * 8));
   TRY(s->ctrl.alloc(sizeof(Ctrl)));
   s->vp_n = vp_n;
   if (open_x && vp_n) {
@@ -1489,16 +1469,14 @@ int osr_sim_create(const osr_sim_desc* desc, osr_sim** out) {
     TRY(s->wall.alloc(wb));
     HIPC(hipMemsetAsync(s->wall.p, 0, wb, s->stream));
   }
-  for (const DBuf* f : {&s->E, &s->B, &s->J, &s->E2, &s->B2, &s->J2})
-    if (f->p && f->own) HIPC(hipMemsetAsync(f->p, 0, f->n, s->stream));
+  HIPC(hipMemsetAsync(s->E.p, 0, 3 * ncp * 4, s->stream));
+  HIPC(hipMemsetAsync(s->B.p, 0, 3 * ncp * 4, s->stream));
+  HIPC(hipMemsetAsync(s->J.p, 0, 3 * ncp * 8, s->stream));
   HIPC(hipMemsetAsync(s->ctrl.p, 0, sizeof(Ctrl), s->stream));
   HIPC(hipStreamSynchronize(s->stream));
   g.E = s->E.as<float>();
   g.B = s->B.as<float>();
   g.J = s->J.as<unsigned long long>();
-  g.E2 = s->E2.as<float>();
-  g.B2 = s->B2.as<float>();
-  g.J2 = s->J2.as<unsigned long long>();
   g.ctrl = s->ctrl.as<Ctrl>();
   s->nblk = (int)((nc + 255) / 256);
   s->nblk_e = (s->nblk + kEneBlk - 1) / kEneBlk;
@@ -2134,11 +2112,9 @@ int osr_sim_relayouts(osr_sim* s, int64_t* count) {
 int osr_sim_footprint(osr_sim* s, int64_t* bytes) {
   TRY(check_sim(s));
   if (!bytes) return fail(OSR_ERR_ARG, "null argument");
-  size_t b = s->fe_part.n + s->hist.n;
-  for (const DBuf* f : {&s->E, &s->B, &s->J, &s->E2, &s->B2, &s->J2}) b += f->own ? f->n : 0;
+  size_t b = s->E.n + s->B.n + s->J.n + s->fe_part.n + s->hist.n;
   for (auto& p : s->sp) {
-    b += p->tables.n;
-    for (const DBuf& d : p->slots) b += d.n;
+    b += p->slots.n + p->tables.n;
   }
   *bytes = (int64_t)b;
   return OSR_OK;

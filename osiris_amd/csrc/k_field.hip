@@ -462,9 +462,10 @@ OSR_DEV void yee2d_tile(const FieldDesc& fd, int item, float* lds) {
   if (halt >= 2) return;
   const int nx = g.nx, ny = g.ny, tid = threadIdx.x;
   const long long nc = g.ncell;
+  const long long in = (long long)par * 3 * nc, out = (long long)(par ^ 1u) * 3 * nc;
   const T tile(item, nx);
-  const float* __restrict__ Ei = par ? g.E2 : g.E;
-  const float* __restrict__ Bi = par ? g.B2 : g.B;
+  const float* __restrict__ Ei = g.E + in;
+  const float* __restrict__ Bi = g.B + in;
   // every load of the thread is issued before its first use (cells of the halo whose B or J
   // is not needed included: no branches between the loads)
   float e[Q][3], b[Q][3], jv[Q][3];
@@ -486,7 +487,7 @@ OSR_DEV void yee2d_tile(const FieldDesc& fd, int item, float* lds) {
 #pragma unroll
       for (int m = 0; m < 3; m++) jv[q][m] = Jf[m * nc + c[q]];
   } else {
-    const unsigned long long* __restrict__ Ji = par ? g.J2 : g.J;
+    const unsigned long long* __restrict__ Ji = g.J + in;
     const double jinv = g.jinv;
     long long v[Q][3];
 #pragma unroll
@@ -541,9 +542,9 @@ OSR_DEV void yee2d_tile(const FieldDesc& fd, int item, float* lds) {
   }
   __syncthreads();
   double acc[6] = {0, 0, 0, 0, 0, 0};
-  float* __restrict__ Eo = par ? g.E : g.E2;
-  float* __restrict__ Bo = par ? g.B : g.B2;
-  unsigned long long* __restrict__ Jo = par ? g.J : g.J2;
+  float* __restrict__ Eo = g.E + out;
+  float* __restrict__ Bo = g.B + out;
+  unsigned long long* __restrict__ Jo = g.J + out;
 #pragma unroll
   for (int q = 0; q < Q; q++) {
     const int i = tid + 256 * q;
@@ -606,8 +607,8 @@ __global__ __launch_bounds__(256) void yee2d_energy(const FieldDesc* __restrict_
   const int nx = g.nx, ny = g.ny;
   const long long nc = g.ncell;
   const T tile(wk.y, nx);
-  const float* __restrict__ E = cur_E(g);
-  const float* __restrict__ B = cur_B(g);
+  const float* __restrict__ E = g.E + cur_copy(g);
+  const float* __restrict__ B = g.B + cur_copy(g);
   double acc[6] = {0, 0, 0, 0, 0, 0};
 #pragma unroll
   for (int q = 0; q < T::Q; q++) {

@@ -90,11 +90,11 @@ __global__ __launch_bounds__(64 * NW, 4) void push_deposit_2d_t(const SpecDesc* 
   const int tile = wk.y;
   const int cx0 = (tile % g.ntx) * TX, cy0 = (tile / g.ntx) * TY;
   const int nx = g.nx, ny = g.ny;
-  const long long nc = g.ncell;
+  const long long nc = g.ncell, co = cur_copy(g);
 
   {
-    const gf32* __restrict__ E = (const gf32*)cur_E(g);
-    const gf32* __restrict__ B = (const gf32*)cur_B(g);
+    const gf32* __restrict__ E = (const gf32*)g.E + co;
+    const gf32* __restrict__ B = (const gf32*)g.B + co;
     for (int i = threadIdx.x; i < GN; i += NT) {
       const int col = i % GX, row = i / GX;
       const int gx = wrapi(cx0 + col - O::GLO, nx), gy = wrapi(cy0 + row - O::GLO, ny);
@@ -403,7 +403,7 @@ __global__ __launch_bounds__(64 * NW, 4) void push_deposit_2d_t(const SpecDesc* 
     d.epart[tile * split + part] = t;
   }
   // ---- fold the LDS current tile into the global fixed-point J (periodic wrap)
-  gu64* __restrict__ GJ = (gu64*)cur_J(g);
+  gu64* __restrict__ GJ = (gu64*)g.J + co;
   for (int i = threadIdx.x; i < JN; i += NT) {
     const int gx = wrapi(cx0 + i % JX - O::JLO, nx), gy = wrapi(cy0 + i / JX - O::JLO, ny);
     const long long gi = gx + (long long)nx * gy;

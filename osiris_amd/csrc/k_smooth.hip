@@ -59,7 +59,7 @@ __global__ __launch_bounds__(256) void smooth_pass(const FieldDesc* __restrict__
   }
   const long long row = idx - (long long)c * st;  // the line's first cell
   const int src = pass == 0 ? fd.sm_src : 2;
-  const unsigned long long* Jq = cur_J(g);
+  const unsigned long long* Jq = g.J + cur_copy(g);
   const float* Jp = (const float*)g.J;
   const float* P = fd.sm_buf[(pass + 1) & 1];  // previous pass's output
   float* dst = fd.sm_buf[pass & 1];
@@ -113,7 +113,7 @@ __global__ __launch_bounds__(256) void smooth2d(const FieldDesc* __restrict__ fd
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int gx = wrap_any(x0 - n[0] + (lane < wd ? lane : wd - 1), nx);
   const long long base = comp * nc + gx;
-  const unsigned long long* __restrict__ Jq = cur_J(g);
+  const unsigned long long* __restrict__ Jq = g.J + cur_copy(g);
   const float* __restrict__ Jp = (const float*)g.J;
   const double jinv = g.jinv;
   for (int r0 = wave; r0 < ht; r0 += 16) {

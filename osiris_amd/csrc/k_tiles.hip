@@ -90,17 +90,15 @@ __global__ __launch_bounds__(NT) void push_deposit_2d(const SpecDesc* __restrict
   float* sF = (float*)(smem + sizeof(unsigned long long) * 3 * JN);  // E[3][GN], B[3][GN]
   const int cx0 = (tile % g.ntx) * TX, cy0 = (tile / g.ntx) * TY;
   const int nx = g.nx, ny = g.ny;
-  const long long nc = g.ncell;
-  const float* const E = cur_E(g);
-  const float* const B = cur_B(g);
+  const long long nc = g.ncell, co = cur_copy(g);
 
   for (int i = threadIdx.x; i < GN; i += NT) {
     int gx = wrapi(cx0 + (i % GX) - O::GLO, nx), gy = wrapi(cy0 + (i / GX) - O::GLO, ny);
     long long gi = gx + (long long)nx * gy;
 #pragma unroll
     for (int c = 0; c < 3; c++) {
-      sF[c * GN + i] = E[c * nc + gi];
-      sF[(3 + c) * GN + i] = B[c * nc + gi];
+      sF[c * GN + i] = g.E[co + c * nc + gi];
+      sF[(3 + c) * GN + i] = g.B[co + c * nc + gi];
     }
   }
   for (int i = threadIdx.x; i < 3 * JN; i += NT) sJ[i] = 0ull;
@@ -261,7 +259,7 @@ __global__ __launch_bounds__(NT) void push_deposit_2d(const SpecDesc* __restrict
 #pragma unroll
     for (int c = 0; c < 3; c++) {
       const unsigned long long v = sJ[c * JN + i];
-      if (v) atomicAdd(&cur_J(g)[c * nc + gi], v);
+      if (v) atomicAdd(&g.J[co + c * nc + gi], v);
     }
   }
 }

@@ -92,11 +92,8 @@ struct GridDesc {
   float* E;
   float* B;
   unsigned long long* J;
-  int pp;            // E, B and J have a second copy E2, B2, J2: the step reads those of
-                     // Ctrl::par, writes E and B of the other and clears its J
-  float* E2;
-  float* B2;
-  unsigned long long* J2;
+  int pp;            // E, B and J hold two copies, 3 ncell values apart: the step reads those
+                     // of Ctrl::par, writes E and B of the other and clears its J
   double jscale;     // 2^jshift
   double jinv;       // 2^-jshift
   float dt_dx[3];    // (float)(dt/dx)
@@ -105,11 +102,10 @@ struct GridDesc {
   FastDiv div_nx, div_ny;  // cell index c -> x = c mod nx, row c / nx; row -> y, z
 };
 
-// the copies the step reads
-__device__ inline bool second_copy(const GridDesc& g) { return g.pp && g.ctrl->par; }
-__device__ inline float* cur_E(const GridDesc& g) { return second_copy(g) ? g.E2 : g.E; }
-__device__ inline float* cur_B(const GridDesc& g) { return second_copy(g) ? g.B2 : g.B; }
-__device__ inline unsigned long long* cur_J(const GridDesc& g) { return second_copy(g) ? g.J2 : g.J; }
+// values from the start of E, B or J to the copy the step reads
+__device__ inline long long cur_copy(const GridDesc& g) {
+  return g.pp ? (long long)g.ctrl->par * 3 * g.ncell : 0;
+}
 
 // the divisors of a grid whose extents are set (host)
 __host__ inline void set_grid_divisors(GridDesc& g) {

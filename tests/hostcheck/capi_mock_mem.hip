@@ -1,16 +1,14 @@
-// capi_mock_mem.hip -- the host check of capi_mock.hip with a device memory that fills up and
-// a log of the large allocations (test infrastructure only).
+// capi_mock_mem.hip -- the host check of capi_mock.hip with a device memory that fills up (test
+// infrastructure only).
 #include "mock_hip.h"
 
 namespace mock {
 inline size_t& limit() { static size_t l = ~size_t(0); return l; }  // bytes of device memory
-inline long long& nlarge() { static long long n = 0; return n; }    // allocations of 2 MiB and more
 inline hipError_t limited_malloc(void** p, size_t n) {
   size_t held = 0;
   for (auto& kv : live())
     if (!kv.second.pinned) held += kv.second.n;
   if (held + n > limit()) return hipErrorOutOfMemory;
-  nlarge() += n >= (size_t(2) << 20);
   return m_hipMalloc(p, n);
 }
 }  // namespace mock
@@ -25,4 +23,3 @@ extern "C" void mock_leave_free(long long bytes) {
     if (!kv.second.pinned) held += kv.second.n;
   mock::limit() = bytes < 0 ? ~size_t(0) : held + (size_t)bytes;
 }
-extern "C" long long mock_large_allocs() { return mock::nlarge(); }

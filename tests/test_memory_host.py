@@ -43,7 +43,7 @@ import osiris_amd._lib as L
 L.LIB_PATH = {lib!r}
 L.lib()
 raw = C.CDLL({lib!r})
-for f in ("mock_errors", "mock_order_errors", "mock_live", "mock_large_allocs"):
+for f in ("mock_errors", "mock_order_errors", "mock_live"):
     getattr(raw, f).restype = C.c_longlong
 raw.mock_leave_free.argtypes = [C.c_longlong]
 from osiris_amd.sim import Simulation
@@ -63,27 +63,6 @@ print(json.dumps(out))
     res = json.loads(r.stdout.strip().splitlines()[-1])
     assert res.pop("errors") == 0 and res.pop("live") == 0, r.stderr[-3000:]
     return res
-
-
-@pytest.mark.parametrize("dims,nx,ppc,species", [(2, (300, 200), (2, 2), 0), (2, (64, 64), (2, 2), 0),
-                                                 (3, (48, 48, 48), (2, 1, 1), 0), (2, (512, 512), (4, 4), 2)])
-def test_no_large_allocation_for_small_arrays(mem_lib, dims, nx, ppc, species):
-    """An allocation of 2 MiB or more takes some 290 us and a smaller one 5 us: arrays below
-    that size (the copies of the fields and the current, the particle arrays) are not put
-    together into larger allocations, and larger ones are one allocation each, or, the particle
-    arrays, one in all (512x512: once for the empty species, once for the particles)."""
-    res = _run(mem_lib, f"""
-with Simulation({dims}, {nx}, (0.1,) * {dims}, 0.05, 2) as s:
-    out["grid"] = raw.mock_large_allocs()
-    sid = s.add_species(-1.0)
-    s.generate(sid, {ppc})
-    out["species"] = raw.mock_large_allocs() - out["grid"]
-    s.run(3)
-""")
-    cells = 1
-    for m in nx:
-        cells *= m
-    assert res == {"grid": 2 * (12 * cells >= 2 << 20) + (24 * cells >= 2 << 20), "species": species}
 
 
 @pytest.mark.parametrize("dims,nx", [(2, (150, 110)), (3, (40, 30, 20))])
