@@ -1785,15 +1785,13 @@ static int fields_xfer(osr_sim* s, float* e, float* b, const int* ld, const int*
   if (!set) {
     // every array cell (guards included) gets its periodic image; with open x walls the x
     // guard cells come from the guard band of the ring.  In pieces of whole rows, at most
-    // about 64 MB each.  Small arrays are rearranged by the host, in less time than the device
-    // memory for it takes (us for E and B, host / device: 69x69 cells 75 / 100, 17^3 66 / 101,
-    // 305x205 289 / 130), and so are all when there is no device memory left.
+    // about 64 MB each.  Without device memory left for that the host rearranges them.
     FieldsOut a{s->g.nx, s->g.ny, s->g.nz, s->g.ncell, ld[0], ld[1],
                 {gcl[0], gcl[1], D == 3 ? gcl[2] : 0}, 0, 0};
     const long long rows = (long long)ld[1] * (D == 3 ? ld[2] : 1);
     const long long piece = std::min(rows, std::max(1ll, (64ll << 20) / (12ll * ld[0])));
     DBuf out;
-    if (rows * ld[0] <= 12000 || out.alloc(12 * (size_t)piece * ld[0]) != OSR_OK)
+    if (out.alloc(12 * (size_t)piece * ld[0]) != OSR_OK)
       return fields_get_host(s, e, b, ld, gcl);
     for (int w = 0; w < 2; w++) {
       float* h = w == 0 ? e : b;
