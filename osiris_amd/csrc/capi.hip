@@ -154,6 +154,7 @@ struct Species {
   int pusher = OSR_BORIS;
   int64_t np = 0;
   int64_t npid = 0;  // particles given at first: their pids are 0 .. npid - 1
+  int used = 0, most = 0;  // tiles that held particles when it was laid out, the fullest one
   int64_t cap_total = 0;
   double qabs = 0.0, qmax = 0.0;
   // The particle and mover arrays and the tile tables are parts of one allocation each: from 2 MiB
@@ -212,10 +213,13 @@ struct osr_sim {
   int yv = 0;             // yee2d_step variant (0: 32x8 cells per workgroup, 1: 64x16)
   int64_t steps = 0;
   int64_t relayouts = 0;
+  bool halted = false;  // a step's movers wait for a re-layout that failed
   bool plain = false;
   size_t lds_push = 0;
   int push_waves = 4;  // waves per push workgroup
-  int split = 1;       // push workgroups per tile (SpecDesc::split)
+  int split = 1;       // push workgroups per tile (SpecDesc::split), at most
+  int split_max = 1;
+  bool pwork_ok = false;  // d_pwork names the present species and split
   int tile_waves() const { return push_waves * split; }
   int reorder = 0;     // tile_reorder period in steps (0: off)
   int sm_order[3] = {0, 0, 0};  // current smoothing per direction (0: none)
@@ -526,20 +530,76 @@ inline void cell_coords(const osr_sim* s, uint32_t c, int* ic) {
 // slots each, and the fill leaves as many (at least those of the largest workgroup).
 int mover_slack(int tile_waves) { return 64 * std::max(kMaxPushWaves, tile_waves); }
 
-// Push workgroups per tile (2D compile-time kernels).  One wave takes about 1.2 us of VALU
-// issue per 64 particles, and about 2 us when it has a SIMD to itself, so a grid with
-// fewer waves than the chip's 1024 SIMDs hold is bound by the longest wave: its tiles are
-// shared by several workgroups.  Each of them stages the tile's fields and folds a current
-// tile of its own, which costs more than it gains once the tiles fill the chip.  us per
-// step, 1 / 2 / 4 workgroups per tile: 16x16 tiles with 4 waves, 64 tiles (128 x 128 x 16)
-// 53.6 / 45.4 / 41.9, 247 tiles (300 x 200 x 16) 94.2 / 87.1 / 90.8, 561 tiles (two species
-// of 9) 90.9 / 92.4 / 107.6, 1024 tiles 216.9 / 228.1 / 245.0; 32x16 tiles with 8 waves
-// (2 workgroups per CU), 102 tiles 84.6 / 76.8, 528 tiles push 69.4 / 57.7 (one workgroup
-// per tile leaves a second round of 16).  3D keeps one: LDS lets two workgroups into a CU,
-// and 378 tiles of 8x8x4 went from 95.8 to 106.8.
-int pick_split(int ntiles, int waves) {
+// The most push workgroups that a tile may get (2D compile-time kernels; 3D keeps one: LDS lets
+// two into a CU, and 378 tiles of 8x8x4 went from 95.8 to 106.8 us).  It sets what the layout
+// keeps free: 1024 slots per tile for 16 waves, only on grids where they can pay.
+int max_split(int ntiles, int waves) {
   if (waves >= 8) return ntiles <= 640 ? 2 : 1;
-  return ntiles <= 128 ? 4 : (ntiles <= 384 ? 2 : 1);
+  return ntiles <= 192 ? 4 : 2;
+}
+
+// Cost of a push launch of `wgs` (species, tile) pairs with sp workgroups each, in iterations of a
+// workgroup (its: 64 particles per wave and iteration, over the waves of one workgroup; most: of
+// the fullest tile).  The busiest CU gets ceil(wgs sp / 256) workgroups, each of which also stages
+// the tile's fields and folds a current tile of its own, 2.2 iterations' worth; alone on its CU one
+// of 4 waves waits on latencies half the time.  A fifth workgroup of 4 waves on a CU waits for one
+// to end, which the short iterations of linear splines do not make up for (640 tiles of 16 per
+// cell 58.6 / 64.3 us).  Species of one launch mostly differ, and the lighter one's workgroups
+// (cold ions) end early and leave the CU to others: part of the mean then.
+// us per step with 1 / 2 / 4 workgroups per tile, quadratic, 16x16 tiles of 4 waves: 64 tiles, 1 per
+// cell 23.2 / 23.2 / 23.3, 4 per cell 28.3 / 26.5 / 25.5, 16 per cell 47.4 / 36.3 / 31.4; 192
+// tiles, 4 per cell 30.2 / 32.1 / 32.5, 16 per cell 50.5 / 45.6 / 42.7; 384 tiles, 16 per cell 64.1
+// / 56.9 / 63.9, as two species of 192 62.7 / 54.9 / 63.0; 512 tiles 64.2 / 66.3 / 71.7, as eight
+// species of 64 63.6 / 65.6 / 72.8, with 4 per cell 35.4 / 42.0 / 49.7; hot electrons and ions of
+// 84, 4 per cell 30.2 / 27.6 / 28.1.  32x16 tiles of 8 waves, 16 per cell: 128 tiles 61.0 / 47.9,
+// 256 67.3 / 70.0, 528 132.7 / 126.5, 768 147.7 / 161.3; 8 per cell between open walls: 272 tiles
+// 73.9 / 63.5, 400 78.2 / 85.1.  Of 2271 measured launches (1 to 8 species, 1 to 64 per cell, u_th
+// 0.01 to 0.3, all orders, both pushers) the choice is 0.1% above the fastest on average, and 13
+// are more than 2% (at most 5.4%) slower than with one workgroup per tile.
+double push_cost(int wgs, double its, double most, int sp, int waves, int order, bool several) {
+  const double x = wgs * sp / 256.0, up = std::ceil(x);
+  if (order == 1 && sp > 1 && up > 4.0) return 1e30;
+  const double per_cu = several ? std::max(1.0, 0.75 * up + 0.25 * x) : up;
+  const double n = std::max(its / sp, waves / 4.0);
+  return std::max(per_cu, waves == 4 ? 1.5 : 1.1) * n + (most - its) / sp + per_cu * 2.2;
+}
+
+// Push workgroups per tile for the particles as they lie: the fewest with the least cost over the
+// step's push launches (with 4 waves the most that still have a CU each: 16 tiles of 2 per cell
+// 24.6 / 24.4 / 23.2 us).  Between open walls, where a laser piles the particles up, the fullest
+// tile is taken to have twice the mean: 1024x256 with 528 tiles 100 us per step either way at
+// first, push 66 / 55 us later; 448x208 5.1 / 5.4 ms per 75 steps, push 54 / 37 us.  The caller
+// uploads the descriptors; the mover lists of a halted step keep the split they were written with.
+void choose_split(osr_sim* s) {
+  if (s->split_max == 1 || s->halted) return;
+  const int ns = (int)s->sp.size();
+  int best = 1;
+  double best_cost = 0.0;
+  for (int sp = 1; sp <= s->split_max; sp *= 2) {
+    double cost = 0.0;
+    bool room = sp > 1 && s->push_waves == 4;
+    for (int a = 0, b; a < ns; a = b) {  // the launches of launch_pushes
+      double np = 0.0, used = 0.0, most = 0.0;
+      for (b = a; b < ns && s->sp[b]->pusher == s->sp[a]->pusher; b++) {
+        np += (double)s->sp[b]->np;
+        used += s->sp[b]->used;
+        most = std::max<double>(most, s->sp[b]->most);
+      }
+      const int wgs = (b - a) * s->ntiles;
+      const double lanes = 64.0 * s->push_waves, its = np / std::max(used, 1.0) / lanes;
+      most = std::max(most / lanes, s->g.open_nx ? 2.0 * its : its);
+      cost += push_cost(wgs, its, most, sp, s->push_waves, s->order, b - a > 1);
+      room = room && wgs * sp <= (its > 1.0 ? 256 : 192);
+    }
+    if (sp == 1 || cost < best_cost * (room ? 1.0 + 1e-9 : 1.0 - 1e-9)) {
+      best = sp;
+      best_cost = cost;
+    }
+  }
+  if (best == s->split) return;
+  s->split = best;
+  s->pwork_ok = false;
+  for (auto& p : s->sp) p->epart_n = s->ntiles * s->split;
 }
 
 // The 19 particle and mover arrays of a species in the order of RegrowArrays
@@ -563,6 +623,15 @@ int alloc_slots(int dims, DBuf& slots, size_t n, uint32_t* (&at)[19]) {
   return OSR_OK;
 }
 
+// what the choice of the push's workgroups needs of the tile counts
+void count_tiles(Species& p, const std::vector<int>& cnt) {
+  p.used = p.most = 0;
+  for (int c : cnt) {
+    p.used += c > 0;
+    p.most = std::max(p.most, c);
+  }
+}
+
 // Allocate a species' arrays for the given per-tile counts and capacities.
 int alloc_species(osr_sim* s, Species& p, const std::vector<int>& cnt) {
   const int nt = s->ntiles;
@@ -570,7 +639,7 @@ int alloc_species(osr_sim* s, Species& p, const std::vector<int>& cnt) {
   int64_t total = 0;
   for (int t = 0; t < nt; t++) {
     const int c = cnt[t];
-    int64_t cp = (int64_t)c + std::max(c / 4, 64) + mover_slack(s->tile_waves());
+    int64_t cp = (int64_t)c + std::max(c / 4, 64) + mover_slack(s->push_waves * s->split_max);
     cp = (cp + 63) / 64 * 64;
     if (total + cp > INT32_MAX) return fail(OSR_ERR_ARG, "species too large for int32 slots");
     cap[t] = (int)cp;
@@ -588,7 +657,7 @@ int alloc_species(osr_sim* s, Species& p, const std::vector<int>& cnt) {
   p.epart_n = s->plain ? (int)((total + 255) / 256) : nt * s->split;
   // the tile tables: off, cnt, cap (uploaded together), then those that start at zero
   const size_t tb = (4 * (size_t)nt + 255) / 256 * 256, mb = tb * kMaxTileWaves;
-  const size_t eb = 8 * (size_t)p.epart_n;
+  const size_t eb = 8 * (size_t)(s->plain ? p.epart_n : nt * s->split_max);
   TRY(p.tables.alloc(6 * tb + mb + eb));
   char* t0 = (char*)p.tables.p;
   DBuf* const tab[6] = {&p.off, &p.cnt, &p.cap, &p.mv_stride, &p.newcnt, &p.inc};
@@ -612,6 +681,7 @@ int alloc_species(osr_sim* s, Species& p, const std::vector<int>& cnt) {
   int64_t np = 0;
   for (int c : cnt) np += c;
   p.np = np;
+  count_tiles(p, cnt);
   return OSR_OK;
 }
 
@@ -840,7 +910,7 @@ int regrow_species(osr_sim* s, int sid, bool* ok) {
     // every tile gets room for half its count again (a density front that overflows one
     // tile usually reaches its neighbours next); no tile shrinks
     const int64_t r = inc[t] < 0 ? need[t] : cnt[t];
-    int64_t c = std::max<int64_t>(p.h_cap[t], r + std::max<int64_t>(r / 2, 64) + mover_slack(s->tile_waves()));
+    int64_t c = std::max<int64_t>(p.h_cap[t], r + std::max<int64_t>(r / 2, 64) + mover_slack(s->push_waves * s->split_max));
     c = (c + 63) / 64 * 64;
     if (total + c > INT32_MAX) return OSR_OK;
     cap[t] = (int)c;
@@ -890,6 +960,7 @@ int regrow_species(osr_sim* s, int sid, bool* ok) {
   int64_t np = 0;
   for (int v : cnt) np += v;
   p.np = np;
+  count_tiles(p, cnt);
   *ok = true;
   return OSR_OK;
 }
@@ -898,6 +969,7 @@ int regrow_species(osr_sim* s, int sid, bool* ok) {
 // device re-layout is tried first and the host one (collect + layout_upload) is the
 // fallback; otherwise the particles are laid out again from the host.
 int relayout(osr_sim* s, bool pending) {
+  s->halted = pending;
   for (size_t i = 0; i < s->sp.size(); i++) {
     if (pending) {
       bool ok = false;
@@ -908,6 +980,8 @@ int relayout(osr_sim* s, bool pending) {
     TRY(collect(s, *s->sp[i], pending, hp));
     TRY(layout_upload(s, *s->sp[i], hp));
   }
+  s->halted = false;
+  choose_split(s);
   TRY(upload_descs(s));
   s->relayouts++;
   return OSR_OK;
@@ -1284,6 +1358,18 @@ int build_graph(osr_sim* s) {
   return OSR_OK;
 }
 
+// The push's work list names every item once per workgroup of the tile.
+int upload_push_list(osr_sim* s) {
+  std::vector<int2> pw;
+  for (int i = 0; i < (int)s->sp.size(); i++)
+    for (int t = 0; t < s->ntiles; t++)
+      pw.insert(pw.end(), s->split, make_int2(i, xcd_tile(s->dims, t, s->ntiles)));
+  TRY(s->d_pwork.alloc(sizeof(int2) * pw.size()));
+  TRY(copy_on(s->stream, s->d_pwork.p, pw.data(), sizeof(int2) * pw.size(), hipMemcpyHostToDevice));
+  s->pwork_ok = true;
+  return OSR_OK;
+}
+
 int ensure_hist(osr_sim* s, int64_t rows) {
   if (rows <= s->hist_cap) return OSR_OK;
   int64_t cap = std::max<int64_t>(rows, std::max<int64_t>(2 * s->hist_cap, 1024));
@@ -1445,7 +1531,7 @@ int osr_sim_create(const osr_sim_desc* desc, osr_sim** out) {
     s->push_waves = push3d_waves(s->order);
   if (!s->plain && dims == 2 && desc->kernel != 1 &&
       pick_push2d_t(s->order, 0, g.tx, g.ty, s->push_waves))
-    s->split = pick_split(g.ntiles, s->push_waves);
+    s->split_max = max_split(g.ntiles, s->push_waves);
   HIPC(hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking));
   const size_t nc = (size_t)g.ncell;
   g.pp = dims == 2 && !s->plain && !open_x;  // grids whose field step is yee2d_step
@@ -1553,11 +1639,8 @@ int osr_sim_add_species(osr_sim* s, float rqm, int pusher, int* sid) {
   for (int i = 0; i < ns; i++)
     for (int t = 0; t < s->ntiles; t++) w[(size_t)i * s->ntiles + t] = make_int2(i, xcd_tile(s->dims, t, s->ntiles));
   TRY(copy_on(s->stream, s->d_work.p, w.data(), sizeof(int2) * w.size(), hipMemcpyHostToDevice));
-  // the push's list names every item once per workgroup of the tile
-  std::vector<int2> pw;
-  for (size_t i = 0; i < nw; i++) pw.insert(pw.end(), s->split, w[i]);
-  TRY(s->d_pwork.alloc(sizeof(int2) * pw.size()));
-  TRY(copy_on(s->stream, s->d_pwork.p, pw.data(), sizeof(int2) * pw.size(), hipMemcpyHostToDevice));
+  s->pwork_ok = false;
+  choose_split(s);
   // history rows gain a column: restart the history buffer
   s->hist.release();
   s->hist_cap = 0;
@@ -1600,6 +1683,7 @@ int osr_species_set(osr_sim* s, int sid, int64_t np, const int* ix, const float*
   TRY(layout_upload(s, *s->sp[sid], hp));
   s->sp[sid]->npid = np;
   update_jscale(s);
+  choose_split(s);
   TRY(upload_descs(s));
   s->graph_ok = false;
   return OSR_OK;
@@ -1718,6 +1802,7 @@ int osr_species_generate(osr_sim* s, int sid, const int* ppc, double density,
   p.qabs = std::fabs((double)q) * (double)p.np;
   p.qmax = std::fabs((double)q);
   update_jscale(s);
+  choose_split(s);
   TRY(upload_descs(s));
   GenArgs a{};
   for (int d = 0; d < 3; d++) {
@@ -1878,6 +1963,7 @@ int osr_sim_run(osr_sim* s, int nsteps) {
   if (nsteps < 0) return fail(OSR_ERR_ARG, "negative step count");
   if (nsteps == 0) return OSR_OK;
   TRY(ensure_hist(s, s->steps + nsteps));
+  if (!s->pwork_ok) TRY(upload_push_list(s));
   if (!s->graph_ok) TRY(build_graph(s));
   TRY(refresh_energy(s));
   int64_t left = nsteps;
@@ -1904,7 +1990,12 @@ int osr_sim_run(osr_sim* s, int nsteps) {
       Ctrl z = c;
       z.halt = 0;
       TRY(copy_on(s->stream, s->ctrl.p, &z, sizeof(Ctrl), hipMemcpyHostToDevice));
-      // the captured steps name the descriptors and work lists, which keep their places
+      // the captured steps name the descriptors and work lists, which keep their places, unless
+      // the fuller tiles are now shared by more workgroups
+      if (!s->pwork_ok) {
+        TRY(upload_push_list(s));
+        TRY(build_graph(s));
+      }
       batch = 8;
     } else if (done != nb) {
       return fail(OSR_ERR_STATE, "step counter advanced by %lld instead of %d",
@@ -2150,6 +2241,7 @@ int osr_sim_time_kernels(osr_sim* s, int nsteps, double* ms) {
   for (int i = 0; i < nev; i++) HIPC(hipEventCreate(&ev[i]));
   double acc[6] = {0, 0, 0, 0, 0, 0};
   int done = 0;
+  if (!s->pwork_ok) TRY(upload_push_list(s));
   TRY(refresh_energy(s));
   for (int k = 0; k < nsteps; k++) {
     if (!s->zp.empty()) {  // the laser walls of the step, not timed
@@ -2184,6 +2276,10 @@ int osr_sim_time_kernels(osr_sim* s, int nsteps, double* ms) {
       Ctrl z = c;
       z.halt = 0;
       TRY(copy_on(s->stream, s->ctrl.p, &z, sizeof(Ctrl), hipMemcpyHostToDevice));
+      if (!s->pwork_ok) {
+        TRY(upload_push_list(s));
+        s->graph_ok = false;
+      }
       continue;  // a re-laid-out step is not representative
     }
     float t;

@@ -96,10 +96,10 @@ int64_t job_footprint(const osr_job_desc& j) {
       const int64_t wy = std::min(tl[1], d.nx[1] - ty * tl[1]);
       const int64_t wz = D == 3 ? std::min(tl[2], d.nx[2] - tz * tl[2]) : 1;
       const int64_t c = wx * wy * wz * ppc;
-      int64_t cp = c + std::max<int64_t>(c / 4, 64) + 64 * kMaxTileWaves;
+      int64_t cp = c + std::max<int64_t>(c / 4, 64) + 64 * kMaxPushWaves;
       slots += (cp + 63) / 64 * 64;
     }
-    b += slots * slot + ntiles * (24 + 4 * kMaxTileWaves + 8 * kMaxSplit);
+    b += slots * slot + ntiles * (24 + 4 * kMaxTileWaves + 8);
   }
   return b + (1 << 20);
 }
@@ -156,6 +156,7 @@ int ens_admit(osr_ensemble* e, EnsJob* j) {
   osr_sim* s = nullptr;
   TRY(osr_sim_create(&jd.sim, &s));
   std::unique_ptr<osr_sim, int (*)(osr_sim*)> guard(s, osr_sim_destroy);
+  s->split_max = 1;  // a batch's launch holds the tiles of all its jobs
   for (int i = 0; i < jd.nspecies; i++) {
     const osr_job_species& sp = jd.species[i];
     int sid = 0;
@@ -222,7 +223,7 @@ int ens_build(osr_ensemble* e, EnsBatch* b) {
   std::vector<SpecDesc> specs;
   std::vector<FieldDesc> fds(b->jobs.size());
   std::vector<int2> wp[2], wf, wy, we, wd;
-  std::vector<int> wn, spec0;
+  std::vector<int> wn;
   for (size_t k = 0; k < b->jobs.size(); k++) {
     osr_sim* s = b->jobs[k]->sim;
     const int base = (int)specs.size();
@@ -231,25 +232,14 @@ int ens_build(osr_ensemble* e, EnsBatch* b) {
     make_field_desc(s, fds[k]);
     for (size_t i = 0; i < s->sp.size(); i++)
       for (int t = 0; t < s->ntiles; t++) {
+        wp[s->sp[i]->pusher == OSR_VAY ? 1 : 0].push_back(make_int2(base + (int)i, t));
         wf.push_back(make_int2(base + (int)i, t));
       }
     for (int blk = 0; blk < s->nblk; blk++) wy.push_back(make_int2((int)k, blk));
     for (int blk = 0; blk < s->nblk_e; blk++) we.push_back(make_int2((int)k, blk));
     for (int c = 0; c < 6 + (int)s->sp.size(); c++) wd.push_back(make_int2((int)k, -1 - c));
     wn.push_back((int)k);
-    spec0.push_back(base);
   }
-  // the push lists, jobs with the most workgroups per tile first: a tile's workgroups then
-  // start at a multiple of their number, from which each finds its part
-  for (int sp = kMaxSplit; sp >= 1; sp /= 2)
-    for (size_t k = 0; k < b->jobs.size(); k++) {
-      const osr_sim* s = b->jobs[k]->sim;
-      if (s->split != sp) continue;
-      for (size_t i = 0; i < s->sp.size(); i++)
-        for (int t = 0; t < s->ntiles; t++)
-          wp[s->sp[i]->pusher == OSR_VAY ? 1 : 0].insert(
-              wp[s->sp[i]->pusher == OSR_VAY ? 1 : 0].end(), sp, make_int2(spec0[k] + (int)i, t));
-    }
   // the launch with the history columns: these, then yee2d_step's tiles (2D) or the E step's
   // cell blocks
   const std::vector<int2>& cells = b->dims == 2 ? we : wy;

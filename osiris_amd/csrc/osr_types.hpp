@@ -29,10 +29,9 @@ constexpr int kMaxSpecies = 8;
 // tiles in LDS are then shared by twice as many waves, so two workgroups (16 waves) fit in
 // a CU's LDS where three 4-wave ones (12 waves) did.
 constexpr int kMaxPushWaves = 8;
-// Workgroups per tile in the 2D push (its split), and the waves of a tile over all of them:
-// a grid of few tiles would leave CUs idle with one workgroup per tile.  Each wave of a tile
-// owns a contiguous slice of its particles and a mover region, whichever workgroup it is in.
-constexpr int kMaxSplit = 4;
+// Waves of a tile over all its workgroups in the 2D push, of which there are up to four (its
+// split): a grid of few tiles would leave CUs idle with one workgroup per tile.  Each wave of a
+// tile owns a contiguous slice of its particles and a mover region, whichever workgroup it is in.
 constexpr int kMaxTileWaves = 16;
 // waves per workgroup of the compile-time 3D push
 __host__ __device__ constexpr int push3d_waves(int order) { return order == 3 ? 4 : 8; }

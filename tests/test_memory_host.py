@@ -1,5 +1,5 @@
-"""The library's use of device memory on the CPU, over the mock runtime of tests/hostcheck with
-a device memory that fills up (capi_mock_mem.hip)."""
+"""The library's use of device memory and the size of its push launches on the CPU, over the mock
+runtime of tests/hostcheck with a device memory that fills up (capi_mock_mem.hip)."""
 import json
 import os
 import subprocess
@@ -89,3 +89,45 @@ with Simulation(dims, nx, (0.1,) * dims, 0.05, 2) as s:
     raw.mock_leave_free(-1)
 """)
     assert res == {"particles": True, "fields": True}
+
+
+@pytest.mark.parametrize("nx,tile,nsp,ppc,split", [
+    ((128, 128), (16, 16), 1, (4, 4), 4), ((256, 128), (16, 16), 1, (1, 1), 1), ((128, 128), (16, 16), 1, (2, 2), 4),
+    ((256, 128), (16, 16), 8, (2, 2), 1), ((128, 128), (16, 16), 8, (4, 4), 1), ((256, 128), (16, 16), 1, (2, 2), 2),
+    ((256, 192), (16, 16), 2, (4, 4), 2), ((256, 192), (16, 16), 1, (2, 2), 1), ((512, 256), (16, 16), 1, (4, 4), 1),
+    ((256, 256), (32, 16), 1, (4, 4), 2), ((512, 256), (32, 16), 1, (4, 4), 1), ((640, 512), (32, 16), 2, (2, 2), 1)])
+def test_push_workgroups_per_tile(mem_lib, nx, tile, nsp, ppc, split):
+    """A push launch has several workgroups per tile where the tiles of all its species leave the
+    chip idle and each wave still has iterations to share, and one elsewhere.  The points are
+    measured ones: in each the number expected here was the fastest."""
+    res = _run(mem_lib, f"""
+with Simulation(2, {nx}, (0.1, 0.1), 0.05, 2, tile={tile}) as s:
+    for k in range({nsp}):
+        s.generate(s.add_species(-1.0), {ppc})
+    s.run(1)
+    out["wgs"] = raw.mock_push_workgroups()
+""")
+    tiles = -(-nx[0] // tile[0]) * -(-nx[1] // tile[1])
+    assert res["wgs"] == tiles * nsp * split
+
+
+def test_split_follows_the_particles(mem_lib):
+    """The number of workgroups is chosen again when species or their particles change, also
+    between runs; every tile table holds the largest number."""
+    res = _run(mem_lib, """
+out["wgs"] = []
+with Simulation(2, (256, 128), (0.1, 0.1), 0.05, 2) as s:
+    s.generate(s.add_species(-1.0), (1, 1))
+    s.run(2)
+    out["wgs"].append(raw.mock_push_workgroups())
+    s.generate(0, (4, 4))
+    s.time_kernels(1)
+    out["wgs"].append(raw.mock_push_workgroups())
+    s.run(3)
+    for k in range(7):
+        s.generate(s.add_species(1.0), (4, 4))
+    s.run(3)
+    out["wgs"].append(raw.mock_push_workgroups())
+    s.get_particles(3)
+""")
+    assert res == {"wgs": [128, 512, 8 * 128]}
