@@ -34,7 +34,7 @@ struct EnsJob {
 };
 
 struct EnsBatch {
-  int dims = 2, order = 2, tile[3] = {1, 1, 1}, kernel = 0, waves = 4, yv = 0;
+  int dims = 2, order = 2, tile[3] = {1, 1, 1}, kernel = 0, waves = 4, yv = 0, pp = 0;
   hipStream_t stream = nullptr;
   hipEvent_t ev = nullptr;
   std::vector<EnsJob*> jobs;     // jobs stepped by the graph
@@ -82,7 +82,7 @@ int64_t job_footprint(const osr_job_desc& j) {
   }
   const int64_t ntiles = (int64_t)nt[0] * nt[1] * nt[2];
   const int64_t nblk = (nc + 255) / 256;
-  int64_t b = nc * (12 + 12 + 24) * (D == 2 ? 2 : 1) + nblk * (2 * 48 + 8);
+  int64_t b = nc * (12 + 12 + 24) * (D == 2 && nc <= (int64_t)kTwoCopyCells ? 2 : 1) + nblk * (2 * 48 + 8);
   const int64_t rows = std::max<int64_t>(j.nsteps, 1024);
   b += rows * (6 + j.nspecies) * 8;
   const int64_t slot = D == 2 ? 68 : 76;
@@ -189,7 +189,7 @@ int ens_admit(osr_ensemble* e, EnsJob* j) {
   for (auto& bb : e->batches)
     if (bb->dims == s->dims && bb->order == s->order && bb->tile[0] == s->g.tx &&
         bb->tile[1] == s->g.ty && bb->tile[2] == s->g.tz && bb->kernel == jd.sim.kernel &&
-        bb->waves == s->push_waves && bb->yv == s->yv) {
+        bb->waves == s->push_waves && bb->yv == s->yv && bb->pp == s->g.pp) {
       b = bb.get();
       break;
     }
@@ -203,6 +203,7 @@ int ens_admit(osr_ensemble* e, EnsJob* j) {
     nb->kernel = jd.sim.kernel;
     nb->waves = s->push_waves;
     nb->yv = s->yv;
+    nb->pp = s->g.pp;
     nb->lds = s->lds_push;
     HIPC(hipStreamCreateWithFlags(&nb->stream, hipStreamNonBlocking));
     HIPC(hipEventCreateWithFlags(&nb->ev, hipEventDisableTiming));
@@ -240,9 +241,9 @@ int ens_build(osr_ensemble* e, EnsBatch* b) {
     for (int c = 0; c < 6 + (int)s->sp.size(); c++) wd.push_back(make_int2((int)k, -1 - c));
     wn.push_back((int)k);
   }
-  // the launch with the history columns: these, then yee2d_step's tiles (2D) or the E step's
-  // cell blocks
-  const std::vector<int2>& cells = b->dims == 2 ? we : wy;
+  // the launch with the history columns: these, then yee2d_step's tiles or the E step's cell
+  // blocks
+  const std::vector<int2>& cells = b->pp ? we : wy;
   wd.insert(wd.end(), cells.begin(), cells.end());
   auto put = [&](DBuf& d, const void* src, size_t bytes) -> int {
     if (bytes == 0) return OSR_OK;
@@ -304,9 +305,13 @@ int ens_build(osr_ensemble* e, EnsBatch* b) {
     const int2* w = b->wyee.as<int2>();
     const int2* we = b->wene.as<int2>();
     const int2* wd = b->wded.as<int2>();
-    if (b->dims == 2) {
+    if (b->pp) {
       hipLaunchKernelGGL(pick_yee2d(b->yv), dim3(b->nded), dim3(256),
                          0, b->stream, fd, wd, 0);
+    } else if (b->dims == 2) {
+      hipLaunchKernelGGL((yee_dbdt<2, true>), dim3(b->nene), dim3(256), 0, b->stream, fd, we);
+      hipLaunchKernelGGL((yee_dedt<2>), dim3(b->nded), dim3(256), 0, b->stream, fd, wd);
+      hipLaunchKernelGGL((yee_dbdt<2, false>), dim3(b->nyee), dim3(256), 0, b->stream, fd, w);
     } else {
       hipLaunchKernelGGL((yee_dbdt<3, true>), dim3(b->nene), dim3(256), 0, b->stream, fd, we);
       hipLaunchKernelGGL((yee_dedt<3>), dim3(b->nded), dim3(256), 0, b->stream, fd, wd);

@@ -131,3 +131,28 @@ with Simulation(2, (256, 128), (0.1, 0.1), 0.05, 2) as s:
     s.get_particles(3)
 """)
     assert res == {"wgs": [128, 512, 8 * 128]}
+
+
+def test_one_copy_of_the_fields_where_two_do_not_fit(mem_lib):
+    """A 2D grid whose fields and current fit the card once, but not twice, is simulated on one
+    copy, and read back; with room for both it takes both."""
+    res = _run(mem_lib, """
+nx = (400, 350)
+one = 48 * nx[0] * nx[1]
+for name, free in (("one", one + one // 2), ("two", 3 * one)):
+    raw.mock_leave_free(free)
+    with Simulation(2, nx, (0.1, 0.1), 0.05, 2) as s:
+        out[name] = s.footprint // one
+        raw.mock_leave_free(-1)
+        s.generate(s.add_species(-1.0), (1, 1))
+        e = np.arange(3 * nx[0] * nx[1], dtype=np.float32).reshape(nx[1], nx[0], 3)
+        s.set_fields(e, -e)
+        raw.mock_leave_free(0)
+        f = s.get_fields()
+        raw.mock_leave_free(-1)
+        out[name + " fields"] = bool(np.array_equal(f[0], e) and np.array_equal(f[1], -e))
+        s.run(9)
+        s.time_kernels(2)
+        out[name + " steps"] = s.steps
+""")
+    assert res == {"one": 1, "one fields": True, "one steps": 11, "two": 2, "two fields": True, "two steps": 11}
