@@ -166,8 +166,9 @@ typedef struct {
   int push_waves; /* fused path: waves per push workgroup, 0 = default (8 for 2D
                      compile-time tiles of 512 cells or more and for the 3D compile-time
                      tile with order 1 or 2, else 4); 4 or 8 for the 2D compile-time tiles
-                     16x16 and 32x16; in 3D 4 is accepted and means the default.  Changes no
-                     result */
+                     16x16 and 32x16; elsewhere the default's number, which
+                     osr_sim_launch_config reports; in 3D 4 also means the default.  Changes
+                     no result */
 } osr_sim_desc;
 
 /* x boundaries of a resident simulation.  Both open types have absorbing particles

@@ -18,7 +18,8 @@ import json
 import os
 
 # (tile, waves per workgroup, kernel): kernel 0 = compile-time tile variant where one is
-# instantiated, 1 = generic kernel (runtime tile shape, any tile that fits the LDS)
+# instantiated, 1 = generic kernel (runtime tile shape, any tile that fits the LDS); waves 0 =
+# the number of the kernel that runs (in 3D it follows from the order)
 DEFAULT_2D = (
     {"tile": (16, 16), "push_waves": 4, "kernel": 0},
     {"tile": (16, 16), "push_waves": 8, "kernel": 0},
@@ -27,7 +28,7 @@ DEFAULT_2D = (
     {"tile": (8, 8), "push_waves": 4, "kernel": 0},
 )
 DEFAULT_3D = (
-    {"tile": (8, 8, 4), "push_waves": 4, "kernel": 0},
+    {"tile": (8, 8, 4), "push_waves": 0, "kernel": 0},
     {"tile": (8, 8, 4), "push_waves": 4, "kernel": 1},
     {"tile": (4, 4, 4), "push_waves": 4, "kernel": 1},
     {"tile": (8, 4, 4), "push_waves": 4, "kernel": 1},

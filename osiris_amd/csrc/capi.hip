@@ -1524,13 +1524,14 @@ int osr_sim_create(const osr_sim_desc* desc, osr_sim** out) {
     const int w = desc->push_waves > 0 ? desc->push_waves : push2d_default_waves(g.tx, g.ty);
     if (pick_push2d_t(s->order, 0, g.tx, g.ty, w)) s->push_waves = w;
   }
-  // 3D takes 4 (what every 3D kernel had before) for its own number, and no other request
-  if (desc->push_waves > 0 && desc->push_waves != (dims == 3 ? kWaves : s->push_waves))
-    return fail(OSR_ERR_ARG, "no push kernel with %d waves per workgroup for this tile and kernel",
-                desc->push_waves);
   if (!s->plain && dims == 3 && desc->kernel != 1 &&
       pick_push3d_t(s->order, 0, g.tx, g.ty, g.tz))
     s->push_waves = push3d_waves(s->order);
+  // 3D also takes 4, which every 3D kernel once had, for its own number
+  if (desc->push_waves > 0 && desc->push_waves != s->push_waves &&
+      !(dims == 3 && desc->push_waves == kWaves))
+    return fail(OSR_ERR_ARG, "no push kernel with %d waves per workgroup for this tile and kernel",
+                desc->push_waves);
   if (!s->plain && dims == 2 && desc->kernel != 1 &&
       pick_push2d_t(s->order, 0, g.tx, g.ty, s->push_waves))
     s->split_max = max_split(g.ntiles, s->push_waves);

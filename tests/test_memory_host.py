@@ -156,3 +156,31 @@ for name, free in (("one", one + one // 2), ("two", 3 * one)):
         out[name + " steps"] = s.steps
 """)
     assert res == {"one": 1, "one fields": True, "one steps": 11, "two": 2, "two fields": True, "two steps": 11}
+
+
+@pytest.mark.parametrize("dims,order,tile,kernel", [
+    (2, 2, (16, 16), 0), (2, 1, (32, 16), 0), (2, 3, (8, 8), 0), (2, 2, (16, 16), 1), (2, 2, (10, 10), 0),
+    (3, 1, (8, 8, 4), 0), (3, 2, (8, 8, 4), 0), (3, 3, (8, 8, 4), 0), (3, 2, (8, 8, 4), 1), (3, 1, (4, 4, 4), 0)])
+def test_reported_launch_configuration_is_accepted(mem_lib, dims, order, tile, kernel):
+    """The waves that launch_config reports can be asked for and give the same configuration; in
+    3D so can 4; another number than 4 and 8 or than the kernel's is refused."""
+    res = _run(mem_lib, f"""
+kw = dict(tile={tile}, kernel={kernel})
+mk = lambda w: Simulation({dims}, (32,) * {dims}, (0.1,) * {dims}, 0.05, {order}, push_waves=w, **kw)
+with mk(0) as s:
+    cfg = s.launch_config
+with mk(cfg["push_waves"]) as s:
+    out["same"] = s.launch_config == cfg
+for w in (2, 4, 8):
+    try:
+        with mk(w) as s:
+            out[str(w)] = s.push_waves
+    except L.OsrError:
+        out[str(w)] = 0
+out["own"] = cfg["push_waves"]
+""")
+    own = res["own"]
+    assert res["same"] and res["2"] == 0
+    either = dims == 2 and kernel == 0 and tile in ((16, 16), (32, 16))
+    assert res["4"] == (4 if own == 4 or either else own if dims == 3 else 0)
+    assert res["8"] == (8 if own == 8 or either else 0)
