@@ -872,8 +872,8 @@ int collect(osr_sim* s, Species& p, bool pending, HostParts& hp) {
   return OSR_OK;
 }
 
-// Fill kernel and its launch shape (4 waves per tile; LDS lists for up to 4096 incoming
-// particles and 32768 holes left in a tile's tail).
+// Fill kernel and its launch shape (4 waves per tile; an LDS list for up to 4096 incoming
+// particles).
 typedef void (*fill_fn)(const SpecDesc*, const int2*);
 struct FillKernel {
   fill_fn f;
@@ -885,8 +885,8 @@ FillKernel pick_fill() { return {tile_fill<256, 4096, 32768>, 256}; }
 // tile gets its count after the step plus half of it again as capacity (no tile
 // shrinks), every tile's particles and pending mover lists move to the
 // new arrays on the device (regrow_move), and the fill of the overflowed tiles runs again
-// there.  *ok = false when that cannot finish the step (a tile's incoming or tail lists
-// exceed the fill kernel's LDS tables, or slots would exceed int32): the species is then
+// there.  *ok = false when that cannot finish the step (a tile's incoming list exceeds
+// the fill kernel's, or slots would exceed int32): the species is then
 // left in the halted state, possibly in the larger layout, for the host re-layout.
 int regrow_species(osr_sim* s, int sid, bool* ok) {
   Species& p = *s->sp[sid];

@@ -575,11 +575,12 @@ OSR_DEV void copy_particle(const SpecDesc& d, int src, int dst, int dims) {
 // sources = incoming movers by (neighbour, wave, slot), then the non-hole particles of
 // the tail [newcnt, cnt) ascending; targets = holes below newcnt ascending, then the
 // appended slots [cnt, newcnt)).  A tile that cannot take its incoming particles (its
-// capacity, or the LDS lists of this kernel, would overflow) changes nothing, marks
+// capacity, or this kernel's LDS list of them, would overflow) changes nothing, marks
 // itself with inc = -1 and raises Ctrl::halt; the host then re-lays the species out from
 // the tiles that did fill plus the mover buffers.
-// NT threads per tile; INC_MAX incoming movers and TAIL_BITS holes left in the tail are the
-// most one fill handles; beyond them the tile flags an overflow.
+// NT threads per tile; INC_MAX incoming movers are the most one fill handles; beyond them the
+// tile flags an overflow.  Any number may leave.  (The third parameter, once a limit on that, is
+// part of the name under which the host checks know the kernel.)
 //
 // Bound: the chain of dependent loads and barriers of a tile (a tile moves few particles),
 // so the loads that depend on the same thing go out together: every list's length and base
@@ -604,7 +605,7 @@ OSR_DEV void seg_find_multi(const int* ofs, const int (&v)[PF], int (&l)[PF]) {
       if (ofs[l[p] + h] <= v[p]) l[p] += h;
 }
 
-template <int NT, int INC_MAX, int TAIL_BITS>
+template <int NT, int INC_MAX, int>
 __global__ __launch_bounds__(NT) void tile_fill(const SpecDesc* __restrict__ descs,
                                                 const int2* __restrict__ work) {
   constexpr int MAXL = 26 * kMaxTileWaves;  // candidate lists: neighbours x waves
@@ -746,12 +747,12 @@ __global__ __launch_bounds__(NT) void tile_fill(const SpecDesc* __restrict__ des
   // every wave's entries of s_inc and s_hole are in LDS before any wave reads them below
   __syncthreads();
   const int nn = n - H + I;
-  if (I > INC_MAX || nn > cap - 64 * NW || H - I > TAIL_BITS) {
+  if (I > INC_MAX || nn > cap - 64 * NW) {
     if (tid == 0) {
       d.inc[tile] = -1;
       // the count the tile needs after this step, or -1 if more capacity would not help
-      // (the incoming or tail lists exceed this kernel's limits)
-      d.newcnt[tile] = (I > INC_MAX || H - I > TAIL_BITS) ? -1 : nn;
+      // (the incoming list exceeds this kernel's limit)
+      d.newcnt[tile] = I > INC_MAX ? -1 : nn;
       atomicOr(&g.ctrl->halt, 1);
     }
     return;
