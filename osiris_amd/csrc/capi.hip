@@ -460,7 +460,7 @@ void make_field_desc(const osr_sim* s, FieldDesc& f) {
     f.sm_src = s->plain ? 1 : 0;
     f.sm_buf[0] = s->sm_buf[0].as<float>();
     f.sm_buf[1] = s->sm_buf[1].as<float>();
-    f.Jf = f.sm_buf[(f.sm_np - 1) & 1];
+    f.Jf = f.sm_buf[s->dims == 3 ? (f.sm_np - 1) & 1 : 0];
     f.jf_zero = 0;
     f.jsrc_clear = s->plain ? 2 : 1;
   }
@@ -1211,7 +1211,7 @@ int refresh_energy(osr_sim* s) {
   if (!s->g.pp || !s->fe_stale) return OSR_OK;
   hipLaunchKernelGGL(pick_yee2d_energy(s->yv), dim3((unsigned)s->nblk_e),
                      dim3(256), 0, s->stream, s->d_fd.as<FieldDesc>(),
-                     s->d_dwork.as<int2>() + kRedCols, 0);
+                     s->d_dwork.as<int2>(), kRedCols);
   HIPC(hipGetLastError());
   s->fe_stale = false;
   return OSR_OK;
@@ -1997,8 +1997,7 @@ int osr_sim_run(osr_sim* s, int nsteps) {
     Ctrl c;
     TRY(read_ctrl(s, c));
     s->par = c.par;
-    if (c.error & 1) return fail(OSR_ERR_LAYOUT, "particle found outside its tile");
-    if (c.error) return fail(OSR_ERR_STATE, "mover lists exceed the tile fill tables");
+    if (c.error) return fail(OSR_ERR_LAYOUT, "particle found outside its tile");
     const int64_t done = c.steps - s->steps;
     s->steps = c.steps;
     left -= done;
@@ -2285,8 +2284,7 @@ int osr_sim_time_kernels(osr_sim* s, int nsteps, double* ms) {
     Ctrl c;
     TRY(read_ctrl(s, c));
     s->par = c.par;
-    if (c.error & 1) return fail(OSR_ERR_LAYOUT, "particle found outside its tile");
-    if (c.error) return fail(OSR_ERR_STATE, "mover lists exceed the tile fill tables");
+    if (c.error) return fail(OSR_ERR_LAYOUT, "particle found outside its tile");
     s->steps = c.steps;
     if (c.halt == 2) {
       TRY(relayout(s, true));
@@ -2980,10 +2978,8 @@ int osr_sim_set_smooth(osr_sim* s, const int* order, const float* coef) {
     for (int j = 0; j < 31; j++) s->sm_coef[d][j] = d < s->dims ? coef[d * OSR_SMOOTH_NCOEF + j] : 0.f;
   }
   const size_t bytes = 12 * (size_t)s->g.ncell;
-  if (any && !s->sm_buf[0].p) {
-    TRY(s->sm_buf[0].alloc(bytes));
-    TRY(s->sm_buf[1].alloc(bytes));
-  }
+  for (int k = 0; k < (s->dims == 3 ? 2 : 1); k++)  // 2D writes its result at once
+    if (any && !s->sm_buf[k].p) TRY(s->sm_buf[k].alloc(bytes));
   TRY(upload_descs(s));
   s->graph_ok = false;
   return OSR_OK;

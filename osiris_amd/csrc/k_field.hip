@@ -38,8 +38,8 @@ struct FieldDesc {
   float* Jf;
   int jf_zero;  // clear Jf after reading it (the plain path accumulates into it)
   // current smoothing: passes (one per filtered direction, x before y before z) from the
-  // source current into the ping-pong buffers; the last output is Jf, and the E step then
-  // clears the source (1: fixed-point J, 2: the plain path's float J)
+  // source current into the ping-pong buffers, in 2D all into the first; the last output is Jf,
+  // and the E step then clears the source (1: fixed-point J, 2: the plain path's float J)
   int sm_np;
   int sm_dir[3];
   int sm_n[3];
@@ -563,12 +563,12 @@ OSR_DEV void yee2d_tile(const FieldDesc& fd, int item, float* lds) {
   tile_energy(acc, fd.fe_part + (long long)(par ^ 1u) * 6 * fd.nblk, fd.nblk, item);
 }
 
-// work items (simulation, tile) or (simulation, -1 - history column)
+// work items from `first` on: (simulation, tile) or (simulation, -1 - history column)
 template <int TX, int TY>
 __global__ __launch_bounds__(256) void yee2d_step(const FieldDesc* __restrict__ fds,
-                                                  const int2* __restrict__ work, int) {
+                                                  const int2* __restrict__ work, int first) {
   __shared__ float lds[kYeeLds<TX, TY>];
-  const int2 wk = work[blockIdx.x];
+  const int2 wk = work[first + blockIdx.x];
   if (wk.y < 0)
     reduce_column(fds[wk.x], -1 - wk.y);
   else
@@ -599,9 +599,9 @@ OSR_DEV void field_beside_fill(const FieldDesc& fd, int kind, int item, float* l
 // same sums): run when the host changed the fields, before the next step.
 template <int TX, int TY>
 __global__ __launch_bounds__(256) void yee2d_energy(const FieldDesc* __restrict__ fds,
-                                                    const int2* __restrict__ work, int) {
+                                                    const int2* __restrict__ work, int first) {
   using T = YeeTile<TX, TY>;
-  const int2 wk = work[blockIdx.x];
+  const int2 wk = work[first + blockIdx.x];
   const FieldDesc& fd = fds[wk.x];
   const GridDesc& g = fd.g;
   const int nx = g.nx, ny = g.ny;

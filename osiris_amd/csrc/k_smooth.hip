@@ -8,11 +8,11 @@
 //
 // Three forms:
 //  * smooth2d: every direction of a 2D simulation in one launch;
-//  * smooth_pass: the resident simulation, planar interior arrays with periodic index
-//    wraps (equal to the reference on the interior, whose guard cells hold the periodic
+//  * smooth_pass: one direction of a 3D simulation, planar interior arrays with periodic
+//    index wraps (equal to the reference on the interior, whose guard cells hold the periodic
 //    images after the current's boundary update, os-simulation.f03:650-657); the first
-//    pass reads the folded current (fixed-point or the plain path's float) and converts it
-//    as the E step would, later passes read the previous output;
+//    pass reads the folded fixed-point current and converts it as the E step would, later
+//    passes read the previous output;
 //  * smooth_vdf_pass: the stateless drop-in, a component-interleaved array with guard
 //    cells, filtered exactly like smooth_vdf: cells closer than n to either end of a line
 //    keep their values.
@@ -58,9 +58,7 @@ __global__ __launch_bounds__(256) void smooth_pass(const FieldDesc* __restrict__
     st = (long long)nx * ny;
   }
   const long long row = idx - (long long)c * st;  // the line's first cell
-  const int src = pass == 0 ? fd.sm_src : 2;
-  const unsigned long long* Jq = g.J + cur_copy(g);
-  const float* Jp = (const float*)g.J;
+  const unsigned long long* Jq = g.J;
   const float* P = fd.sm_buf[(pass + 1) & 1];  // previous pass's output
   float* dst = fd.sm_buf[pass & 1];
   const double jinv = g.jinv;
@@ -69,9 +67,7 @@ __global__ __launch_bounds__(256) void smooth_pass(const FieldDesc* __restrict__
     const long long off = comp * nc + row;
     auto val = [&](int k) -> float {
       const long long id = off + (long long)wrapn(c + k, len) * st;
-      if (src == 0) return (float)((double)(long long)Jq[id] * jinv);
-      if (src == 1) return Jp[id];
-      return P[id];
+      return pass == 0 ? (float)((double)(long long)Jq[id] * jinv) : P[id];
     };
     float acc = val(-n) * s[-n];
     for (int k = -n + 1; k <= n; k++) acc = acc + val(k) * s[k];

@@ -184,3 +184,29 @@ out["own"] = cfg["push_waves"]
     either = dims == 2 and kernel == 0 and tile in ((16, 16), (32, 16))
     assert res["4"] == (4 if own == 4 or either else own if dims == 3 else 0)
     assert res["8"] == (8 if own == 8 or either else 0)
+
+
+@pytest.mark.parametrize("dims,nx,buffers", [(2, (300, 250), 1), (3, (40, 36, 30), 2)])
+def test_smoothing_buffers(mem_lib, dims, nx, buffers):
+    """Smoothing in 2D takes one float copy of the current, in 3D two; a call that finds no room
+    for them leaves the next one to try again."""
+    res = _run(mem_lib, f"""
+from osiris_amd.sim import smooth_setup
+dims, nx = {dims}, {nx}
+one = 12 * int(np.prod(nx))
+filt = smooth_setup(dims, ["binomial"] * dims, (1,) * dims, (0.1,) * dims)
+with Simulation(dims, nx, (0.1,) * dims, 0.05, 2) as s:
+    s.generate(s.add_species(-1.0), (1,) * dims)
+    out["fails"] = 0
+    for room in (0, one + one // 2):
+        raw.mock_leave_free(room)
+        try:
+            s.set_smooth(*filt)
+        except L.OsrError:
+            out["fails"] += 1
+    raw.mock_leave_free(-1)
+    s.set_smooth(*filt)
+    s.run(5)
+    out["steps"] = s.steps
+""")
+    assert res == {"fails": buffers, "steps": 5}
