@@ -240,11 +240,14 @@ int osr_sim_gauss(osr_sim *sim, double *res, double *rho, double *maxabs);
 int osr_sim_relayouts(osr_sim *sim, int64_t *count);
 
 /* Per-kernel timing of nsteps steps, measured with HIP events on the simulation's
- * stream (the steps are really advanced).  ms[k] = mean duration per step of kernel
- * class k: 0 push+deposit (all species), 1 tile fill and re-order, 2 field advance
- * (smoothing, Yee sub-steps, wall updates), 3 step end (energy reduction; with Lindman
- * walls it runs in the last wall kernel and this is 0); ms[4] = mean time per step from
- * the first to the last event; ms[5] = 0. */
+ * stream (the steps are really advanced).  Every kernel class has launches of its own here,
+ * with an event between them: osr_sim_run puts the first part of the field advance, and the
+ * history sums with it, on the tile fill's launch, a laser wall's values on the last field
+ * launch of the step before, and leaves no gaps, so that its steps take less than ms[4].
+ * ms[k] = mean duration per step of kernel class k: 0 push+deposit (all species),
+ * 1 tile fill and re-order, 2 field advance (smoothing, Yee sub-steps, wall updates),
+ * 3 step end (energy reduction; with Lindman walls it runs in the last wall kernel and this
+ * is 0); ms[4] = mean time per step from the first to the last event; ms[5] = 0. */
 int osr_sim_time_kernels(osr_sim *sim, int nsteps, double *ms);
 /* Bytes of device memory held by a simulation. */
 int osr_sim_footprint(osr_sim *sim, int64_t *bytes);

@@ -1362,6 +1362,7 @@ int build_graph(osr_sim* s) {
 
 // The push's work list names every item once per workgroup of the tile.
 int upload_push_list(osr_sim* s) {
+  s->graph_ok = false;  // captured launches hold the list's address and length
   std::vector<int2> pw;
   for (int i = 0; i < (int)s->sp.size(); i++)
     for (int t = 0; t < s->ntiles; t++)
@@ -1514,7 +1515,10 @@ int osr_sim_create(const osr_sim_desc* desc, osr_sim** out) {
   // / 418, 0.02 434 / 416 / 413 / 424 / 457, 0.1 501 / 492 / 492 / 496 / 496; 160^3, 0.3 2681 /
   // 2621 / 2597 / 2585 / 2565.  The linear push is not bound by the order: 160^3, 0.01 1195 /
   // 1074 / 1005 / 976 / 946, 52x44x36 70.6 / 66.7 / 64.8 / 64.1 / 61.6 (a launch that finds
-  // nothing to do costs 2.5 us).
+  // nothing to do costs 2.5 us).  It stays so in long runs: 96^3, steps 1200 to 1264 (linear: 3000
+  // to 3064), linear u_th 0.002 / 0.01 / 0.05, none 217 / 228 / 259, 64 218 / 232 / 265, 16 228 /
+  // 240 / 275, 4 271 / 283 / 317; quadratic 0.005 / 0.02 / 0.1, none 445 / 457 / 499, 64 386 / 439
+  // / 502, 16 370 / 413 / 495, 4 403 / 431 / 504.
   const int period = dims == 3 ? (s->order == 3 ? 4 : (s->order == 2 ? 16 : 0)) : 0;
   s->reorder = desc->reorder > 0 ? desc->reorder : (desc->reorder == 0 ? period : 0);
   s->push_waves = kWaves;
@@ -2291,10 +2295,7 @@ int osr_sim_time_kernels(osr_sim* s, int nsteps, double* ms) {
       Ctrl z = c;
       z.halt = 0;
       TRY(copy_on(s->stream, s->ctrl.p, &z, sizeof(Ctrl), hipMemcpyHostToDevice));
-      if (!s->pwork_ok) {
-        TRY(upload_push_list(s));
-        s->graph_ok = false;
-      }
+      if (!s->pwork_ok) TRY(upload_push_list(s));
       continue;  // a re-laid-out step is not representative
     }
     float t;

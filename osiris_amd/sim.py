@@ -341,8 +341,7 @@ class Simulation:
     def time_kernels(self, nsteps):
         ms = np.zeros(6)
         check(lib().osr_sim_time_kernels(self._h, int(nsteps), _p(ms)))
-        # tile_fill runs beside yee (the field advance with its walls); finalize is the
-        # step end after both
+        # each kernel in a launch of its own, unlike a run's; finalize is the step end
         return {"push_deposit": ms[0], "tile_fill": ms[1], "yee": ms[2], "finalize": ms[3],
                 "step": ms[4]}
 
