@@ -31,9 +31,10 @@ HBM_PEAK_GBS = 8000.0
 # ix2+x2+u3 = 28 B; per cell the gather reads E,B (24 B) and the deposit writes J (12 B).
 BYTES_PER_PARTICLE = 60.0
 BYTES_PER_CELL_PUSH = 36.0
-# Yee per cell: B half step 36 B (read E, B; write B), E step 48 B (read E, B; write E;
-# J counted with the deposit), B half step 36 B
-BYTES_PER_CELL_YEE = 120.0
+# Field step of a periodic 2D grid per cell, one launch: read E, B (24 B) and the three
+# fixed-point sums of J (24 B), write E, B to their other copy (24 B) and clear the next
+# step's sums (24 B)
+BYTES_PER_CELL_YEE = 96.0
 
 
 def log(*a):

@@ -18,10 +18,10 @@
 // What bounds it: LDS (bank conflicts of the 64-bit adds, whose lanes point at random nodes
 // once the particles have moved: 12.7 cycles of a CU per add against 7.4 without conflicts)
 // and VALU issue, together.  Two-stream 1024x1024, 64 per cell, quadratic, per 64 particles:
-// 557 -> 460 VALU instructions (raw fixed-point bits, 21; split and further VPs on full waves
-// only, about 70), 36 -> 18 LDS reads; 1.270 -> 1.147 ms per step (3.1 TB/s of the 52 B a
-// particle moves), VALU 71% and LDS about 80% of the cycles.  512x512, 16 per cell, cubic, Vay
-// 170 -> 153 us, 515x267 quadratic 58 -> 54.5, 300x200 37 -> 31.6.
+// 557 -> 443 VALU instructions (raw fixed-point bits, split and further VPs on full waves
+// only), 36 -> 18 LDS reads; 1.270 -> 1.110 ms per step (3.63 TB/s of the 60 B a particle
+// moves), VALU issue 83% of the cycles, bank conflicts 32%.  512x512, 16 per cell, cubic, Vay
+// 170 -> 148 us, 515x267 quadratic 58 -> 54.5, 300x200 37 -> 31.6.
 // The arithmetic of gather, push, position advance and split is the one of the generic
 // kernel (the reference's AVX2 kernel, simd/os-spec-push-avx2.c:471-760).
 #include <type_traits>
@@ -54,8 +54,8 @@ OSR_DEV int wrap1(int i, int n) { return i < 0 ? i + n : (i >= n ? i - n : i); }
 // in the order a few steps leave them do not give).  So a 16-byte element per node holds what
 // the node's x line needs next: the two components that share a stencil at the node and its
 // right neighbour ((E1, B2) at half x, full y; (E2, B1) at full x, half y), and for E3 (full,
-// full) and B3 (half, half) the node and the next three, or, with linear and cubic splines,
-// the node and the next one (which keeps 4 workgroups in a CU).
+// full) and B3 (half, half) the node and the next three, or, with linear splines, whose line
+// is two nodes, the node and the next one.
 template <int ORDER>
 struct Line2 {
   static constexpr int W = ORDER >= 2 ? 4 : 2;  // E3, B3 values per node
